@@ -64,27 +64,6 @@ struct DCut {
     int32_t nLeaves, used;
 };
 
-// Leaf signature of the reference (rewrite.cu:68, 262: bit leaf & 31).  In a
-// batched pass sigBits holds each node's bit as it would be in its own AIG
-// (its id there & 31), so that the prefilter of rewrite.cu:283 sees the same
-// signatures as when that AIG is rewritten alone.
-// Without branches per leaf: the sigBits test is uniform, and in the batched
-// case the four byte loads are issued at once (absent leaves read entry 0).
-__device__ __forceinline__ uint32_t cut_sign_of(const DCut &c, const uint8_t *__restrict__ sigBits) {
-    uint32_t b[4];
-    if (sigBits) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) b[i] = sigBits[i < c.nLeaves ? c.leaves[i] : 0u];
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; i++) b[i] = c.leaves[i] & 31;
-    }
-    uint32_t s = 0;
-#pragma unroll
-    for (int i = 0; i < 4; i++) s |= i < c.nLeaves ? 1u << b[i] : 0u;
-    return s;
-}
-
 // the reference counts of a cut's leaves, all four loads in flight at once;
 // absent leaves read node 0's entry
 __device__ __forceinline__ void leaf_refs(const DCut &c, const int32_t *nRef, int (&r)[4]) {
@@ -92,22 +71,7 @@ __device__ __forceinline__ void leaf_refs(const DCut &c, const int32_t *nRef, in
     for (int i = 0; i < 4; i++) r[i] = nRef[i < c.nLeaves ? c.leaves[i] : 0u];
 }
 
-// CutFindValue (rewrite.cu:49-61) of a cut of nLeaves leaves whose reference
-// counts are r[0..nLeaves-1]
-__device__ __forceinline__ uint32_t cut_value_of(int nLeaves, const int (&r)[4]) {
-    int value = 0, nOnes = 0;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        if (i < nLeaves) {
-            value += r[i];
-            nOnes += (r[i] == 1);
-        }
-    if (nLeaves < 2) return 1001;
-    if (value > 1000) value = 1000;
-    if (nOnes > 3) value = 5 - nOnes;
-    return (uint32_t)value;
-}
-
+// CutFindValue (rewrite.cu:49-61)
 __device__ __forceinline__ uint32_t cut_value(const DCut &c, const int32_t *nRef) {
     int r[4];
     leaf_refs(c, nRef, r);
@@ -124,119 +88,12 @@ __device__ __forceinline__ uint32_t cut_value(const DCut &c, const int32_t *nRef
     return (uint32_t)value;
 }
 
-__device__ __forceinline__ void unpack_cut(const uint32_t *p, DCut &c) {
-    c.leaves[0] = p[0]; c.leaves[1] = p[1]; c.leaves[2] = p[2]; c.leaves[3] = p[3];
-    uint32_t m = p[4];
-    c.tt = m & 0xFFFF;
-    c.value = (m >> 16) & 0x7FF;
-    c.nLeaves = (m >> 27) & 7;
-    c.used = (m >> 30) & 1;
-}
-
-// Sorted union of two sorted leaf sets (rewrite.cu:112-163), the reference's
-// two-pointer walk unrolled over the four output positions; fails above 4
-// leaves.  The current element of each set is selected with constant indexes,
-// so the leaf arrays stay in registers.
-__device__ __forceinline__ uint32_t sel4(const uint32_t *l, int i) {
-    return i == 0 ? l[0] : i == 1 ? l[1] : i == 2 ? l[2] : l[3];
-}
-
-// phA / phB: the output positions that hold a's / b's leaves (the truth-table
-// phases of rewrite.cu:195-201, read off the walk itself).  Selects only, no
-// branches: c is written whether or not the union fits in 4 leaves (the
-// return value says), so a failed merge leaves leaves of a and b in c.
-__device__ __forceinline__ int merge_ordered(const DCut &a, const DCut &b, DCut &c, int &phA, int &phB) {
-    int i = 0, k = 0, n = 0;
-    phA = 0;
-    phB = 0;
-    uint32_t o[4];
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-        const bool ha = i < a.nLeaves, hb = k < b.nLeaves;
-        const uint32_t ai = sel4(a.leaves, i < 3 ? i : 3), bk = sel4(b.leaves, k < 3 ? k : 3);
-        const bool takeA = ha & (!hb | (ai <= bk));
-        const bool takeB = hb & (!ha | (bk <= ai));
-        o[s] = (ha | hb) ? (takeA ? ai : bk) : 0u;
-        phA |= (int)takeA << s;
-        phB |= (int)takeB << s;
-        n += (int)(ha | hb);
-        i += (int)takeA;
-        k += (int)takeB;
-    }
-    // positions past the count repeat the first leaf (the containment tests of
-    // the slot replay rely on it; stored records zero them)
-#pragma unroll
-    for (int p = 0; p < 4; p++) c.leaves[p] = p < n ? o[p] : o[0];
-    c.nLeaves = n;
-    return (i >= a.nLeaves) & (k >= b.nLeaves);
-}
-
-// Placement of truth-table variables (tt_place.h): one entry per phase,
-// held in lanes 0..15 of two registers and read with ds_bpermute, so a lane
-// finds its phase's swaps without a memory access and without a loop.
+// Reduction of truth-table variables (tt_place.h): the swaps of each phase.
 __constant__ uint64_t kTtPlace[16] = {
     tt_place_entry(0),  tt_place_entry(1),  tt_place_entry(2),  tt_place_entry(3),
     tt_place_entry(4),  tt_place_entry(5),  tt_place_entry(6),  tt_place_entry(7),
     tt_place_entry(8),  tt_place_entry(9),  tt_place_entry(10), tt_place_entry(11),
     tt_place_entry(12), tt_place_entry(13), tt_place_entry(14), tt_place_entry(15)};
-
-struct PlaceTab {
-    uint32_t lo, hi;    // lane i (i < 16): kTtPlace[i]
-};
-
-__device__ __forceinline__ PlaceTab place_tab(int lane) {
-    const uint64_t e = kTtPlace[lane & 15];
-    return PlaceTab{(uint32_t)e, (uint32_t)(e >> 32)};
-}
-
-// the entry of `phase` (0..15); every lane of the wavefront must be active
-__device__ __forceinline__ uint64_t place_of(const PlaceTab &tab, int phase) {
-    const int a = phase << 2;
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(a, (int)tab.lo);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(a, (int)tab.hi);
-    return (uint64_t)hi << 32 | lo;
-}
-
-// Support reduction (rewrite.cu:223-266): the leaves the table does not
-// depend on are dropped, the others keep their order, and the table's
-// variables move down with them.  Without branches per lane: when every leaf
-// stays, the shrink has no swaps and the compaction keeps the leaves where
-// they are (positions past the count already repeat the first leaf, as after
-// the merge).  The shrink and the compaction run only if some lane whose
-// result is used (`used_here`) shrinks; otherwise every such lane's cut is
-// already its result, and the others' results are not read.  r holds the
-// leaves' reference counts and moves with them.  Returns 1 if the cut shrank
-// (0 in lanes left as they were).
-__device__ __forceinline__ int minimize_support(DCut &c, const PlaceTab &tab, bool used_here, int (&r)[4]) {
-    const uint32_t m0[4] = {0x5555, 0x3333, 0x0F0F, 0x00FF};
-    const uint32_t m1[4] = {0xAAAA, 0xCCCC, 0xF0F0, 0xFF00};
-    const uint32_t t = c.tt & 0xFFFF;
-    int phase = 0;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-        phase |= (int)((i < c.nLeaves) & ((t & m0[i]) != ((t & m1[i]) >> (1 << i)))) << i;
-    const int nL = __popc((uint32_t)phase);
-    if (__ballot(used_here && nL != c.nLeaves) == 0) return 0;     // wave-uniform
-    c.tt = tt_place_shrink(t, place_of(tab, phase)) & 0xFFFF;
-    // compaction: kept leaf i moves to slot popc(phase below i); the slots past
-    // the new count repeat the first leaf
-    uint32_t o[4];
-    int q[4];
-#pragma unroll
-    for (int p = 0; p < 4; p++) { o[p] = c.leaves[p]; q[p] = r[p]; }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int pos = __popc((uint32_t)phase & ((1u << i) - 1u));
-#pragma unroll
-        for (int p = 0; p < 4; p++)
-            if (p == pos && ((phase >> i) & 1)) { o[p] = c.leaves[i]; q[p] = r[i]; }
-    }
-#pragma unroll
-    for (int p = 0; p < 4; p++) { c.leaves[p] = p < nL ? o[p] : o[0]; r[p] = q[p]; }
-    const int shrunk = nL != c.nLeaves;
-    c.nLeaves = nL;
-    return shrunk;
-}
 
 __device__ void store_cuts(uint32_t *out, const DCut *cs) {
     for (int s = 0; s < NCUT; s++) {
@@ -257,89 +114,87 @@ __global__ void k_cuts_pi(int32_t nPIs, const int32_t *__restrict__ nRef, uint32
     store_cuts(cuts + (size_t)v * NCUT * 5, c);
 }
 
-// One wavefront per node.  Lane l = 8*i + j owns the pair (cut i of fanin0,
-// cut j of fanin1): the 64 merges, truth tables, support reductions and cut
-// values are computed in parallel.  The reference inserts the candidates one
+// One wavefront per node.  A node's candidate cuts are the pairs (cut i of
+// fanin 0, cut j of fanin 1) that pass the signature prefilter, inserted one
 // by one in (i, j) order with an order-dependent slot policy (FindCut evicts,
-// CutFilter drops dominated cuts, rewrite.cu:84-193, 268-294); that replay runs
-// wave-uniformly over the surviving candidates with the 8 slots held in lanes
-// 0..7, using ballots for the per-slot tests, so the result equals the
-// sequential one exactly.
+// CutFilter drops dominated cuts, rewrite.cu:84-193, 268-294).
+//   - lane 4 s + k (+ 32 for fanin 1) loads leaf k of the fanin's slot s; the
+//     signatures are an OR over the quad, lane 8 i + j tests pair (i, j);
+//   - the candidates (about 10 of the 64 pairs on most graphs, 2 on most nodes
+//     of the 10M deep AIG) are compacted to one quad of lanes each, 16 at a
+//     time: lane k of a quad holds leaf k of both cuts, ranks its leaves in the
+//     union, computes bits 4 k .. 4 k + 3 of the truth table and tests variable
+//     k for support;
+//   - on most nodes no two candidates compare, so the containment tests are
+//     made up front, all candidates against one per step, and the candidates
+//     before the first comparable pair take their slots by rank (or, with every
+//     slot in use, by the smallest eviction key);
+//   - the others are inserted one by one, slot s's leaf k in lane 4 s + k and
+//     the slot's state in its quad.  A free slot's key is below every used
+//     one's, so the slot a candidate takes, free or evicted, is the smallest
+//     key, and a failed merge is the insertion of an empty slot.  The number of
+//     slot leaves that the new cut holds decides containment both ways: the
+//     smaller cut lies in the larger one when it equals the smaller leaf count.
+// What bounds it is the length of one wavefront's instruction stream: a
+// level's nodes are far fewer than the SIMDs, and the next level waits for
+// the slowest.  Measured on a lone wavefront: 4 cycles an instruction, 16 more
+// where a scalar instruction reads what a vector one wrote, about 14 a branch,
+// 60 a lane permute.  One insertion in turn costs about 300 cycles, a
+// containment step about 50.
 constexpr int CUTW_BLOCK = 256;
 // the per-level kernel runs one wavefront per workgroup: a level's ~200 nodes
 // then spread over as many CUs, each wavefront with its own L1 and memory
 // pipeline (4 wavefronts per workgroup measured 10% slower on the 10M AIG)
 constexpr int CUTL_BLOCK = 64;
-enum : int { C_SKIP = 0, C_FAIL = 1, C_OK = 2 };
 
 __device__ __forceinline__ int rl(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
-// x with lane l replaced by the wave-uniform v: the llvm.amdgcn.writelane
-// intrinsic (v_writelane_b32), which this compiler has no builtin name for
-extern "C" __device__ int gls_writelane_i32(int v, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
-__device__ __forceinline__ uint32_t wl(uint32_t v, int l, uint32_t x) {
-    return (uint32_t)gls_writelane_i32((int)v, l, (int)x);
+__device__ __forceinline__ uint32_t bperm(uint32_t byteAddr, uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_ds_bpermute((int)byteAddr, (int)v);
+}
+// the lanes where x holds, from the comparison's own lane mask, and back
+__device__ __forceinline__ uint64_t lanes_of(bool x) { return __builtin_amdgcn_ballot_w64(x); }
+__device__ __forceinline__ bool in_lanes(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+// lane j of the quad, to its four lanes; the quad's OR and sum
+template <int CTRL> __device__ __forceinline__ uint32_t quad_perm(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+}
+template <int J> __device__ __forceinline__ uint32_t quad_lane(uint32_t v) { return quad_perm<J * 0x55>(v); }
+__device__ __forceinline__ uint32_t quad_or(uint32_t v) {
+    v |= quad_perm<0xB1>(v);
+    return v | quad_perm<0x4E>(v);
+}
+__device__ __forceinline__ uint32_t quad_add(uint32_t v) {
+    v += quad_perm<0xB1>(v);
+    return v + quad_perm<0x4E>(v);
 }
 
-// Minimum of v over lanes 0..7, valid in lane 0: two quad_perm steps (xor 1,
-// xor 2) and row rotations by 4 and 12, so lane 0 also sees lanes 4..7 in
-// either rotation direction.  DPP moves, no LDS round trip.
-__device__ __forceinline__ uint32_t min8_lane0(uint32_t v) {
-    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp((int)0xFFFFFFFF, (int)v, 0xB1, 0xF, 0xF, false));
-    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp((int)0xFFFFFFFF, (int)v, 0x4E, 0xF, 0xF, false));
+// Minimum over lanes 0..31 (in each of them), and over the wavefront, of v,
+// which is the same in a quad: row rotations by 4 and 8 within 16 lanes, then
+// the other rows.
+__device__ __forceinline__ uint32_t min_quads32(uint32_t v) {
     v = min(v, (uint32_t)__builtin_amdgcn_update_dpp((int)0xFFFFFFFF, (int)v, 0x124, 0xF, 0xF, false));
-    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp((int)0xFFFFFFFF, (int)v, 0x12C, 0xF, 0xF, false));
-    return v;
+    v = min(v, (uint32_t)__builtin_amdgcn_update_dpp((int)0xFFFFFFFF, (int)v, 0x128, 0xF, 0xF, false));
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return min((uint32_t)r[0], (uint32_t)r[1]);
+}
+__device__ __forceinline__ uint32_t min_quads(uint32_t v) {
+    v = min_quads32(v);
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return min((uint32_t)r[0], (uint32_t)r[1]);
 }
 
-// One slot of the cut set under construction, held by lane = slot index; which
-// slots are in use is the wave-uniform bit mask `used` of the replay.
-struct Slot {
-    uint32_t l0, l1, l2, l3, tt, value;
-    int n;
-    uint32_t sig;       // bit (leaf & 31) of every leaf: a prefilter for containment
-};
-
-
-// Leaf signature of a merged or support-minimized cut: its leaf list is padded
-// with its first leaf, so a padded position adds no bit; an empty cut has none.
-__device__ __forceinline__ uint32_t sig4(uint32_t n0, uint32_t n1, uint32_t n2, uint32_t n3, int nn) {
-    const uint32_t s = (1u << (n0 & 31)) | (1u << (n1 & 31)) | (1u << (n2 & 31)) | (1u << (n3 & 31));
-    return nn > 0 ? s : 0u;
-}
-
-// CutFilter (rewrite.cu:178-193) of the cut in slot `id` (leaves N, nn) against
-// the other used slots.  Scanning slots in order, a larger slot that contains N
-// is dropped; the first slot of no more leaves that N contains drops N and ends
-// the scan.  Returns true if N was dropped.
-__device__ __forceinline__ bool filter_wave(Slot &s, int lane, int id, uint32_t n0, uint32_t n1, uint32_t n2,
-                                            uint32_t n3, int nn, uint32_t nsig, uint32_t &used) {
-    const bool mine = lane < NCUT && lane != id && ((used >> (lane & 7)) & 1u);
-    const bool bigger = s.n > nn;
-    // containment implies containment of the leaf signatures (CutFilter's own
-    // prefilter, rewrite.cu:181, 185): when no slot passes it, nothing changes
-    const bool maybe = mine & ((s.sig & nsig) == (bigger ? nsig : s.sig));
-    if (__ballot(maybe) == 0) return false;
-    // exact containment both ways from one 4x4 equality matrix: leaf lists are
-    // padded with their first leaf past their count, so a padded entry repeats
-    // a real one and no count enters the test (bitwise, without branches)
-    const bool e00 = n0 == s.l0, e01 = n0 == s.l1, e02 = n0 == s.l2, e03 = n0 == s.l3;
-    const bool e10 = n1 == s.l0, e11 = n1 == s.l1, e12 = n1 == s.l2, e13 = n1 == s.l3;
-    const bool e20 = n2 == s.l0, e21 = n2 == s.l1, e22 = n2 == s.l2, e23 = n2 == s.l3;
-    const bool e30 = n3 == s.l0, e31 = n3 == s.l1, e32 = n3 == s.l2, e33 = n3 == s.l3;
-    const bool nInS = (nn == 0) | ((e00 | e01 | e02 | e03) & (e10 | e11 | e12 | e13) & (e20 | e21 | e22 | e23) &
-                                   (e30 | e31 | e32 | e33));
-    const bool sInN = (s.n == 0) | ((nn != 0) & (e00 | e10 | e20 | e30) & (e01 | e11 | e21 | e31) &
-                                    (e02 | e12 | e22 | e32) & (e03 | e13 | e23 | e33));
-    const bool d1 = maybe & bigger & nInS;
-    const bool d2 = maybe & !bigger & sInN;
-    const uint64_t m2 = __ballot(d2);
-    const int k = m2 ? __ffsll((unsigned long long)m2) - 1 : NCUT;
-    used &= ~(uint32_t)(__ballot(d1 && lane < k) & 0xFFull);
-    if (k < NCUT) {
-        used &= ~(1u << id);
-        return true;
-    }
-    return false;
+// Bits 4 k .. 4 k + 3 of a table over the variables at the set bits of
+// `phase`, from the table t over variables 0, 1, ..: entry b of the result is
+// entry pext(b, phase) of t.  The two high index bits (k) give a shift of t,
+// the two low ones spread at most four of its bits over the nibble.
+__device__ __forceinline__ uint32_t tt_nibble(uint32_t t, uint32_t phase, uint32_t ext) {
+    const uint32_t lo = phase & 3u, sh8 = lo << 3;
+    const uint32_t px = (ext >> ((phase >> 1) & 6u)) & 3u;
+    const uint32_t pc = (0x94u >> (lo << 1)) & 3u;                   // bits set in lo
+    const uint32_t x = (t >> (px << pc)) & 15u;
+    // lo 0: bit 0 to all four; 1: bits 1, 0 twice; 2: bits 0 and 1 doubled; 3: as they are
+    return (x & (0x0F010301u >> sh8)) * ((0x0103050Fu >> sh8) & 15u) + (x & (0x00020000u >> sh8)) * 6u;
 }
 
 // Fence-free record format of the dataflow schedule: every 64-bit word of a
@@ -349,34 +204,24 @@ __device__ __forceinline__ bool filter_wave(Slot &s, int lane, int id, uint32_t 
 constexpr unsigned long long TAG_V = 1ull << 63;
 constexpr uint32_t DF_SPIN_LIMIT = 1u << 22;
 
-__device__ __forceinline__ bool load_tagged(const unsigned long long *rec, DCut &c) {
-    const unsigned long long w0 = __hip_atomic_load(rec + 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long w1 = __hip_atomic_load(rec + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned long long w2 = __hip_atomic_load(rec + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (!(w0 & w1 & w2 & TAG_V)) return false;
-    c.leaves[0] = (uint32_t)(w0 & 0x7FFFFFFFull);
-    c.leaves[1] = (uint32_t)((w0 >> 31) & 0x7FFFFFFFull);
-    c.leaves[2] = (uint32_t)(w1 & 0x7FFFFFFFull);
-    c.leaves[3] = (uint32_t)((w1 >> 31) & 0x7FFFFFFFull);
-    const uint32_t m = (uint32_t)w2;
-    c.tt = m & 0xFFFF;
-    c.value = (m >> 16) & 0x7FF;
-    c.nLeaves = (m >> 27) & 7;
-    c.used = (m >> 30) & 1;
-    return true;
+__device__ __forceinline__ unsigned long long load_tagged(const unsigned long long *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-
-__device__ __forceinline__ void store_tagged(unsigned long long *rec, uint32_t l0, uint32_t l1, uint32_t l2,
-                                             uint32_t l3, uint32_t meta) {
-    __hip_atomic_store(rec + 0, (unsigned long long)l0 | (unsigned long long)l1 << 31 | TAG_V, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(rec + 1, (unsigned long long)l2 | (unsigned long long)l3 << 31 | TAG_V, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(rec + 2, (unsigned long long)meta | TAG_V, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void store_tagged(unsigned long long *p, unsigned long long v) {
+    __hip_atomic_store(p, v | TAG_V, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // cut_node record modes
 enum : int { REC_PLAIN = 0, REC_TAGGED = 1 };
+
+// leaf words that are no leaf: of a slot, of a candidate (never equal)
+constexpr uint32_t SLOT_PAD = 0xFFFFFFFEu, CAND_PAD = 0xFFFFFFFFu;
+constexpr uint64_t QUAD_LANE0 = 0x1111111111111111ull;
+// state of a slot, and what a candidate brings to it: leaf count << 24 |
+// SLOT_NEW (its meta word is still with the candidate) | SLOT_USED | candidate
+// << 16 | category << 14 | value << 3.  The bits of SLOT_KEY with the slot's
+// index order the slots for eviction, free ones first.
+constexpr uint32_t SLOT_FREE = 15u << 24, SLOT_NEW = 1u << 21, SLOT_USED = 1u << 20, SLOT_KEY = 0x10FFFFu;
 
 // Cut set of node idx (fanin literals l0, l1), computed by one whole wavefront
 // (lane = thread lane).  MODE REC_PLAIN: the fanins' 8-slot records (20 bytes
@@ -386,20 +231,20 @@ enum : int { REC_PLAIN = 0, REC_TAGGED = 1 };
 // is written in it (tcuts, 24 bytes per slot).
 // Returns false if a poll exceeded its bound (*err set), true otherwise.
 template <int MODE>
-__device__ __forceinline__ bool cut_node(const int idx, const int lane, const uint32_t l0, const uint32_t l1,
+__device__ __forceinline__ bool cut_node(const int idx, const uint32_t lane, const uint32_t l0, const uint32_t l1,
                                          const uint32_t *ra, const uint32_t *rb, uint32_t *out,
                                          const int32_t *__restrict__ nRef, unsigned long long *tcuts, uint32_t *err,
                                          const uint8_t *__restrict__ sigBits, uint32_t *out2 = nullptr) {
-    const uint32_t in0 = LID(l0), in1 = LID(l1), c0 = LC(l0), c1 = LC(l1);
-    const PlaceTab tab = place_tab(lane);
-    DCut a, b;
+    const uint32_t k = lane & 3u, slot = (lane >> 2) & 7u, quad0 = lane & 60u, k4 = 4u * k;
+    uint32_t leaf, meta;
     if (MODE == REC_TAGGED) {
-        const unsigned long long *ra = tcuts + ((size_t)in0 * NCUT + (lane >> 3)) * 3;
-        const unsigned long long *rb = tcuts + ((size_t)in1 * NCUT + (lane & 7)) * 3;
+        const unsigned long long *r = tcuts + ((size_t)(lane < 32 ? LID(l0) : LID(l1)) * NCUT + slot) * 3;
         uint32_t spins = 0;
+        unsigned long long wl, wm;
         for (;;) {
-            const bool ok = load_tagged(ra, a) && load_tagged(rb, b);
-            if (__ballot(!ok) == 0) break;
+            wl = load_tagged(r + (k >> 1));
+            wm = load_tagged(r + 2);
+            if (lanes_of(!(wl & wm & TAG_V)) == 0) break;
             if (++spins > DF_SPIN_LIMIT ||
                 ((spins & 1023u) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
                 if (lane == 0) atomicOr(err, 4u);
@@ -407,110 +252,253 @@ __device__ __forceinline__ bool cut_node(const int idx, const int lane, const ui
             }
             __builtin_amdgcn_s_sleep(1);
         }
+        leaf = (uint32_t)((k & 1u) ? wl >> 31 : wl) & 0x7FFFFFFFu;
+        meta = (uint32_t)wm;
     } else {
-        unpack_cut(ra + (lane >> 3) * 5, a);
-        unpack_cut(rb + (lane & 7) * 5, b);
+        const uint32_t *r = (lane < 32 ? ra : rb) + slot * 5;
+        leaf = r[k];
+        meta = r[4];
     }
-    // ---- phase 1: every pair in parallel
-    int status = C_SKIP, shrunk = 0;
-    DCut m, mm;
-    m.leaves[0] = m.leaves[1] = m.leaves[2] = m.leaves[3] = 0;
-    m.nLeaves = 0; m.tt = 0; m.value = 0; m.used = 0;
-    mm = m;
-    {
-        // every lane runs the whole computation (no divergent branches; a
-        // failed merge leaves leaves of a and b in m, so every leaf read below
-        // is a valid id) and the status says which results the replay may use
-        const bool cand = a.used && b.used && __popc(cut_sign_of(a, sigBits) | cut_sign_of(b, sigBits)) <= 4;
-        int phA, phB;
-        const int ok = merge_ordered(a, b, m, phA, phB);
-        // the merged leaves' reference counts, in flight during the truth
-        // tables; a reduced cut's leaves are some of them
-        int r[4];
-        leaf_refs(m, nRef, r);
-        uint32_t t0 = c0 ? ~a.tt : a.tt, t1 = c1 ? ~b.tt : b.tt;
-        t0 = tt_place_stretch(t0, place_of(tab, phA));
-        t1 = tt_place_stretch(t1, place_of(tab, phB));
-        m.tt = (t0 & t1) & 0xFFFF;
-        mm = m;
-        shrunk = minimize_support(mm, tab, cand && ok, r);
-        mm.value = cut_value_of(mm.nLeaves, r);
-        status = !cand ? C_SKIP : !ok ? C_FAIL : C_OK;
-    }
-    // per-candidate words read by the replay: status, shrink flag, leaf counts
-    // and value in one; both truth tables in one; both leaf signatures
-    const uint32_t info = (uint32_t)status | (uint32_t)shrunk << 2 | (uint32_t)(m.nLeaves & 7) << 3 |
-                          (uint32_t)(mm.nLeaves & 7) << 6 | (mm.value & 0x7FFu) << 9;
-    const uint32_t tts = (m.tt & 0xFFFFu) | (mm.tt & 0xFFFFu) << 16;
-    const uint32_t msig = sig4(m.leaves[0], m.leaves[1], m.leaves[2], m.leaves[3], m.nLeaves);
-    const uint32_t mmsig = sig4(mm.leaves[0], mm.leaves[1], mm.leaves[2], mm.leaves[3], mm.nLeaves);
-    // ---- phase 2: replay the insertions in (i, j) order
-    Slot s;
-    s.l0 = lane == 0 ? (uint32_t)idx : 0u;
-    s.l1 = s.l2 = s.l3 = s.l0;          // padded with the first leaf
-    s.n = lane == 0 ? 1 : 0;
-    s.tt = lane == 0 ? 0xAAAAu : 0u;
-    s.value = lane == 0 ? 1001u : 0u;
-    s.sig = lane == 0 ? 1u << ((uint32_t)idx & 31) : 0u;
-    uint32_t used = 1u;                 // slots in use (bit = slot), wave-uniform
-    uint64_t todo = __ballot(status != C_SKIP);
+    // lane constants: the quad's lanes before this one, pext(k, 0..3) in 2 bits
+    // each, the table entries with variable k clear
+    const uint32_t below = (1u << k) - 1u, ext = k << 6 | (k >> 1) << 4 | (k & 1u) << 2;
+    const uint32_t vmask = (uint32_t)(0x00FF0F0F33335555ull >> (16u * k)) & 0xFFFFu;
+    // leaf signatures of the reference (rewrite.cu:68, 262: bit leaf & 31).  In
+    // a batched pass sigBits holds each node's bit as it would be in its own
+    // AIG (its id there & 31), so that the prefilter of rewrite.cu:283 sees the
+    // same signatures as when that AIG is rewritten alone.  An empty slot gets
+    // all bits, so that no pair with it passes.
+    const bool has = k < ((meta >> 27) & 7u);
+    const uint32_t bit = sigBits ? (uint32_t)sigBits[has ? leaf : 0u] : leaf & 31u;
+    uint32_t sig = quad_or(has ? 1u << bit : 0u);
+    sig = (meta >> 30) & 1u ? sig : 0xFFFFFFFFu;
+    const uint32_t sa = bperm((lane >> 3) * 16u, sig), sb = bperm(128u + (lane & 7u) * 16u, sig);
+    bool cand = __popc(sa | sb) <= 4;
+    uint64_t todo = lanes_of(cand);
+    // the slots, slot 0 holding the trivial cut; sval: their meta words
+    uint32_t sl = lane == 0 ? (uint32_t)idx : SLOT_PAD;
+    uint32_t st = lane < 4 ? 1u << 24 | SLOT_USED | 2u << 14 | 1001u << 3 : SLOT_FREE;
+    uint32_t sval = 1u << 30 | 1u << 27 | 1001u << 16 | 0xAAAAu;
+    const uint32_t keyLow = lane < 32 ? slot : 0xFFFFFFFFu;     // lanes 32 and up hold no slot
+    bool first = true;
     while (todo) {
-        const int l = __ffsll((unsigned long long)todo) - 1;
-        todo &= todo - 1;
-        const uint32_t inf = (uint32_t)rl((int)info, l);
-        const int st = (int)(inf & 3u);
-        // FindCut (rewrite.cu:84-109)
-        int id;
-        if (used != 0xFFu) {
-            id = __ffs(~used & 0xFFu) - 1;
-        } else {
-            // categories in order (more than 2 leaves, 2, fewer), then the
-            // smallest value, then the first slot: one minimum of that key
-            const uint32_t cat = s.n > 2 ? 0u : s.n == 2 ? 1u : 2u;
-            const uint32_t key = lane < NCUT ? (cat << 14 | (s.value & 0x7FF) << 3 | (uint32_t)lane) : 0xFFFFFFFFu;
-            id = (int)((uint32_t)rl((int)min8_lane0(key), 0) & 7u);
+        // ---- the next 16 candidates, one quad of lanes each
+        const uint32_t order = __builtin_amdgcn_mbcnt_hi((uint32_t)(todo >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)todo, 0u));
+        const uint32_t cnt = min((uint32_t)__popcll(todo), 16u);
+        const bool now = cand && order < 16u;
+        cand = cand && !now;
+        // lane 1 takes what the lanes without a candidate send
+        const uint32_t pair = quad_lane<0>((uint32_t)__builtin_amdgcn_ds_permute(now ? (int)(order * 16u) : 4, (int)lane));
+        todo = lanes_of(cand);
+        const uint32_t pa = (pair & 56u) * 2u + k4, pb = 128u + (pair & 7u) * 16u + k4;
+        const uint32_t a = bperm(pa, leaf), b = bperm(pb, leaf), ma = bperm(pa, meta), mb = bperm(pb, meta);
+        // sorted union (rewrite.cu:112-163): a leaf's position is the number
+        // of distinct leaves before it (ids are below 2^31 - 16)
+        const uint32_t na = (ma >> 27) & 7u, nb = (mb >> 27) & 7u;
+        const uint32_t aa = k < na ? a : 0x7FFFFFFFu, bb = k < nb ? b : 0x7FFFFFFEu;
+        const uint32_t b0 = quad_lane<0>(bb), b1 = quad_lane<1>(bb), b2 = quad_lane<2>(bb), b3 = quad_lane<3>(bb);
+        const bool common = min(min(aa ^ b0, aa ^ b1), min(aa ^ b2, aa ^ b3)) == 0;
+        const uint32_t both = quad_or((common ? 1u : 0u) << k);
+        const uint32_t rank = k + ((b0 - aa) >> 31) + ((b1 - aa) >> 31) + ((b2 - aa) >> 31) + ((b3 - aa) >> 31) -
+                              (uint32_t)__popc(both & below);
+        const uint32_t n = na + nb - (uint32_t)__popc(both);
+        const bool ok = (lane >> 2) < cnt && n <= 4u;
+        // positions that hold a's leaves, and (high half) those that only a has
+        const uint32_t kind = common ? 1u : 0x10001u;
+        const uint32_t pos = quad_or((k < na ? kind : 0u) << (rank & 15u));
+        const uint32_t phA = pos & 15u, phB = ~(pos >> 16) & ((1u << n) - 1u) & 15u;
+        const uint32_t la = bperm(4u * (quad0 + (uint32_t)__popc(phA & below)), a);
+        const uint32_t lb = bperm(4u * (quad0 + (uint32_t)__popc(phB & below)), b);
+        // truth table over the union, four bits per lane
+        const uint32_t ta = (ma ^ (0u - LC(l0))) & 0xFFFFu, tb = (mb ^ (0u - LC(l1))) & 0xFFFFu;
+        const uint32_t tt = quad_or((tt_nibble(ta, phA, ext) & tt_nibble(tb, phB, ext)) << k4);
+        const uint32_t m = (phA >> k) & 1u ? la : lb;
+        // support reduction (rewrite.cu:223-266): fm, fn, ftt the final cut, the
+        // leaves that the table does not depend on dropped, the others moved down
+        const bool dep = ((tt ^ (tt >> (1u << k))) & vmask) != 0;
+        uint32_t fm = m, ftt = tt, fn = n;
+        if (lanes_of(ok && k < n && !dep) != 0) {      // some candidate shrinks
+            const uint32_t keep = quad_or((k < n && dep ? 1u : 0u) << k);
+            fn = (uint32_t)__popc(keep);
+            // the kept leaves first, in order, then the dropped ones
+            const uint32_t before = (uint32_t)__popc(keep & below);
+            const uint32_t to = (keep >> k) & 1u ? before : fn + k - before;
+            fm = (uint32_t)__builtin_amdgcn_ds_permute((int)(4u * (quad0 + to)), (int)m);
+            ftt = tt_place_shrink(tt, kTtPlace[keep]) & 0xFFFFu;
         }
-        used &= ~(1u << id);
-        if (st == C_FAIL) continue;
-        // the slot takes the merged cut (selects on one lane compare)
-        const int nn = (int)((inf >> 3) & 7u);
-        const uint32_t n0 = (uint32_t)rl((int)m.leaves[0], l), n1 = (uint32_t)rl((int)m.leaves[1], l);
-        const uint32_t n2 = (uint32_t)rl((int)m.leaves[2], l), n3 = (uint32_t)rl((int)m.leaves[3], l);
-        const uint32_t nsig = (uint32_t)rl((int)msig, l);
-        // slot id takes the values (all wave-uniform): one v_writelane each
-        s.l0 = wl(n0, id, s.l0); s.l1 = wl(n1, id, s.l1); s.l2 = wl(n2, id, s.l2); s.l3 = wl(n3, id, s.l3);
-        s.n = (int)wl((uint32_t)nn, id, (uint32_t)s.n); s.sig = wl(nsig, id, s.sig);
-        used |= 1u << id;
-        if (filter_wave(s, lane, id, n0, n1, n2, n3, nn, nsig, used)) continue;
-        const uint32_t ttw = (uint32_t)rl((int)tts, l);
-        s.tt = wl(ttw & 0xFFFFu, id, s.tt);
-        int fn = nn;
-        if ((inf >> 2) & 1u) {
-            fn = (int)((inf >> 6) & 7u);
-            const uint32_t q0 = (uint32_t)rl((int)mm.leaves[0], l), q1 = (uint32_t)rl((int)mm.leaves[1], l);
-            const uint32_t q2 = (uint32_t)rl((int)mm.leaves[2], l), q3 = (uint32_t)rl((int)mm.leaves[3], l);
-            const uint32_t qsig = (uint32_t)rl((int)mmsig, l);
-            s.l0 = wl(q0, id, s.l0); s.l1 = wl(q1, id, s.l1); s.l2 = wl(q2, id, s.l2); s.l3 = wl(q3, id, s.l3);
-            s.n = (int)wl((uint32_t)fn, id, (uint32_t)s.n); s.tt = wl(ttw >> 16, id, s.tt); s.sig = wl(qsig, id, s.sig);
-            filter_wave(s, lane, id, q0, q1, q2, q3, fn, qsig, used);
+        // the final leaves' reference counts are in flight meanwhile: only an
+        // eviction and the end of the batch need the values
+        int ref = nRef[k < fn ? fm : 0u];
+        const uint32_t cat = fn > 2u ? 0u : fn == 2u ? 1u : 2u;
+        uint32_t info = ok ? fn << 24 | SLOT_NEW | SLOT_USED | (lane >> 2) << 16 | cat << 14 : SLOT_FREE;
+        uint32_t fmeta = 0;
+        bool valued = false;
+        auto value = [&]() {            // meta words: CutFindValue (rewrite.cu:49-61)
+            asm volatile("" : "+v"(ref));       // the load is waited for here, not before a branch to here
+            const int sum = (int)quad_add(k < fn ? (uint32_t)ref : 0u);
+            const uint32_t ones = quad_add(k < fn && ref == 1 ? 1u : 0u);
+            uint32_t v = (uint32_t)(sum > 1000 ? 1000 : sum);
+            v = ones > 3u ? 5u - ones : v;
+            v = fn < 2u ? 1001u : v;
+            fmeta = ftt | (v & 0x7FFu) << 16 | (fn & 7u) << 27 | 1u << 30;
+            info |= ok ? (v & 0x7FFu) << 3 : 0u;
+            const uint32_t g = bperm((st >> 12) & 0xF0u, info);
+            st = st & SLOT_NEW ? g : st;
+            valued = true;
+        };
+        const uint64_t okm = lanes_of(ok) & QUAD_LANE0;
+        // candidates that shrink or end the insertions
+        uint64_t odd = lanes_of(ok && (fn != n || fn < 2u)) & QUAD_LANE0;
+        const uint32_t cl = ok && k < n ? m : CAND_PAD;
+        uint32_t c = 0;
+        if (!first) {
+            value();
+        } else if (cnt > 2u) {
+            // ---- the candidates before the first odd one, and of these the
+            // ones before the later of the first two that compare
+            const uint32_t quad = lane >> 2;
+            uint32_t end = odd ? (uint32_t)__builtin_ctzll(odd) >> 2 : cnt;
+            // bit q of sub: candidate q's leaves all lie in this quad's cut
+            const uint32_t m0 = quad_lane<0>(m);
+            const uint32_t c0 = ok ? (k < n ? m : m0) : CAND_PAD;
+            const uint32_t c1 = quad_perm<0x39>(c0), c2 = quad_perm<0x4E>(c0), c3 = quad_perm<0x93>(c0);
+            uint32_t sub = 0;
+            for (uint32_t q = (end + 3u) & ~3u; q; q -= 4) {
+                const uint32_t at = 16u * q - 64u + k4;
+                uint32_t d[4];
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++) d[j] = bperm(at + 16u * j, c0);
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++)
+                    d[j] = quad_or(min(min(c0 ^ d[j], c1 ^ d[j]), min(c2 ^ d[j], c3 ^ d[j])));
+#pragma unroll
+                for (int j = 3; j >= 0; j--) sub = 2u * sub + (d[j] == 0 ? 1u : 0u);
+            }
+            const uint32_t early = (1u << quad) - 1u;
+            sub = ok && quad < end ? sub & ((1u << end) - 1u) & ~(1u << quad) : 0u;
+            if (lanes_of(sub != 0) != 0)
+                end = (uint32_t)__builtin_amdgcn_readfirstlane(
+                    (int)min_quads(sub == 0 ? 255u : sub & early ? quad : (uint32_t)__builtin_ctz(sub)));
+            // the first seven that merged, to slots 1..7
+            const uint64_t take = okm & (end < 16u ? (1ull << (4u * end)) - 1ull : ~0ull);
+            const uint32_t r = quad_lane<0>(__builtin_amdgcn_mbcnt_hi((uint32_t)(take >> 32),
+                                                                      __builtin_amdgcn_mbcnt_lo((uint32_t)take, 0u)));
+            const bool slotted = ok && quad < end && r < (uint32_t)(NCUT - 1);
+            const int to = (int)(slotted ? 16u * r + 16u + k4 : 128u + k4);    // lanes 32 and up take the rest
+            const uint32_t nTake = (uint32_t)__popcll(take);
+            const uint32_t pl = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)cl);
+            const uint32_t pi = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)info);
+            const bool filled = slot >= 1u && slot <= nTake && lane < 32;
+            sl = filled ? min(pl, SLOT_PAD) : sl;
+            st = filled ? pi : st;
+            c = end;
+            if (nTake >= (uint32_t)(NCUT - 1)) {
+                // every slot is in use: each further one evicts (also if it
+                // failed to merge), FindCut (rewrite.cu:84-109)
+                c = (uint32_t)__builtin_ctzll(lanes_of(slotted && r == (uint32_t)(NCUT - 2))) / 4u + 1u;
+                if (c < end) {
+                    value();
+                    uint32_t inf = bperm(16u * c, info);
+                    for (; c < end; c++) {
+                        const uint32_t next = bperm(16u * c + 16u, info);
+                        const uint32_t key = (st & SLOT_KEY) | keyLow;
+                        st = key == min_quads32(key) ? inf : st;
+                        inf = next;
+                        asm volatile("" : "+v"(inf));      // moved before the loop's branch
+                    }
+                    const uint32_t gl = bperm(((st >> 12) & 0xF0u) + k4, cl);
+                    sl = st & SLOT_NEW ? min(gl, SLOT_PAD) : st & SLOT_USED ? sl : SLOT_PAD;
+                }
+            }
+            if (!valued && nTake + (cnt - c) >= (uint32_t)NCUT && c < cnt) value();
         }
-        s.value = wl((inf >> 9) & 0x7FFu, id, s.value);
-        if (fn < 2) break;
+        first = false;
+        // ---- the others one by one.
+        // CutFilter (rewrite.cu:178-193) of a cut (leaf k in x, nn leaves)
+        // against the slots where `hit` holds: scanning slots in order, a
+        // larger slot that contains it is dropped; the first slot of no more
+        // leaves that it contains drops it and ends the scan.  True if dropped.
+        auto shared_with = [&](uint32_t x) -> uint32_t {
+            const uint32_t d = min(min(sl ^ x, sl ^ quad_perm<0x39>(x)), min(sl ^ quad_perm<0x4E>(x), sl ^ quad_perm<0x93>(x)));
+            return quad_add(d == 0 ? 1u : 0u);
+        };
+        auto filter = [&](uint32_t hit, uint32_t nn) -> bool {
+            const uint32_t drops = hit & (uint32_t)lanes_of((st >> 24) <= nn);
+            const uint32_t gone = hit & ~drops & ((drops & (0u - drops)) - 1u);     // before the first that drops it
+            const bool g = in_lanes((uint64_t)gone);
+            sl = g ? SLOT_PAD : sl;
+            st = g ? SLOT_FREE : st;
+            return drops != 0;
+        };
+        bool stop = false;
+        uint32_t x = bperm(16u * c + k4, cl), inf = bperm(16u * c, info);
+        odd &= c < 16u ? ~0ull << (4u * c) : 0ull;
+        while (c < cnt) {
+            const uint32_t end = odd ? (uint32_t)__builtin_ctzll(odd) >> 2 : cnt;
+            for (; c < end; c++) {
+                const uint32_t nx = bperm(16u * c + 16u + k4, cl), ninf = bperm(16u * c + 16u, info);
+                // FindCut (rewrite.cu:84-109): the smallest key
+                const uint32_t key = (st & SLOT_KEY) | keyLow;
+                const bool here = key == min_quads32(key);
+                const uint32_t nn = inf >> 24;
+                const uint32_t shared = shared_with(x) + (here ? 64u : 0u);
+                const uint32_t hit = (uint32_t)lanes_of(shared == min(st >> 24, nn));
+                if (hit != 0 && filter(hit, nn)) {
+                    x = CAND_PAD;
+                    inf = SLOT_FREE;
+                }
+                sl = here ? min(x, SLOT_PAD) : sl;
+                st = here ? inf : st;
+                x = nx;
+                inf = ninf;
+                asm volatile("" : "+v"(x), "+v"(inf));     // moved before the loop's branch
+            }
+            if (c == cnt) break;
+            const uint32_t key = (st & SLOT_KEY) | keyLow;
+            const bool here = key == min_quads32(key);
+            const uint32_t n1 = (uint32_t)rl((int)n, (int)(4u * c)), n2 = (uint32_t)rl((int)fn, (int)(4u * c));
+            auto hits = [&](uint32_t y, uint32_t nn) {
+                const uint32_t shared = shared_with(y) + (here ? 64u : 0u);
+                return (uint32_t)lanes_of(shared == min(st >> 24, nn)) & (uint32_t)lanes_of((st & SLOT_USED) != 0);
+            };
+            bool dropped = filter(hits(x, n1), n1);
+            if (!dropped) {
+                if (n2 != n1) {
+                    x = bperm(16u * c + k4, k < fn ? fm : CAND_PAD);
+                    dropped = filter(hits(x, n2), n2);
+                }
+                stop = n2 < 2u;
+            }
+            sl = here ? (dropped ? SLOT_PAD : min(x, SLOT_PAD)) : sl;
+            st = here ? (dropped ? SLOT_FREE : inf) : st;
+            if (stop) break;
+            odd &= odd - 1;
+            c++;
+            x = bperm(16u * c + k4, cl);
+            inf = bperm(16u * c, info);
+        }
+        if (!valued) value();
+        const uint32_t g = bperm((st >> 12) & 0xF0u, fmeta);
+        sval = st & SLOT_NEW ? g : sval;
+        st &= ~SLOT_NEW;
+        if (stop) break;
     }
-    // ---- phase 3: lanes 0..7 store the slots
-    if (lane < NCUT) {
-        const bool u = (used >> lane) & 1u;
-        const uint32_t o0 = (u && s.n > 0) ? s.l0 : 0u, o1 = (u && s.n > 1) ? s.l1 : 0u;
-        const uint32_t o2 = (u && s.n > 2) ? s.l2 : 0u, o3 = (u && s.n > 3) ? s.l3 : 0u;
-        const uint32_t meta = u ? ((s.tt & 0xFFFF) | (s.value & 0x7FF) << 16 | (uint32_t)(s.n & 7) << 27 | 1u << 30) : 0u;
+    // ---- lanes 0..31 store the slots
+    if (lane < 32) {
+        const uint32_t o = sl == SLOT_PAD ? 0u : sl;
+        const uint32_t om = st & SLOT_USED ? sval : 0u;
         if (MODE == REC_TAGGED) {
-            store_tagged(tcuts + ((size_t)idx * NCUT + lane) * 3, o0, o1, o2, o3, meta);
+            const uint32_t o1 = quad_perm<0xB1>(o);
+            unsigned long long *q = tcuts + ((size_t)idx * NCUT + slot) * 3;
+            if (!(k & 1u)) store_tagged(q + (k >> 1), (unsigned long long)o | (unsigned long long)o1 << 31);
+            else if (k == 1u) store_tagged(q + 2, om);
         } else {
-            uint32_t *o = out + lane * 5;
-            o[0] = o0; o[1] = o1; o[2] = o2; o[3] = o3; o[4] = meta;
+            out[slot * 5 + k] = o;
+            if (k == 0) out[slot * 5 + 4] = om;
             if (out2) {
-                uint32_t *q = out2 + lane * 5;
-                q[0] = o0; q[1] = o1; q[2] = o2; q[3] = o3; q[4] = meta;
+                out2[slot * 5 + k] = o;
+                if (k == 0) out2[slot * 5 + 4] = om;
             }
         }
     }
@@ -592,7 +580,7 @@ __device__ __forceinline__ const uint32_t *rec_or_lds(uint32_t x, const uint32_t
     return cuts + (size_t)x * NCUT * 5;
 }
 
-__global__ void __launch_bounds__(CUT3_BLOCK) k_cuts_triple(int32_t s0_, int32_t s1_, int32_t s2_,
+__global__ void __launch_bounds__(CUT3_BLOCK) k_cuts_triple(int32_t s0_, int32_t s1_, int32_t s2_, uint32_t n,
                                                             const uint32_t *__restrict__ f0,
                                                             const uint32_t *__restrict__ f1,
                                                             const int32_t *__restrict__ nRef, uint32_t *cuts,
@@ -605,7 +593,18 @@ __global__ void __launch_bounds__(CUT3_BLOCK) k_cuts_triple(int32_t s0_, int32_t
     // dependent steps and bounds the launch, a first-level node's runs one
     if (v < s1) {                               // uniform per workgroup
         __builtin_amdgcn_s_setprio(0);
-        if (w == 0) cut_node_global((int)v, lane, f0, f1, nRef, cuts, sigBits);
+        if (w == 0) {
+            cut_node_global((int)v, lane, f0, f1, nRef, cuts, sigBits);
+        } else if (w == 1) {
+            // the next launch's fanins into this XCD's L2 (workgroups go round
+            // the 8 XCDs; a line holds 32 nodes): a cone walk there starts with
+            // three dependent loads of them
+            const uint32_t q = s0 + gridDim.x + (blockIdx.x >> 3) * 32u;
+            if (lane < 2 && q < n) {
+                const uint32_t l = lane == 0 ? f0[q] : f1[q];
+                if (l == 0xFFFFFFFFu) cuts[0] = 0u;     // no literal: keeps the load
+            }
+        }
         return;
     }
     if (v >= s2) __builtin_amdgcn_s_setprio(2);
@@ -952,9 +951,10 @@ __global__ void k_cuts_pi_tagged(int32_t nPIs, const int32_t *__restrict__ nRef,
     if (i >= (int64_t)nPIs * NCUT) return;
     const int64_t v = 1 + i / NCUT;
     const int slot = (int)(i % NCUT);
-    uint32_t meta = 0;
-    if (slot == 0) meta = 0xAAAAu | (1001u << 16) | (1u << 27) | (1u << 30);
-    store_tagged(tcuts + ((size_t)v * NCUT + slot) * 3, slot == 0 ? (uint32_t)v : 0u, 0, 0, 0, meta);
+    unsigned long long *q = tcuts + ((size_t)v * NCUT + slot) * 3;
+    store_tagged(q + 0, slot == 0 ? (unsigned long long)v : 0ull);
+    store_tagged(q + 1, 0ull);
+    store_tagged(q + 2, slot == 0 ? 0xAAAAull | (1001ull << 16) | (1ull << 27) | (1ull << 30) : 0ull);
     (void)nRef;
 }
 
@@ -2003,7 +2003,7 @@ int dev_enumerate_cuts(gls_ctx *ctx, const DevGraph &g, const std::vector<int32_
                                           (const uint32_t *)g.f1, (const int32_t *)d_nref, d_cuts, sigBits);
                 else if (c.kind == 3)
                     hipExtLaunchKernelGGL(k_cuts_triple, grid, dim3(CUT3_BLOCK), 0, st, evStart, evStop, 0, c.s, c.m,
-                                          c.m2, (const uint32_t *)g.f0, (const uint32_t *)g.f1,
+                                          c.m2, (uint32_t)n, (const uint32_t *)g.f0, (const uint32_t *)g.f1,
                                           (const int32_t *)d_nref, d_cuts, sigBits);
                 else if (c.kind == 2)
                     hipExtLaunchKernelGGL(k_cuts_pair, grid, dim3(CUTP_BLOCK), 0, st, evStart, evStop, 0, c.s,
@@ -2019,7 +2019,7 @@ int dev_enumerate_cuts(gls_ctx *ctx, const DevGraph &g, const std::vector<int32_
                 k_cuts_quad<<<grid, CUT4_BLOCK, 0, st>>>(c.s, c.m, c.m2, levelStart[std::min(c.l + 3, L)], g.f0, g.f1,
                                                          d_nref, d_cuts, sigBits);
             } else if (c.kind == 3) {
-                k_cuts_triple<<<grid, CUT3_BLOCK, 0, st>>>(c.s, c.m, c.m2, g.f0, g.f1, d_nref, d_cuts, sigBits);
+                k_cuts_triple<<<grid, CUT3_BLOCK, 0, st>>>(c.s, c.m, c.m2, (uint32_t)n, g.f0, g.f1, d_nref, d_cuts, sigBits);
             } else if (c.kind == 2) {
                 k_cuts_pair<<<grid, CUTP_BLOCK, 0, st>>>(c.s, c.m - c.s, c.m, g.f0, g.f1, d_nref, d_cuts, sigBits);
             } else {
