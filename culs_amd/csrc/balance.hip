@@ -24,18 +24,22 @@
 // Literal values decide ties in the input order; there the reference's own
 // values are used (lit 0 = TRUE, common.h:285-286), not the AIGER ones.
 //
-// Mapping to MI355X: cover discovery is two frontier sweeps (reachability,
-// then a topological sweep of the cover graph; each root is touched twice,
-// several rounds per host check).  Reconstruction of
-// narrow levels runs in ONE persistent workgroup across levels and steps, so
-// a step costs a few workgroup barriers instead of kernel launches and a host
-// round trip; the hash tables are global and all of their traffic is atomics,
-// which the L2 serves.  Wide levels (more than balance_narrow_max covers, a
-// gls_tuning setting) run each phase of a step as a grid-wide kernel.
+// Mapping to MI355X.  Only the order of the created ids matters, so a step's
+// new nodes take consecutive ids by a prefix sum over its covers: the ids are
+// then the output's, levels travel with the literals and the table's values,
+// and nothing is renumbered.  Which ANDs are roots is a property of their
+// fanout edges, so all covers are computed in one launch; roots that no
+// reached cover has as input are dropped by a cascade over the cover graph,
+// and a synchronous topological sweep gives the levels.  Both sweeps, and the
+// reconstruction of a level that fits its LDS, run in one persistent workgroup
+// per member of a batched arena (one in all for a single AIG): a step is bound
+// by the latency of its lookups, and the members do not depend on each other.
+// Other levels run each phase of a step as a grid-wide kernel.
 #include "gls_internal.h"
 #include "dev_common.h"
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_reduce.hpp>
+#include <rocprim/device/device_scan.hpp>
 #include <rocprim/device/device_select.hpp>
 #include <rocprim/iterator/counting_iterator.hpp>
 #include <algorithm>
@@ -48,13 +52,17 @@ constexpr int kB = 256;
 constexpr int BAL_STACK = 128;        // DFS_COVER_STACK_SIZE, balance.cu:18
 constexpr int BAL_MAX_COVER = 1024;   // MAX_LOCAL_COVER_SIZE, balance.cu:17
 constexpr int BAL_BATCH = 32768;      // iterLen, balance.cu:1129
-constexpr int BAL_WG = 1024;          // threads of the persistent reconstruction workgroup
-constexpr int COVER_THREADS = 16384;  // threads of a cover-discovery launch (each owns COVER_SCRATCH slots),
-constexpr int COVER_THREADS_MAX = 131072;   // scaled up to this with the graph (a level's frontier in one round)
+constexpr int BAL_WG = 1024;          // threads of the persistent workgroups
+constexpr int COVER_THREADS = 65536;  // most threads of a cover launch (each owns COVER_SCRATCH slots)
 // the size limit is checked before an expansion, so a cover can end up to a
 // few inputs above BAL_MAX_COVER: room for that
 constexpr int COVER_SCRATCH = BAL_MAX_COVER + 64;
-constexpr int COVER_LEVELS_PER_CHECK = 32;  // cover-discovery levels launched per host check
+constexpr int COVER_FAST = 16;        // first inputs of a cover, kept in LDS during its DFS
+// a frontier wider than this runs as grid-wide rounds, SWEEP_GRID_ROUNDS per
+// host check (a round costs about 1 us per 1024 covers in one workgroup, and
+// about 9 us as a launch)
+constexpr uint32_t SWEEP_WIDE = 8192;
+constexpr int SWEEP_GRID_ROUNDS = 8;
 constexpr uint32_t UNSET = 0xFFFFFFFFu;
 constexpr unsigned long long EMPTY64 = ~0ull;
 
@@ -62,129 +70,127 @@ inline int nblocks(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_
 
 __device__ __forceinline__ uint32_t culs_val(uint32_t l) { return l < 2u ? 1u - l : l; }
 
+// Literal and level of a signal, as one word.
+__device__ __forceinline__ unsigned long long sig(uint32_t lit, uint32_t lev) {
+    return (unsigned long long)lev << 32 | lit;
+}
+__device__ __forceinline__ uint32_t sig_lit(unsigned long long s) { return (uint32_t)s; }
+__device__ __forceinline__ uint32_t sig_lev(unsigned long long s) { return (uint32_t)(s >> 32); }
+
 // ---------------------------------------------------------------------------
-// hash tables (open addressing, linear probing; keys never removed)
+// table of created nodes: key lit0 << 32 | lit1 (lit0 < lit1) -> positive
+// literal and level of the node (open addressing, linear probing; slot s is
+// the words 2 s, 2 s + 1).  Written with atomics and read past the L1, so a
+// workgroup sees its own insertions after a wait and a barrier.
 // ---------------------------------------------------------------------------
-struct Tables {
-    unsigned long long *rk;   // reconstruct table: key (lit0 << 32 | lit1)
-    uint32_t *rv;             //   value: the node's id (smallest on a tie)
-    uint64_t rmask;
-    uint32_t *lk, *lv;        // level table: id -> level
-    uint64_t lmask;
+struct NodeTable {
+    unsigned long long *w;
+    uint64_t mask;
 };
 
-__device__ __forceinline__ uint32_t r_find(const Tables &t, unsigned long long key) {
-    for (uint64_t s = mix64(key) & t.rmask, probes = 0; probes <= t.rmask; s = (s + 1) & t.rmask, probes++) {
-        const unsigned long long k = __hip_atomic_load(&t.rk[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (k == key) return __hip_atomic_load(&t.rv[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (k == EMPTY64) return UNSET;
-    }
-    return UNSET;
+__device__ __forceinline__ unsigned long long t_word(const NodeTable &t, uint64_t i) {
+    return __hip_atomic_load(&t.w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// insert key with value val, keeping the smallest value; returns false if full
-__device__ __forceinline__ bool r_insert_min(const Tables &t, unsigned long long key, uint32_t val) {
-    for (uint64_t s = mix64(key) & t.rmask, probes = 0; probes <= t.rmask; s = (s + 1) & t.rmask, probes++) {
+// the node with this key, or EMPTY64; s and k: its first slot and the word there
+__device__ __forceinline__ unsigned long long t_find_from(const NodeTable &t, unsigned long long key, uint64_t s,
+                                                          unsigned long long k) {
+    for (uint64_t probes = 0; probes <= t.mask; probes++) {
+        if (k == key) return t_word(t, 2 * s + 1);
+        if (k == EMPTY64) return EMPTY64;
+        s = (s + 1) & t.mask;
+        k = t_word(t, 2 * s);
+    }
+    return EMPTY64;
+}
+
+// slot of the key, inserted if it is new; UNSET if the table is full
+__device__ __forceinline__ uint32_t t_slot(const NodeTable &t, unsigned long long key) {
+    uint64_t s = mix64(key) & t.mask;
+    for (uint64_t probes = 0; probes <= t.mask; probes++, s = (s + 1) & t.mask) {
         unsigned long long prev = EMPTY64;
-        __hip_atomic_compare_exchange_strong(&t.rk[s], &prev, key, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+        __hip_atomic_compare_exchange_strong(&t.w[2 * s], &prev, key, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT);
-        if (prev == EMPTY64 || prev == key) {
-            __hip_atomic_fetch_min(&t.rv[s], val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return true;
-        }
-    }
-    return false;
-}
-
-__device__ __forceinline__ bool l_insert(const Tables &t, uint32_t id, uint32_t lev) {
-    for (uint64_t s = mix64(id) & t.lmask, probes = 0; probes <= t.lmask; s = (s + 1) & t.lmask, probes++) {
-        uint32_t prev = UNSET;
-        __hip_atomic_compare_exchange_strong(&t.lk[s], &prev, id, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
-        if (prev == UNSET || prev == id) {
-            __hip_atomic_fetch_min(&t.lv[s], lev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return true;
-        }
-    }
-    return false;
-}
-
-__device__ __forceinline__ uint32_t l_find(const Tables &t, uint32_t id) {
-    for (uint64_t s = mix64(id) & t.lmask, probes = 0; probes <= t.lmask; s = (s + 1) & t.lmask, probes++) {
-        const uint32_t k = __hip_atomic_load(&t.lk[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (k == id) return __hip_atomic_load(&t.lv[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (k == UNSET) return UNSET;
+        if (prev == EMPTY64 || prev == key) return (uint32_t)s;
     }
     return UNSET;
 }
 
-// trivial AND rules (hash_table.h:435-449) in AIGER literals; UNSET if none
-__device__ __forceinline__ uint32_t and_trivial(uint32_t a, uint32_t b) {
-    if (a == b) return a;
-    if (a == (b ^ 1u)) return 0u;
-    if (a == 1u) return b;
-    if (b == 1u) return a;
-    if (a == 0u || b == 0u) return 0u;
-    return UNSET;
+// trivial AND rules (hash_table.h:435-449) in AIGER literals; EMPTY64 if none.
+// The result is one of the two signals or the constant (level 0).
+__device__ __forceinline__ unsigned long long and_trivial(unsigned long long a, unsigned long long b) {
+    const uint32_t x = sig_lit(a), y = sig_lit(b);
+    if (x == y) return a;
+    if (x == (y ^ 1u)) return 0ull;
+    if (x == 1u) return b;
+    if (y == 1u) return a;
+    if (x == 0u || y == 0u) return 0ull;
+    return EMPTY64;
 }
 
-// retrieveAndNode (balance.cu:87-111): trivial result, existing node, or UNSET
-__device__ __forceinline__ uint32_t and_lookup(const Tables &t, uint32_t a, uint32_t b) {
-    const uint32_t tr = and_trivial(a, b);
-    if (tr != UNSET) return tr;
-    if (a > b) { const uint32_t x = a; a = b; b = x; }
-    const uint32_t v = r_find(t, (unsigned long long)a << 32 | b);
-    return v == UNSET ? UNSET : 2u * v;
-}
-
-__device__ __forceinline__ uint32_t lit_level(const Tables &t, uint32_t lit, int32_t nPIs) {
-    const uint32_t id = lit >> 1;
-    if ((int32_t)id <= nPIs) return 0u;
-    const uint32_t l = l_find(t, id);
-    return l == UNSET ? 0u : l;
+__device__ __forceinline__ unsigned long long and_key_of(uint32_t x, uint32_t y) {
+    return x < y ? (unsigned long long)x << 32 | y : (unsigned long long)y << 32 | x;
 }
 
 // ---------------------------------------------------------------------------
 // phase 1: covers
 // ---------------------------------------------------------------------------
+enum : uint8_t { RM_STOP = 1, RM_PO = 2 };      // marks of a node: a complemented edge or a PO stops a cover there; a PO
+
 __global__ void k_fanouts(int32_t n, int32_t nPIs, const uint32_t *__restrict__ f0, const uint32_t *__restrict__ f1,
-                          int32_t nPOs, const uint32_t *__restrict__ pos, uint32_t *nFo) {
+                          int32_t nPOs, const uint32_t *__restrict__ pos, uint32_t *nFo, uint32_t *mark) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t v = nPIs + 1 + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += stride) {
-        atomicAdd(&nFo[LID(f0[v])], 1u);
-        atomicAdd(&nFo[LID(f1[v])], 1u);
+        const uint32_t a = f0[v], b = f1[v];
+        atomicAdd(&nFo[LID(a)], 1u);
+        atomicAdd(&nFo[LID(b)], 1u);
+        if (LC(a)) mark[LID(a)] = RM_STOP;
+        if (LC(b)) mark[LID(b)] = RM_STOP;
     }
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nPOs; i += stride)
         atomicAdd(&nFo[LID(pos[i])], 1u);
 }
 
-// first frontier: the AND nodes driving POs, each once
-__global__ void k_po_frontier(int32_t nPOs, int32_t nPIs, const uint32_t *__restrict__ pos, uint32_t *stamp,
-                              uint32_t *front, uint32_t *frontLen) {
+__global__ void k_po_marks(int32_t nPOs, const uint32_t *__restrict__ pos, uint32_t *mark) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nPOs; i += stride) {
-        const uint32_t id = LID(pos[i]);
-        const bool add = (int32_t)id > nPIs && atomicExch(&stamp[id], 1u) != 1u;
-        const uint32_t q = wave_append(frontLen, add);
-        if (add) front[q] = id;
-    }
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nPOs; i += stride)
+        mark[LID(pos[i])] = RM_STOP | RM_PO;
+}
+
+// The ANDs at which every cover that meets them stops: their covers are
+// needed if any cover or PO reaches them.
+__global__ void k_root_flags(int32_t n, int32_t nPIs, const uint32_t *__restrict__ nFo,
+                             const uint32_t *__restrict__ mark, uint8_t *flag) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += stride)
+        flag[v] = v > nPIs && (nFo[v] > 1u || mark[v] != 0u);
 }
 
 struct CoverArgs {
     const uint32_t *f0, *f1, *nFo;
     int32_t nPIs;
-    uint32_t *coverOff, *coverLen;   // coverLen UNSET: not computed
+    uint2 *cover;                    // per root: first input in pool, inputs
     uint32_t *pool, *poolNext;
     uint64_t poolCap;
     uint32_t *scratch;               // COVER_SCRATCH entries per thread
-    uint32_t *lastLevel, *stamp;
-    uint32_t *indeg;                 // parent covers of a root not yet taken by the topological sweep
+    uint8_t *isRoot;
+    uint32_t *indeg;                 // covers that have a root as input and are not yet taken by a sweep
+    uint32_t *extra, *extraLen;      // roots met at the stack / size limits
     uint32_t *err;                   // 1: cover pool full
+};
+
+// a cover's inputs during its DFS
+struct CoverIn {
+    uint32_t *fast;      // column of an LDS array [COVER_FAST][kB]
+    uint32_t *slow;
+    __device__ __forceinline__ uint32_t &operator[](uint32_t i) const {
+        return i < (uint32_t)COVER_FAST ? fast[i * kB] : slow[i];
+    }
 };
 
 // localCoverTravToTable (balance.cu:666-750) of root v into in[]; returns len
 // (0 = constant FALSE)
-__device__ uint32_t cover_dfs(const CoverArgs &a, uint32_t v, uint32_t *in) {
+__device__ uint32_t cover_dfs(const CoverArgs &a, uint32_t v, const CoverIn &in) {
     uint32_t stack[BAL_STACK];
     int top = -1;
     uint32_t len = 0;
@@ -211,123 +217,244 @@ __device__ uint32_t cover_dfs(const CoverArgs &a, uint32_t v, uint32_t *in) {
     return len;
 }
 
-// Root levels.  The reference sweeps levels from the POs, putting on level
-// L + 1 every AND input of a cover on level L (again on every level it is
-// reached on), and keeps for each root the last level it appeared on
-// (balance.cu:958-1037): a root's level is the length of the longest cover
-// path from a PO to it, and the number of levels is one more than the
-// longest.  Here each root is visited twice instead of once per path length:
-//   reach: a sweep from the POs in which each root is put on a frontier the
-//          first time it is seen; its cover is computed then, and each AND
-//          input of the cover counts one more parent cover;
-//   kahn:  a synchronous topological sweep of the cover graph: round 0 holds
-//          the roots without a parent cover (PO drivers), and a root goes on
-//          the next round's frontier when its last parent cover is taken.
-// A root taken in round L has its longest path from a PO equal to L.
-// flen[r] = size of round r's frontier, kept on the device so that several
-// rounds are launched per host check; round r's frontier is in
-// fronts[r & 1].
-__global__ void k_cover_reach(CoverArgs a, uint32_t *front0, uint32_t *front1, uint32_t *flen, uint32_t round) {
-    const uint32_t frontLen = flen[round];
-    const uint32_t *front = (round & 1u) ? front1 : front0;
-    uint32_t *next = (round & 1u) ? front0 : front1;
-    uint32_t *nextLen = &flen[round + 1];
+// The covers of the listed roots.
+__global__ void __launch_bounds__(kB) k_covers(CoverArgs a, uint32_t nList, const uint32_t *__restrict__ list) {
+    __shared__ uint32_t s_in[COVER_FAST * kB];
     const int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
-    uint32_t *in = a.scratch + (size_t)tid * COVER_SCRATCH;
+    const CoverIn in{s_in + threadIdx.x, a.scratch + (size_t)tid * COVER_SCRATCH};
     const int64_t lane = threadIdx.x & 63;
     // the wavefront runs the same number of iterations (its first lane's
     // index decides), so the pool reservation sees all 64 lanes
-    for (int64_t k = tid; k - lane < (int64_t)frontLen; k += stride) {
-        const bool has = k < (int64_t)frontLen;
-        const uint32_t v = has ? front[k] : 0u;
+    for (int64_t k = tid; k - lane < (int64_t)nList; k += stride) {
+        const bool has = k < (int64_t)nList;
+        const uint32_t v = has ? list[k] : 0u;
         const uint32_t len = has ? cover_dfs(a, v, in) : 0u;
         const uint32_t off = wave_reserve(a.poolNext, len);
         if (!has) continue;
         if ((uint64_t)off + len > a.poolCap) {
             atomicOr(a.err, 1u);
-            a.coverLen[v] = 0;
+            a.cover[v] = make_uint2(0u, 0u);
             continue;
         }
         for (uint32_t i = 0; i < len; i++) {
             const uint32_t lit = in[i], id = lit >> 1;
             a.pool[off + i] = lit;
-            bool add = false;
             if ((int32_t)id > a.nPIs) {
                 atomicAdd(&a.indeg[id], 1u);
-                add = atomicExch(&a.stamp[id], 1u) != 1u;
+                // an AND that is no root by its edges: a limit cut the cover there
+                if (a.isRoot[id] == 0) {
+                    uint32_t *word = reinterpret_cast<uint32_t *>(a.isRoot + (id & ~3u));
+                    const uint32_t bit = 1u << (8u * (id & 3u));
+                    if (!(atomicOr(word, bit) & bit)) a.extra[atomicAdd(a.extraLen, 1u)] = id;
+                }
             }
-            const uint32_t q = wave_append(nextLen, add);
-            if (add) next[q] = id;
         }
-        a.coverOff[v] = off;
-        a.coverLen[v] = len;
+        a.cover[v] = make_uint2(off, len);
     }
 }
 
-// round 0 of the topological sweep: the PO drivers that no cover has as input
-__global__ void k_kahn_first(int32_t nPOs, int32_t nPIs, const uint32_t *__restrict__ pos,
-                             const uint32_t *__restrict__ indeg, uint32_t *stamp, uint32_t *front,
-                             uint32_t *frontLen) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nPOs; i += stride) {
-        const uint32_t id = LID(pos[i]);
-        const bool add = (int32_t)id > nPIs && indeg[id] == 0u && atomicExch(&stamp[id], 2u) != 2u;
-        const uint32_t q = wave_append(frontLen, add);
-        if (add) front[q] = id;
+// ---- sweeps over the cover graph.  A sweep starts from the listed roots
+// without a parent cover and takes a root when its last parent cover is taken:
+//   drop: from the roots that no PO drives; they are unreached (a constant
+//         cover has no inputs, and dangling logic no PO);
+//   levels: from the PO drivers; a root taken in round L has its longest path
+//         from a PO equal to L, which is the last level the reference's
+//         sweep puts it on (again on every level it is reached on,
+//         balance.cu:958-1037).
+struct SweepArgs {
+    const uint2 *cover;
+    const uint32_t *pool;
+    int32_t nPIs;
+    const uint32_t *mark;
+    uint32_t *indeg;
+    uint32_t *lastLevel;             // round of a taken root; UNSET, or DROPPED
+    uint32_t *front[2];              // round r's frontier, in front[r & 1] from the segment's first root
+    uint32_t drop;
+};
+constexpr uint32_t DROPPED = 0xFFFFFFFEu;
+
+// Takes root v; add(id, want) appends an input that it was the last parent of
+// (called with want false too: appends go by wavefront).
+template <class Add>
+__device__ __forceinline__ void sweep_take(const SweepArgs &a, bool has, uint32_t v, uint32_t round, Add add) {
+    uint2 c = make_uint2(0u, 0u);
+    if (has) {
+        a.lastLevel[v] = a.drop ? DROPPED : round;
+        c = a.cover[v];
+    }
+    for (uint32_t i = 0; __ballot(i < c.y) != 0; i++) {
+        bool want = false;
+        uint32_t id = 0;
+        if (i < c.y) {
+            id = a.pool[c.x + i] >> 1;
+            want = (int32_t)id > a.nPIs && atomicSub(&a.indeg[id], 1u) == 1u && !(a.drop && (a.mark[id] & RM_PO));
+        }
+        add(id, want);
     }
 }
 
-__global__ void k_cover_kahn(CoverArgs a, uint32_t *front0, uint32_t *front1, uint32_t *flen, uint32_t round) {
-    const uint32_t frontLen = flen[round];
-    const uint32_t *front = (round & 1u) ? front1 : front0;
-    uint32_t *next = (round & 1u) ? front0 : front1;
-    uint32_t *nextLen = &flen[round + 1];
+// round 0 of a sweep
+__global__ void k_sweep_first(uint32_t nRoots, const uint32_t *__restrict__ roots, SweepArgs a,
+                              const uint32_t *__restrict__ tag, const uint32_t *__restrict__ segFirst,
+                              uint32_t *segLen) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < frontLen; k += stride) {
-        const uint32_t v = front[k];
-        a.lastLevel[v] = round;
-        const uint32_t len = a.coverLen[v], off = a.coverOff[v];
-        for (uint32_t i = 0; i < len; i++) {
-            const uint32_t id = a.pool[off + i] >> 1;
-            const bool add = (int32_t)id > a.nPIs && atomicSub(&a.indeg[id], 1u) == 1u;
-            const uint32_t q = wave_append(nextLen, add);
-            if (add) next[q] = id;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i - (threadIdx.x & 63) < (int64_t)nRoots;
+         i += stride) {
+        const bool has = i < (int64_t)nRoots;
+        const uint32_t v = has ? roots[i] : 0u;
+        const bool want = has && a.indeg[v] == 0u && a.lastLevel[v] == UNSET && ((a.mark[v] & RM_PO) == 0) == (a.drop != 0);
+        if (tag) {
+            if (want) {
+                const uint32_t s = tag[v];
+                a.front[0][segFirst[s] + atomicAdd(&segLen[s], 1u)] = v;
+            }
+        } else {
+            const uint32_t q = wave_append(segLen, want);
+            if (want) a.front[0][q] = v;
         }
     }
 }
 
-__global__ void k_root_flags(int32_t n, const uint32_t *__restrict__ lastLevel, uint8_t *flag) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += stride)
-        flag[v] = lastLevel[v] != UNSET;
+// One workgroup per segment: rounds until the frontier is empty (or, for a
+// single segment, wider than `wide`).  segLen: the frontier's size, in and
+// out; segRound: rounds done.
+__global__ void __launch_bounds__(BAL_WG) k_sweep_wg(SweepArgs a, const uint32_t *__restrict__ segFirst,
+                                                     uint32_t *segLen, uint32_t *segRound, uint32_t wide) {
+    __shared__ uint32_t s_next;
+    const uint32_t seg = blockIdx.x, base = segFirst[seg], tid = threadIdx.x;
+    uint32_t round = segRound[seg], cur = segLen[seg];
+    while (cur != 0 && cur <= wide) {
+        if (tid == 0) s_next = 0;
+        __syncthreads();
+        const uint32_t *front = a.front[round & 1u] + base;
+        uint32_t *next = a.front[(round & 1u) ^ 1u] + base;
+        for (uint32_t k = tid; k - (tid & 63u) < cur; k += BAL_WG) {
+            const bool has = k < cur;
+            sweep_take(a, has, has ? front[k] : 0u, round, [&](uint32_t id, bool want) {
+                const uint32_t q = wave_append(&s_next, want);
+                if (want) next[q] = id;
+            });
+        }
+        __syncthreads();
+        cur = s_next;
+        round++;
+        __syncthreads();
+    }
+    if (tid == 0) {
+        segLen[seg] = cur;
+        segRound[seg] = round;
+    }
 }
 
-__global__ void k_gather_level(int32_t m, const uint32_t *__restrict__ ids, const uint32_t *__restrict__ lastLevel,
-                               uint32_t *keys) {
+// One grid-wide round: len[0] the frontier's size, len[1] collects the next
+// one's (cleared by the host's batch).
+__global__ void k_sweep_grid(SweepArgs a, uint32_t round, uint32_t *len) {
+    const uint32_t cur = len[0];
+    const uint32_t *front = a.front[round & 1u];
+    uint32_t *next = a.front[(round & 1u) ^ 1u];
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m; i += stride) keys[i] = lastLevel[ids[i]];
+    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k - (threadIdx.x & 63) < (int64_t)cur; k += stride) {
+        const bool has = k < (int64_t)cur;
+        sweep_take(a, has, has ? front[k] : 0u, round, [&](uint32_t id, bool want) {
+            const uint32_t q = wave_append(&len[1], want);
+            if (want) next[q] = id;
+        });
+    }
+}
+
+__global__ void k_taken_flags(int32_t n, const uint32_t *__restrict__ lastLevel, uint8_t *flag) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += stride) flag[v] = lastLevel[v] < DROPPED;
+}
+
+__global__ void __launch_bounds__(kBlock) k_count_tags(uint32_t m, const uint32_t *__restrict__ roots,
+                                                       const uint32_t *__restrict__ tag, uint32_t *cnt) {
+    __shared__ uint32_t s_bins[TAG_BINS];
+    TagBins tb{s_bins};
+    tb.init();
+    int64_t b, e;
+    tag_chunk(0, m, b, e);
+    for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) tb.add(cnt, tag[roots[i]], 1u);
+    tb.flush_add(cnt, 0xFFFFFFFFu);
+}
+
+// sort key of every root: its level, after the levels of the segments before
+// its own (levOff) where they are given
+__global__ void k_level_keys(uint32_t m, const uint32_t *__restrict__ roots, const uint32_t *__restrict__ lastLevel,
+                             const uint32_t *__restrict__ tag, const uint32_t *__restrict__ levOff, uint32_t *keys) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m; i += stride)
+        keys[i] = lastLevel[roots[i]] + (levOff ? levOff[tag[roots[i]]] : 0u);
+}
+
+// first position of every key (each occurs), and one past the last
+__global__ void k_key_starts(uint32_t m, const uint32_t *__restrict__ keys, uint32_t nKeys, uint32_t *starts) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= m; i += stride) {
+        if (i == m) starts[nKeys] = m;
+        else if (i == 0 || keys[i] != keys[i - 1]) starts[keys[i]] = (uint32_t)i;
+    }
+}
+
+// every cover's inputs, and the most ANDs it can create (none from a constant)
+__global__ void k_cover_lens(uint32_t m, const uint32_t *__restrict__ roots, const uint2 *__restrict__ cover,
+                             uint32_t *len, uint32_t *most) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= m; i += stride) {
+        const uint32_t k = i < m ? cover[roots[i]].y : 0u;
+        len[i] = k;
+        most[i] = k ? k - 1u : 0u;
+    }
+}
+
+// the covers' inputs in the order in which they are rebuilt
+__global__ void k_pack_inputs(uint32_t m, const uint32_t *__restrict__ roots, const uint2 *__restrict__ cover,
+                              const uint32_t *__restrict__ pool, const uint32_t *__restrict__ off, uint32_t *in) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m; i += stride) {
+        const uint2 c = cover[roots[i]];
+        for (uint32_t j = 0; j < c.y; j++) in[off[i] + j] = pool[c.x + j];
+    }
+}
+
+// largest level: covers, inputs, ANDs it can create; and per level the inputs
+// and the ANDs
+__global__ void k_level_sizes(uint32_t nKeys, const uint32_t *__restrict__ starts, const uint32_t *__restrict__ off,
+                              const uint32_t *__restrict__ newOff, uint2 *levSize, uint32_t *most) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < nKeys; k += stride) {
+        const uint32_t a = starts[k], b = starts[k + 1];
+        const uint2 z = make_uint2(off[b] - off[a], newOff[b] - newOff[a]);
+        levSize[k] = z;
+        atomicMax(&most[0], b - a);
+        atomicMax(&most[1], z.x);
+        atomicMax(&most[2], z.y);
+    }
 }
 
 // ---------------------------------------------------------------------------
 // phase 2: reconstruction
 // ---------------------------------------------------------------------------
 struct RecArgs {
-    Tables t;
+    NodeTable t;
     int32_t nPIs;
-    const uint32_t *roots;            // roots by (level, id)
-    const uint32_t *coverOff, *coverLen, *pool;
-    uint32_t *newLit;                 // per root id
-    uint32_t *arr, *alv;              // batch workspace: maxLen entries per cover
-    uint32_t *alen;
-    uint32_t maxLen;
-    uint8_t *mask;
-    unsigned long long *skey;
-    uint32_t *sval, *slev;
-    uint32_t *counter;                // [0] next tentative id, [1] step max, [2] any, [3] created
+    const uint32_t *roots;            // roots by (segment, level, id)
+    const uint32_t *off, *in;         // their covers' inputs
+    const uint2 *levSize;             // per (segment, level): inputs, ANDs it can create
+    const uint32_t *starts;           // first root of every (segment, level)
+    unsigned long long *newSig;       // per root id: the result
+    uint32_t *of0, *of1;              // fanins of the created nodes, by id
+    uint32_t *tagOut;                 // optional: their tags
+    const uint32_t *tagIn;
     uint32_t *err;                    // 2: table full
-    const uint32_t *tagIn;            // optional: per-node tag of the input (batched balance)
-    Tables tagTab;                    // created id -> tag of the cover that made it
     uint32_t shuffle;                 // 1: `b -s` input order (sortDecId = 0)
+    // grid-wide phases: a batch's covers and their state
+    unsigned long long *arr;          // inputs, packed as in `in` from the batch's first
+    uint32_t *alen;
+    uint8_t *mask;
+    unsigned long long *skey, *sres;
+    uint32_t *slot, *bcnt;
+    uint32_t *counter;                // next id, alternating between two words by step
 };
 
 // thrust::shuffle(thrust::seq, ..., default_random_engine(seed)) as an index
@@ -371,298 +498,448 @@ struct ThrustShuffle {
     }
 };
 
-__device__ __forceinline__ void rec_tag(const RecArgs &r, uint32_t c, uint32_t root) {
-    if (r.tagIn && r.mask[c] == 1 && !l_insert(r.tagTab, r.sval[c], r.tagIn[root])) atomicOr(r.err, 2u);
+// the input before which another one stands: level descending, then (`b`) the
+// reference's literal value descending; equal ones keep their order
+__device__ __forceinline__ bool sorts_before(uint32_t shuffle, unsigned long long a, unsigned long long b) {
+    if (sig_lev(a) != sig_lev(b)) return sig_lev(a) > sig_lev(b);
+    return !shuffle && culs_val(sig_lit(a)) > culs_val(sig_lit(b));
 }
 
-// prepareReconstructArrays (balance.cu:272-427), one cover
-__device__ void rec_gather(const RecArgs &r, uint32_t c, uint32_t root) {
-    uint32_t *A = r.arr + (size_t)c * r.maxLen, *LV = r.alv + (size_t)c * r.maxLen;
-    const uint32_t len = r.coverLen[root], off = r.coverOff[root];
-    r.alen[c] = len;
-    auto put = [&](uint32_t k, uint32_t src) {
-        const uint32_t lit = r.pool[off + src], id = lit >> 1;
-        const uint32_t nl = (int32_t)id <= r.nPIs ? lit : (r.newLit[id] ^ (lit & 1u));
-        A[k] = nl;
-        LV[k] = lit_level(r.t, nl, r.nPIs);
-    };
-    if (r.shuffle) {
-        // `b -s`: the inputs in the order of the shuffle seeded with the
-        // cover's index in its batch
-        if (len > 0) {
-            const ThrustShuffle sh(len, c);
-            uint32_t k = 0;
-            for (uint32_t j = 0; j < sh.span && k < len; j++) {
-                const uint32_t src = sh(j);
-                if (src < len) put(k++, src);
-            }
-        }
-    } else {
-        for (uint32_t i = 0; i < len; i++) put(i, i);
-    }
-    // level descending, then (`b`) the reference's literal value descending;
-    // insertion sort keeps equal keys in order, as thrust's sequential sort does
-    for (uint32_t i = 1; i < len; i++) {
-        const uint32_t x = A[i], xl = LV[i];
-        int j = (int)i - 1;
-        while (j >= 0 && (LV[j] < xl || (!r.shuffle && LV[j] == xl && culs_val(A[j]) < culs_val(x)))) {
-            A[j + 1] = A[j];
-            LV[j + 1] = LV[j];
-            j--;
-        }
-        A[j + 1] = x;
-        LV[j + 1] = xl;
-    }
+__device__ __forceinline__ unsigned long long input_sig(const RecArgs &r, uint32_t lit) {
+    const uint32_t id = lit >> 1;
+    return (int32_t)id <= r.nPIs ? sig(lit, 0u) : r.newSig[id] ^ (lit & 1u);
 }
 
-// sharedNodeDrivenPermute then prepareDataToInsert, one cover; returns mask
-__device__ uint32_t rec_prepare(const RecArgs &r, uint32_t c, uint32_t counter) {
-    uint32_t *A = r.arr + (size_t)c * r.maxLen, *LV = r.alv + (size_t)c * r.maxLen;
-    const uint32_t L = r.alen[c];
-    if (L <= 1) { r.mask[c] = 0; return 0; }
-    int left;
-    if (L < 3) {
-        left = 0;
-    } else {
-        left = (int)L - 2;
-        const uint32_t border = LV[left];
-        for (left--; left >= 0; left--)
-            if (LV[left] != border) break;
-        left++;
-    }
-    const int right = (int)L - 2;
-    if (left < right) {
-        const uint32_t l1 = A[right + 1], l2 = A[right];
-        for (int i = right; i >= left; i--) {
-            const uint32_t l3 = A[i];
-            if (and_lookup(r.t, l1, l3) != UNSET) {
-                if (l3 != l2) {
-                    A[i] = l2;
-                    A[right] = l3;
-                    const uint32_t tl = LV[i];
-                    LV[i] = LV[right];
-                    LV[right] = tl;
+// ---- one workgroup per segment, levels within its LDS
+constexpr uint32_t LT_INPUTS = 4096;      // inputs of a level
+constexpr uint32_t LT_COVERS = 2048;      // covers of a level
+constexpr uint32_t LT_NEW = 3072;         // ANDs that a level can create
+constexpr uint32_t LT_HASH = 4096;        // entries of the level's own node table
+constexpr uint32_t LN_FINAL = 0x80000000u;
+
+// Rebuilds levels lFirst, lFirst - 1, .., lLast of its segment (levOff: the
+// segments' first levels in starts; levels beyond the segment's are skipped).
+// A level's cover inputs, sorted by rank among the cover's, and the nodes it
+// creates live in LDS; the table in memory holds the nodes of the levels
+// before and takes this level's at its end, so a pair with a literal of this
+// level is looked up in LDS only.  The candidates of the permutation are looked
+// up four at a time.  Per step three barriers: keys inserted; winners (the
+// smallest cover index of a key) counted; ids given.
+// What bounds it: a level costs three dependent trips to memory (inputs,
+// their results, lookups) and the insertions, and a step some LDS trips,
+// whatever the number of covers; measured before: 83 us per level of 675
+// covers and six steps with all state and every lookup in memory.
+__global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *__restrict__ levOff,
+                                                    const uint32_t *__restrict__ idBase, uint32_t *made, int32_t lFirst,
+                                                    int32_t lLast) {
+    __shared__ unsigned long long s_key[LT_HASH];
+    __shared__ uint32_t s_val[LT_HASH];              // smallest cover index, then LN_FINAL | node of the level
+    __shared__ unsigned long long s_arr[LT_INPUTS];  // the covers' current inputs
+    __shared__ uint32_t s_nlev[LT_NEW];
+    __shared__ uint16_t s_cov[LT_INPUTS], s_off[LT_COVERS + 1], s_len[LT_COVERS], s_slot[LT_COVERS];
+    __shared__ uint32_t s_wcnt[2][BAL_WG / 64];
+    const uint32_t tid = threadIdx.x, seg = blockIdx.x, wave = tid >> 6, lane = tid & 63u;
+    const uint32_t lev0 = levOff[seg], nLev = levOff[seg + 1] - lev0, base0 = idBase[seg];
+    uint32_t counter = base0 + made[seg];            // next id
+    for (int32_t l = min(lFirst, (int32_t)nLev - 1); l >= lLast; l--) {
+        const uint32_t s = r.starts[lev0 + l], nb = r.starts[lev0 + l + 1] - s;
+        const uint32_t in0 = r.off[s], T = r.off[s + nb] - in0;
+        const uint32_t levBase = counter;
+        // a power of two with room for every AND the level can create (LT_NEW at most)
+        const uint32_t most = r.levSize[lev0 + l].y;
+        uint32_t hsize = 256;
+        while (hsize < LT_HASH && hsize < 2u * most) hsize <<= 1;
+        // covers' ranges, and every input's cover
+        for (uint32_t c = tid; c < nb; c += BAL_WG) {
+            const uint32_t o = r.off[s + c] - in0, e = r.off[s + c + 1] - in0;
+            s_off[c] = (uint16_t)o;
+            s_len[c] = (uint16_t)(e - o);
+            for (uint32_t j = o; j < e; j++) s_cov[j] = (uint16_t)c;
+            if (r.shuffle && e > o) {
+                // `b -s`: the inputs in the order of the shuffle seeded with
+                // the cover's index in its batch
+                const ThrustShuffle sh(e - o, c);
+                uint32_t k = o;
+                for (uint32_t j = 0; j < sh.span && k < e; j++) {
+                    const uint32_t src = sh(j);
+                    if (src < e - o) s_arr[k++] = input_sig(r, r.in[in0 + o + src]);
                 }
-                break;
             }
         }
-    }
-    uint32_t l1 = A[L - 1], l2 = A[L - 2];
-    const uint32_t v1 = LV[L - 1], v2 = LV[L - 2];
-    r.alen[c] = L - 2;
-    const uint32_t found = and_lookup(r.t, l1, l2);
-    if (found != UNSET) {
-        r.mask[c] = 2;
-        r.sval[c] = found;
-        r.slev[c] = lit_level(r.t, found, r.nPIs);
-        return 2;
-    }
-    if (l1 > l2) { const uint32_t x = l1; l1 = l2; l2 = x; }
-    r.mask[c] = 1;
-    r.skey[c] = (unsigned long long)l1 << 32 | l2;
-    r.sval[c] = counter + c;
-    r.slev[c] = (v1 > v2 ? v1 : v2) + 1u;
-    return 1;
-}
-
-// addBackLocalArrays (balance.cu:429-467), one cover
-__device__ void rec_add_back(const RecArgs &r, uint32_t c) {
-    const uint8_t m = r.mask[c];
-    if (m == 0) return;
-    uint32_t *A = r.arr + (size_t)c * r.maxLen, *LV = r.alv + (size_t)c * r.maxLen;
-    const uint32_t lit = m == 2 ? r.sval[c] : 2u * r.sval[c];
-    const uint32_t L = r.alen[c];
-    for (uint32_t i = 0; i < L; i++)
-        if (A[i] == lit) return;
-    A[L] = lit;
-    LV[L] = r.slev[c];
-    r.alen[c] = L + 1;
-    for (uint32_t i = L; i > 0; i--) {
-        if (LV[i] <= LV[i - 1]) break;
-        const uint32_t x = A[i];
-        A[i] = A[i - 1];
-        A[i - 1] = x;
-        const uint32_t y = LV[i];
-        LV[i] = LV[i - 1];
-        LV[i - 1] = y;
-    }
-}
-
-__device__ __forceinline__ void rec_record(const RecArgs &r, uint32_t c, uint32_t root) {
-    r.newLit[root] = r.alen[c] == 0 ? 0u : r.arr[(size_t)c * r.maxLen];
-}
-
-// The persistent workgroup: levels [lFirst .. lLast] (descending), every one
-// at most balance_narrow_max covers wide; starts[l] = first index of level l
-// in roots.
-__global__ void __launch_bounds__(BAL_WG) k_rec_narrow(RecArgs r, const uint32_t *__restrict__ starts, int32_t lFirst,
-                                                       int32_t lLast) {
-    __shared__ uint32_t s_any, s_max, s_counter;
-    const uint32_t tid = threadIdx.x;
-    if (tid == 0) s_counter = __hip_atomic_load(&r.counter[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int32_t l = lFirst; l >= lLast; l--) {
-        const uint32_t s = starts[l], nb = starts[l + 1] - s;
-        for (uint32_t c = tid; c < nb; c += BAL_WG) rec_gather(r, c, r.roots[s + c]);
+        if (tid == 0) s_off[nb] = (uint16_t)T;
+        for (uint32_t i = tid; i < hsize; i += BAL_WG) { s_key[i] = EMPTY64; s_val[i] = UNSET; }
+        unsigned long long mine[LT_INPUTS / BAL_WG];
+        if (!r.shuffle) {
+#pragma unroll
+            for (uint32_t q = 0; q < LT_INPUTS / BAL_WG; q++) {
+                const uint32_t i = tid + q * BAL_WG;
+                mine[q] = i < T ? input_sig(r, r.in[in0 + i]) : 0ull;
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < LT_INPUTS / BAL_WG; q++)
+                if (tid + q * BAL_WG < T) s_arr[tid + q * BAL_WG] = mine[q];
+        }
         __syncthreads();
+        // each input's place in its cover's order
+        uint32_t place[LT_INPUTS / BAL_WG];
+#pragma unroll
+        for (uint32_t q = 0; q < LT_INPUTS / BAL_WG; q++) {
+            const uint32_t i = tid + q * BAL_WG;
+            place[q] = i;
+            if (i < T) {
+                if (r.shuffle) mine[q] = s_arr[i];
+                const uint32_t c = s_cov[i], o = s_off[c], e = s_off[c + 1];
+                uint32_t p = o;
+                for (uint32_t j = o; j < e; j++) {
+                    const unsigned long long x = s_arr[j];
+                    p += (sorts_before(r.shuffle, x, mine[q]) || (j < i && !sorts_before(r.shuffle, mine[q], x))) ? 1u : 0u;
+                }
+                place[q] = p;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t q = 0; q < LT_INPUTS / BAL_WG; q++)
+            if (tid + q * BAL_WG < T) s_arr[place[q]] = mine[q];
+        __syncthreads();
+        // a node of this level with this key, or EMPTY64
+        auto level_find = [&](unsigned long long key) -> unsigned long long {
+            for (uint32_t h = (uint32_t)mix64(key) & (hsize - 1);; h = (h + 1) & (hsize - 1)) {
+                const unsigned long long k = *(volatile unsigned long long *)&s_key[h];
+                if (k == EMPTY64) return EMPTY64;
+                if (k != key) continue;
+                const uint32_t v = *(volatile uint32_t *)&s_val[h];
+                // inserted in this step: not there yet
+                if (v == UNSET || !(v & LN_FINAL)) return EMPTY64;
+                return sig(2u * (levBase + (v & ~LN_FINAL)), s_nlev[v & ~LN_FINAL]);
+            }
+        };
+        // addBackLocalArrays (balance.cu:429-467)
+        auto add_back = [&](uint32_t c, unsigned long long x) {
+            const uint32_t o = s_off[c], L = s_len[c];
+            for (uint32_t i = 0; i < L; i++)
+                if (sig_lit(s_arr[o + i]) == sig_lit(x)) return;
+            uint32_t i = L;
+            while (i > 0 && sig_lev(x) > sig_lev(s_arr[o + i - 1])) {
+                s_arr[o + i] = s_arr[o + i - 1];
+                i--;
+            }
+            s_arr[o + i] = x;
+            s_len[c] = (uint16_t)(L + 1);
+        };
         for (;;) {
-            if (tid == 0) { s_any = 0; s_max = 0; }
+            // sharedNodeDrivenPermute and prepareDataToInsert (balance.cu:113-247)
+            int active = 0;
+            for (uint32_t c = tid; c < nb; c += BAL_WG) {
+                const uint32_t o = s_off[c], L = s_len[c];
+                s_slot[c] = 0;
+                if (L <= 1) continue;
+                active = 1;
+                const int right = (int)L - 2;
+                int left = right;
+                const uint32_t border = sig_lev(s_arr[o + right]);
+                while (left > 0 && sig_lev(s_arr[o + left - 1]) == border) left--;
+                const unsigned long long l1 = s_arr[o + L - 1], l2 = s_arr[o + right];
+                const uint32_t x1 = sig_lit(l1);
+                const bool old1 = (x1 >> 1) < levBase;
+                unsigned long long found = EMPTY64;
+                for (int i = right; i >= left && found == EMPTY64; i -= 4) {
+                    unsigned long long l3[4], key[4], k0[4];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        l3[q] = i - q >= left ? s_arr[o + i - q] : l1;
+                        key[q] = and_key_of(x1, sig_lit(l3[q]));
+                        const bool old = old1 && (sig_lit(l3[q]) >> 1) < levBase && i - q >= left;
+                        k0[q] = old ? t_word(r.t, 2 * (mix64(key[q]) & r.t.mask)) : EMPTY64;
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        if (found != EMPTY64 || i - q < left) continue;
+                        unsigned long long f = and_trivial(l1, l3[q]);
+                        if (f == EMPTY64) f = level_find(key[q]);
+                        if (f == EMPTY64 && k0[q] != EMPTY64)
+                            f = t_find_from(r.t, key[q], mix64(key[q]) & r.t.mask, k0[q]);
+                        if (f == EMPTY64) continue;
+                        found = f;
+                        // the partner goes next to last; the order by level stays
+                        s_arr[o + i - q] = l2;
+                    }
+                }
+                s_len[c] = (uint16_t)(L - 2);
+                if (found != EMPTY64) {
+                    add_back(c, found);
+                    continue;
+                }
+                const unsigned long long key = and_key_of(x1, sig_lit(l2));
+                const uint32_t lv = (sig_lev(l1) > sig_lev(l2) ? sig_lev(l1) : sig_lev(l2)) + 1u;
+                uint32_t h = (uint32_t)mix64(key) & (hsize - 1);
+                for (;; h = (h + 1) & (hsize - 1)) {
+                    unsigned long long prev = EMPTY64;
+                    __hip_atomic_compare_exchange_strong(&s_key[h], &prev, key, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_WORKGROUP);
+                    if (prev == EMPTY64 || prev == key) break;
+                }
+                atomicMin(&s_val[h], c);
+                s_slot[c] = (uint16_t)(h + 1);
+                s_arr[o + L - 1] = key;                  // the popped pair, and its level
+                s_arr[o + right] = lv;
+            }
+            if (!__syncthreads_or(active)) break;
+            // winners, counted in cover order
+            uint32_t rank[LT_COVERS / BAL_WG];
+#pragma unroll
+            for (uint32_t q = 0; q < LT_COVERS / BAL_WG; q++) {
+                const uint32_t c = tid + q * BAL_WG;
+                const bool win = c < nb && s_slot[c] != 0 && s_val[s_slot[c] - 1] == c;
+                const uint64_t m = __ballot(win);
+                rank[q] = win ? (uint32_t)__popcll(m & ((1ull << lane) - 1ull)) : UNSET;
+                if (lane == 0) s_wcnt[q][wave] = (uint32_t)__popcll(m);
+            }
             __syncthreads();
-            const uint32_t counter = s_counter;
-            bool any = false;
-            for (uint32_t c = tid; c < nb; c += BAL_WG) any |= rec_prepare(r, c, counter) != 0;
-            if (any) atomicOr(&s_any, 1u);
+            uint32_t total = 0;
+#pragma unroll
+            for (uint32_t q = 0; q < LT_COVERS / BAL_WG; q++) {
+                uint32_t before = total;
+                for (uint32_t w = 0; w < BAL_WG / 64; w++) {
+                    const uint32_t x = s_wcnt[q][w];
+                    before += w < wave ? x : 0u;
+                    total += x;
+                }
+                if (rank[q] != UNSET) {
+                    const uint32_t c = tid + q * BAL_WG, o = s_off[c], L = s_len[c];
+                    const uint32_t id = counter + before + rank[q];
+                    const unsigned long long key = s_arr[o + L + 1];
+                    s_nlev[id - levBase] = (uint32_t)s_arr[o + L];
+                    s_val[s_slot[c] - 1] = LN_FINAL | (id - levBase);
+                    r.of0[id] = (uint32_t)(key >> 32);
+                    r.of1[id] = (uint32_t)key;
+                    if (r.tagOut) r.tagOut[id] = r.tagIn[r.roots[s + c]];
+                }
+            }
+            counter += total;
             __syncthreads();
-            if (!s_any) break;
             for (uint32_t c = tid; c < nb; c += BAL_WG)
-                if (r.mask[c] == 1 && !r_insert_min(r.t, r.skey[c], r.sval[c])) atomicOr(r.err, 2u);
-            __syncthreads();
-            uint32_t mx = 0;
-            for (uint32_t c = tid; c < nb; c += BAL_WG) {
-                if (r.mask[c] != 1) continue;
-                const uint32_t got = r_find(r.t, r.skey[c]);
-                if (got == r.sval[c]) atomicAdd(&r.counter[3], 1u);
-                r.sval[c] = got;
-                mx = got > mx ? got : mx;
-            }
-            if (mx) atomicMax(&s_max, mx);
-            __syncthreads();
-            if (tid == 0 && s_max) s_counter = s_max + 1u;
-            for (uint32_t c = tid; c < nb; c += BAL_WG) {
-                if (r.mask[c] == 1 && !l_insert(r.t, r.sval[c], r.slev[c])) atomicOr(r.err, 2u);
-                rec_tag(r, c, r.roots[s + c]);
-                rec_add_back(r, c);
-            }
-            __syncthreads();
+                if (s_slot[c] != 0) {
+                    const uint32_t v = s_val[s_slot[c] - 1] & ~LN_FINAL;
+                    add_back(c, sig(2u * (levBase + v), s_nlev[v]));
+                }
         }
-        for (uint32_t c = tid; c < nb; c += BAL_WG) rec_record(r, c, r.roots[s + c]);
+        // results, and this level's nodes into the table
+        for (uint32_t c = tid; c < nb; c += BAL_WG)
+            r.newSig[r.roots[s + c]] = s_len[c] == 0 ? 0ull : s_arr[s_off[c]];
+        for (uint32_t i = tid; i < hsize; i += BAL_WG) {
+            const unsigned long long key = s_key[i];
+            if (key == EMPTY64) continue;
+            const uint32_t v = s_val[i] & ~LN_FINAL;
+            const uint32_t slot = t_slot(r.t, key);
+            if (slot == UNSET) { atomicOr(r.err, 2u); continue; }
+            __hip_atomic_store(&r.t.w[2 * (size_t)slot + 1], sig(2u * (levBase + v), s_nlev[v]), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);     // vmcnt(0): the table's words are written
         __syncthreads();
     }
-    if (tid == 0) __hip_atomic_store(&r.counter[0], s_counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) made[seg] = counter - base0;
 }
 
-// wide levels: one kernel per phase
+// ---- wide levels: a batch of covers, one kernel per phase of a step
+
+// prepareReconstructArrays (balance.cu:272-427)
 __global__ void k_rec_gather(RecArgs r, uint32_t s, uint32_t nb) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nb; c += stride)
-        rec_gather(r, (uint32_t)c, r.roots[s + c]);
+    const uint32_t in0 = r.off[s];
+    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nb; c += stride) {
+        const uint32_t o = r.off[s + c], len = r.off[s + c + 1] - o;
+        unsigned long long *A = r.arr + (o - in0);
+        r.alen[c] = len;
+        if (r.shuffle) {
+            // `b -s`: the inputs in the order of the shuffle seeded with the
+            // cover's index in its batch
+            if (len > 0) {
+                const ThrustShuffle sh(len, (uint32_t)c);
+                uint32_t k = 0;
+                for (uint32_t j = 0; j < sh.span && k < len; j++) {
+                    const uint32_t src = sh(j);
+                    if (src < len) A[k++] = input_sig(r, r.in[o + src]);
+                }
+            }
+        } else {
+            for (uint32_t i = 0; i < len; i++) A[i] = input_sig(r, r.in[o + i]);
+        }
+        // insertion sort keeps equal keys in order, as thrust's sequential sort does
+        for (uint32_t i = 1; i < len; i++) {
+            const unsigned long long x = A[i];
+            int j = (int)i - 1;
+            while (j >= 0 && sorts_before(r.shuffle, x, A[j])) {
+                A[j + 1] = A[j];
+                j--;
+            }
+            A[j + 1] = x;
+        }
+    }
 }
 
-__global__ void k_rec_prepare(RecArgs r, uint32_t nb) {
-    const uint32_t counter = r.counter[0];
+// sharedNodeDrivenPermute then prepareDataToInsert: mask 0 done, 1 a new key
+// (skey, its level in sres), 2 an existing signal (sres)
+__global__ void k_rec_prepare(RecArgs r, uint32_t s, uint32_t nb) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    bool any = false;
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nb; c += stride)
-        any |= rec_prepare(r, (uint32_t)c, counter) != 0;
-    if (any) atomicOr(&r.counter[2], 1u);
+    const uint32_t in0 = r.off[s];
+    auto lookup = [&](unsigned long long a, unsigned long long b) -> unsigned long long {
+        const unsigned long long t = and_trivial(a, b);
+        if (t != EMPTY64) return t;
+        const unsigned long long key = and_key_of(sig_lit(a), sig_lit(b));
+        const uint64_t h = mix64(key) & r.t.mask;
+        return t_find_from(r.t, key, h, t_word(r.t, 2 * h));
+    };
+    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nb; c += stride) {
+        unsigned long long *A = r.arr + (r.off[s + c] - in0);
+        const uint32_t L = r.alen[c];
+        if (L <= 1) { r.mask[c] = 0; continue; }
+        const int right = (int)L - 2;
+        int left = right;
+        const unsigned long long l1 = A[right + 1], l2 = A[right];
+        while (left > 0 && sig_lev(A[left - 1]) == sig_lev(l2)) left--;
+        unsigned long long found = EMPTY64;
+        for (int i = right; i >= left && found == EMPTY64; i--) {
+            found = lookup(l1, A[i]);
+            if (found != EMPTY64) A[i] = l2;        // the partner goes next to last
+        }
+        r.alen[c] = L - 2;
+        if (found != EMPTY64) {
+            r.mask[c] = 2;
+            r.sres[c] = found;
+            continue;
+        }
+        r.mask[c] = 1;
+        r.skey[c] = and_key_of(sig_lit(l1), sig_lit(l2));
+        r.sres[c] = (sig_lev(l1) > sig_lev(l2) ? sig_lev(l1) : sig_lev(l2)) + 1u;
+    }
 }
 
 __global__ void k_rec_insert(RecArgs r, uint32_t nb) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nb; c += stride)
-        if (r.mask[c] == 1 && !r_insert_min(r.t, r.skey[c], r.sval[c])) atomicOr(r.err, 2u);
-}
-
-__global__ void k_rec_retrieve(RecArgs r, uint32_t nb) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    uint32_t mx = 0, made = 0;
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nb; c += stride) {
         if (r.mask[c] != 1) continue;
-        const uint32_t got = r_find(r.t, r.skey[c]);
-        made += got == r.sval[c] ? 1u : 0u;
-        r.sval[c] = got;
-        mx = got > mx ? got : mx;
-    }
-    // one atomic per workgroup for each counter
-    __shared__ uint32_t s_made, s_mx;
-    if (threadIdx.x == 0) { s_made = 0; s_mx = 0; }
-    __syncthreads();
-    if (made) atomicAdd(&s_made, made);
-    if (mx) atomicMax(&s_mx, mx);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        if (s_made) atomicAdd(&r.counter[3], s_made);
-        if (s_mx) atomicMax(&r.counter[1], s_mx);
+        const uint32_t slot = t_slot(r.t, r.skey[c]);
+        r.slot[c] = slot;
+        if (slot == UNSET) { atomicOr(r.err, 2u); r.mask[c] = 0; continue; }
+        atomicMin(&r.t.w[2 * (size_t)slot + 1], (unsigned long long)c);
     }
 }
 
+// winners (the smallest cover index of a key) of every workgroup's kB covers
+__global__ void __launch_bounds__(kB) k_rec_winners(RecArgs r, uint32_t nb) {
+    const uint32_t c = blockIdx.x * kB + threadIdx.x;
+    const bool win = c < nb && r.mask[c] == 1 && r.t.w[2 * (size_t)r.slot[c] + 1] == (unsigned long long)c;
+    const int n = __syncthreads_count(win);
+    if (c < nb && win) r.mask[c] = 3;
+    if (threadIdx.x == 0) r.bcnt[blockIdx.x] = (uint32_t)n;
+}
+
+// ids of the winners: the counter, the winners of the workgroups before, the
+// rank inside the workgroup
+__global__ void __launch_bounds__(kB) k_rec_ids(RecArgs r, uint32_t s, uint32_t nb, uint32_t step) {
+    __shared__ uint32_t s_sum, s_w[kB / 64];
+    if (threadIdx.x == 0) s_sum = 0;
+    __syncthreads();
+    uint32_t x = 0;
+    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kB) x += r.bcnt[b];
+    if (x) atomicAdd(&s_sum, x);
+    const uint32_t c = blockIdx.x * kB + threadIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const bool win = c < nb && r.mask[c] == 3;
+    const uint64_t m = __ballot(win);
+    if (lane == 0) s_w[wave] = (uint32_t)__popcll(m);
+    __syncthreads();
+    uint32_t id = r.counter[step & 1u] + s_sum + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+    for (uint32_t w = 0; w < wave; w++) id += s_w[w];
+    if (win) {
+        const unsigned long long key = r.skey[c];
+        r.of0[id] = (uint32_t)(key >> 32);
+        r.of1[id] = (uint32_t)key;
+        if (r.tagOut) r.tagOut[id] = r.tagIn[r.roots[s + c]];
+        r.t.w[2 * (size_t)r.slot[c] + 1] = sig(2u * id, (uint32_t)r.sres[c]);
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        uint32_t n = r.counter[step & 1u] + s_sum;
+        for (uint32_t w = 0; w < kB / 64; w++) n += s_w[w];
+        r.counter[(step & 1u) ^ 1u] = n;
+    }
+}
+
+// addBackLocalArrays (balance.cu:429-467)
 __global__ void k_rec_add_back(RecArgs r, uint32_t s, uint32_t nb) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const uint32_t in0 = r.off[s];
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nb; c += stride) {
-        if (r.mask[c] == 1 && !l_insert(r.t, r.sval[c], r.slev[c])) atomicOr(r.err, 2u);
-        rec_tag(r, (uint32_t)c, r.roots[s + c]);
-        rec_add_back(r, (uint32_t)c);
+        const uint8_t m = r.mask[c];
+        if (m == 0) continue;
+        unsigned long long *A = r.arr + (r.off[s + c] - in0);
+        const unsigned long long x = m == 2 ? r.sres[c] : r.t.w[2 * (size_t)r.slot[c] + 1];
+        const uint32_t L = r.alen[c];
+        bool there = false;
+        for (uint32_t i = 0; i < L; i++) there |= sig_lit(A[i]) == sig_lit(x);
+        if (there) continue;
+        uint32_t i = L;
+        while (i > 0 && sig_lev(x) > sig_lev(A[i - 1])) {
+            A[i] = A[i - 1];
+            i--;
+        }
+        A[i] = x;
+        r.alen[c] = L + 1;
     }
-}
-
-// counter[0] = step max + 1 when a node was made; clears the step fields
-__global__ void k_rec_step_end(uint32_t *counter) {
-    if (counter[1]) counter[0] = counter[1] + 1u;
-    counter[1] = 0;
-    counter[2] = 0;
 }
 
 __global__ void k_rec_record(RecArgs r, uint32_t s, uint32_t nb) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const uint32_t in0 = r.off[s];
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nb; c += stride)
-        rec_record(r, (uint32_t)c, r.roots[s + c]);
+        r.newSig[r.roots[s + c]] = r.alen[c] == 0 ? 0ull : r.arr[r.off[s + c] - in0];
 }
 
 // ---------------------------------------------------------------------------
-// phase 3: renumbering
+// phase 3: output.  A segment's ids are consecutive; they move down by its gap
+// (its first id less the first of its output) behind the segments before it.
 // ---------------------------------------------------------------------------
-__global__ void k_created(uint64_t cap, const unsigned long long *__restrict__ rk, const uint32_t *__restrict__ rv,
-                          unsigned long long *keys, uint32_t *ids, uint32_t *count) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < (int64_t)cap; s += stride) {
-        const bool full = rk[s] != EMPTY64;
-        const uint32_t k = wave_append(count, full);
-        if (!full) continue;
-        keys[k] = rk[s];
-        ids[k] = rv[s];
-    }
+__device__ __forceinline__ uint32_t moved(uint32_t lit, int32_t nPIs, uint32_t gap) {
+    return (int32_t)(lit >> 1) <= nPIs ? lit : lit - 2u * gap;
 }
 
-// ids sorted ascending: created node q gets output id nPIs + 1 + q
-__global__ void k_out_map(int32_t m, int32_t nPIs, const uint32_t *__restrict__ sortedIds, Tables t, uint32_t *err) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < m; q += stride)
-        if (!l_insert(t, sortedIds[q], (uint32_t)(nPIs + 1 + q))) atomicOr(err, 2u);
-}
-
-__device__ __forceinline__ uint32_t out_lit(const Tables &outMap, uint32_t lit, int32_t nPIs) {
-    const uint32_t id = lit >> 1;
-    if ((int32_t)id <= nPIs) return lit;
-    return 2u * l_find(outMap, id) | (lit & 1u);
-}
-
-__global__ void k_out_emit(int32_t m, int32_t nPIs, const unsigned long long *__restrict__ sortedKeys,
-                           const uint32_t *__restrict__ sortedIds, Tables outMap, uint32_t *of0, uint32_t *of1,
-                           uint32_t *olevel, const uint32_t *__restrict__ tagIn, Tables tagTab, uint32_t *tagOut) {
+__global__ void k_out_emit(uint32_t m, int32_t nPIs, uint32_t nSeg, const uint32_t *__restrict__ outOff,
+                           const uint32_t *__restrict__ idBase, const uint32_t *__restrict__ if0,
+                           const uint32_t *__restrict__ if1, uint32_t *of0, uint32_t *of1, uint32_t *olevel,
+                           const uint32_t *__restrict__ tagIn, const uint32_t *__restrict__ itag, uint32_t *otag) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < m; q += stride) {
-        const unsigned long long k = sortedKeys[q];
-        const int64_t o = nPIs + 1 + q;
-        of0[o] = out_lit(outMap, (uint32_t)(k >> 32), nPIs);
-        of1[o] = out_lit(outMap, (uint32_t)k, nPIs);
+        uint32_t lo = 0, hi = nSeg - 1;          // the segment whose output holds q
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1) >> 1;
+            if (outOff[mid] <= (uint32_t)q) lo = mid;
+            else hi = mid - 1;
+        }
+        const uint32_t gap = idBase[lo] - (uint32_t)(nPIs + 1) - outOff[lo];
+        const uint32_t o = (uint32_t)(nPIs + 1) + (uint32_t)q, v = o + gap;
+        of0[o] = moved(if0[v], nPIs, gap);
+        of1[o] = moved(if1[v], nPIs, gap);
         olevel[o] = 0;
-        if (tagOut) tagOut[o] = l_find(tagTab, sortedIds[q]);
+        if (otag) otag[o] = itag[v];
     }
     for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v <= nPIs; v += stride) {
         of0[v] = 0;
         of1[v] = 0;
         olevel[v] = 0;
-        if (tagOut) tagOut[v] = tagIn[v];
+        if (otag) otag[v] = tagIn[v];
     }
 }
 
 __global__ void k_out_pos(int32_t nPOs, int32_t nPIs, const uint32_t *__restrict__ pos,
-                          const uint32_t *__restrict__ newLit, Tables outMap, uint32_t *opos) {
+                          const unsigned long long *__restrict__ newSig, const uint32_t *__restrict__ segTag,
+                          const uint32_t *__restrict__ outOff, const uint32_t *__restrict__ idBase, uint32_t *opos) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nPOs; i += stride) {
         const uint32_t l = pos[i], id = l >> 1;
         if ((int32_t)id <= nPIs) { opos[i] = l; continue; }
-        const uint32_t nl = newLit[id];
-        opos[i] = out_lit(outMap, nl, nPIs) ^ (l & 1u);
+        const uint32_t seg = segTag ? segTag[id] : 0u;
+        opos[i] = moved(sig_lit(newSig[id]), nPIs, idBase[seg] - (uint32_t)(nPIs + 1) - outOff[seg]) ^ (l & 1u);
     }
 }
 
@@ -691,40 +968,29 @@ __global__ void k_split_tags(uint32_t nRoots, const unsigned long long *__restri
     }
 }
 
-// the largest set cover length (at least 1)
-__global__ void k_max_cover_len(int32_t n, const uint32_t *__restrict__ coverLen, uint32_t *out) {
-    __shared__ uint32_t s_m;
-    if (threadIdx.x == 0) s_m = 1;
-    __syncthreads();
-    uint32_t m = 1;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += stride) {
-        const uint32_t l = coverLen[v];
-        if (l != UNSET && l > m) m = l;
-    }
-    atomicMax(&s_m, m);
-    __syncthreads();
-    if (threadIdx.x == 0) atomicMax(out, s_m);
-}
-
 // steps of every reconstruction batch of the wide levels: the largest
 // (cover length - 1) of its roots; batchOff[l] = first batch of level l
 // (UNSET for a level that the persistent workgroup takes)
-__global__ void k_batch_steps(uint32_t nRoots, const uint32_t *__restrict__ levels,
-                              const uint32_t *__restrict__ roots, const uint32_t *__restrict__ coverLen,
+__global__ void k_batch_steps(uint32_t nRoots, const uint32_t *__restrict__ levels, const uint32_t *__restrict__ off,
                               const uint32_t *__restrict__ starts, const uint32_t *__restrict__ batchOff,
                               uint32_t batchLimit, uint32_t *steps) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nRoots; i += stride) {
         const uint32_t l = levels[i], bo = batchOff[l];
         if (bo == UNSET) continue;
-        const uint32_t len = coverLen[roots[i]];
+        const uint32_t len = off[i + 1] - off[i];
         const uint32_t st = len > 1 ? len - 1 : 0u;
         // most roots of a batch see a maximum at least as large already: the
         // atomic is taken only by those that raise it
         uint32_t *dst = &steps[bo + ((uint32_t)i - starts[l]) / batchLimit];
         if (st > __hip_atomic_load(dst, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(dst, st);
     }
+}
+
+// the wide levels' counter from the nodes made so far, or (to = 0) back
+__global__ void k_counter_made(uint32_t *counter, uint32_t *made, uint32_t firstId, uint32_t to) {
+    if (to) *made = *counter - firstId;
+    else *counter = firstId + *made;
 }
 
 struct Tmp {
@@ -751,263 +1017,325 @@ uint32_t bits_of(uint32_t x) {
 } // namespace
 
 int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *info, const uint32_t *tagIn,
-                uint32_t **tagOut, std::vector<uint32_t> *splitTags, int sortDecId) {
+                uint32_t **tagOut, std::vector<uint32_t> *splitTags, int sortDecId, int32_t nTags) {
     const bool tagged = tagIn && tagOut;
     if (sortDecId != 0 && sortDecId != 1) return gls_fail(ctx, GLS_ERR_ARG, "balance: sortDecId must be 0 or 1");
     // the shuffle is seeded with a cover's index in its batch, which in a
     // batched arena is not its index when balanced alone
     if (sortDecId == 0 && tagged) return gls_fail(ctx, GLS_ERR_ARG, "balance: `b -s` is not batched");
+    if (tagged && nTags <= 0) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: tags without their number");
     const int32_t n = in.nObjs, nPIs = in.nPIs, nPOs = in.nPOs;
+    const uint32_t nSeg = tagged ? (uint32_t)nTags : 1u;
     const uint32_t narrowMax = (uint32_t)tuning_for(ctx, n).balance_narrow_max;
     hipStream_t st = ctx->stream;
     Tmp t{ctx};
     const auto t0 = std::chrono::steady_clock::now();
-    // ---- phase 1: covers and root levels
-    uint32_t *nFo = t.get<uint32_t>(n), *coverOff = t.get<uint32_t>(n), *coverLen = t.get<uint32_t>(n);
-    uint32_t *lastLevel = t.get<uint32_t>(n), *stamp = t.get<uint32_t>(n), *indeg = t.get<uint32_t>(n);
-    uint32_t *frontA = t.get<uint32_t>(n), *frontB = t.get<uint32_t>(n);
-    uint32_t *ctr = t.get<uint32_t>(8);   // [1] pool next, [2] err, [4..7] reconstruction counter
-    uint32_t *flen = t.get<uint32_t>((size_t)n + 2 + COVER_LEVELS_PER_CHECK);   // frontier size per level
+    // ---- phase 1: covers
+    uint32_t *nFo = t.get<uint32_t>(n), *mark = t.get<uint32_t>(n), *indeg = t.get<uint32_t>(n);
+    uint2 *cover = t.get<uint2>(n);
+    uint32_t *lastLevel = t.get<uint32_t>(n), *roots = t.get<uint32_t>(n), *rootsSorted = t.get<uint32_t>(n);
+    uint8_t *flag = t.get<uint8_t>((size_t)n + 4), *flag2 = t.get<uint8_t>(n);
+    uint32_t *extra = t.get<uint32_t>(n);
+    // [0] pool next, [1] error, [2] extra roots, [3] roots, [4..6] largest level, [8..9] counter
+    uint32_t *ctr = t.get<uint32_t>(16);
     const uint64_t poolCap = 2ull * (uint64_t)n + 64;   // cover inputs are distinct fanin edges
     uint32_t *pool = t.get<uint32_t>(poolCap);
-    // one cover-discovery thread per 8 objects within the bounds: a wide
-    // level's frontier is then walked in one or two rounds per thread
-    const int coverThreads = (int)std::min<int64_t>(
-        COVER_THREADS_MAX, std::max<int64_t>(COVER_THREADS, ((int64_t)n / 8 + kB - 1) / kB * kB));
+    const int coverThreads = (int)std::min<int64_t>(COVER_THREADS, (int64_t)nblocks(n) * kB);
     uint32_t *scratch = t.get<uint32_t>((size_t)coverThreads * COVER_SCRATCH);
+    uint32_t *segInfo = t.get<uint32_t>(4 * (size_t)nSeg + 4), *flen = t.get<uint32_t>(SWEEP_GRID_ROUNDS + 1);
     if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: allocation (n=%d)", n);
+    uint32_t *segFirst = segInfo, *segLen = segInfo + nSeg + 1, *segRound = segLen + nSeg, *segCnt = segRound + nSeg;
     GLS_HIP(ctx, hipMemsetAsync(nFo, 0, sizeof(uint32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(coverLen, 0xFF, sizeof(uint32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(lastLevel, 0xFF, sizeof(uint32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(stamp, 0, sizeof(uint32_t) * n, st));
+    GLS_HIP(ctx, hipMemsetAsync(mark, 0, sizeof(uint32_t) * n, st));
     GLS_HIP(ctx, hipMemsetAsync(indeg, 0, sizeof(uint32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(ctr, 0, sizeof(uint32_t) * 8, st));
-    GLS_HIP(ctx, hipMemsetAsync(flen, 0, sizeof(uint32_t) * ((size_t)n + 2 + COVER_LEVELS_PER_CHECK), st));
-    k_fanouts<<<nblocks(n), kB, 0, st>>>(n, nPIs, in.f0, in.f1, nPOs, in.pos, nFo);
-    if (nPOs > 0) k_po_frontier<<<nblocks(nPOs), kB, 0, st>>>(nPOs, nPIs, in.pos, stamp, frontA, &flen[0]);
+    GLS_HIP(ctx, hipMemsetAsync(lastLevel, 0xFF, sizeof(uint32_t) * n, st));
+    GLS_HIP(ctx, hipMemsetAsync(ctr, 0, sizeof(uint32_t) * 16, st));
+    GLS_HIP(ctx, hipMemsetAsync(segInfo, 0, sizeof(uint32_t) * (4 * (size_t)nSeg + 4), st));
+    k_fanouts<<<nblocks(n), kB, 0, st>>>(n, nPIs, in.f0, in.f1, nPOs, in.pos, nFo, mark);
+    if (nPOs > 0) k_po_marks<<<nblocks(nPOs), kB, 0, st>>>(nPOs, in.pos, mark);
+    k_root_flags<<<nblocks(n), kB, 0, st>>>(n, nPIs, nFo, mark, flag);
     GLS_HIP(ctx, hipGetLastError());
-    CoverArgs ca{in.f0, in.f1, nFo, nPIs, coverOff, coverLen, pool, &ctr[1], poolCap, scratch, lastLevel, stamp,
-                 indeg, &ctr[2]};
-    // rounds are launched COVER_LEVELS_PER_CHECK at a time; a launch past the
-    // last round finds an empty frontier and does nothing.  Returns the
-    // number of rounds with a non-empty frontier.
-    auto sweep = [&](bool kahn, uint32_t &rounds) -> int {
-        for (uint32_t base = 0;; base += COVER_LEVELS_PER_CHECK) {
-            if ((uint64_t)base > (uint64_t)n) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: cover levels do not end");
-            for (uint32_t r = base; r < base + COVER_LEVELS_PER_CHECK; r++) {
-                if (kahn) k_cover_kahn<<<coverThreads / kB, kB, 0, st>>>(ca, frontA, frontB, flen, r);
-                else k_cover_reach<<<coverThreads / kB, kB, 0, st>>>(ca, frontA, frontB, flen, r);
-            }
-            GLS_HIP(ctx, hipGetLastError());
-            uint32_t h[COVER_LEVELS_PER_CHECK + 1];
-            GLS_TRY(stream_copy(ctx, h, &flen[base], sizeof(h), hipMemcpyDeviceToHost));
-            for (int i = 0; i <= COVER_LEVELS_PER_CHECK; i++)
-                if (h[i] == 0) { rounds = base + (uint32_t)i; return GLS_OK; }
-        }
-    };
-    uint32_t reachRounds = 0, levels = 0;
-    GLS_TRY(sweep(false, reachRounds));
-    // every reached root now has its cover and its count of parent covers
-    GLS_HIP(ctx, hipMemsetAsync(flen, 0, sizeof(uint32_t) * ((size_t)reachRounds + 2), st));
-    if (nPOs > 0) k_kahn_first<<<nblocks(nPOs), kB, 0, st>>>(nPOs, nPIs, in.pos, indeg, stamp, frontA, &flen[0]);
-    GLS_HIP(ctx, hipGetLastError());
-    GLS_TRY(sweep(true, levels));
-    uint32_t herr = 0, poolUsed = 0;
-    GLS_TRY(stream_copy(ctx, &herr, &ctr[2], sizeof(uint32_t), hipMemcpyDeviceToHost));
-    GLS_TRY(stream_copy(ctx, &poolUsed, &ctr[1], sizeof(uint32_t), hipMemcpyDeviceToHost));
-    if (herr) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: cover pool overflow");
-
-    // roots by (level, id)
-    uint8_t *flag = t.get<uint8_t>(n);
-    uint32_t *roots = t.get<uint32_t>(n), *rootsSorted = t.get<uint32_t>(n);
-    uint32_t *keys = t.get<uint32_t>(n), *keysSorted = t.get<uint32_t>(n), *d_cnt = t.get<uint32_t>(2);
-    if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: allocation");
-    k_root_flags<<<nblocks(n), kB, 0, st>>>(n, lastLevel, flag);
-    size_t tb = 0;
     rocprim::counting_iterator<uint32_t> ids(0u);
-    GLS_HIP(ctx, rocprim::select(nullptr, tb, ids, flag, roots, d_cnt, (size_t)n, st));
+    size_t tb = 0;
+    GLS_HIP(ctx, rocprim::select(nullptr, tb, ids, flag, roots, &ctr[3], (size_t)n, st));
     void *tmp = t.get<uint8_t>(tb);
     if (!tmp) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: select storage");
-    GLS_HIP(ctx, rocprim::select(tmp, tb, ids, flag, roots, d_cnt, (size_t)n, st));
-    uint32_t nRoots = 0;
-    GLS_TRY(stream_copy(ctx, &nRoots, d_cnt, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    std::vector<uint32_t> starts(levels + 2, 0);
-    if (nRoots > 0) {
-        k_gather_level<<<nblocks(nRoots), kB, 0, st>>>((int32_t)nRoots, roots, lastLevel, keys);
-        size_t tb2 = 0;
-        const uint32_t eb = bits_of(levels);
+    auto select_ids = [&](const uint8_t *f, uint32_t &count) -> int {
+        GLS_HIP(ctx, rocprim::select(tmp, tb, ids, f, roots, &ctr[3], (size_t)n, st));
+        return stream_copy(ctx, &count, &ctr[3], sizeof(uint32_t), hipMemcpyDeviceToHost);
+    };
+    uint32_t nCand = 0;
+    GLS_TRY(select_ids(flag, nCand));
+    const CoverArgs ca{in.f0, in.f1, nFo, nPIs, cover, pool, &ctr[0], poolCap, scratch, flag, indeg, extra, &ctr[2],
+                       &ctr[1]};
+    // covers of the roots by their edges; then of those a limit made, until
+    // no cover meets another one
+    uint32_t misc[4] = {};
+    bool limited = false;
+    const uint32_t *list = roots;
+    for (uint32_t todo = nCand, done = 0; todo > 0;) {
+        k_covers<<<(int)std::min<int64_t>(nblocks(todo), coverThreads / kB), kB, 0, st>>>(ca, todo, list);
+        GLS_HIP(ctx, hipGetLastError());
+        GLS_TRY(stream_copy(ctx, misc, ctr, sizeof(misc), hipMemcpyDeviceToHost));
+        if (misc[1]) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: cover pool overflow");
+        list = extra + done;
+        todo = misc[2] - done;
+        done = misc[2];
+        limited |= todo > 0;
+    }
+    const uint32_t poolUsed = misc[0];
+    if (limited) GLS_TRY(select_ids(flag, nCand));
+    // ---- the sweeps: unreached roots dropped, then levels
+    if (tagged && nCand > 0) {
+        k_count_tags<<<tag_grid(nCand), kBlock, 0, st>>>(nCand, roots, tagIn, segCnt);
+        size_t tbs = 0;
+        GLS_HIP(ctx, rocprim::exclusive_scan(nullptr, tbs, segCnt, segFirst, 0u, (size_t)nSeg, rocprim::plus<uint32_t>(), st));
+        void *ts = t.get<uint8_t>(std::max<size_t>(tbs, 1));
+        if (!ts) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: scan storage");
+        GLS_HIP(ctx, rocprim::exclusive_scan(ts, tbs, segCnt, segFirst, 0u, (size_t)nSeg, rocprim::plus<uint32_t>(), st));
+    }
+    SweepArgs sa{cover, pool, nPIs, mark, indeg, lastLevel, {extra, rootsSorted}, 0u};
+    std::vector<uint32_t> segLevels(nSeg, 0);
+    auto sweep = [&](bool drop) -> int {
+        sa.drop = drop ? 1u : 0u;
+        GLS_HIP(ctx, hipMemsetAsync(segLen, 0, sizeof(uint32_t) * 2 * nSeg, st));
+        k_sweep_first<<<nblocks(nCand), kB, 0, st>>>(nCand, roots, sa, tagged ? tagIn : nullptr, segFirst, segLen);
+        for (;;) {
+            k_sweep_wg<<<nSeg, BAL_WG, 0, st>>>(sa, segFirst, segLen, segRound, nSeg == 1 ? SWEEP_WIDE : UNSET);
+            GLS_HIP(ctx, hipGetLastError());
+            if (nSeg > 1) break;
+            uint32_t h[2] = {};      // the frontier's size, rounds done (segLen[0], segRound[0])
+            GLS_TRY(stream_copy(ctx, h, segLen, sizeof(h), hipMemcpyDeviceToHost));
+            while (h[0] > SWEEP_WIDE) {
+                if (h[1] > (uint32_t)n) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: cover levels do not end");
+                GLS_HIP(ctx, hipMemsetAsync(flen, 0, sizeof(uint32_t) * (SWEEP_GRID_ROUNDS + 1), st));
+                GLS_HIP(ctx, hipMemcpyAsync(flen, segLen, sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
+                for (int i = 0; i < SWEEP_GRID_ROUNDS; i++)
+                    k_sweep_grid<<<nblocks(2 * (int64_t)h[0]), kB, 0, st>>>(sa, h[1] + (uint32_t)i, flen + i);
+                GLS_HIP(ctx, hipGetLastError());
+                uint32_t sizes[SWEEP_GRID_ROUNDS + 1];
+                GLS_TRY(stream_copy(ctx, sizes, flen, sizeof(sizes), hipMemcpyDeviceToHost));
+                // rounds past the last non-empty frontier did nothing
+                int last = 0;
+                while (last < SWEEP_GRID_ROUNDS && sizes[last] != 0) last++;
+                h[0] = sizes[last];
+                h[1] += (uint32_t)last;
+                GLS_TRY(stream_copy(ctx, segLen, h, sizeof(h), hipMemcpyHostToDevice));
+            }
+            if (h[0] == 0) break;
+        }
+        return GLS_OK;
+    };
+    uint32_t nRoots = 0, levels = 0;
+    if (nCand > 0) {
+        GLS_TRY(sweep(true));
+        GLS_TRY(sweep(false));
+        GLS_TRY(stream_copy(ctx, segLevels.data(), segRound, sizeof(uint32_t) * nSeg, hipMemcpyDeviceToHost));
+        for (uint32_t x : segLevels) levels = std::max(levels, x);
+        k_taken_flags<<<nblocks(n), kB, 0, st>>>(n, lastLevel, flag2);
+        GLS_TRY(select_ids(flag2, nRoots));
+    }
+    // ---- roots in the order in which they are rebuilt: by (segment, level,
+    // id) where every level fits the persistent workgroup, else by (level, id)
+    const uint32_t fitCovers = std::min<uint32_t>(narrowMax, LT_COVERS);
+    uint32_t *keys = t.get<uint32_t>(std::max(nRoots, 1u)), *keysSorted = t.get<uint32_t>(std::max(nRoots, 1u));
+    uint32_t *off = t.get<uint32_t>((size_t)nRoots + 1), *len = t.get<uint32_t>((size_t)nRoots + 1);
+    uint32_t *newLen = t.get<uint32_t>((size_t)nRoots + 1), *newOff = t.get<uint32_t>((size_t)nRoots + 1);
+    uint32_t *inputs = t.get<uint32_t>(std::max<size_t>(poolUsed, 1));
+    if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: order allocation");
+    uint32_t *d_starts = nullptr, *d_levOff = nullptr;
+    uint2 *d_levSize = nullptr;
+    uint32_t most[3] = {};
+    std::vector<uint32_t> levOff;
+    auto order = [&](bool bySeg) -> int {
+        const uint32_t ns = bySeg ? nSeg : 1u;
+        levOff.assign(ns + 1, 0);
+        for (uint32_t k = 0; k < ns; k++) levOff[k + 1] = levOff[k] + (bySeg ? segLevels[k] : levels);
+        const uint32_t nKeys = levOff[ns];
+        d_levOff = t.get<uint32_t>(ns + 1);
+        d_starts = t.get<uint32_t>((size_t)nKeys + 1);
+        d_levSize = t.get<uint2>((size_t)nKeys + 1);
+        if (!d_levOff || !d_starts || !d_levSize) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: levels");
+        GLS_TRY(stream_copy(ctx, d_levOff, levOff.data(), sizeof(uint32_t) * (ns + 1), hipMemcpyHostToDevice));
+        k_level_keys<<<nblocks(nRoots), kB, 0, st>>>(nRoots, roots, lastLevel, tagIn,
+                                                     bySeg && tagged ? d_levOff : nullptr, keys);
+        size_t tb2 = 0, tb3 = 0;
+        const uint32_t eb = bits_of(nKeys);
         GLS_HIP(ctx, rocprim::radix_sort_pairs(nullptr, tb2, keys, keysSorted, roots, rootsSorted, (size_t)nRoots, 0u,
                                                eb, st));
-        void *tmp2 = t.get<uint8_t>(tb2);
+        GLS_HIP(ctx, rocprim::exclusive_scan(nullptr, tb3, len, off, 0u, (size_t)nRoots + 1, rocprim::plus<uint32_t>(), st));
+        void *tmp2 = t.get<uint8_t>(std::max<size_t>(std::max(tb2, tb3), 1));
         if (!tmp2) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: sort storage");
         GLS_HIP(ctx, rocprim::radix_sort_pairs(tmp2, tb2, keys, keysSorted, roots, rootsSorted, (size_t)nRoots, 0u,
                                                eb, st));
-        std::vector<uint32_t> hk(nRoots);
-        GLS_TRY(stream_copy(ctx, hk.data(), keysSorted, sizeof(uint32_t) * nRoots, hipMemcpyDeviceToHost));
-        for (uint32_t i = 0; i < nRoots; i++) starts[hk[i] + 1]++;
-        for (uint32_t l = 1; l <= levels + 1; l++) starts[l] += starts[l - 1];
-    }
-    // Batches: 32768 covers of a level at a time.  With tags (a union of
-    // independent AIGs) a level is one batch, which gives every AIG the batches
-    // it gets alone as long as none has more than 32768 covers on a level: the
-    // (level, tag) keys of the roots are sorted on the device, and a tag with
-    // a longer run is reported to the caller (splitTags), which balances it
-    // alone.
-    if (tagged && nRoots > (uint32_t)BAL_BATCH) {
-        unsigned long long *gk = t.get<unsigned long long>(nRoots), *gkS = t.get<unsigned long long>(nRoots);
-        uint32_t *lst = t.get<uint32_t>(1024), *lcnt = t.get<uint32_t>(1);
-        if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: split check");
-        k_level_tag_keys<<<nblocks(nRoots), kB, 0, st>>>(nRoots, keysSorted, rootsSorted, tagIn, gk);
-        size_t tbk = 0;
-        GLS_HIP(ctx, rocprim::radix_sort_keys(nullptr, tbk, gk, gkS, (size_t)nRoots, 0u, 64u, st));
-        void *tmpk = t.get<uint8_t>(tbk);
-        if (!tmpk) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: split check sort");
-        GLS_HIP(ctx, rocprim::radix_sort_keys(tmpk, tbk, gk, gkS, (size_t)nRoots, 0u, 64u, st));
-        GLS_HIP(ctx, hipMemsetAsync(lcnt, 0, sizeof(uint32_t), st));
-        k_split_tags<<<nblocks(nRoots), kB, 0, st>>>(nRoots, gkS, lst, 1024u, lcnt);
+        k_key_starts<<<nblocks((int64_t)nRoots + 1), kB, 0, st>>>(nRoots, keysSorted, nKeys, d_starts);
+        k_cover_lens<<<nblocks((int64_t)nRoots + 1), kB, 0, st>>>(nRoots, rootsSorted, cover, len, newLen);
+        GLS_HIP(ctx, rocprim::exclusive_scan(tmp2, tb3, len, off, 0u, (size_t)nRoots + 1, rocprim::plus<uint32_t>(), st));
+        GLS_HIP(ctx, rocprim::exclusive_scan(tmp2, tb3, newLen, newOff, 0u, (size_t)nRoots + 1,
+                                             rocprim::plus<uint32_t>(), st));
+        GLS_HIP(ctx, hipMemsetAsync(&ctr[4], 0, sizeof(uint32_t) * 3, st));
+        k_level_sizes<<<nblocks(nKeys), kB, 0, st>>>(nKeys, d_starts, off, newOff, d_levSize, &ctr[4]);
+        k_pack_inputs<<<nblocks(nRoots), kB, 0, st>>>(nRoots, rootsSorted, cover, pool, off, inputs);
         GLS_HIP(ctx, hipGetLastError());
-        uint32_t nsplit = 0;
-        GLS_TRY(stream_copy(ctx, &nsplit, lcnt, sizeof(uint32_t), hipMemcpyDeviceToHost));
-        if (nsplit > 0) {
-            if (splitTags) {
-                splitTags->assign(std::min<uint32_t>(nsplit, 1024u), 0u);
-                GLS_TRY(stream_copy(ctx, splitTags->data(), lst, sizeof(uint32_t) * splitTags->size(),
-                                    hipMemcpyDeviceToHost));
-                if (nsplit > 1024u) splitTags->clear();   // too many to list: the caller splits them all
+        return stream_copy(ctx, most, &ctr[4], sizeof(most), hipMemcpyDeviceToHost);
+    };
+    bool bySeg = true, fits = true;
+    if (nRoots > 0) {
+        GLS_TRY(order(true));
+        fits = most[0] <= fitCovers && most[1] <= LT_INPUTS && most[2] <= LT_NEW;
+        if (!fits && tagged) {
+            // Batches: 32768 covers of a level at a time.  With tags (a union of
+            // independent AIGs) a level is one batch, which gives every AIG the
+            // batches it gets alone as long as none has more than 32768 covers
+            // on a level: the (level, tag) keys of the roots are sorted on the
+            // device, and a tag with a longer run is reported to the caller
+            // (splitTags), which balances it alone.
+            bySeg = false;
+            GLS_TRY(order(false));
+            if (nRoots > (uint32_t)BAL_BATCH) {
+                unsigned long long *gk = t.get<unsigned long long>(nRoots), *gkS = t.get<unsigned long long>(nRoots);
+                uint32_t *lst = t.get<uint32_t>(1024), *lcnt = t.get<uint32_t>(1);
+                if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: split check");
+                k_level_tag_keys<<<nblocks(nRoots), kB, 0, st>>>(nRoots, keysSorted, rootsSorted, tagIn, gk);
+                size_t tbk = 0;
+                GLS_HIP(ctx, rocprim::radix_sort_keys(nullptr, tbk, gk, gkS, (size_t)nRoots, 0u, 64u, st));
+                void *tmpk = t.get<uint8_t>(tbk);
+                if (!tmpk) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: split check sort");
+                GLS_HIP(ctx, rocprim::radix_sort_keys(tmpk, tbk, gk, gkS, (size_t)nRoots, 0u, 64u, st));
+                GLS_HIP(ctx, hipMemsetAsync(lcnt, 0, sizeof(uint32_t), st));
+                k_split_tags<<<nblocks(nRoots), kB, 0, st>>>(nRoots, gkS, lst, 1024u, lcnt);
+                GLS_HIP(ctx, hipGetLastError());
+                uint32_t nsplit = 0;
+                GLS_TRY(stream_copy(ctx, &nsplit, lcnt, sizeof(uint32_t), hipMemcpyDeviceToHost));
+                if (nsplit > 0) {
+                    if (splitTags) {
+                        splitTags->assign(std::min<uint32_t>(nsplit, 1024u), 0u);
+                        GLS_TRY(stream_copy(ctx, splitTags->data(), lst, sizeof(uint32_t) * splitTags->size(),
+                                            hipMemcpyDeviceToHost));
+                        if (nsplit > 1024u) splitTags->clear();   // too many to list: the caller splits them all
+                    }
+                    return GLS_ERR_BATCH_SPLIT;
+                }
             }
-            return GLS_ERR_BATCH_SPLIT;
         }
     }
+    const uint32_t ns = bySeg ? nSeg : 1u;
     const uint32_t batchLimit = tagged ? 0xFFFFFFFFu : (uint32_t)BAL_BATCH;
-    // the persistent workgroup takes a whole level as one batch, so a level
-    // goes there only if it is not wider than a batch
-    const uint32_t narrowCap = std::min(narrowMax, batchLimit);
-    // cover lengths: the workspace width, and the steps a batch needs (a step
-    // takes two inputs of every unfinished cover and gives back at most one),
-    // reduced on the device
-    uint32_t maxLen = 1;
-    {
-        uint32_t *d_ml = t.get<uint32_t>(1);
-        if (!d_ml) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: cover length");
-        GLS_HIP(ctx, hipMemsetAsync(d_ml, 0, sizeof(uint32_t), st));
-        k_max_cover_len<<<std::min<int64_t>(nblocks(n), 1024), kB, 0, st>>>(n, coverLen, d_ml);
-        GLS_HIP(ctx, hipGetLastError());
-        GLS_TRY(stream_copy(ctx, &maxLen, d_ml, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    }
-    // the wide levels' batches and their step counts
-    std::vector<uint32_t> batchOff(levels + 1, UNSET), batchSteps;
-    uint32_t nBatches = 0;
-    for (uint32_t l = 0; l < levels; l++) {
-        const uint32_t cnt = starts[l + 1] - starts[l];
-        if (cnt <= narrowCap) continue;
-        batchOff[l] = nBatches;
-        nBatches += (cnt + std::min(cnt, batchLimit) - 1) / std::min(cnt, batchLimit);
-    }
-    if (nBatches > 0) {
-        uint32_t *d_off = t.get<uint32_t>(levels + 1), *d_st = t.get<uint32_t>(levels + 2);
-        uint32_t *d_steps = t.get<uint32_t>(nBatches);
-        if (!d_off || !d_st || !d_steps) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: batch steps");
-        GLS_TRY(stream_copy(ctx, d_off, batchOff.data(), sizeof(uint32_t) * (levels + 1), hipMemcpyHostToDevice));
-        GLS_TRY(stream_copy(ctx, d_st, starts.data(), sizeof(uint32_t) * (levels + 2), hipMemcpyHostToDevice));
-        GLS_HIP(ctx, hipMemsetAsync(d_steps, 0, sizeof(uint32_t) * nBatches, st));
-        k_batch_steps<<<nblocks(nRoots), kB, 0, st>>>(nRoots, keysSorted, rootsSorted, coverLen, d_st, d_off,
-                                                      batchLimit, d_steps);
-        GLS_HIP(ctx, hipGetLastError());
-        batchSteps.resize(nBatches);
-        GLS_TRY(stream_copy(ctx, batchSteps.data(), d_steps, sizeof(uint32_t) * nBatches, hipMemcpyDeviceToHost));
-    }
 
     // ---- phase 2: reconstruction
     uint64_t cap = 1024;
-    while (cap < 2ull * ((uint64_t)poolUsed + 16)) cap <<= 1;
-    unsigned long long *rk = t.get<unsigned long long>(cap);
-    uint32_t *rv = t.get<uint32_t>(cap), *lk = t.get<uint32_t>(cap), *lv = t.get<uint32_t>(cap);
-    uint32_t *newLit = t.get<uint32_t>(n);
-    size_t maxBatch = 1;
-    for (uint32_t l = 0; l < levels; l++)
-        maxBatch = std::max<size_t>(maxBatch, std::min<uint32_t>(starts[l + 1] - starts[l], batchLimit));
-    uint32_t *arr = t.get<uint32_t>(maxBatch * maxLen), *alv = t.get<uint32_t>(maxBatch * maxLen);
-    uint32_t *alen = t.get<uint32_t>(maxBatch);
-    uint8_t *mask = t.get<uint8_t>(maxBatch);
-    unsigned long long *skey = t.get<unsigned long long>(maxBatch);
-    uint32_t *sval = t.get<uint32_t>(maxBatch), *slev = t.get<uint32_t>(maxBatch);
-    uint32_t *d_starts = t.get<uint32_t>(levels + 2);
+    while (cap < 2ull * ((uint64_t)poolUsed + 16)) cap <<= 1;       // a cover of k inputs creates at most k - 1 nodes
+    const size_t idEnd = (size_t)nPIs + 1 + poolUsed;
+    unsigned long long *tab = t.get<unsigned long long>(2 * cap), *newSig = t.get<unsigned long long>(n);
+    uint32_t *cf0 = t.get<uint32_t>(idEnd), *cf1 = t.get<uint32_t>(idEnd);
+    uint32_t *ctag = tagged ? t.get<uint32_t>(idEnd) : nullptr;
+    uint32_t *segIds = t.get<uint32_t>(3 * (size_t)ns + 3);
     if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: reconstruction allocation");
-    GLS_HIP(ctx, hipMemsetAsync(rk, 0xFF, sizeof(unsigned long long) * cap, st));
-    GLS_HIP(ctx, hipMemsetAsync(rv, 0xFF, sizeof(uint32_t) * cap, st));
-    GLS_HIP(ctx, hipMemsetAsync(lk, 0xFF, sizeof(uint32_t) * cap, st));
-    GLS_HIP(ctx, hipMemsetAsync(lv, 0xFF, sizeof(uint32_t) * cap, st));
-    GLS_HIP(ctx, hipMemsetAsync(newLit, 0xFF, sizeof(uint32_t) * n, st));
-    GLS_TRY(stream_copy(ctx, d_starts, starts.data(), sizeof(uint32_t) * (levels + 2), hipMemcpyHostToDevice));
-    const uint32_t firstId = (uint32_t)nPIs + 1u;
-    GLS_TRY(stream_copy(ctx, &ctr[4], &firstId, sizeof(uint32_t), hipMemcpyHostToDevice));
-    Tables tabs{rk, rv, cap - 1, lk, lv, cap - 1};
-    Tables tagTab{nullptr, nullptr, 0, nullptr, nullptr, 0};
-    if (tagged) {
-        uint32_t *tk = t.get<uint32_t>(cap), *tv = t.get<uint32_t>(cap);
-        if (!tk || !tv) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: tag table");
-        GLS_HIP(ctx, hipMemsetAsync(tk, 0xFF, sizeof(uint32_t) * cap, st));
-        GLS_HIP(ctx, hipMemsetAsync(tv, 0xFF, sizeof(uint32_t) * cap, st));
-        tagTab = Tables{nullptr, nullptr, 0, tk, tv, cap - 1};
-    }
-    RecArgs ra{tabs, nPIs, rootsSorted, coverOff, coverLen, pool, newLit, arr, alv, alen, maxLen, mask, skey,
-               sval, slev, &ctr[4], &ctr[2], tagged ? tagIn : nullptr, tagTab, sortDecId == 0 ? 1u : 0u};
-    int32_t l = (int32_t)levels - 1;
-    while (l >= 0) {
-        // a run of narrow levels goes to the persistent workgroup
-        int32_t e = l;
-        while (e >= 0 && starts[e + 1] - starts[e] <= narrowCap) e--;
-        if (e < l) {
-            k_rec_narrow<<<1, BAL_WG, 0, st>>>(ra, d_starts, l, e + 1);
-            GLS_HIP(ctx, hipGetLastError());
-            l = e;
-            continue;
+    uint32_t *d_idBase = segIds, *d_made = segIds + ns, *d_outOff = segIds + 2 * (size_t)ns;
+    GLS_HIP(ctx, hipMemsetAsync(tab, 0xFF, sizeof(unsigned long long) * 2 * cap, st));
+    std::vector<uint32_t> idBase(ns, (uint32_t)nPIs + 1u), made(ns, 0u);
+    if (bySeg && ns > 1 && nRoots > 0) {
+        // a segment's ids start after room for all that those before it can create
+        std::vector<uint2> hl(levOff[ns]);
+        GLS_TRY(stream_copy(ctx, hl.data(), d_levSize, sizeof(uint2) * hl.size(), hipMemcpyDeviceToHost));
+        uint32_t sum = (uint32_t)nPIs + 1u;
+        for (uint32_t k = 0; k < ns; k++) {
+            idBase[k] = sum;
+            for (uint32_t l = levOff[k]; l < levOff[k + 1]; l++) sum += hl[l].y;
         }
-        // one wide level, in batches, one kernel per phase
-        uint32_t bi = batchOff[l];
-        for (uint32_t b0 = starts[l]; b0 < starts[l + 1]; b0 += std::min<uint32_t>(starts[l + 1] - b0, batchLimit)) {
-            const uint32_t nb = std::min<uint32_t>(starts[l + 1] - b0, batchLimit);
-            const uint32_t steps = batchSteps[bi++];
-            k_rec_gather<<<nblocks(nb), kB, 0, st>>>(ra, b0, nb);
-            for (uint32_t stp = 0; stp < steps; stp++) {
-                k_rec_prepare<<<nblocks(nb), kB, 0, st>>>(ra, nb);
-                k_rec_insert<<<nblocks(nb), kB, 0, st>>>(ra, nb);
-                k_rec_retrieve<<<nblocks(nb), kB, 0, st>>>(ra, nb);
-                k_rec_add_back<<<nblocks(nb), kB, 0, st>>>(ra, b0, nb);
-                k_rec_step_end<<<1, 1, 0, st>>>(&ctr[4]);
+    }
+    GLS_TRY(stream_copy(ctx, d_idBase, idBase.data(), sizeof(uint32_t) * ns, hipMemcpyHostToDevice));
+    GLS_HIP(ctx, hipMemsetAsync(d_made, 0, sizeof(uint32_t) * ns, st));
+    RecArgs ra{NodeTable{tab, cap - 1}, nPIs, rootsSorted, off, inputs, d_levSize, d_starts, newSig, cf0, cf1, ctag, tagIn, &ctr[1],
+               sortDecId == 0 ? 1u : 0u, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, &ctr[8]};
+    if (nRoots > 0 && fits) {
+        k_rec_lds<<<ns, BAL_WG, 0, st>>>(ra, d_levOff, d_idBase, d_made, (int32_t)levels - 1, 0);
+        GLS_HIP(ctx, hipGetLastError());
+    } else if (nRoots > 0) {
+        std::vector<uint32_t> starts((size_t)levels + 1);
+        std::vector<uint2> size(levels);
+        GLS_TRY(stream_copy(ctx, starts.data(), d_starts, sizeof(uint32_t) * ((size_t)levels + 1), hipMemcpyDeviceToHost));
+        GLS_TRY(stream_copy(ctx, size.data(), d_levSize, sizeof(uint2) * levels, hipMemcpyDeviceToHost));
+        // a level goes to the persistent workgroup if it fits its LDS (it is
+        // one batch then)
+        auto narrow = [&](uint32_t l) {
+            return starts[l + 1] - starts[l] <= fitCovers && size[l].x <= LT_INPUTS && size[l].y <= LT_NEW;
+        };
+        // the wide levels' batches and their step counts
+        std::vector<uint32_t> batchOff(levels + 1, UNSET), batchSteps;
+        uint32_t nBatches = 0, maxBatch = 1;
+        for (uint32_t l = 0; l < levels; l++) {
+            const uint32_t cnt = starts[l + 1] - starts[l], per = std::min(cnt, batchLimit);
+            if (narrow(l)) continue;
+            batchOff[l] = nBatches;
+            nBatches += (cnt + per - 1) / per;
+            maxBatch = std::max(maxBatch, per);
+        }
+        uint32_t *d_off = t.get<uint32_t>(levels + 1), *d_steps = t.get<uint32_t>(std::max(nBatches, 1u));
+        ra.arr = t.get<unsigned long long>(most[1]);
+        ra.alen = t.get<uint32_t>(maxBatch);
+        ra.mask = t.get<uint8_t>(maxBatch);
+        ra.skey = t.get<unsigned long long>(maxBatch);
+        ra.sres = t.get<unsigned long long>(maxBatch);
+        ra.slot = t.get<uint32_t>(maxBatch);
+        ra.bcnt = t.get<uint32_t>((size_t)nblocks(maxBatch));
+        if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: wide levels");
+        GLS_TRY(stream_copy(ctx, d_off, batchOff.data(), sizeof(uint32_t) * (levels + 1), hipMemcpyHostToDevice));
+        GLS_HIP(ctx, hipMemsetAsync(d_steps, 0, sizeof(uint32_t) * std::max(nBatches, 1u), st));
+        k_batch_steps<<<nblocks(nRoots), kB, 0, st>>>(nRoots, keysSorted, off, d_starts, d_off, batchLimit, d_steps);
+        GLS_HIP(ctx, hipGetLastError());
+        batchSteps.resize(nBatches);
+        if (nBatches > 0)
+            GLS_TRY(stream_copy(ctx, batchSteps.data(), d_steps, sizeof(uint32_t) * nBatches, hipMemcpyDeviceToHost));
+        const uint32_t firstId = (uint32_t)nPIs + 1u;
+        uint32_t step = 0;               // counter[step & 1] is the next id of the wide levels
+        GLS_TRY(stream_copy(ctx, &ctr[8], &firstId, sizeof(uint32_t), hipMemcpyHostToDevice));
+        int32_t l = (int32_t)levels - 1;
+        while (l >= 0) {
+            // a run of narrow levels goes to the persistent workgroup
+            int32_t e = l;
+            while (e >= 0 && narrow((uint32_t)e)) e--;
+            if (e < l) {
+                k_counter_made<<<1, 1, 0, st>>>(&ctr[8 + (step & 1u)], d_made, firstId, 1u);
+                k_rec_lds<<<1, BAL_WG, 0, st>>>(ra, d_levOff, d_idBase, d_made, l, e + 1);
+                k_counter_made<<<1, 1, 0, st>>>(&ctr[8 + (step & 1u)], d_made, firstId, 0u);
+                GLS_HIP(ctx, hipGetLastError());
+                l = e;
+                continue;
+            }
+            // one wide level, in batches, one kernel per phase
+            uint32_t bi = batchOff[l];
+            for (uint32_t b0 = starts[l]; b0 < starts[l + 1]; b0 += std::min<uint32_t>(starts[l + 1] - b0, batchLimit)) {
+                const uint32_t nb = std::min<uint32_t>(starts[l + 1] - b0, batchLimit);
+                const uint32_t steps = batchSteps[bi++];
+                const int gb = (int)((nb + kB - 1) / kB);
+                k_rec_gather<<<gb, kB, 0, st>>>(ra, b0, nb);
+                for (uint32_t s2 = 0; s2 < steps; s2++, step++) {
+                    k_rec_prepare<<<gb, kB, 0, st>>>(ra, b0, nb);
+                    k_rec_insert<<<gb, kB, 0, st>>>(ra, nb);
+                    k_rec_winners<<<gb, kB, 0, st>>>(ra, nb);
+                    k_rec_ids<<<gb, kB, 0, st>>>(ra, b0, nb, step);
+                    k_rec_add_back<<<gb, kB, 0, st>>>(ra, b0, nb);
+                    GLS_HIP(ctx, hipGetLastError());
+                }
+                k_rec_record<<<gb, kB, 0, st>>>(ra, b0, nb);
                 GLS_HIP(ctx, hipGetLastError());
             }
-            k_rec_record<<<nblocks(nb), kB, 0, st>>>(ra, b0, nb);
-            GLS_HIP(ctx, hipGetLastError());
+            l--;
         }
-        l--;
+        k_counter_made<<<1, 1, 0, st>>>(&ctr[8 + (step & 1u)], d_made, firstId, 1u);
+        GLS_HIP(ctx, hipGetLastError());
     }
-    GLS_TRY(stream_copy(ctx, &herr, &ctr[2], sizeof(uint32_t), hipMemcpyDeviceToHost));
+    uint32_t herr = 0;
+    GLS_TRY(stream_copy(ctx, &herr, &ctr[1], sizeof(uint32_t), hipMemcpyDeviceToHost));
     if (herr) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: table overflow (%u)", herr);
 
-    // ---- phase 3: created nodes in id order
-    uint32_t created = 0;
-    GLS_TRY(stream_copy(ctx, &created, &ctr[7], sizeof(uint32_t), hipMemcpyDeviceToHost));
-    unsigned long long *ckeys = t.get<unsigned long long>(created), *ckeysS = t.get<unsigned long long>(created);
-    uint32_t *cids = t.get<uint32_t>(created), *cidsS = t.get<uint32_t>(created);
-    uint32_t *ok = t.get<uint32_t>(cap), *ov = t.get<uint32_t>(cap);
-    if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: output allocation");
-    GLS_HIP(ctx, hipMemsetAsync(d_cnt, 0, sizeof(uint32_t), st));
-    k_created<<<nblocks((int64_t)cap), kB, 0, st>>>(cap, rk, rv, ckeys, cids, d_cnt);
-    uint32_t m = 0;
-    GLS_TRY(stream_copy(ctx, &m, d_cnt, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    if (m != created) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: %u nodes in the table, %u created", m, created);
-    if (m > 0) {
-        size_t tb3 = 0;
-        GLS_HIP(ctx, rocprim::radix_sort_pairs(nullptr, tb3, cids, cidsS, ckeys, ckeysS, (size_t)m, 0u, 32u, st));
-        void *tmp3 = t.get<uint8_t>(tb3);
-        if (!tmp3) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: sort storage");
-        GLS_HIP(ctx, rocprim::radix_sort_pairs(tmp3, tb3, cids, cidsS, ckeys, ckeysS, (size_t)m, 0u, 32u, st));
-    }
-    GLS_HIP(ctx, hipMemsetAsync(ok, 0xFF, sizeof(uint32_t) * cap, st));
-    GLS_HIP(ctx, hipMemsetAsync(ov, 0xFF, sizeof(uint32_t) * cap, st));
-    Tables outMap{nullptr, nullptr, 0, ok, ov, cap - 1};
-    if (m > 0) k_out_map<<<nblocks(m), kB, 0, st>>>((int32_t)m, nPIs, cidsS, outMap, &ctr[2]);
+    // ---- phase 3: output
+    GLS_TRY(stream_copy(ctx, made.data(), d_made, sizeof(uint32_t) * ns, hipMemcpyDeviceToHost));
+    std::vector<uint32_t> outOff(ns + 1, 0u);
+    for (uint32_t k = 0; k < ns; k++) outOff[k + 1] = outOff[k] + made[k];
+    const uint32_t m = outOff[ns];
+    GLS_TRY(stream_copy(ctx, d_outOff, outOff.data(), sizeof(uint32_t) * (ns + 1), hipMemcpyHostToDevice));
     if ((int64_t)nPIs + 1 + m > 0x7FFFFFF0LL) return gls_fail(ctx, GLS_ERR_ARG, "balance: result too large");
     GLS_TRY(dev_graph_alloc(ctx, out, nPIs + 1 + (int32_t)m, nPIs, nPOs));
     uint32_t *tags = nullptr;
@@ -1016,12 +1344,13 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
         if (!tags) { dev_graph_free(ctx, out); return gls_fail(ctx, GLS_ERR_NOMEM, "balance: tags"); }
         *tagOut = tags;
     }
-    k_out_emit<<<nblocks(std::max<int64_t>(m, nPIs + 1)), kB, 0, st>>>((int32_t)m, nPIs, ckeysS, cidsS, outMap,
-                                                                     out.f0, out.f1, out.level, tagIn, tagTab, tags);
-    if (nPOs > 0) k_out_pos<<<nblocks(nPOs), kB, 0, st>>>(nPOs, nPIs, in.pos, newLit, outMap, out.pos);
+    k_out_emit<<<nblocks(std::max<int64_t>(m, nPIs + 1)), kB, 0, st>>>(m, nPIs, ns, d_outOff, d_idBase, cf0, cf1, out.f0,
+                                                                     out.f1, out.level, tagIn, ctag, tags);
+    if (nPOs > 0)
+        k_out_pos<<<nblocks(nPOs), kB, 0, st>>>(nPOs, nPIs, in.pos, newSig, bySeg && tagged ? tagIn : nullptr, d_outOff,
+                                                d_idBase, out.pos);
     GLS_HIP(ctx, hipGetLastError());
-    GLS_TRY(stream_copy(ctx, &herr, &ctr[2], sizeof(uint32_t), hipMemcpyDeviceToHost));
-    if (herr) { dev_graph_free(ctx, out); return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: output map overflow"); }
+    GLS_HIP(ctx, hipStreamSynchronize(st));
     if (info) {
         info->total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         info->levels_enumerated = levels;

@@ -276,7 +276,7 @@ int batch_pass(gls_ctx *ctx, gls_aig **aigs, int32_t count, Pass pass, int32_t u
     std::vector<uint32_t> splitTags;
     int rc = pass == Pass::Strash    ? dev_strash(ctx, U, R, &depth, &info, utag, &rtag, dep)
              : pass == Pass::Rewrite ? dev_rewrite(ctx, U, useZeros, flags, R, &depth, &info, utag, &rtag, dep)
-                                     : dev_balance(ctx, U, R, &info, utag, &rtag, &splitTags);
+                                     : dev_balance(ctx, U, R, &info, utag, &rtag, &splitTags, 1, count);
     if (rtag) pb.ptrs.push_back(rtag);
     if (rc == GLS_ERR_BATCH_SPLIT) {
         // members with a level wider than one balance batch go alone (their

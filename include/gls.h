@@ -243,8 +243,9 @@ int gls_batch_balance(gls_ctx *ctx, gls_aig **aigs, int32_t count, int32_t sort_
  *   strash_wave_batch: wide strash waves launched per host check, 1-64
  *     (default 4);
  *   balance_narrow_max: balance levels of at most this many covers are
- *     rebuilt in one persistent workgroup, wider ones by grid-wide phase
- *     kernels (default 4096);
+ *     rebuilt in one persistent workgroup where they fit its LDS (2048 covers,
+ *     4096 inputs, 3072 possible ANDs), others by grid-wide phase kernels
+ *     (default 4096);
  *   cut_levels: levels per cut launch of the planned schedule
  *     (GLS_RW_PLAN_CUTS, currently disabled), 1-6 (default 3). */
 typedef struct {
