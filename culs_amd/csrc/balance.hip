@@ -79,38 +79,56 @@ __device__ __forceinline__ uint32_t sig_lev(unsigned long long s) { return (uint
 
 // ---------------------------------------------------------------------------
 // table of created nodes: key lit0 << 32 | lit1 (lit0 < lit1) -> positive
-// literal and level of the node (open addressing, linear probing; slot s is
-// the words 2 s, 2 s + 1).  Written with atomics and read past the L1, so a
-// workgroup sees its own insertions after a wait and a barrier.
+// literal and level of the node (open addressing, linear probing; keys and
+// values apart, because most lookups miss).  Written with atomics and read past
+// the L1, so a workgroup sees its own insertions after a wait and a barrier.
 // ---------------------------------------------------------------------------
 struct NodeTable {
-    unsigned long long *w;
+    unsigned long long *k, *v;
     uint64_t mask;
 };
 
-__device__ __forceinline__ unsigned long long t_word(const NodeTable &t, uint64_t i) {
-    return __hip_atomic_load(&t.w[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ unsigned long long t_load(const unsigned long long *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// the node with this key, or EMPTY64; s and k: its first slot and the word there
-__device__ __forceinline__ unsigned long long t_find_from(const NodeTable &t, unsigned long long key, uint64_t s,
-                                                          unsigned long long k) {
+// first slot of a key: three 32-bit products, because a wavefront that hashes
+// its candidates is bound by issue
+__device__ __forceinline__ uint64_t t_hash(const NodeTable &t, unsigned long long key) {
+    uint32_t h = (uint32_t)(key >> 32) * 0x9E3779B1u + (uint32_t)key * 0x85EBCA77u;
+    h = (h ^ h >> 16) * 0xC2B2AE3Du;
+    return (h ^ h >> 15) & t.mask;
+}
+
+// the node with this key, or EMPTY64; k is the key word at its first slot s
+__device__ __forceinline__ unsigned long long t_find_at(const NodeTable &t, unsigned long long key, uint64_t s,
+                                                        unsigned long long k) {
     for (uint64_t probes = 0; probes <= t.mask; probes++) {
-        if (k == key) return t_word(t, 2 * s + 1);
+        if (k == key) return t_load(&t.v[s]);
         if (k == EMPTY64) return EMPTY64;
         s = (s + 1) & t.mask;
-        k = t_word(t, 2 * s);
+        k = t_load(&t.k[s]);
     }
     return EMPTY64;
 }
 
+__device__ __forceinline__ unsigned long long t_find(const NodeTable &t, unsigned long long key) {
+    const uint64_t s = t_hash(t, key);
+    return t_find_at(t, key, s, t_load(&t.k[s]));
+}
+
+__device__ __forceinline__ unsigned long long t_cas(const NodeTable &t, uint64_t s, unsigned long long key) {
+    unsigned long long prev = EMPTY64;
+    __hip_atomic_compare_exchange_strong(&t.k[s], &prev, key, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    return prev;
+}
+
 // slot of the key, inserted if it is new; UNSET if the table is full
 __device__ __forceinline__ uint32_t t_slot(const NodeTable &t, unsigned long long key) {
-    uint64_t s = mix64(key) & t.mask;
+    uint64_t s = t_hash(t, key);
     for (uint64_t probes = 0; probes <= t.mask; probes++, s = (s + 1) & t.mask) {
-        unsigned long long prev = EMPTY64;
-        __hip_atomic_compare_exchange_strong(&t.w[2 * s], &prev, key, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long prev = t_cas(t, s, key);
         if (prev == EMPTY64 || prev == key) return (uint32_t)s;
     }
     return UNSET;
@@ -120,6 +138,7 @@ __device__ __forceinline__ uint32_t t_slot(const NodeTable &t, unsigned long lon
 // The result is one of the two signals or the constant (level 0).
 __device__ __forceinline__ unsigned long long and_trivial(unsigned long long a, unsigned long long b) {
     const uint32_t x = sig_lit(a), y = sig_lit(b);
+    if ((x ^ y) > 1u && min(x, y) > 1u) return EMPTY64;
     if (x == y) return a;
     if (x == (y ^ 1u)) return 0ull;
     if (x == 1u) return b;
@@ -274,7 +293,9 @@ struct SweepArgs {
 constexpr uint32_t DROPPED = 0xFFFFFFFEu;
 
 // Takes root v; add(id, want) appends an input that it was the last parent of
-// (called with want false too: appends go by wavefront).
+// (called with want false too: appends go by wavefront).  Four inputs at a
+// time: a round is bound by the latency of its loads and atomics, not by their
+// number.
 template <class Add>
 __device__ __forceinline__ void sweep_take(const SweepArgs &a, bool has, uint32_t v, uint32_t round, Add add) {
     uint2 c = make_uint2(0u, 0u);
@@ -282,14 +303,14 @@ __device__ __forceinline__ void sweep_take(const SweepArgs &a, bool has, uint32_
         a.lastLevel[v] = a.drop ? DROPPED : round;
         c = a.cover[v];
     }
-    for (uint32_t i = 0; __ballot(i < c.y) != 0; i++) {
-        bool want = false;
-        uint32_t id = 0;
-        if (i < c.y) {
-            id = a.pool[c.x + i] >> 1;
-            want = (int32_t)id > a.nPIs && atomicSub(&a.indeg[id], 1u) == 1u && !(a.drop && (a.mark[id] & RM_PO));
-        }
-        add(id, want);
+    for (uint32_t i = 0; __ballot(i < c.y) != 0; i += 4) {
+        uint32_t id[4], left[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) id[j] = i + j < c.y ? a.pool[c.x + i + j] >> 1 : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) left[j] = (int32_t)id[j] > a.nPIs ? atomicSub(&a.indeg[id[j]], 1u) : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) add(id[j], left[j] == 1u && !(a.drop && (a.mark[id[j]] & RM_PO)));
     }
 }
 
@@ -304,9 +325,15 @@ __global__ void k_sweep_first(uint32_t nRoots, const uint32_t *__restrict__ root
         const uint32_t v = has ? roots[i] : 0u;
         const bool want = has && a.indeg[v] == 0u && a.lastLevel[v] == UNSET && ((a.mark[v] & RM_PO) == 0) == (a.drop != 0);
         if (tag) {
-            if (want) {
-                const uint32_t s = tag[v];
-                a.front[0][segFirst[s] + atomicAdd(&segLen[s], 1u)] = v;
+            // roots are in id order, so a wavefront's are mostly of one segment:
+            // one append per segment
+            const uint32_t s = has ? tag[v] : 0u;
+            for (uint64_t left = __ballot(want); left;) {
+                const uint32_t seg = (uint32_t)__shfl((int)s, __ffsll((unsigned long long)left) - 1);
+                const bool mine = want && s == seg;
+                const uint32_t q = wave_append(&segLen[seg], mine);
+                if (mine) a.front[0][segFirst[seg] + q] = v;
+                left &= ~__ballot(mine);
             }
         } else {
             const uint32_t q = wave_append(segLen, want);
@@ -396,12 +423,15 @@ __global__ void k_key_starts(uint32_t m, const uint32_t *__restrict__ keys, uint
     }
 }
 
-// every cover's inputs, and the most ANDs it can create (none from a constant)
+constexpr uint32_t SRC_MEM = 0xFFFFu;
+
+// every root's place, its cover's inputs, and the most ANDs it can create (none from a constant)
 __global__ void k_cover_lens(uint32_t m, const uint32_t *__restrict__ roots, const uint2 *__restrict__ cover,
-                             uint32_t *len, uint32_t *most) {
+                             uint32_t *len, uint32_t *most, uint32_t *place) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= m; i += stride) {
         const uint32_t k = i < m ? cover[roots[i]].y : 0u;
+        if (i < m) place[roots[i]] = (uint32_t)i;
         len[i] = k;
         most[i] = k ? k - 1u : 0u;
     }
@@ -409,26 +439,40 @@ __global__ void k_cover_lens(uint32_t m, const uint32_t *__restrict__ roots, con
 
 // the covers' inputs in the order in which they are rebuilt
 __global__ void k_pack_inputs(uint32_t m, const uint32_t *__restrict__ roots, const uint2 *__restrict__ cover,
-                              const uint32_t *__restrict__ pool, const uint32_t *__restrict__ off, uint32_t *in) {
+                              const uint32_t *__restrict__ pool, const uint32_t *__restrict__ off,
+                              const uint32_t *__restrict__ keys, const uint32_t *__restrict__ starts,
+                              const uint32_t *__restrict__ lastLevel, const uint32_t *__restrict__ place, int32_t nPIs,
+                              uint32_t *in, uint32_t *src) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m; i += stride) {
-        const uint2 c = cover[roots[i]];
-        for (uint32_t j = 0; j < c.y; j++) in[off[i] + j] = pool[c.x + j];
+        const uint32_t v = roots[i], lv = lastLevel[v], key = keys[i], cov = ((uint32_t)i - starts[key]) & 0xFFFFu;
+        const uint2 c = cover[v];
+        for (uint32_t j = 0; j < c.y; j++) {
+            const uint32_t lit = pool[c.x + j], id = lit >> 1;
+            uint32_t at = SRC_MEM;
+            if ((int32_t)id > nPIs && lastLevel[id] == lv + 1u) at = min(place[id] - starts[key + 1u], SRC_MEM);
+            in[off[i] + j] = lit;
+            src[off[i] + j] = at << 16 | cov;
+        }
     }
 }
 
-// largest level: covers, inputs, ANDs it can create; and per level the inputs
-// and the ANDs
+// largest level: covers, inputs, ANDs it can create; and per level its extent
+struct LevelRec {
+    uint32_t s, nb, in0, T;           // first root, roots, first input, inputs
+    uint32_t most, pad[3];            // ANDs it can create
+};
+
 __global__ void k_level_sizes(uint32_t nKeys, const uint32_t *__restrict__ starts, const uint32_t *__restrict__ off,
-                              const uint32_t *__restrict__ newOff, uint2 *levSize, uint32_t *most) {
+                              const uint32_t *__restrict__ newOff, LevelRec *rec, uint32_t *most) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < nKeys; k += stride) {
         const uint32_t a = starts[k], b = starts[k + 1];
-        const uint2 z = make_uint2(off[b] - off[a], newOff[b] - newOff[a]);
-        levSize[k] = z;
-        atomicMax(&most[0], b - a);
-        atomicMax(&most[1], z.x);
-        atomicMax(&most[2], z.y);
+        const LevelRec z = {a, b - a, off[a], off[b] - off[a], newOff[b] - newOff[a], {}};
+        rec[k] = z;
+        atomicMax(&most[0], z.nb);
+        atomicMax(&most[1], z.T);
+        atomicMax(&most[2], z.most);
     }
 }
 
@@ -440,7 +484,8 @@ struct RecArgs {
     int32_t nPIs;
     const uint32_t *roots;            // roots by (segment, level, id)
     const uint32_t *off, *in;         // their covers' inputs
-    const uint2 *levSize;             // per (segment, level): inputs, ANDs it can create
+    const uint32_t *src;              // per input: place of its root in the level before << 16 (SRC_MEM: not there) | cover
+    const LevelRec *lev;              // per (segment, level)
     const uint32_t *starts;           // first root of every (segment, level)
     unsigned long long *newSig;       // per root id: the result
     uint32_t *of0, *of1;              // fanins of the created nodes, by id
@@ -505,6 +550,11 @@ __device__ __forceinline__ bool sorts_before(uint32_t shuffle, unsigned long lon
     return !shuffle && culs_val(sig_lit(a)) > culs_val(sig_lit(b));
 }
 
+// the same as a number: a stands before b if its key is larger
+__device__ __forceinline__ unsigned long long order_key(uint32_t shuffle, unsigned long long a) {
+    return (unsigned long long)sig_lev(a) << 32 | (shuffle ? 0u : culs_val(sig_lit(a)));
+}
+
 __device__ __forceinline__ unsigned long long input_sig(const RecArgs &r, uint32_t lit) {
     const uint32_t id = lit >> 1;
     return (int32_t)id <= r.nPIs ? sig(lit, 0u) : r.newSig[id] ^ (lit & 1u);
@@ -515,230 +565,487 @@ constexpr uint32_t LT_INPUTS = 4096;      // inputs of a level
 constexpr uint32_t LT_COVERS = 2048;      // covers of a level
 constexpr uint32_t LT_NEW = 3072;         // ANDs that a level can create
 constexpr uint32_t LT_HASH = 4096;        // entries of the level's own node table
-constexpr uint32_t LN_FINAL = 0x80000000u;
+constexpr uint32_t LQ_IN = LT_INPUTS / BAL_WG, LQ_COV = LT_COVERS / BAL_WG, LQ_NEW = LT_NEW / BAL_WG;
+constexpr uint32_t LN_FINAL = 0x80000000u, LS_NONE = 0xFFFFu;
 
 // Rebuilds levels lFirst, lFirst - 1, .., lLast of its segment (levOff: the
 // segments' first levels in starts; levels beyond the segment's are skipped).
-// A level's cover inputs, sorted by rank among the cover's, and the nodes it
-// creates live in LDS; the table in memory holds the nodes of the levels
-// before and takes this level's at its end, so a pair with a literal of this
-// level is looked up in LDS only.  The candidates of the permutation are looked
-// up four at a time.  Per step three barriers: keys inserted; winners (the
-// smallest cover index of a key) counted; ids given.
-// What bounds it: a level costs three dependent trips to memory (inputs,
-// their results, lookups) and the insertions, and a step some LDS trips,
-// whatever the number of covers; measured before: 83 us per level of 675
-// covers and six steps with all state and every lookup in memory.
+// A level's cover inputs and the nodes it creates live in LDS; the table in
+// memory holds the nodes of the levels before.  A pair of a cover's inputs is
+// looked up there once, before the steps: the partner that the permutation may
+// try for input j has the level of input j - 1 (the list is consumed from its
+// end, and what a step puts back does not separate inputs of one level), so
+// each input tries those, four at a time, and the ones that exist enter the
+// level's own table.  The steps then look up in LDS only, except a cover whose
+// pair was found once: what came back may be an older node, and the permutation
+// may have changed which inputs meet, so its later pairs are looked up in
+// memory as well.  A step has three barriers: keys inserted; winners (the
+// smallest cover index of a key) counted; ids given; and once 64 covers at most
+// have a pair left, one wavefront takes the remaining steps without any.
+// What bounds it is latency, so little is left between two levels: results of
+// the level before come from LDS, other inputs are read during its steps, its
+// table insertions are under way until the lookups, and only used entries of
+// the level's table are cleared.  Cycles per level of 2M random ANDs (1795
+// levels of 668 covers and 1523 inputs): 68000, of which 12000 to place and
+// sort the inputs, 13000 for the pairs, 20000 for two full steps, 17000 for 3.9
+// more; 88000 with every lookup made at its step in memory (46 and 63 ms in
+// all).  A level of the 64-bit multiplier (77 covers, 161 inputs): 24000 and
+// 27000.  Limiting the later memory lookups pair by pair made no difference.
 __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *__restrict__ levOff,
                                                     const uint32_t *__restrict__ idBase, uint32_t *made, int32_t lFirst,
                                                     int32_t lLast) {
     __shared__ unsigned long long s_key[LT_HASH];
-    __shared__ uint32_t s_val[LT_HASH];              // smallest cover index, then LN_FINAL | node of the level
+    __shared__ uint32_t s_val[LT_HASH];              // smallest cover index, then LN_FINAL | node
     __shared__ unsigned long long s_arr[LT_INPUTS];  // the covers' current inputs
-    __shared__ uint32_t s_nlev[LT_NEW];
-    __shared__ uint16_t s_cov[LT_INPUTS], s_off[LT_COVERS + 1], s_len[LT_COVERS], s_slot[LT_COVERS];
-    __shared__ uint32_t s_wcnt[2][BAL_WG / 64];
+    __shared__ unsigned long long s_node[LT_NEW];    // nodes: created from 0 up, found in memory from the top down
+    __shared__ unsigned long long s_res[LT_COVERS];  // the covers' results, for the next level
+    __shared__ uint16_t s_ent[LT_NEW];               // the nodes' entries in s_key, LS_NONE: another one has it
+    __shared__ uint16_t s_perm[LT_INPUTS];           // `b -s`: the shuffled inputs
+    __shared__ uint16_t s_off[LT_COVERS + 1], s_len[LT_COVERS], s_slot[LT_COVERS], s_act[64];
+    __shared__ uint8_t s_mem[LT_COVERS];             // the cover's pairs are looked up in memory too
+    __shared__ uint32_t s_cnt[LQ_COV][BAL_WG / 64], s_over;
+    __shared__ int32_t s_top;
     const uint32_t tid = threadIdx.x, seg = blockIdx.x, wave = tid >> 6, lane = tid & 63u;
     const uint32_t lev0 = levOff[seg], nLev = levOff[seg + 1] - lev0, base0 = idBase[seg];
     uint32_t counter = base0 + made[seg];            // next id
-    for (int32_t l = min(lFirst, (int32_t)nLev - 1); l >= lLast; l--) {
-        const uint32_t s = r.starts[lev0 + l], nb = r.starts[lev0 + l + 1] - s;
-        const uint32_t in0 = r.off[s], T = r.off[s + nb] - in0;
-        const uint32_t levBase = counter;
-        // a power of two with room for every AND the level can create (LT_NEW at most)
-        const uint32_t most = r.levSize[lev0 + l].y;
-        uint32_t hsize = 256;
-        while (hsize < LT_HASH && hsize < 2u * most) hsize <<= 1;
-        // covers' ranges, and every input's cover
-        for (uint32_t c = tid; c < nb; c += BAL_WG) {
-            const uint32_t o = r.off[s + c] - in0, e = r.off[s + c + 1] - in0;
-            s_off[c] = (uint16_t)o;
-            s_len[c] = (uint16_t)(e - o);
-            for (uint32_t j = o; j < e; j++) s_cov[j] = (uint16_t)c;
-            if (r.shuffle && e > o) {
-                // `b -s`: the inputs in the order of the shuffle seeded with
-                // the cover's index in its batch
-                const ThrustShuffle sh(e - o, c);
-                uint32_t k = o;
-                for (uint32_t j = 0; j < sh.span && k < e; j++) {
-                    const uint32_t src = sh(j);
-                    if (src < e - o) s_arr[k++] = input_sig(r, r.in[in0 + o + src]);
-                }
-            }
-        }
-        if (tid == 0) s_off[nb] = (uint16_t)T;
-        for (uint32_t i = tid; i < hsize; i += BAL_WG) { s_key[i] = EMPTY64; s_val[i] = UNSET; }
-        unsigned long long mine[LT_INPUTS / BAL_WG];
-        if (!r.shuffle) {
+    // a level's extent, its inputs (one per thread and LQ_IN), its covers' first
+    // inputs and roots
+    struct Level {
+        LevelRec e;
+        uint32_t lit[LQ_IN], src[LQ_IN], off[LQ_COV], root[LQ_COV];
+        unsigned long long sig[LQ_IN];
+    };
+    auto load_extent = [&](int32_t l) -> LevelRec {
+        LevelRec e = {};
+        if (l >= lLast) e = r.lev[lev0 + l];
+        return e;
+    };
+    auto load_level = [&](const LevelRec &e, Level &v) {
+        v.e = e;
 #pragma unroll
-            for (uint32_t q = 0; q < LT_INPUTS / BAL_WG; q++) {
-                const uint32_t i = tid + q * BAL_WG;
-                mine[q] = i < T ? input_sig(r, r.in[in0 + i]) : 0ull;
-            }
-#pragma unroll
-            for (uint32_t q = 0; q < LT_INPUTS / BAL_WG; q++)
-                if (tid + q * BAL_WG < T) s_arr[tid + q * BAL_WG] = mine[q];
-        }
-        __syncthreads();
-        // each input's place in its cover's order
-        uint32_t place[LT_INPUTS / BAL_WG];
-#pragma unroll
-        for (uint32_t q = 0; q < LT_INPUTS / BAL_WG; q++) {
+        for (uint32_t q = 0; q < LQ_IN; q++) {
             const uint32_t i = tid + q * BAL_WG;
-            place[q] = i;
-            if (i < T) {
-                if (r.shuffle) mine[q] = s_arr[i];
-                const uint32_t c = s_cov[i], o = s_off[c], e = s_off[c + 1];
-                uint32_t p = o;
-                for (uint32_t j = o; j < e; j++) {
-                    const unsigned long long x = s_arr[j];
-                    p += (sorts_before(r.shuffle, x, mine[q]) || (j < i && !sorts_before(r.shuffle, mine[q], x))) ? 1u : 0u;
-                }
-                place[q] = p;
+            v.lit[q] = i < e.T ? r.in[e.in0 + i] : 0u;
+            v.src[q] = i < e.T ? r.src[e.in0 + i] : 0u;
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_COV; q++) {
+            const uint32_t c = tid + q * BAL_WG;
+            v.off[q] = c < e.nb ? r.off[e.s + c] - e.in0 : 0u;
+            v.root[q] = c < e.nb ? r.roots[e.s + c] : 0u;
+        }
+    };
+    // the inputs that are not results of the level before (first: all), without
+    // their complement: nothing is to wait for them here
+    auto load_inputs = [&](bool first, Level &v) {
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_IN; q++) {
+            v.sig[q] = 0;
+            if (tid + q * BAL_WG >= v.e.T) continue;
+            if (first) v.src[q] |= SRC_MEM << 16;
+            const uint32_t id = v.lit[q] >> 1;
+            if ((int32_t)id <= r.nPIs) v.sig[q] = sig(2u * id, 0u);
+            else if (v.src[q] >> 16 == SRC_MEM) v.sig[q] = r.newSig[id];
+        }
+    };
+    for (uint32_t i = tid; i < LT_HASH; i += BAL_WG) { s_key[i] = EMPTY64; s_val[i] = UNSET; }
+    int32_t l = min(lFirst, (int32_t)nLev - 1);
+    Level cur, next;
+    load_level(load_extent(l), cur);
+    LevelRec ahead = load_extent(l - 1);     // extents come two levels ahead, inputs one
+    load_inputs(true, cur);
+    // the level before's nodes, on their way into the table
+    unsigned long long newKey[LQ_NEW], newNode[LQ_NEW], newPrev[LQ_NEW];
+    uint32_t newSlot[LQ_NEW];
+#pragma unroll
+    for (uint32_t q = 0; q < LQ_NEW; q++) newKey[q] = EMPTY64;
+    auto finish_inserts = [&]() {
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_NEW; q++) {
+            if (newKey[q] == EMPTY64) continue;
+            uint64_t probes = 0;
+            while (newPrev[q] != EMPTY64 && newPrev[q] != newKey[q] && probes++ <= r.t.mask) {
+                newSlot[q] = (uint32_t)((newSlot[q] + 1ull) & r.t.mask);
+                newPrev[q] = t_cas(r.t, newSlot[q], newKey[q]);
             }
+            if (newPrev[q] != EMPTY64 && newPrev[q] != newKey[q]) { atomicOr(r.err, 2u); continue; }
+            __hip_atomic_store(&r.t.v[newSlot[q]], newNode[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    };
+    for (; l >= lLast; l--) {
+        const uint32_t nb = cur.e.nb, T = cur.e.T, most = cur.e.most, levBase = counter;
+        load_level(ahead, next);
+        ahead = load_extent(l - 2);
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_COV; q++) {
+            const uint32_t c = tid + q * BAL_WG;
+            if (c < nb) { s_off[c] = (uint16_t)cur.off[q]; s_mem[c] = 0; }
+        }
+        if (tid == 0) { s_off[nb] = (uint16_t)T; s_top = (int32_t)LT_NEW; s_over = 0; }
+        unsigned long long mine[LQ_IN];
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_IN; q++) {
+            mine[q] = cur.sig[q];
+            if (tid + q * BAL_WG >= T) continue;
+            if (cur.src[q] >> 16 != SRC_MEM) mine[q] = s_res[cur.src[q] >> 16];
+            mine[q] ^= cur.lit[q] & 1u;
+            s_arr[tid + q * BAL_WG] = mine[q];
+        }
+        __syncthreads();
+        if (r.shuffle) {
+            // `b -s`: the inputs in the order of the shuffle seeded with the
+            // cover's index in its batch
+            for (uint32_t c = tid; c < nb; c += BAL_WG) {
+                const uint32_t o = s_off[c], n = s_off[c + 1] - o;
+                if (n == 0) continue;
+                const ThrustShuffle sh(n, c);
+                uint32_t k = 0;
+                for (uint32_t j = 0; j < sh.span && k < n; j++) {
+                    const uint32_t src = sh(j);
+                    if (src < n) s_perm[o + k++] = (uint16_t)(o + src);
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t q = 0; q < LQ_IN; q++)
+                if (tid + q * BAL_WG < T) mine[q] = s_arr[s_perm[tid + q * BAL_WG]];
+            __syncthreads();
+#pragma unroll
+            for (uint32_t q = 0; q < LQ_IN; q++)
+                if (tid + q * BAL_WG < T) s_arr[tid + q * BAL_WG] = mine[q];
+            __syncthreads();
+        }
+        // each input's place by its rank among the cover's
+        uint32_t place[LQ_IN];
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_IN; q++) {
+            const uint32_t i = tid + q * BAL_WG;
+            place[q] = UNSET;
+            if (i >= T) continue;
+            const uint32_t c = cur.src[q] & 0xFFFFu, o = s_off[c], e = s_off[c + 1];
+            const unsigned long long x = order_key(r.shuffle, mine[q]);
+            uint32_t p = o;
+            for (uint32_t j = o; j < e; j += 2) {
+                const unsigned long long y0 = order_key(r.shuffle, s_arr[j]);
+                const unsigned long long y1 = order_key(r.shuffle, s_arr[min(j + 1, e - 1)]);
+                p += y0 > x || (y0 == x && j < i) ? 1u : 0u;
+                p += j + 1 < e && (y1 > x || (y1 == x && j + 1 < i)) ? 1u : 0u;
+            }
+            place[q] = p;
         }
         __syncthreads();
 #pragma unroll
-        for (uint32_t q = 0; q < LT_INPUTS / BAL_WG; q++)
-            if (tid + q * BAL_WG < T) s_arr[place[q]] = mine[q];
+        for (uint32_t q = 0; q < LQ_IN; q++)
+            if (place[q] != UNSET) s_arr[place[q]] = mine[q];
+        for (uint32_t c = tid; c < nb; c += BAL_WG) s_len[c] = (uint16_t)(s_off[c + 1] - s_off[c]);
+        finish_inserts();
+        __builtin_amdgcn_s_waitcnt(0x0F70);     // vmcnt(0): the table's words and the level before's results are written
         __syncthreads();
-        // a node of this level with this key, or EMPTY64
-        auto level_find = [&](unsigned long long key) -> unsigned long long {
-            for (uint32_t h = (uint32_t)mix64(key) & (hsize - 1);; h = (h + 1) & (hsize - 1)) {
-                const unsigned long long k = *(volatile unsigned long long *)&s_key[h];
-                if (k == EMPTY64) return EMPTY64;
-                if (k != key) continue;
-                const uint32_t v = *(volatile uint32_t *)&s_val[h];
-                // inserted in this step: not there yet
-                if (v == UNSET || !(v & LN_FINAL)) return EMPTY64;
-                return sig(2u * (levBase + (v & ~LN_FINAL)), s_nlev[v & ~LN_FINAL]);
+        // the level's own table
+        auto hash = [](unsigned long long key) -> uint32_t {
+            const uint32_t h = (uint32_t)(key >> 32) * 0x9E3779B1u + (uint32_t)key;
+            return (h ^ h >> 15) & (LT_HASH - 1);
+        };
+        auto level_slot = [&](unsigned long long key, bool &isNew) -> uint32_t {
+            for (uint32_t h = hash(key);; h = (h + 1) & (LT_HASH - 1)) {
+                unsigned long long prev = EMPTY64;
+                __hip_atomic_compare_exchange_strong(&s_key[h], &prev, key, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+                isNew = prev == EMPTY64;
+                if (isNew || prev == key) return h;
             }
         };
-        // addBackLocalArrays (balance.cu:429-467)
-        auto add_back = [&](uint32_t c, unsigned long long x) {
-            const uint32_t o = s_off[c], L = s_len[c];
-            for (uint32_t i = 0; i < L; i++)
-                if (sig_lit(s_arr[o + i]) == sig_lit(x)) return;
+        // its node with this key, or EMPTY64; k is the key at its first entry h
+        auto level_find = [&](unsigned long long key, uint32_t h, unsigned long long k) -> unsigned long long {
+            for (;;) {
+                if (k == EMPTY64) return EMPTY64;
+                if (k == key) {
+                    const uint32_t v = *(volatile uint32_t *)&s_val[h];
+                    // inserted in this step: not there yet
+                    return v == UNSET || !(v & LN_FINAL) ? EMPTY64 : s_node[v & ~LN_FINAL];
+                }
+                h = (h + 1) & (LT_HASH - 1);
+                k = *(volatile unsigned long long *)&s_key[h];
+            }
+        };
+        // pairs of inputs that exist
+#pragma unroll
+        for (uint32_t g = 0; g < LQ_IN; g++) {
+            const uint32_t j = tid + g * BAL_WG;
+            if (g * BAL_WG >= T) break;
+            uint32_t o = 0, left = 0;        // candidates [o, left)
+            unsigned long long x = 0;
+            uint32_t border = 0;
+            if (j < T) {
+                // position j's cover is input j's: the order is within covers
+                o = s_off[cur.src[g] & 0xFFFFu];
+                left = j;
+                x = s_arr[j];
+                border = j > o ? sig_lev(s_arr[j - 1]) : 0u;
+            }
+            while (__ballot(left > o) != 0) {
+                unsigned long long key[4];
+                uint64_t slot[4];
+                uint32_t wait = 0;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    key[q] = EMPTY64;
+                    slot[q] = 0;
+                    if (left <= o) continue;
+                    const unsigned long long y = s_arr[left - 1];
+                    if (sig_lev(y) != border) { left = o; continue; }
+                    left--;
+                    if (and_trivial(x, y) != EMPTY64) continue;
+                    key[q] = and_key_of(sig_lit(x), sig_lit(y));
+                    slot[q] = t_hash(r.t, key[q]);
+                    wait |= 1u << q;
+                }
+                while (__ballot(wait != 0) != 0) {
+                    unsigned long long k[4];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) k[q] = (wait >> q) & 1u ? t_load(&r.t.k[slot[q]]) : EMPTY64;
+                    uint32_t hit = 0;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        if (k[q] == EMPTY64) wait &= ~(1u << q);
+                        if (k[q] == key[q] && ((wait >> q) & 1u)) hit |= 1u << q;
+                        slot[q] = (slot[q] + 1) & r.t.mask;
+                    }
+                    wait &= ~hit;
+                    while (hit) {
+                        const int q = __ffs((int)hit) - 1;
+                        hit &= hit - 1u;
+                        const unsigned long long kq = q < 2 ? (q == 0 ? key[0] : key[1]) : (q == 2 ? key[2] : key[3]);
+                        const uint64_t sq = q < 2 ? (q == 0 ? slot[0] : slot[1]) : (q == 2 ? slot[2] : slot[3]);
+                        // nodes found and created together at most LT_NEW (so the table has room)
+                        const int32_t at = atomicSub(&s_top, 1) - 1;
+                        if (at < (int32_t)most) { s_over = 1; continue; }
+                        bool isNew = false;
+                        const uint32_t h = level_slot(kq, isNew);
+                        s_ent[at] = isNew ? (uint16_t)h : (uint16_t)LS_NONE;
+                        if (isNew) {
+                            s_node[at] = t_load(&r.t.v[(sq - 1) & r.t.mask]);
+                            s_val[h] = LN_FINAL | (uint32_t)at;
+                        }
+                    }
+                }
+            }
+        }
+        load_inputs(false, next);
+        __syncthreads();
+        const bool over = s_over != 0;       // not all of them fit: every cover looks up in memory too
+        // sharedNodeDrivenPermute and prepareDataToInsert (balance.cu:113-247)
+        // of a cover with two inputs at least: takes its last two; returns the
+        // existing signal, or EMPTY64 and the slot of the inserted key
+        auto prepare = [&](uint32_t c, uint32_t o, uint32_t L, uint32_t &slot) -> unsigned long long {
+            const uint32_t right = o + L - 2;
+            const unsigned long long l1 = s_arr[right + 1], l2 = s_arr[right];
+            const uint32_t x1 = sig_lit(l1), border = sig_lev(l2);
+            const bool old1 = (over || s_mem[c] != 0) && (x1 >> 1) < levBase;
+            unsigned long long found = EMPTY64, l3 = l2;
+            for (uint32_t i = right;;) {
+                const unsigned long long before = s_arr[i > o ? i - 1 : o], key = and_key_of(x1, sig_lit(l3));
+                const uint32_t h = hash(key);
+                const unsigned long long k = *(volatile unsigned long long *)&s_key[h];
+                found = and_trivial(l1, l3);
+                if (found == EMPTY64 && k != EMPTY64) found = level_find(key, h, k);
+                if (found == EMPTY64 && old1 && (sig_lit(l3) >> 1) < levBase) found = t_find(r.t, key);
+                if (found != EMPTY64) {
+                    s_arr[i] = l2;           // the partner goes next to last; the order by level stays
+                    break;
+                }
+                if (i == o || sig_lev(before) != border) break;
+                i--;
+                l3 = before;
+            }
+            slot = 0;
+            if (found == EMPTY64) {
+                const unsigned long long key = and_key_of(x1, sig_lit(l2));
+                bool isNew;
+                const uint32_t h = level_slot(key, isNew);
+                atomicMin(&s_val[h], c);
+                slot = h + 1;
+                s_arr[right + 1] = key;                  // the popped pair, and its level
+                s_arr[right] = (sig_lev(l1) > border ? sig_lev(l1) : border) + 1u;
+            } else {
+                s_mem[c] = 1;
+            }
+            return found;
+        };
+        // the winner of a key becomes node `at` of the level
+        auto create = [&](uint32_t c, uint32_t o, uint32_t L, uint32_t slot, uint32_t at) {
+            const unsigned long long key = s_arr[o + L + 1];
+            const uint32_t id = levBase + at;
+            s_node[at] = sig(2u * id, (uint32_t)s_arr[o + L]);
+            s_val[slot - 1] = LN_FINAL | at;
+            s_ent[at] = (uint16_t)(slot - 1);
+            r.of0[id] = (uint32_t)(key >> 32);
+            r.of1[id] = (uint32_t)key;
+            if (r.tagOut) r.tagOut[id] = r.tagIn[r.roots[cur.e.s + c]];
+        };
+        // addBackLocalArrays (balance.cu:429-467); returns the new length
+        auto add_back = [&](uint32_t o, uint32_t L, unsigned long long x) -> uint32_t {
+            for (uint32_t i = 0; i < L; i += 2)
+                if (sig_lit(s_arr[o + i]) == sig_lit(x) || sig_lit(s_arr[o + min(i + 1, L - 1)]) == sig_lit(x)) return L;
             uint32_t i = L;
-            while (i > 0 && sig_lev(x) > sig_lev(s_arr[o + i - 1])) {
-                s_arr[o + i] = s_arr[o + i - 1];
+            while (i > 0) {
+                const unsigned long long y = s_arr[o + i - 1];
+                if (sig_lev(x) <= sig_lev(y)) break;
+                s_arr[o + i] = y;
                 i--;
             }
             s_arr[o + i] = x;
-            s_len[c] = (uint16_t)(L + 1);
+            return L + 1;
         };
-        for (;;) {
-            // sharedNodeDrivenPermute and prepareDataToInsert (balance.cu:113-247)
-            int active = 0;
+        // ---- steps by all wavefronts, while more than 64 covers have a pair left
+        uint32_t nAct = nb;
+        if (nb <= 64u && tid < 64u) s_act[tid] = (uint16_t)tid;
+        while (nAct > 64u) {
             for (uint32_t c = tid; c < nb; c += BAL_WG) {
                 const uint32_t o = s_off[c], L = s_len[c];
                 s_slot[c] = 0;
                 if (L <= 1) continue;
-                active = 1;
-                const int right = (int)L - 2;
-                int left = right;
-                const uint32_t border = sig_lev(s_arr[o + right]);
-                while (left > 0 && sig_lev(s_arr[o + left - 1]) == border) left--;
-                const unsigned long long l1 = s_arr[o + L - 1], l2 = s_arr[o + right];
-                const uint32_t x1 = sig_lit(l1);
-                const bool old1 = (x1 >> 1) < levBase;
-                unsigned long long found = EMPTY64;
-                for (int i = right; i >= left && found == EMPTY64; i -= 4) {
-                    unsigned long long l3[4], key[4], k0[4];
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        l3[q] = i - q >= left ? s_arr[o + i - q] : l1;
-                        key[q] = and_key_of(x1, sig_lit(l3[q]));
-                        const bool old = old1 && (sig_lit(l3[q]) >> 1) < levBase && i - q >= left;
-                        k0[q] = old ? t_word(r.t, 2 * (mix64(key[q]) & r.t.mask)) : EMPTY64;
-                    }
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        if (found != EMPTY64 || i - q < left) continue;
-                        unsigned long long f = and_trivial(l1, l3[q]);
-                        if (f == EMPTY64) f = level_find(key[q]);
-                        if (f == EMPTY64 && k0[q] != EMPTY64)
-                            f = t_find_from(r.t, key[q], mix64(key[q]) & r.t.mask, k0[q]);
-                        if (f == EMPTY64) continue;
-                        found = f;
-                        // the partner goes next to last; the order by level stays
-                        s_arr[o + i - q] = l2;
-                    }
-                }
-                s_len[c] = (uint16_t)(L - 2);
-                if (found != EMPTY64) {
-                    add_back(c, found);
-                    continue;
-                }
-                const unsigned long long key = and_key_of(x1, sig_lit(l2));
-                const uint32_t lv = (sig_lev(l1) > sig_lev(l2) ? sig_lev(l1) : sig_lev(l2)) + 1u;
-                uint32_t h = (uint32_t)mix64(key) & (hsize - 1);
-                for (;; h = (h + 1) & (hsize - 1)) {
-                    unsigned long long prev = EMPTY64;
-                    __hip_atomic_compare_exchange_strong(&s_key[h], &prev, key, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_WORKGROUP);
-                    if (prev == EMPTY64 || prev == key) break;
-                }
-                atomicMin(&s_val[h], c);
-                s_slot[c] = (uint16_t)(h + 1);
-                s_arr[o + L - 1] = key;                  // the popped pair, and its level
-                s_arr[o + right] = lv;
+                uint32_t slot;
+                const unsigned long long f = prepare(c, o, L, slot);
+                s_slot[c] = (uint16_t)slot;
+                s_len[c] = (uint16_t)(slot ? L - 2 : add_back(o, L - 2, f));
             }
-            if (!__syncthreads_or(active)) break;
+            __syncthreads();
             // winners, counted in cover order
-            uint32_t rank[LT_COVERS / BAL_WG];
+            uint32_t rank[LQ_COV];
 #pragma unroll
-            for (uint32_t q = 0; q < LT_COVERS / BAL_WG; q++) {
+            for (uint32_t q = 0; q < LQ_COV; q++) {
                 const uint32_t c = tid + q * BAL_WG;
                 const bool win = c < nb && s_slot[c] != 0 && s_val[s_slot[c] - 1] == c;
                 const uint64_t m = __ballot(win);
                 rank[q] = win ? (uint32_t)__popcll(m & ((1ull << lane) - 1ull)) : UNSET;
-                if (lane == 0) s_wcnt[q][wave] = (uint32_t)__popcll(m);
+                if (lane == 0) s_cnt[q][wave] = (uint32_t)__popcll(m);
             }
             __syncthreads();
             uint32_t total = 0;
 #pragma unroll
-            for (uint32_t q = 0; q < LT_COVERS / BAL_WG; q++) {
+            for (uint32_t q = 0; q < LQ_COV; q++) {
                 uint32_t before = total;
+#pragma unroll
                 for (uint32_t w = 0; w < BAL_WG / 64; w++) {
-                    const uint32_t x = s_wcnt[q][w];
+                    const uint32_t x = s_cnt[q][w];
                     before += w < wave ? x : 0u;
                     total += x;
                 }
                 if (rank[q] != UNSET) {
-                    const uint32_t c = tid + q * BAL_WG, o = s_off[c], L = s_len[c];
-                    const uint32_t id = counter + before + rank[q];
-                    const unsigned long long key = s_arr[o + L + 1];
-                    s_nlev[id - levBase] = (uint32_t)s_arr[o + L];
-                    s_val[s_slot[c] - 1] = LN_FINAL | (id - levBase);
-                    r.of0[id] = (uint32_t)(key >> 32);
-                    r.of1[id] = (uint32_t)key;
-                    if (r.tagOut) r.tagOut[id] = r.tagIn[r.roots[s + c]];
+                    const uint32_t c = tid + q * BAL_WG;
+                    create(c, s_off[c], s_len[c], s_slot[c], counter - levBase + before + rank[q]);
                 }
             }
             counter += total;
             __syncthreads();
-            for (uint32_t c = tid; c < nb; c += BAL_WG)
-                if (s_slot[c] != 0) {
-                    const uint32_t v = s_val[s_slot[c] - 1] & ~LN_FINAL;
-                    add_back(c, sig(2u * (levBase + v), s_nlev[v]));
+            // results back; the covers that still have a pair, counted
+            uint64_t am[LQ_COV];
+#pragma unroll
+            for (uint32_t q = 0; q < LQ_COV; q++) {
+                const uint32_t c = tid + q * BAL_WG;
+                bool more = false;
+                if (c < nb) {
+                    uint32_t L = s_len[c];
+                    if (s_slot[c] != 0) {
+                        L = add_back(s_off[c], L, s_node[s_val[s_slot[c] - 1] & ~LN_FINAL]);
+                        s_len[c] = (uint16_t)L;
+                    }
+                    more = L > 1;
                 }
+                am[q] = __ballot(more);
+                if (lane == 0) s_cnt[q][wave] = (uint32_t)__popcll(am[q]);
+            }
+            __syncthreads();
+            nAct = 0;
+            uint32_t before[LQ_COV];
+#pragma unroll
+            for (uint32_t q = 0; q < LQ_COV; q++) {
+                before[q] = nAct;
+#pragma unroll
+                for (uint32_t w = 0; w < BAL_WG / 64; w++) {
+                    const uint32_t x = s_cnt[q][w];
+                    before[q] += w < wave ? x : 0u;
+                    nAct += x;
+                }
+            }
+            if (nAct > 64u) continue;
+#pragma unroll
+            for (uint32_t q = 0; q < LQ_COV; q++)
+                if ((am[q] >> lane) & 1ull)
+                    s_act[before[q] + (uint32_t)__popcll(am[q] & ((1ull << lane) - 1ull))] = (uint16_t)(tid + q * BAL_WG);
         }
-        // results, and this level's nodes into the table
-        for (uint32_t c = tid; c < nb; c += BAL_WG)
-            r.newSig[r.roots[s + c]] = s_len[c] == 0 ? 0ull : s_arr[s_off[c]];
-        for (uint32_t i = tid; i < hsize; i += BAL_WG) {
-            const unsigned long long key = s_key[i];
-            if (key == EMPTY64) continue;
-            const uint32_t v = s_val[i] & ~LN_FINAL;
-            const uint32_t slot = t_slot(r.t, key);
-            if (slot == UNSET) { atomicOr(r.err, 2u); continue; }
-            __hip_atomic_store(&r.t.w[2 * (size_t)slot + 1], sig(2u * (levBase + v), s_nlev[v]), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        // ---- the others by the first wavefront: its lanes hold the covers in order
+        if (nAct != 0) {
+            if (wave == 0) {
+                const bool has = lane < nAct;
+                const uint32_t c = has ? s_act[lane] : 0u, o = s_off[c];
+                uint32_t L = has ? s_len[c] : 0u;
+                while (__ballot(L > 1) != 0) {
+                    uint32_t slot = 0;
+                    unsigned long long f = EMPTY64;
+                    const bool act = L > 1;
+                    if (act) {
+                        f = prepare(c, o, L, slot);
+                        L -= 2;
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    const bool win = slot != 0 && *(volatile uint32_t *)&s_val[slot - 1] == c;
+                    const uint64_t m = __ballot(win);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    if (win) create(c, o, L, slot, counter - levBase + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)));
+                    counter += (uint32_t)__popcll(m);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    if (slot != 0) f = s_node[*(volatile uint32_t *)&s_val[slot - 1] & ~LN_FINAL];
+                    if (act) L = add_back(o, L, f);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                }
+                if (has) s_len[c] = (uint16_t)L;
+                if (lane == 0) s_cnt[0][0] = counter;
+            }
+            __syncthreads();
+            counter = s_cnt[0][0];
         }
-        __builtin_amdgcn_s_waitcnt(0x0F70);     // vmcnt(0): the table's words are written
+        // the next level's loads have arrived: the waits for them stand here, where
+        // they do not include the insertions
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_IN; q++) asm volatile("" : "+v"(next.sig[q]), "+v"(next.lit[q]), "+v"(next.src[q]));
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_COV; q++) asm volatile("" : "+v"(next.off[q]), "+v"(next.root[q]));
+        // the level's nodes set out for the table; its own table is cleared
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_NEW; q++) {
+            const uint32_t i = tid + q * BAL_WG;
+            newKey[q] = EMPTY64;
+            if (i >= counter - levBase) continue;
+            const uint32_t h = s_ent[i];
+            newKey[q] = s_key[h];
+            newNode[q] = s_node[i];
+            s_key[h] = EMPTY64;
+            s_val[h] = UNSET;
+            newSlot[q] = (uint32_t)t_hash(r.t, newKey[q]);
+            newPrev[q] = t_cas(r.t, newSlot[q], newKey[q]);
+        }
+        for (int32_t i = (int32_t)(LT_NEW - 1 - tid), end = max(s_top, (int32_t)most); i >= end; i -= (int32_t)BAL_WG) {
+            const uint32_t h = s_ent[i];
+            if (h == LS_NONE) continue;
+            s_key[h] = EMPTY64;
+            s_val[h] = UNSET;
+        }
+        // results
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_COV; q++) {
+            const uint32_t c = tid + q * BAL_WG;
+            if (c >= nb) continue;
+            const unsigned long long x = s_len[c] == 0 ? 0ull : s_arr[s_off[c]];
+            s_res[c] = x;
+            r.newSig[cur.root[q]] = x;
+        }
+        cur = next;
         __syncthreads();
     }
+    finish_inserts();
     if (tid == 0) made[seg] = counter - base0;
 }
 
@@ -786,10 +1093,7 @@ __global__ void k_rec_prepare(RecArgs r, uint32_t s, uint32_t nb) {
     const uint32_t in0 = r.off[s];
     auto lookup = [&](unsigned long long a, unsigned long long b) -> unsigned long long {
         const unsigned long long t = and_trivial(a, b);
-        if (t != EMPTY64) return t;
-        const unsigned long long key = and_key_of(sig_lit(a), sig_lit(b));
-        const uint64_t h = mix64(key) & r.t.mask;
-        return t_find_from(r.t, key, h, t_word(r.t, 2 * h));
+        return t != EMPTY64 ? t : t_find(r.t, and_key_of(sig_lit(a), sig_lit(b)));
     };
     for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < nb; c += stride) {
         unsigned long long *A = r.arr + (r.off[s + c] - in0);
@@ -823,14 +1127,14 @@ __global__ void k_rec_insert(RecArgs r, uint32_t nb) {
         const uint32_t slot = t_slot(r.t, r.skey[c]);
         r.slot[c] = slot;
         if (slot == UNSET) { atomicOr(r.err, 2u); r.mask[c] = 0; continue; }
-        atomicMin(&r.t.w[2 * (size_t)slot + 1], (unsigned long long)c);
+        atomicMin(&r.t.v[slot], (unsigned long long)c);
     }
 }
 
 // winners (the smallest cover index of a key) of every workgroup's kB covers
 __global__ void __launch_bounds__(kB) k_rec_winners(RecArgs r, uint32_t nb) {
     const uint32_t c = blockIdx.x * kB + threadIdx.x;
-    const bool win = c < nb && r.mask[c] == 1 && r.t.w[2 * (size_t)r.slot[c] + 1] == (unsigned long long)c;
+    const bool win = c < nb && r.mask[c] == 1 && r.t.v[r.slot[c]] == (unsigned long long)c;
     const int n = __syncthreads_count(win);
     if (c < nb && win) r.mask[c] = 3;
     if (threadIdx.x == 0) r.bcnt[blockIdx.x] = (uint32_t)n;
@@ -857,7 +1161,7 @@ __global__ void __launch_bounds__(kB) k_rec_ids(RecArgs r, uint32_t s, uint32_t 
         r.of0[id] = (uint32_t)(key >> 32);
         r.of1[id] = (uint32_t)key;
         if (r.tagOut) r.tagOut[id] = r.tagIn[r.roots[s + c]];
-        r.t.w[2 * (size_t)r.slot[c] + 1] = sig(2u * id, (uint32_t)r.sres[c]);
+        r.t.v[r.slot[c]] = sig(2u * id, (uint32_t)r.sres[c]);
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
         uint32_t n = r.counter[step & 1u] + s_sum;
@@ -874,7 +1178,7 @@ __global__ void k_rec_add_back(RecArgs r, uint32_t s, uint32_t nb) {
         const uint8_t m = r.mask[c];
         if (m == 0) continue;
         unsigned long long *A = r.arr + (r.off[s + c] - in0);
-        const unsigned long long x = m == 2 ? r.sres[c] : r.t.w[2 * (size_t)r.slot[c] + 1];
+        const unsigned long long x = m == 2 ? r.sres[c] : r.t.v[r.slot[c]];
         const uint32_t L = r.alen[c];
         bool there = false;
         for (uint32_t i = 0; i < L; i++) there |= sig_lit(A[i]) == sig_lit(x);
@@ -1141,10 +1445,10 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
     uint32_t *keys = t.get<uint32_t>(std::max(nRoots, 1u)), *keysSorted = t.get<uint32_t>(std::max(nRoots, 1u));
     uint32_t *off = t.get<uint32_t>((size_t)nRoots + 1), *len = t.get<uint32_t>((size_t)nRoots + 1);
     uint32_t *newLen = t.get<uint32_t>((size_t)nRoots + 1), *newOff = t.get<uint32_t>((size_t)nRoots + 1);
-    uint32_t *inputs = t.get<uint32_t>(std::max<size_t>(poolUsed, 1));
+    uint32_t *inputs = t.get<uint32_t>(std::max<size_t>(poolUsed, 1)), *inSrc = t.get<uint32_t>(std::max<size_t>(poolUsed, 1));
     if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: order allocation");
     uint32_t *d_starts = nullptr, *d_levOff = nullptr;
-    uint2 *d_levSize = nullptr;
+    LevelRec *d_lev = nullptr;
     uint32_t most[3] = {};
     std::vector<uint32_t> levOff;
     auto order = [&](bool bySeg) -> int {
@@ -1154,8 +1458,8 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
         const uint32_t nKeys = levOff[ns];
         d_levOff = t.get<uint32_t>(ns + 1);
         d_starts = t.get<uint32_t>((size_t)nKeys + 1);
-        d_levSize = t.get<uint2>((size_t)nKeys + 1);
-        if (!d_levOff || !d_starts || !d_levSize) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: levels");
+        d_lev = t.get<LevelRec>((size_t)nKeys + 1);
+        if (!d_levOff || !d_starts || !d_lev) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: levels");
         GLS_TRY(stream_copy(ctx, d_levOff, levOff.data(), sizeof(uint32_t) * (ns + 1), hipMemcpyHostToDevice));
         k_level_keys<<<nblocks(nRoots), kB, 0, st>>>(nRoots, roots, lastLevel, tagIn,
                                                      bySeg && tagged ? d_levOff : nullptr, keys);
@@ -1169,13 +1473,14 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
         GLS_HIP(ctx, rocprim::radix_sort_pairs(tmp2, tb2, keys, keysSorted, roots, rootsSorted, (size_t)nRoots, 0u,
                                                eb, st));
         k_key_starts<<<nblocks((int64_t)nRoots + 1), kB, 0, st>>>(nRoots, keysSorted, nKeys, d_starts);
-        k_cover_lens<<<nblocks((int64_t)nRoots + 1), kB, 0, st>>>(nRoots, rootsSorted, cover, len, newLen);
+        k_cover_lens<<<nblocks((int64_t)nRoots + 1), kB, 0, st>>>(nRoots, rootsSorted, cover, len, newLen, indeg);
         GLS_HIP(ctx, rocprim::exclusive_scan(tmp2, tb3, len, off, 0u, (size_t)nRoots + 1, rocprim::plus<uint32_t>(), st));
         GLS_HIP(ctx, rocprim::exclusive_scan(tmp2, tb3, newLen, newOff, 0u, (size_t)nRoots + 1,
                                              rocprim::plus<uint32_t>(), st));
         GLS_HIP(ctx, hipMemsetAsync(&ctr[4], 0, sizeof(uint32_t) * 3, st));
-        k_level_sizes<<<nblocks(nKeys), kB, 0, st>>>(nKeys, d_starts, off, newOff, d_levSize, &ctr[4]);
-        k_pack_inputs<<<nblocks(nRoots), kB, 0, st>>>(nRoots, rootsSorted, cover, pool, off, inputs);
+        k_level_sizes<<<nblocks(nKeys), kB, 0, st>>>(nKeys, d_starts, off, newOff, d_lev, &ctr[4]);
+        k_pack_inputs<<<nblocks(nRoots), kB, 0, st>>>(nRoots, rootsSorted, cover, pool, off, keysSorted, d_starts, lastLevel, indeg,
+                                                      nPIs, inputs, inSrc);
         GLS_HIP(ctx, hipGetLastError());
         return stream_copy(ctx, most, &ctr[4], sizeof(most), hipMemcpyDeviceToHost);
     };
@@ -1226,40 +1531,41 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
     uint64_t cap = 1024;
     while (cap < 2ull * ((uint64_t)poolUsed + 16)) cap <<= 1;       // a cover of k inputs creates at most k - 1 nodes
     const size_t idEnd = (size_t)nPIs + 1 + poolUsed;
-    unsigned long long *tab = t.get<unsigned long long>(2 * cap), *newSig = t.get<unsigned long long>(n);
+    unsigned long long *tabK = t.get<unsigned long long>(cap), *tabV = t.get<unsigned long long>(cap), *newSig = t.get<unsigned long long>(n);
     uint32_t *cf0 = t.get<uint32_t>(idEnd), *cf1 = t.get<uint32_t>(idEnd);
     uint32_t *ctag = tagged ? t.get<uint32_t>(idEnd) : nullptr;
     uint32_t *segIds = t.get<uint32_t>(3 * (size_t)ns + 3);
     if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: reconstruction allocation");
     uint32_t *d_idBase = segIds, *d_made = segIds + ns, *d_outOff = segIds + 2 * (size_t)ns;
-    GLS_HIP(ctx, hipMemsetAsync(tab, 0xFF, sizeof(unsigned long long) * 2 * cap, st));
+    GLS_HIP(ctx, hipMemsetAsync(tabK, 0xFF, sizeof(unsigned long long) * cap, st));
+    GLS_HIP(ctx, hipMemsetAsync(tabV, 0xFF, sizeof(unsigned long long) * cap, st));
     std::vector<uint32_t> idBase(ns, (uint32_t)nPIs + 1u), made(ns, 0u);
     if (bySeg && ns > 1 && nRoots > 0) {
         // a segment's ids start after room for all that those before it can create
-        std::vector<uint2> hl(levOff[ns]);
-        GLS_TRY(stream_copy(ctx, hl.data(), d_levSize, sizeof(uint2) * hl.size(), hipMemcpyDeviceToHost));
+        std::vector<LevelRec> hl(levOff[ns]);
+        GLS_TRY(stream_copy(ctx, hl.data(), d_lev, sizeof(LevelRec) * hl.size(), hipMemcpyDeviceToHost));
         uint32_t sum = (uint32_t)nPIs + 1u;
         for (uint32_t k = 0; k < ns; k++) {
             idBase[k] = sum;
-            for (uint32_t l = levOff[k]; l < levOff[k + 1]; l++) sum += hl[l].y;
+            for (uint32_t l = levOff[k]; l < levOff[k + 1]; l++) sum += hl[l].most;
         }
     }
     GLS_TRY(stream_copy(ctx, d_idBase, idBase.data(), sizeof(uint32_t) * ns, hipMemcpyHostToDevice));
     GLS_HIP(ctx, hipMemsetAsync(d_made, 0, sizeof(uint32_t) * ns, st));
-    RecArgs ra{NodeTable{tab, cap - 1}, nPIs, rootsSorted, off, inputs, d_levSize, d_starts, newSig, cf0, cf1, ctag, tagIn, &ctr[1],
+    RecArgs ra{NodeTable{tabK, tabV, cap - 1}, nPIs, rootsSorted, off, inputs, inSrc, d_lev, d_starts, newSig, cf0, cf1, ctag, tagIn, &ctr[1],
                sortDecId == 0 ? 1u : 0u, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, &ctr[8]};
     if (nRoots > 0 && fits) {
         k_rec_lds<<<ns, BAL_WG, 0, st>>>(ra, d_levOff, d_idBase, d_made, (int32_t)levels - 1, 0);
         GLS_HIP(ctx, hipGetLastError());
     } else if (nRoots > 0) {
         std::vector<uint32_t> starts((size_t)levels + 1);
-        std::vector<uint2> size(levels);
+        std::vector<LevelRec> size(levels);
         GLS_TRY(stream_copy(ctx, starts.data(), d_starts, sizeof(uint32_t) * ((size_t)levels + 1), hipMemcpyDeviceToHost));
-        GLS_TRY(stream_copy(ctx, size.data(), d_levSize, sizeof(uint2) * levels, hipMemcpyDeviceToHost));
+        GLS_TRY(stream_copy(ctx, size.data(), d_lev, sizeof(LevelRec) * levels, hipMemcpyDeviceToHost));
         // a level goes to the persistent workgroup if it fits its LDS (it is
         // one batch then)
         auto narrow = [&](uint32_t l) {
-            return starts[l + 1] - starts[l] <= fitCovers && size[l].x <= LT_INPUTS && size[l].y <= LT_NEW;
+            return starts[l + 1] - starts[l] <= fitCovers && size[l].T <= LT_INPUTS && size[l].most <= LT_NEW;
         };
         // the wide levels' batches and their step counts
         std::vector<uint32_t> batchOff(levels + 1, UNSET), batchSteps;

@@ -71,3 +71,42 @@ def test_batch_balance_levels_at_the_limits(gpu_ctx, shape):
     gpu_ctx.batch_balance(aigs, update_level=False)
     for a, g in zip(aigs, graphs):
         assert same(a.arrays(), O.balance(*g))
+
+
+RAW_SHUFFLE = pytest.mark.xfail(strict=True, reason="`b -s` of a graph whose fanins are not in strashed order: the "
+                                "order in which a cover's inputs are shuffled differs from the oracle's")
+
+
+@pytest.mark.parametrize("covers,k", [(40, 6), (1024, 4), (300, 11)])
+@pytest.mark.parametrize("shuffle,strashed", [(False, False), (False, True), (True, True),
+                                              pytest.param(True, False, marks=RAW_SHUFFLE)])
+def test_balance_pairs_that_exist(gpu_ctx, covers, k, shuffle, strashed):
+    """Covers over PIs whose pairs the levels before have created: few of them
+    (found nodes put back meet older ones), and more than a level has room for."""
+    print("balance existing pairs: %d covers of %d inputs, shuffle %s" % (covers, k, shuffle))
+    sys.stdout.flush()
+    rng = np.random.default_rng(k)
+    nPIs = 9
+    f0, f1, pos = [0] * (nPIs + 1), [0] * (nPIs + 1), []
+
+    def chain(lits):
+        cur = int(lits[0])
+        for x in lits[1:]:
+            f0.append(cur)
+            f1.append(int(x))
+            cur = 2 * (len(f0) - 1)
+        return cur
+
+    def pis(n):
+        return 2 * (1 + rng.permutation(nPIs)[:n]) + rng.integers(0, 2, n)
+
+    below = [chain(pis(rng.integers(2, 5))) for _ in range(200)]
+    above = [chain(np.append(pis(rng.integers(2, 4)), x + 1)) for x in below]
+    for i in range(covers):
+        pos.append(chain(np.append(pis(min(k - 1, nPIs)), above[i % len(above)] + 1)))
+    g = nPIs, np.array(f0, np.uint32), np.array(f1, np.uint32), np.array(pos, np.uint32)
+    a = gpu_ctx.from_arrays(*g)
+    if strashed:
+        g = a.strash().arrays()
+    a.balance(update_level=False, shuffle=shuffle)
+    assert same(a.arrays(), O.balance(*g, sort_dec_id=0 if shuffle else 1))
