@@ -38,6 +38,7 @@ constexpr int NCUT = 8;
 constexpr int MFFC_TAB = 8;
 constexpr int NMATCH = 54;
 constexpr int EVAL_BLOCK = 64;
+constexpr int32_t EVAL_FEW = 49152;
 constexpr int PLAN_MAXM = 16;
 
 struct Lib {
@@ -1186,47 +1187,129 @@ __device__ __forceinline__ void cut_leaves4(const uint32_t *p, int *leaves, int 
     if (nL == 3) { leaves[3] = 0; nL = 4; }
 }
 
-template <typename LV>
-__global__ void __launch_bounds__(EVAL_BLOCK) k_eval(int32_t n, int32_t nPIs, GraphView g, Lib L,
-                                                      const uint32_t *__restrict__ cuts, int useZeros,
-                                                      int4 *best) {
-    __shared__ int32_t s_match[NMATCH * EVAL_BLOCK];
-    __shared__ LV s_mlev[NMATCH * EVAL_BLOCK];
-    int64_t v = nPIs + 1 + blockIdx.x * (int64_t)EVAL_BLOCK + threadIdx.x;
-    if (v >= n) return;
-    Col match{s_match + threadIdx.x};
-    ColT<LV> mlev{s_mlev + threadIdx.x};
-    const int id = (int)v;
-    int reduction = -1, bestLevel = 99999999, bestCut = -1, bestOut = 0;
-    const uint32_t *cs = cuts + (size_t)v * NCUT * 5;
-    for (int i = 0; i < NCUT; i++) {
-        const uint32_t *p = cs + 5 * i;
-        uint32_t meta = p[4];
-        if (!((meta >> 30) & 1) || ((meta >> 27) & 7) < 3) continue;
-        int leaves[4], nL;
-        uint32_t tt;
-        cut_leaves4(p, leaves, nL, tt);
-        Mffc t;
-        int saved = calc_mffc(g, id, leaves, nL, t, match);
-        uint32_t isC;
-        uint64_t matched;
-        int cls = match_cut(g, L, id, tt, leaves, t, match, mlev, isC, matched);
-        const int nr = lib_nr(L, cls);
-        for (int out = 0; out < nr; out++) {
-            int rt = lib_root(L, cls, out);
-            if (match[rt] == id) continue;
-            int added = __popcll(added_set(L, cls, rt, matched));
-            int gain = saved - added;
-            if (gain < 0 || (gain == 0 && !useZeros)) continue;
-            int rl = (int)mlev[rt];
-            if (gain < reduction || (gain == reduction && rl >= bestLevel)) continue;
-            reduction = gain;
-            bestLevel = rl;
-            bestCut = i;
-            bestOut = out;
+// Evaluation of every cut of a node (Eval, rewrite.cu:328-424): the gain of the
+// best root, then its level, then the first cut and root decide.
+// One wavefront takes NODES nodes.  First every lane computes the fanout-free
+// cone of one of their cuts; then 16 lanes match one cut each time, four cuts
+// side by side: a lane takes the class's forest nodes gl, gl + 16, .. and
+// waits for a node's children (done: the forest nodes that are finished), and
+// the set of nodes that a forest node would create is the union of its
+// children's and itself unless it exists, so a root costs one popcount.
+// What bounds it is the chain of lookups: a class has 15 forest nodes on
+// average and 50 at most, but these need 3.5 rounds of 16 lanes.  State is per
+// cut and not per lane, so 28 wavefronts fit a CU's LDS instead of 7.  With a
+// node per lane, its cuts one after the other: 2k random ANDs 211 us (now 26),
+// 200k windowed 575 (242), 4M windowed 6090 (1605), 10M in a batch of random
+// AIGs 23500.
+struct EvalCut {           // of one forest entry
+    int32_t match, lev;    // the existing node or -1; its level, or that it would get
+    uint64_t add;          // the entries it would create
+};
+
+constexpr int EG = 16, EGS = 64 / EG;      // lanes per cut, cuts side by side
+
+template <int NODES>
+__global__ void __launch_bounds__(64) k_eval(int32_t n, int32_t nPIs, GraphView g, Lib L,
+                                             const uint32_t *__restrict__ cuts, int useZeros, int4 *best) {
+    __shared__ EvalCut s_ent[EGS * NMATCH];            // first the cones' DFS stacks
+    __shared__ int32_t s_del[MFFC_TAB * 64];           // the cones' nodes besides the root
+    __shared__ unsigned long long s_best[NODES];
+    __shared__ uint8_t s_list[64];
+    static_assert(sizeof(EvalCut) * EGS * NMATCH >= 4 * (MFFC_TAB + 2) * EVAL_BLOCK, "stacks");
+    static_assert(EVAL_BLOCK == 64 && NODES * NCUT <= 64 && NMATCH <= 64, "one wavefront");
+    const int lane = threadIdx.x, grp = lane / EG, gl = lane % EG;
+    const int64_t base = nPIs + 1 + blockIdx.x * (int64_t)NODES;
+    if (lane < NODES) s_best[lane] = ~0ull;
+    // ---- a cut per lane
+    int leaves[4] = {}, nL = 0;
+    uint32_t pack = 0, offs = 0;
+    bool valid = false;
+    if (lane < NODES * NCUT && base + lane / NCUT < n) {
+        const uint32_t *p = cuts + ((size_t)(base + lane / NCUT) * NCUT + lane % NCUT) * 5;
+        const uint32_t meta = p[4];
+        valid = ((meta >> 30) & 1) && ((meta >> 27) & 7) >= 3;
+        if (valid) {
+            uint32_t tt;
+            cut_leaves4(p, leaves, nL, tt);
+            const uint32_t w = L.npn[tt];
+            const int cls = (w >> 10) & 255;
+            Mffc t;
+            const int saved = calc_mffc(g, (int)(base + lane / NCUT), leaves, nL, t, Col{(int32_t *)s_ent + lane});
+            int nd = 0;
+#pragma unroll
+            for (int i = 0; i < MFFC_TAB; i++)
+                if (i < t.size && t.num[i] == 0) s_del[64 * nd++ + lane] = t.id[i];
+            pack = (w & 0x3FFu) | (uint32_t)saved << 10 | (uint32_t)nd << 14 | (uint32_t)lib_nn(L, cls) << 18 |
+                   (uint32_t)lib_nr(L, cls) << 24;
+            offs = (uint32_t)L.nodeOff[cls] | (uint32_t)L.rootOff[cls] << 16;
         }
     }
-    best[v] = bestCut >= 0 ? make_int4(bestCut, bestOut, reduction, bestLevel) : make_int4(-1, 0, 0, 0);
+    const uint64_t vm = __ballot(valid);
+    const int count = __popcll(vm);
+    if (valid) s_list[__popcll(vm & ((1ull << lane) - 1ull))] = (uint8_t)lane;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // ---- a cut per 16 lanes
+    EvalCut *ent = s_ent + grp * NMATCH;
+    for (int c0 = 0; c0 < count; c0 += EGS) {
+        const bool act = c0 + grp < count;
+        const int src = s_list[act ? c0 + grp : 0];
+        const uint32_t pk = (uint32_t)__shfl((int)pack, src), of = (uint32_t)__shfl((int)offs, src);
+        const int l0 = __shfl(leaves[0], src), l1 = __shfl(leaves[1], src), l2 = __shfl(leaves[2], src),
+                  l3 = __shfl(leaves[3], src);
+        const int id = (int)(base + src / NCUT), saved = (int)((pk >> 10) & 15), nd = (int)((pk >> 14) & 15);
+        const int nn = act ? (int)((pk >> 18) & 63) : 0, nr = act ? (int)(pk >> 24) : 0;
+        const uint32_t isC = pk & 15u;
+        const uint16_t *words = L.nodes + (of & 0xFFFFu);
+        const int rt = gl < nr ? L.roots[(of >> 16) + gl] : 0;
+        uint32_t wd = gl < nn ? words[gl] : 0u;
+        if (act && gl < 4) {
+            const int q = L.perms4[4 * ((pk >> 5) & 31) + gl];
+            const int leaf = q == 0 ? l0 : q == 1 ? l1 : q == 2 ? l2 : l3;
+            ent[gl] = EvalCut{leaf, (int32_t)g.level[leaf], 0ull};
+        }
+        uint64_t done = 0xFull;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        for (int j0 = 0; __ballot(j0 < nn) != 0; j0 += EG) {
+            const int j = j0 + gl, a = wd & 63, b = (wd >> 6) & 63;
+            const int ca = (wd >> 12) & 1, cb = (wd >> 13) & 1;
+            bool pend = j < nn;
+            wd = j + EG < nn ? words[j + EG] : 0u;
+            while (__ballot(pend) != 0) {
+                const bool ready = pend && ((done >> a) & (done >> b) & 1u);
+                if (ready) {
+                    const EvalCut x = ent[a], y = ent[b];
+                    EvalCut e{-1, 1 + max(x.lev, y.lev), x.add | y.add | 1ull << (j + 4)};
+                    if (x.match != -1 && y.match != -1 && x.match != id && y.match != id) {
+                        const int nid = table_lookup(g, x.match, y.match, (int)isc_bit(isC, a) ^ ca,
+                                                     (int)isc_bit(isC, b) ^ cb);
+                        bool gone = nid == -1;
+                        for (int i = 0; i < nd && !gone; i++) gone = s_del[64 * i + src] == nid;
+                        if (!gone) e = EvalCut{nid, (int32_t)g.level[nid], 0ull};
+                    }
+                    ent[j + 4] = e;
+                }
+                const uint64_t m = __ballot(ready);
+                done |= ((m >> (EG * grp)) & ((1ull << EG) - 1ull)) << (j0 + 4);
+                pend = pend && !ready;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            }
+        }
+        if (gl < nr) {
+            const EvalCut e = ent[rt];
+            const int gain = saved - __popcll(e.add);
+            if (e.match != id && (gain > 0 || (gain == 0 && useZeros)))
+                atomicMin(&s_best[src / NCUT], (unsigned long long)(255 - gain) << 48 |
+                                                   (unsigned long long)(uint32_t)e.lev << 16 |
+                                                   (unsigned long long)((src % NCUT) << 8 | gl));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    if (lane < NODES && base + lane < n) {
+        const unsigned long long k = s_best[lane];
+        best[base + lane] = k == ~0ull ? make_int4(-1, 0, 0, 0)
+                                       : make_int4((int)((k >> 8) & 255), (int)(k & 255), 255 - (int)(k >> 48),
+                                                   (int)(uint32_t)(k >> 16));
+    }
 }
 
 // ------------------------------------------------------------------------
@@ -2050,6 +2133,18 @@ int dev_enumerate_cuts(gls_ctx *ctx, const DevGraph &g, const std::vector<int32_
     return GLS_OK;
 }
 
+// Few nodes: two per wavefront, so that more wavefronts share the chain of
+// lookups; many: eight, so that the cones use every lane.  Two against eight,
+// us: 2k random ANDs 26 / 56, 32k 53 / 69, a 50k windowed AIG 92 / 89, 64k
+// random 95 / 91, 500k 638 / 512.
+static void launch_eval(hipStream_t st, int32_t n, int32_t nPIs, const GraphView &g, const Lib &L, const uint32_t *cuts,
+                        int useZeros, int4 *best) {
+    const int32_t nAnd = n - nPIs - 1;
+    if (nAnd <= 0) return;
+    if (nAnd <= EVAL_FEW) k_eval<2><<<blocks(nAnd, 2), 64, 0, st>>>(n, nPIs, g, L, cuts, useZeros, best);
+    else k_eval<8><<<blocks(nAnd, 8), 64, 0, st>>>(n, nPIs, g, L, cuts, useZeros, best);
+}
+
 static int build_table(gls_ctx *ctx, Tmp &t, const DevGraph &g, GraphView &gv) {
     hipStream_t st = ctx->stream;
     const int32_t n = g.nObjs;
@@ -2080,14 +2175,11 @@ int dev_evaluate(gls_ctx *ctx, const DevGraph &g, const uint32_t *d_cuts, const 
     GraphView gv{g.f0, g.f1, d_nref, g.level, nullptr, nullptr};
     GLS_TRY(build_table(ctx, t, g, gv));
     GLS_HIP(ctx, hipMemsetAsync(d_best, 0xFF, sizeof(int4) * 1, st));
-    int32_t nAnd = g.nObjs - g.nPIs - 1;
     // PIs and the constant have no candidate
     GLS_HIP(ctx, hipMemsetAsync(d_best, 0, sizeof(int4) * (size_t)(g.nPIs + 1), st));
     std::vector<int4> none(g.nPIs + 1, make_int4(-1, 0, 0, 0));
     GLS_HIP(ctx, hipMemcpyAsync(d_best, none.data(), sizeof(int4) * none.size(), hipMemcpyHostToDevice, st));
-    if (nAnd > 0)
-        k_eval<int32_t><<<blocks(nAnd, EVAL_BLOCK), EVAL_BLOCK, 0, st>>>(g.nObjs, g.nPIs, gv, lib_of(ctx), d_cuts, useZeros,
-                                                                reinterpret_cast<int4 *>(d_best));
+    launch_eval(st, g.nObjs, g.nPIs, gv, lib_of(ctx), d_cuts, useZeros, reinterpret_cast<int4 *>(d_best));
     GLS_HIP(ctx, hipGetLastError());
     GLS_HIP(ctx, hipStreamSynchronize(st));
     return GLS_OK;
@@ -2142,14 +2234,8 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
         tm.mark(); // 3
         std::vector<int4> none(nPIs + 1, make_int4(-1, 0, 0, 0));
         GLS_HIP(ctx, hipMemcpyAsync(best, none.data(), sizeof(int4) * none.size(), hipMemcpyHostToDevice, st));
-        const int32_t nAnd = n - nPIs - 1;
         const Lib L = lib_of(ctx);
-        // a structure node's level exceeds the graph's deepest by at most
-        // NMATCH, so below 65000 levels every value fits 16 bits under 0xFFFF
-        if (nAnd > 0 && levelStart.size() < 65000)
-            k_eval<uint16_t><<<blocks(nAnd, EVAL_BLOCK), EVAL_BLOCK, 0, st>>>(n, nPIs, gv, L, cuts, useZeros, best);
-        else if (nAnd > 0)
-            k_eval<int32_t><<<blocks(nAnd, EVAL_BLOCK), EVAL_BLOCK, 0, st>>>(n, nPIs, gv, L, cuts, useZeros, best);
+        launch_eval(st, n, nPIs, gv, L, cuts, useZeros, best);
         GLS_HIP(ctx, hipGetLastError());
         tm.mark(); // 4
         // candidates in id order
