@@ -155,6 +155,7 @@ struct RwDelta {
     const uint32_t *g0, *g1, *glevel;
     const uint32_t *tOff;
     const uint2 *tEnt;
+    bool allRounds = false;     // as many hashing rounds as it takes
 };
 int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &out, int32_t *depth,
                   gls_op_info *info, const uint32_t *tagIn = nullptr, uint32_t **tagOut = nullptr,

@@ -912,8 +912,22 @@ constexpr int SW_RING = 32768;              // 128 KiB of LDS
 constexpr uint32_t NOFAN = 0xFFFFFFFFu;
 constexpr uint32_t SW_NOLEV = 0xFFFFFFFFu;
 constexpr uint32_t SW_SPIN_LIMIT = 1u << 22;
-// rounds of the incremental strash before it gives way to the wave sweep
-constexpr uint32_t kRwRoundLimit = 4096;
+// Rounds of the incremental strash before it gives way to the wave sweep.  A
+// round merges duplicates one level further up, so a graph that holds the same
+// deep logic twice needs one per level.  Whole graphs measured take one to
+// three, large narrow ones eight; a graph that needs more pays for the rounds
+// tried (the 32-bit multiplier twice over the same inputs 1.7 ms against 1.2 by
+// waves at once, a windowed AIG of 200k ANDs twice 9 against 5.7).
+constexpr uint32_t kRwRoundLimit = 4096, kRwManyRounds = 32, kRwFewRounds = 5;
+// objects from which a whole narrow graph may take many rounds
+constexpr int32_t kRwLarge = 1 << 18;
+// The line for a rewrite of one AIG lies at this many times rw_sweep_width
+// objects per level (8192 by default).  Incremental against wave sweep, ms:
+// 1248 objects per level 1.6 / 9.6, 2309 1.7 / 6.2, 4294 1.6 / 4.2, 6640 3.9 /
+// 4.6, 10967 3.4 / 3.4, 23077 35.2 / 25.8.  A batched arena has its deepest
+// member's levels, most of them nearly empty, and keeps rw_sweep_width (3893
+// per level 4.8 / 4.2 ms for the whole pass, 72602 46.5 / 31.4).
+constexpr int64_t kRwSweepScale = 8;
 
 __device__ __forceinline__ uint32_t sw_lds_load(const uint32_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1626,11 +1640,12 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
         if (info) info->final_strash = 2;
         return rc;
     };
-    // The level sweeps below run in one workgroup, about 3 ns per object for
-    // the two of them; the wave sweep costs about 2.6 us per level plus its
-    // per-node work.  On wide graphs (many objects per level, as in a batched
-    // arena) the wave sweep is the faster one.
-    if (!full && (int64_t)N > (int64_t)tuning_for(ctx, d.n).rw_sweep_width * (int64_t)std::max(d.depth, 1)) {
+    // The level sweeps below run in one workgroup, about 1 ns per object each;
+    // the wave sweep costs 2.6 us per level of few nodes, 13 us of a thousand,
+    // and its per-node work.  On wide graphs the wave sweep is the faster one.
+    const int64_t width = full ? 0 : (int64_t)tuning_for(ctx, d.n).rw_sweep_width;
+    const int64_t depth0 = std::max(d.depth, 1);
+    if (!full && (int64_t)N > width * depth0 * (tagIn ? 1 : kRwSweepScale)) {
         const int rc = dev_strash(ctx, in, out, depthOut, info, tagIn, tagOut, tagDepth);
         if (info) info->final_strash = 0;
         return rc;
@@ -1696,12 +1711,6 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
             GLS_HIP(ctx, hipGetLastError());
             GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
             if (misc[0]) return fallback("ids not topological");
-            // wide graphs are faster by the grid-wide wave sweep
-            if ((int64_t)N > (int64_t)tuning_for(ctx, N).rw_sweep_width * (int64_t)std::max<uint32_t>(misc[1], 1u)) {
-                const int rc = dev_strash(ctx, in, out, depthOut, info, tagIn, tagOut, tagDepth);
-                if (info) info->final_strash = 0;
-                return rc;
-            }
         } else {
         k_rw_key_init<<<gN, kBlock, 0, st>>>(n, N, d.glevel, fa);
         uint32_t keyRounds = 0;
@@ -1746,6 +1755,12 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
         }
         }
         const int32_t depth = (int32_t)misc[1];
+        const bool narrow = full ? N >= kRwLarge && (int64_t)N <= (int64_t)tuning_for(ctx, N).rw_sweep_width * std::max(depth, 1)
+                                 : (int64_t)N <= width * depth0;
+        // the wave sweep's limit on objects holds where it used to run
+        if (!narrow && !d.allRounds && (uint64_t)tuning_for(ctx, N).strash_table_factor * (uint64_t)N > (1ull << 31))
+            return fallback("table range");
+        const uint32_t roundLimit = d.allRounds || (narrow && !full) ? kRwRoundLimit : narrow ? kRwManyRounds : kRwFewRounds;
         k_rw_seed<<<gN, kBlock, 0, st>>>(n, N, nPIs, in.f0, in.f1, d.g0, d.g1, dead, posOf, levPos, wave, rep, inD);
         GLS_HIP(ctx, hipGetLastError());
         {
@@ -1766,7 +1781,7 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
         uint32_t *dslot = nullptr, *nrep = nullptr;
         uint32_t prevD = 0, r = 0;
         for (; nD > 0; ++r) {
-            if (r >= kRwRoundLimit) return fallback("rounds");
+            if (r >= roundLimit) return fallback("rounds");
             uint64_t want = 1024;
             while (want < 4ull * nD) want <<= 1;
             if (want > cap) {

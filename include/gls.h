@@ -236,8 +236,8 @@ int gls_batch_balance(gls_ctx *ctx, gls_aig **aigs, int32_t count, int32_t sort_
  *   cut_wide: a group of levels (three, or cut_levels when planned) whose
  *     widest level has more nodes runs one cut launch per level (default 2048);
  *   rw_sweep_width: rw finishes with the incremental strash while the input
- *     has at most this many objects per level on average, else with the
- *     wave sweep (default 1024);
+ *     has at most eight times this many objects per level on average (the
+ *     arena of a batch: this many), else with the wave sweep (default 1024);
  *   strash_table_factor: the strash table has at least this many slots per
  *     object, a power of two, 4 or 8 (default 4);
  *   strash_wave_batch: wide strash waves launched per host check, 1-64
