@@ -561,6 +561,10 @@ __device__ __forceinline__ unsigned long long input_sig(const RecArgs &r, uint32
 }
 
 // ---- one workgroup per segment, levels within its LDS
+// (a volatile pointer would make these FLAT loads, which wait for all memory)
+template <class T> __device__ __forceinline__ T lds_load(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 constexpr uint32_t LT_INPUTS = 4096;      // inputs of a level
 constexpr uint32_t LT_COVERS = 2048;      // covers of a level
 constexpr uint32_t LT_NEW = 3072;         // ANDs that a level can create
@@ -760,12 +764,12 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
             for (;;) {
                 if (k == EMPTY64) return EMPTY64;
                 if (k == key) {
-                    const uint32_t v = *(volatile uint32_t *)&s_val[h];
+                    const uint32_t v = lds_load(&s_val[h]);
                     // inserted in this step: not there yet
                     return v == UNSET || !(v & LN_FINAL) ? EMPTY64 : s_node[v & ~LN_FINAL];
                 }
                 h = (h + 1) & (LT_HASH - 1);
-                k = *(volatile unsigned long long *)&s_key[h];
+                k = lds_load(&s_key[h]);
             }
         };
         // pairs of inputs that exist
@@ -846,7 +850,7 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
             for (uint32_t i = right;;) {
                 const unsigned long long before = s_arr[i > o ? i - 1 : o], key = and_key_of(x1, sig_lit(l3));
                 const uint32_t h = hash(key);
-                const unsigned long long k = *(volatile unsigned long long *)&s_key[h];
+                const unsigned long long k = lds_load(&s_key[h]);
                 found = and_trivial(l1, l3);
                 if (found == EMPTY64 && k != EMPTY64) found = level_find(key, h, k);
                 if (found == EMPTY64 && old1 && (sig_lit(l3) >> 1) < levBase) found = t_find(r.t, key);
@@ -991,13 +995,13 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
                         L -= 2;
                     }
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    const bool win = slot != 0 && *(volatile uint32_t *)&s_val[slot - 1] == c;
+                    const bool win = slot != 0 && lds_load(&s_val[slot - 1]) == c;
                     const uint64_t m = __ballot(win);
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     if (win) create(c, o, L, slot, counter - levBase + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)));
                     counter += (uint32_t)__popcll(m);
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    if (slot != 0) f = s_node[*(volatile uint32_t *)&s_val[slot - 1] & ~LN_FINAL];
+                    if (slot != 0) f = s_node[lds_load(&s_val[slot - 1]) & ~LN_FINAL];
                     if (act) L = add_back(o, L, f);
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 }
