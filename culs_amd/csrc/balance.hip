@@ -1353,12 +1353,14 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
     uint32_t *segInfo = t.get<uint32_t>(4 * (size_t)nSeg + 4), *flen = t.get<uint32_t>(SWEEP_GRID_ROUNDS + 1);
     if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: allocation (n=%d)", n);
     uint32_t *segFirst = segInfo, *segLen = segInfo + nSeg + 1, *segRound = segLen + nSeg, *segCnt = segRound + nSeg;
-    GLS_HIP(ctx, hipMemsetAsync(nFo, 0, sizeof(uint32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(mark, 0, sizeof(uint32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(indeg, 0, sizeof(uint32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(lastLevel, 0xFF, sizeof(uint32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(ctr, 0, sizeof(uint32_t) * 16, st));
-    GLS_HIP(ctx, hipMemsetAsync(segInfo, 0, sizeof(uint32_t) * (4 * (size_t)nSeg + 4), st));
+    GLS_TRY(Fills(ctx)
+                .add(nFo, 0, sizeof(uint32_t) * n)
+                .add(mark, 0, sizeof(uint32_t) * n)
+                .add(indeg, 0, sizeof(uint32_t) * n)
+                .add(lastLevel, 0xFF, sizeof(uint32_t) * n)
+                .add(ctr, 0, sizeof(uint32_t) * 16)
+                .add(segInfo, 0, sizeof(uint32_t) * (4 * (size_t)nSeg + 4))
+                .run());
     k_fanouts<<<nblocks(n), kB, 0, st>>>(n, nPIs, in.f0, in.f1, nPOs, in.pos, nFo, mark);
     if (nPOs > 0) k_po_marks<<<nblocks(nPOs), kB, 0, st>>>(nPOs, in.pos, mark);
     k_root_flags<<<nblocks(n), kB, 0, st>>>(n, nPIs, nFo, mark, flag);
@@ -1406,7 +1408,7 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
     std::vector<uint32_t> segLevels(nSeg, 0);
     auto sweep = [&](bool drop) -> int {
         sa.drop = drop ? 1u : 0u;
-        GLS_HIP(ctx, hipMemsetAsync(segLen, 0, sizeof(uint32_t) * 2 * nSeg, st));
+        GLS_TRY(Fills(ctx).add(segLen, 0, sizeof(uint32_t) * 2 * nSeg).run());
         k_sweep_first<<<nblocks(nCand), kB, 0, st>>>(nCand, roots, sa, tagged ? tagIn : nullptr, segFirst, segLen);
         for (;;) {
             k_sweep_wg<<<nSeg, BAL_WG, 0, st>>>(sa, segFirst, segLen, segRound, nSeg == 1 ? SWEEP_WIDE : UNSET);
@@ -1416,8 +1418,8 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
             GLS_TRY(stream_copy(ctx, h, segLen, sizeof(h), hipMemcpyDeviceToHost));
             while (h[0] > SWEEP_WIDE) {
                 if (h[1] > (uint32_t)n) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: cover levels do not end");
-                GLS_HIP(ctx, hipMemsetAsync(flen, 0, sizeof(uint32_t) * (SWEEP_GRID_ROUNDS + 1), st));
-                GLS_HIP(ctx, hipMemcpyAsync(flen, segLen, sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
+                GLS_TRY(Fills(ctx).add(flen, 0, sizeof(uint32_t) * (SWEEP_GRID_ROUNDS + 1)).run());
+                GLS_TRY(stream_copy(ctx, flen, &h[0], sizeof(uint32_t), hipMemcpyHostToDevice));
                 for (int i = 0; i < SWEEP_GRID_ROUNDS; i++)
                     k_sweep_grid<<<nblocks(2 * (int64_t)h[0]), kB, 0, st>>>(sa, h[1] + (uint32_t)i, flen + i);
                 GLS_HIP(ctx, hipGetLastError());
@@ -1481,7 +1483,7 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
         GLS_HIP(ctx, rocprim::exclusive_scan(tmp2, tb3, len, off, 0u, (size_t)nRoots + 1, rocprim::plus<uint32_t>(), st));
         GLS_HIP(ctx, rocprim::exclusive_scan(tmp2, tb3, newLen, newOff, 0u, (size_t)nRoots + 1,
                                              rocprim::plus<uint32_t>(), st));
-        GLS_HIP(ctx, hipMemsetAsync(&ctr[4], 0, sizeof(uint32_t) * 3, st));
+        GLS_TRY(Fills(ctx).add(&ctr[4], 0, sizeof(uint32_t) * 3).run());
         k_level_sizes<<<nblocks(nKeys), kB, 0, st>>>(nKeys, d_starts, off, newOff, d_lev, &ctr[4]);
         k_pack_inputs<<<nblocks(nRoots), kB, 0, st>>>(nRoots, rootsSorted, cover, pool, off, keysSorted, d_starts, lastLevel, indeg,
                                                       nPIs, inputs, inSrc);
@@ -1511,7 +1513,7 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
                 void *tmpk = t.get<uint8_t>(tbk);
                 if (!tmpk) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: split check sort");
                 GLS_HIP(ctx, rocprim::radix_sort_keys(tmpk, tbk, gk, gkS, (size_t)nRoots, 0u, 64u, st));
-                GLS_HIP(ctx, hipMemsetAsync(lcnt, 0, sizeof(uint32_t), st));
+                GLS_TRY(Fills(ctx).add(lcnt, 0, sizeof(uint32_t)).run());
                 k_split_tags<<<nblocks(nRoots), kB, 0, st>>>(nRoots, gkS, lst, 1024u, lcnt);
                 GLS_HIP(ctx, hipGetLastError());
                 uint32_t nsplit = 0;
@@ -1541,8 +1543,10 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
     uint32_t *segIds = t.get<uint32_t>(3 * (size_t)ns + 3);
     if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: reconstruction allocation");
     uint32_t *d_idBase = segIds, *d_made = segIds + ns, *d_outOff = segIds + 2 * (size_t)ns;
-    GLS_HIP(ctx, hipMemsetAsync(tabK, 0xFF, sizeof(unsigned long long) * cap, st));
-    GLS_HIP(ctx, hipMemsetAsync(tabV, 0xFF, sizeof(unsigned long long) * cap, st));
+    GLS_TRY(Fills(ctx)
+                .add(tabK, 0xFF, sizeof(unsigned long long) * cap)
+                .add(tabV, 0xFF, sizeof(unsigned long long) * cap)
+                .run());
     std::vector<uint32_t> idBase(ns, (uint32_t)nPIs + 1u), made(ns, 0u);
     if (bySeg && ns > 1 && nRoots > 0) {
         // a segment's ids start after room for all that those before it can create
@@ -1555,7 +1559,7 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
         }
     }
     GLS_TRY(stream_copy(ctx, d_idBase, idBase.data(), sizeof(uint32_t) * ns, hipMemcpyHostToDevice));
-    GLS_HIP(ctx, hipMemsetAsync(d_made, 0, sizeof(uint32_t) * ns, st));
+    GLS_TRY(Fills(ctx).add(d_made, 0, sizeof(uint32_t) * ns).run());
     RecArgs ra{NodeTable{tabK, tabV, cap - 1}, nPIs, rootsSorted, off, inputs, inSrc, d_lev, d_starts, newSig, cf0, cf1, ctag, tagIn, &ctr[1],
                sortDecId == 0 ? 1u : 0u, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, &ctr[8]};
     if (nRoots > 0 && fits) {
@@ -1591,7 +1595,7 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
         ra.bcnt = t.get<uint32_t>((size_t)nblocks(maxBatch));
         if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: wide levels");
         GLS_TRY(stream_copy(ctx, d_off, batchOff.data(), sizeof(uint32_t) * (levels + 1), hipMemcpyHostToDevice));
-        GLS_HIP(ctx, hipMemsetAsync(d_steps, 0, sizeof(uint32_t) * std::max(nBatches, 1u), st));
+        GLS_TRY(Fills(ctx).add(d_steps, 0, sizeof(uint32_t) * std::max(nBatches, 1u)).run());
         k_batch_steps<<<nblocks(nRoots), kB, 0, st>>>(nRoots, keysSorted, off, d_starts, d_off, batchLimit, d_steps);
         GLS_HIP(ctx, hipGetLastError());
         batchSteps.resize(nBatches);

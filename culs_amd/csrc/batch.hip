@@ -323,8 +323,7 @@ int batch_pass(gls_ctx *ctx, gls_aig **aigs, int32_t count, Pass pass, int32_t u
         GLS_HIP(ctx, rocprim::radix_sort_pairs(tmp, tb, keys, skeys, ids, sids, (size_t)Ar, 0u, eb, st));
     }
     std::vector<uint32_t> hcnt(count), hdep(count);
-    GLS_TRY(stream_copy(ctx, hcnt.data(), cnt, sizeof(uint32_t) * count, hipMemcpyDeviceToHost));
-    GLS_TRY(stream_copy(ctx, hdep.data(), dep, sizeof(uint32_t) * count, hipMemcpyDeviceToHost));
+    GLS_TRY(fetch(ctx, {{hcnt.data(), cnt, sizeof(uint32_t) * count}, {hdep.data(), dep, sizeof(uint32_t) * count}}));
 
     // outputs
     std::vector<DevGraph> outs(count);
@@ -367,7 +366,7 @@ int batch_pass(gls_ctx *ctx, gls_aig **aigs, int32_t count, Pass pass, int32_t u
         a->nObjs = outs[k].nObjs;
         a->dev_valid = true;
         a->dev_level_valid = pass != Pass::Balance;
-        a->host_valid = false;
+        a->host_valid = a->fetched = false;
         a->host_level_valid = false;
         a->levels = pass != Pass::Balance ? (int32_t)hdep[k] : -1;
         a->strashed = pass != Pass::Balance;

@@ -2,6 +2,7 @@
 #include "gls_internal.h"
 #include <chrono>
 #include "rwlib_forest.h"
+#include <algorithm>
 #include <cstdarg>
 #include <cstring>
 #include <fstream>
@@ -68,14 +69,6 @@ void DevPool::release_all() {
 }
 
 void pool_put(gls_ctx *ctx, void *p) { ctx->pool.put(p); }
-
-// Every copy is ordered on the context stream: the stream is non-blocking, so
-// copies on the legacy default stream would not wait for its kernels.
-int stream_copy(gls_ctx *ctx, void *dst, const void *src, size_t bytes, hipMemcpyKind kind) {
-    GLS_HIP(ctx, hipMemcpyAsync(dst, src, bytes, kind, ctx->stream));
-    GLS_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return GLS_OK;
-}
 
 int dev_graph_alloc(gls_ctx *ctx, DevGraph &g, int32_t nObjs, int32_t nPIs, int32_t nPOs) {
     g.nObjs = nObjs;
@@ -144,6 +137,7 @@ extern "C" void gls_ctx_destroy(gls_ctx *ctx) {
             if (e) (void)hipEventDestroy(e);
         for (auto &e : ctx->kev)
             if (e) (void)hipEventDestroy(e);
+        transfer_free(ctx);
         (void)hipStreamDestroy(ctx->stream);
     }
     delete ctx;
@@ -291,6 +285,16 @@ void aig_drop_device(gls_aig *a) {
 
 extern "C" int gls_aig_to_arrays(gls_aig *a, uint32_t *fanin0, uint32_t *fanin1, uint32_t *pos, int32_t conv) {
     if (!a) return GLS_ERR_ARG;
+    // the first time straight to the caller's arrays; if they are asked for
+    // again the handle keeps its own
+    if (!a->host_valid && !a->fetched) {
+        GLS_TRY(dev_graph_fetch(a->ctx, a->dev, fanin0, fanin1, pos, conv));
+        a->fetched = true;
+        const size_t first = (size_t)std::min(a->nPIs + 1, a->nObjs);
+        if (fanin0) std::fill_n(fanin0, first, 0u);
+        if (fanin1) std::fill_n(fanin1, first, 0u);
+        return GLS_OK;
+    }
     GLS_TRY(aig_ensure_host(a));
     for (int32_t v = 0; v < a->nObjs; v++) {
         if (fanin0) fanin0[v] = v <= a->nPIs ? 0 : conv_lit(a->h_f0[v], conv);
@@ -308,7 +312,7 @@ extern "C" int gls_aig_stats(gls_aig *a, gls_stats *s) {
     s->nObjs = a->nObjs;
     s->nAnds = a->nObjs - a->nPIs - 1;
     s->levels = a->levels;
-    s->on_device = a->dev_valid && !a->host_valid ? 1 : 0;
+    s->on_device = a->dev_valid && !a->host_valid && !a->fetched ? 1 : 0;
     return GLS_OK;
 }
 
@@ -326,20 +330,14 @@ extern "C" int gls_aig_copy(gls_aig *src, gls_aig **out) {
         a->strashed = src->strashed;
         int rc = dev_graph_alloc(ctx, a->dev, src->nObjs, src->nPIs, src->nPOs);
         if (rc != GLS_OK) { delete a; return rc; }
-        const size_t nb = sizeof(uint32_t) * (size_t)src->nObjs;
-        hipStream_t st = ctx->stream;
-        if (hipMemcpyAsync(a->dev.f0, src->dev.f0, nb, hipMemcpyDeviceToDevice, st) != hipSuccess ||
-            hipMemcpyAsync(a->dev.f1, src->dev.f1, nb, hipMemcpyDeviceToDevice, st) != hipSuccess ||
-            hipMemcpyAsync(a->dev.level, src->dev.level, nb, hipMemcpyDeviceToDevice, st) != hipSuccess ||
-            (src->nPOs && hipMemcpyAsync(a->dev.pos, src->dev.pos, sizeof(uint32_t) * src->nPOs,
-                                         hipMemcpyDeviceToDevice, st) != hipSuccess)) {
+        if (dev_graph_copy(ctx, src->dev, a->dev) != GLS_OK) {
             dev_graph_free(ctx, a->dev);
             delete a;
             return gls_fail(ctx, GLS_ERR_HIP, "device copy failed");
         }
         a->dev_valid = true;
         a->dev_level_valid = src->dev_level_valid;
-        a->host_valid = false;
+        a->host_valid = a->fetched = false;
         *out = a;
         return GLS_OK;
     }
@@ -413,7 +411,7 @@ static void adopt(gls_aig *a, DevGraph &out, int32_t depth) {
     a->nObjs = out.nObjs;
     a->dev_valid = true;
     a->dev_level_valid = true;
-    a->host_valid = false;
+    a->host_valid = a->fetched = false;
     a->host_level_valid = false;
     a->levels = depth;
 }

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <cstdio>
+#include <initializer_list>
 #include <map>
 #include <string>
 #include <vector>
@@ -68,6 +69,11 @@ struct gls_ctx {
     // entry point chose for the pass it runs (TuneScope), else null
     gls_tuning tune[64];
     const gls_tuning *active = nullptr;
+    // pinned memory (transfer.hip): small results and their sequence number;
+    // arrays on their way to the caller
+    uint8_t *mail = nullptr, *stage = nullptr;
+    uint32_t mail_seq = 0;
+    size_t stage_bytes = 0;
 };
 
 // the defaults of gls_tuning
@@ -100,6 +106,7 @@ struct gls_aig {
     int32_t levels = -1;
     bool strashed = false;
     bool host_valid = false, dev_valid = false;
+    bool fetched = false;                       // the device copy's arrays went to the caller
     std::vector<uint32_t> h_f0, h_f1, h_pos;  // AIGER convention
     DevGraph dev;                               // device copy (pool memory)
     bool dev_level_valid = false;
@@ -113,7 +120,37 @@ template <class T> T *pool_get(gls_ctx *ctx, size_t n) {
     return static_cast<T *>(ctx->pool.get(n * sizeof(T) + 16));
 }
 void pool_put(gls_ctx *ctx, void *p);
+// transfer.hip
 int stream_copy(gls_ctx *ctx, void *dst, const void *src, size_t bytes, hipMemcpyKind kind);
+// several small results; the stream's work is done when it returns
+constexpr int FETCH_PIECES = 4;
+struct FetchPiece {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+int fetch(gls_ctx *ctx, std::initializer_list<FetchPiece> pieces);
+// fills of up to FILL_SEGS arrays in one launch
+constexpr int FILL_SEGS = 12;
+struct Fills {
+    struct Seg {
+        void *p;
+        size_t bytes;
+        uint32_t byte;
+    };
+    gls_ctx *ctx;
+    int n = 0;
+    Seg s[FILL_SEGS];
+    explicit Fills(gls_ctx *c) : ctx(c) {}
+    Fills &add(void *p, int byte, size_t bytes) {
+        if (bytes) s[n++] = Seg{p, bytes, (uint32_t)(byte & 0xFF)};
+        return *this;
+    }
+    int run();
+};
+int dev_graph_copy(gls_ctx *ctx, const DevGraph &src, const DevGraph &dst);
+int dev_graph_fetch(gls_ctx *ctx, const DevGraph &g, uint32_t *f0, uint32_t *f1, uint32_t *pos, int32_t conv);
+void transfer_free(gls_ctx *ctx);
 
 // host strash of `st -c` (cpu_strash.cpp)
 int host_strash_cpu(int32_t nPIs, const std::vector<uint32_t> &f0, const std::vector<uint32_t> &f1,

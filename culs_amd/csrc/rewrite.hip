@@ -1427,8 +1427,9 @@ struct Claims {
 };
 
 __global__ void k_sel_claim(uint32_t round, int32_t nCand, const Plan *__restrict__ plans,
-                            const uint8_t *__restrict__ state, Claims cl) {
+                            const uint8_t *__restrict__ state, Claims cl, uint32_t *activeLeft) {
     int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (c == 0) *activeLeft = 0;             // counted by this round's k_sel_elim
     if (c >= nCand || state[c] != ST_ACTIVE) return;
     const Plan &p = plans[c];
     unsigned long long s = stamp(round, p);
@@ -1482,13 +1483,23 @@ __global__ void k_sel_elim(int32_t nCand, const Plan *__restrict__ plans, uint8_
     else atomicAdd(activeLeft, 1u);
 }
 
+// cnt: new nodes per candidate (0 past the last); sum: the selected ones' gain
+// and number
 __global__ void k_new_counts(int32_t nCand, const Plan *__restrict__ plans, const uint8_t *__restrict__ state,
-                             uint32_t *cnt, unsigned long long *gainSum) {
+                             uint32_t *cnt, unsigned long long *sum) {
     int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (c == nCand) cnt[c] = 0;
+    const bool s = c < nCand && state[c] == ST_SELECTED;
+    const uint64_t m = __ballot(s);
+    if (m && (threadIdx.x & 63u) == 0) atomicAdd(&sum[1], (unsigned long long)__popcll(m));
     if (c >= nCand) return;
-    bool s = state[c] == ST_SELECTED;
     cnt[c] = s ? (uint32_t)plans[c].nNew : 0u;
-    if (s) atomicAdd(gainSum, (unsigned long long)plans[c].gain);
+    if (s) atomicAdd(&sum[0], (unsigned long long)plans[c].gain);
+}
+
+__global__ void k_no_candidate(int32_t n, int4 *best) {
+    const int32_t v = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (v < n) best[v] = make_int4(-1, 0, 0, 0);
 }
 
 __global__ void k_iota2(int32_t n, uint32_t *repl) {
@@ -1710,7 +1721,7 @@ static int sig_bits_for_tags(gls_ctx *ctx, int32_t n, const uint32_t *tag, uint8
     uint32_t *keys = t.get<uint32_t>(m), *vals = t.get<uint32_t>(m), *skeys = t.get<uint32_t>(m);
     uint32_t *svals = t.get<uint32_t>(m), *hist = t.get<uint32_t>(maxTag + 2), *start = t.get<uint32_t>(maxTag + 2);
     if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "signature bits: allocation");
-    GLS_HIP(ctx, hipMemsetAsync(hist, 0, sizeof(uint32_t) * (maxTag + 2), st));
+    GLS_TRY(Fills(ctx).add(hist, 0, sizeof(uint32_t) * (maxTag + 2)).run());
     k_sig_keys<<<tag_grid(m), kBlock, 0, st>>>(n, tag, keys, vals, hist);
     size_t tb2 = 0;
     const uint32_t eb = bits_for(maxTag + 1);
@@ -1752,8 +1763,7 @@ int dev_reorder(gls_ctx *ctx, const DevGraph &in, DevGraph &out, std::vector<int
         void *tmp = t.get<uint8_t>(tb);
         if (!tmp) return gls_fail(ctx, GLS_ERR_NOMEM, "reorder: reduce storage");
         GLS_HIP(ctx, rocprim::reduce(tmp, tb, keys, keys2, 0u, (size_t)m, rocprim::maximum<uint32_t>(), st));
-        GLS_HIP(ctx, hipMemcpyAsync(&maxLevel, keys2, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        GLS_HIP(ctx, hipStreamSynchronize(st));
+        GLS_TRY(stream_copy(ctx, &maxLevel, keys2, sizeof(uint32_t), hipMemcpyDeviceToHost));
         size_t tb2 = 0;
         uint32_t eb = bits_for(maxLevel);
         GLS_HIP(ctx, rocprim::radix_sort_pairs(nullptr, tb2, keys, keys2, ids, ids2, (size_t)m, 0u, eb, st));
@@ -1763,21 +1773,22 @@ int dev_reorder(gls_ctx *ctx, const DevGraph &in, DevGraph &out, std::vector<int
         k_reorder_ids<<<blocks(m, kBlock), kBlock, 0, st>>>(m, ids2, newId);
         int32_t *d_starts = t.get<int32_t>(maxLevel + 2);
         if (!d_starts) return gls_fail(ctx, GLS_ERR_NOMEM, "reorder: starts");
-        GLS_HIP(ctx, hipMemsetAsync(d_starts, 0, sizeof(int32_t) * (maxLevel + 2), st));
+        GLS_TRY(Fills(ctx).add(d_starts, 0, sizeof(int32_t) * (maxLevel + 2)).run());
         k_level_starts<<<blocks(m, kBlock), kBlock, 0, st>>>(m, keys2, d_starts);
         levelStart.assign(maxLevel + 2, 0);
-        GLS_HIP(ctx, hipMemcpyAsync(levelStart.data(), d_starts, sizeof(int32_t) * (maxLevel + 1), hipMemcpyDeviceToHost, st));
         k_reorder_emit<<<blocks(n, kBlock), kBlock, 0, st>>>(n, in.nPIs, in.f0, in.f1, in.level, newId, out.f0,
                                                               out.f1, out.level, tagIn, tags);
         if (in.nPOs > 0)
             k_reorder_pos<<<blocks(in.nPOs, kBlock), kBlock, 0, st>>>(in.nPOs, in.pos, newId, out.pos);
         GLS_HIP(ctx, hipGetLastError());
-        GLS_HIP(ctx, hipStreamSynchronize(st));
+        GLS_TRY(stream_copy(ctx, levelStart.data(), d_starts, sizeof(int32_t) * (maxLevel + 1), hipMemcpyDeviceToHost));
         levelStart[maxLevel + 1] = n;  // one past the last id
     } else {
-        GLS_HIP(ctx, hipMemsetAsync(out.f0, 0, sizeof(uint32_t) * n, st));
-        GLS_HIP(ctx, hipMemsetAsync(out.f1, 0, sizeof(uint32_t) * n, st));
-        GLS_HIP(ctx, hipMemsetAsync(out.level, 0, sizeof(uint32_t) * n, st));
+        GLS_TRY(Fills(ctx)
+                    .add(out.f0, 0, sizeof(uint32_t) * n)
+                    .add(out.f1, 0, sizeof(uint32_t) * n)
+                    .add(out.level, 0, sizeof(uint32_t) * n)
+                    .run());
         if (in.nPOs > 0)
             GLS_HIP(ctx, hipMemcpyAsync(out.pos, in.pos, sizeof(uint32_t) * in.nPOs, hipMemcpyDeviceToDevice, st));
         if (tags) GLS_HIP(ctx, hipMemcpyAsync(tags, tagIn, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st));
@@ -1816,8 +1827,10 @@ static int build_cut_plan(gls_ctx *ctx, Tmp &t, const DevGraph &g, int32_t K, co
     uint32_t *cnt = t.get<uint32_t>((size_t)nL + 1), *dOff = t.get<uint32_t>((size_t)nL + 1);
     if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "cuts: plan storage");
     GLS_HIP(ctx, hipMemcpyAsync(dlv, lv.data(), sizeof(int32_t) * lv.size(), hipMemcpyHostToDevice, st));
-    GLS_HIP(ctx, hipMemsetAsync(nodeLaunch, 0xFF, sizeof(int32_t) * (size_t)n, st));
-    GLS_HIP(ctx, hipMemsetAsync(own, 0xFF, sizeof(uint32_t) * (size_t)n, st));
+    GLS_TRY(Fills(ctx)
+                .add(nodeLaunch, 0xFF, sizeof(int32_t) * (size_t)n)
+                .add(own, 0xFF, sizeof(uint32_t) * (size_t)n)
+                .run());
     k_plan_fill<<<nL, kBlock, 0, st>>>(K, dlv, nodeLaunch);
     for (int p = K - 1; p >= 1; p--)
         k_plan_roots<<<grid_for(n), kBlock, 0, st>>>(n, g.nPIs, K, p, g.f0, g.f1, dlv, nodeLaunch, own, coneSize);
@@ -1842,7 +1855,7 @@ static int build_cut_plan(gls_ctx *ctx, Tmp &t, const DevGraph &g, int32_t K, co
     GLS_HIP(ctx, rocprim::exclusive_scan(nullptr, tb3, ecnt, eoff, 0u, nT + 1, rocprim::plus<uint32_t>(), st));
     void *tmp3 = t.get<uint8_t>(std::max<size_t>(tb3, 1));
     if (!ecnt || !eoff || !heads || !tmp3) return gls_fail(ctx, GLS_ERR_NOMEM, "cuts: plan tasks (%zu)", nT);
-    GLS_HIP(ctx, hipMemsetAsync(ecnt, 0, sizeof(uint32_t) * (nT + 1), st));
+    GLS_TRY(Fills(ctx).add(ecnt, 0, sizeof(uint32_t) * (nT + 1)).run());
     k_plan_ecount<<<grid_for(n), kBlock, 0, st>>>(n, g.nPIs, K, dlv, nodeLaunch, own, S, dOff, coneSize, ecnt);
     GLS_HIP(ctx, rocprim::exclusive_scan(tmp3, tb3, ecnt, eoff, 0u, nT + 1, rocprim::plus<uint32_t>(), st));
     // entries: every node once as a root or packed node, plus the cone
@@ -1878,8 +1891,10 @@ int dev_enumerate_cuts(gls_ctx *ctx, const DevGraph &g, const std::vector<int32_
         return gls_fail(ctx, GLS_ERR_ARG, "GLS_RW_PLAN_CUTS is disabled (its kernel faulted the GPU; cause not found)");
     const bool graphed = (mode & GLS_RW_GRAPH_CUTS) != 0;
     mode &= ~GLS_RW_GRAPH_CUTS;
-    GLS_HIP(ctx, hipMemsetAsync(d_nref, 0, sizeof(int32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(d_cuts, 0, sizeof(uint32_t) * (size_t)n * NCUT * 5, st));
+    GLS_TRY(Fills(ctx)
+                .add(d_nref, 0, sizeof(int32_t) * n)
+                .add(d_cuts, 0, sizeof(uint32_t) * (size_t)n * NCUT * 5)
+                .run());
     k_nref<<<grid_for(n), kBlock, 0, st>>>(n, g.nPIs, g.f0, g.f1, g.nPOs, g.pos, d_nref);
     if (g.nPIs > 0) k_cuts_pi<<<blocks(g.nPIs, kBlock), kBlock, 0, st>>>(g.nPIs, d_nref, d_cuts);
     // levelStart[l] = first id of level l (ids 1.. are level-major); the last
@@ -1896,8 +1911,10 @@ int dev_enumerate_cuts(gls_ctx *ctx, const DevGraph &g, const std::vector<int32_
         unsigned long long *tcuts = pool_get<unsigned long long>(ctx, nslots * 3);
         uint32_t *ctr = pool_get<uint32_t>(ctx, 4);
         if (!tcuts || !ctr) { pool_put(ctx, tcuts); pool_put(ctx, ctr); return gls_fail(ctx, GLS_ERR_NOMEM, "cuts: tagged records"); }
-        GLS_HIP(ctx, hipMemsetAsync(tcuts, 0, sizeof(unsigned long long) * nslots * 3, st));
-        GLS_HIP(ctx, hipMemsetAsync(ctr, 0, sizeof(uint32_t) * 4, st));
+        GLS_TRY(Fills(ctx)
+                    .add(tcuts, 0, sizeof(unsigned long long) * nslots * 3)
+                    .add(ctr, 0, sizeof(uint32_t) * 4)
+                    .run());
         if (g.nPIs > 0)
             k_cuts_pi_tagged<<<blocks((int64_t)g.nPIs * NCUT, kBlock), kBlock, 0, st>>>(g.nPIs, d_nref, tcuts);
         k_cuts_dataflow<<<G, CUTW_BLOCK, 0, st>>>(g.nPIs + 1, n, g.f0, g.f1, d_nref, tcuts, &ctr[0], &ctr[1],
@@ -1927,7 +1944,7 @@ int dev_enumerate_cuts(gls_ctx *ctx, const DevGraph &g, const std::vector<int32_
         if (!d_starts || !ctl) { pool_put(ctx, d_starts); pool_put(ctx, ctl); return gls_fail(ctx, GLS_ERR_NOMEM, "cuts: xcd control"); }
         GLS_HIP(ctx, hipMemcpyAsync(d_starts, levelStart.data(), sizeof(int32_t) * levelStart.size(),
                                     hipMemcpyHostToDevice, st));
-        GLS_HIP(ctx, hipMemsetAsync(ctl, 0, sizeof(uint32_t) * 4, st));
+        GLS_TRY(Fills(ctx).add(ctl, 0, sizeof(uint32_t) * 4).run());
         const dim3 grid((unsigned)(nwg * XCD_COUNT));
         if (kSampleLaunches) {
             const size_t k = 2 * (size_t)ctx->ksamp_n;
@@ -1959,7 +1976,7 @@ int dev_enumerate_cuts(gls_ctx *ctx, const DevGraph &g, const std::vector<int32_
         ctx->ksamp_n = 0;
         ctx->ksamp_units.clear();
         ctx->ksamp_launches.clear();
-        GLS_HIP(ctx, hipMemsetAsync(d_cuts, 0, sizeof(uint32_t) * (size_t)n * NCUT * 5, st));
+        GLS_TRY(Fills(ctx).add(d_cuts, 0, sizeof(uint32_t) * (size_t)n * NCUT * 5).run());
         if (g.nPIs > 0) k_cuts_pi<<<blocks(g.nPIs, kBlock), kBlock, 0, st>>>(g.nPIs, d_nref, d_cuts);
         mode = 0;
     }
@@ -2152,14 +2169,14 @@ static int build_table(gls_ctx *ctx, Tmp &t, const DevGraph &g, GraphView &gv) {
     uint32_t *cnt = t.get<uint32_t>((size_t)n + 1), *off = t.get<uint32_t>((size_t)n + 1);
     uint2 *ent = t.get<uint2>(std::max<size_t>(nAnd, 1));
     if (!cnt || !off || !ent) return gls_fail(ctx, GLS_ERR_NOMEM, "table allocation");
-    GLS_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(uint32_t) * ((size_t)n + 1), st));
+    GLS_TRY(Fills(ctx).add(cnt, 0, sizeof(uint32_t) * ((size_t)n + 1)).run());
     k_table_count<<<grid_for(n), kBlock, 0, st>>>(n, g.nPIs, g.f1, cnt);
     size_t tb = 0;
     GLS_HIP(ctx, rocprim::exclusive_scan(nullptr, tb, cnt, off, 0u, (size_t)n + 1, rocprim::plus<uint32_t>(), st));
     void *tmp = t.get<uint8_t>(std::max<size_t>(tb, 1));
     if (!tmp) return gls_fail(ctx, GLS_ERR_NOMEM, "table scan storage");
     GLS_HIP(ctx, rocprim::exclusive_scan(tmp, tb, cnt, off, 0u, (size_t)n + 1, rocprim::plus<uint32_t>(), st));
-    GLS_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(uint32_t) * ((size_t)n + 1), st));
+    GLS_TRY(Fills(ctx).add(cnt, 0, sizeof(uint32_t) * ((size_t)n + 1)).run());
     k_table_fill<<<grid_for(n), kBlock, 0, st>>>(n, g.nPIs, g.f0, g.f1, off, cnt, ent);
     GLS_HIP(ctx, hipGetLastError());
     gv.tOff = off;
@@ -2174,11 +2191,8 @@ int dev_evaluate(gls_ctx *ctx, const DevGraph &g, const uint32_t *d_cuts, const 
     Tmp t{ctx};
     GraphView gv{g.f0, g.f1, d_nref, g.level, nullptr, nullptr};
     GLS_TRY(build_table(ctx, t, g, gv));
-    GLS_HIP(ctx, hipMemsetAsync(d_best, 0xFF, sizeof(int4) * 1, st));
     // PIs and the constant have no candidate
-    GLS_HIP(ctx, hipMemsetAsync(d_best, 0, sizeof(int4) * (size_t)(g.nPIs + 1), st));
-    std::vector<int4> none(g.nPIs + 1, make_int4(-1, 0, 0, 0));
-    GLS_HIP(ctx, hipMemcpyAsync(d_best, none.data(), sizeof(int4) * none.size(), hipMemcpyHostToDevice, st));
+    k_no_candidate<<<blocks(g.nPIs + 1, kBlock), kBlock, 0, st>>>(g.nPIs + 1, reinterpret_cast<int4 *>(d_best));
     launch_eval(st, g.nObjs, g.nPIs, gv, lib_of(ctx), d_cuts, useZeros, reinterpret_cast<int4 *>(d_best));
     GLS_HIP(ctx, hipGetLastError());
     GLS_HIP(ctx, hipStreamSynchronize(st));
@@ -2213,9 +2227,9 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
         uint8_t *flag = t.get<uint8_t>(n);
         uint32_t *candIds = t.get<uint32_t>(n), *d_cnt = t.get<uint32_t>(4), *d_err = t.get<uint32_t>(4);
         uint32_t *repl = t.get<uint32_t>(n);
-        unsigned long long *d_gain = t.get<unsigned long long>(1);
+        unsigned long long *d_gain = t.get<unsigned long long>(2);
         if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "rewrite: allocation (n=%d)", n);
-        GLS_HIP(ctx, hipMemsetAsync(d_err, 0, 16, st));
+        GLS_TRY(Fills(ctx).add(d_err, 0, 16).run());
         uint8_t *sigBits = nullptr;
         if (tagged) {
             sigBits = t.get<uint8_t>(n);
@@ -2232,8 +2246,7 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
         GraphView gv{g.f0, g.f1, nref, g.level, nullptr, nullptr};
         GLS_TRY(build_table(ctx, t, g, gv));
         tm.mark(); // 3
-        std::vector<int4> none(nPIs + 1, make_int4(-1, 0, 0, 0));
-        GLS_HIP(ctx, hipMemcpyAsync(best, none.data(), sizeof(int4) * none.size(), hipMemcpyHostToDevice, st));
+        k_no_candidate<<<blocks(nPIs + 1, kBlock), kBlock, 0, st>>>(nPIs + 1, best);
         const Lib L = lib_of(ctx);
         launch_eval(st, n, nPIs, gv, L, cuts, useZeros, best);
         GLS_HIP(ctx, hipGetLastError());
@@ -2247,8 +2260,7 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
         if (!tmp) return gls_fail(ctx, GLS_ERR_NOMEM, "rewrite: select storage");
         GLS_HIP(ctx, rocprim::select(tmp, tb, ids, flag, candIds, d_cnt, (size_t)n, st));
         uint32_t nCand = 0;
-        GLS_HIP(ctx, hipMemcpyAsync(&nCand, d_cnt, 4, hipMemcpyDeviceToHost, st));
-        GLS_HIP(ctx, hipStreamSynchronize(st));
+        GLS_TRY(stream_copy(ctx, &nCand, d_cnt, 4, hipMemcpyDeviceToHost));
         uint32_t herr = 0;
         uint32_t nSel = 0, rounds = 0, totalNew = 0;
         unsigned long long estGain = 0;
@@ -2266,39 +2278,35 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
             if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "rewrite: plan allocation");
             k_plan<<<blocks(nCand, EVAL_BLOCK), EVAL_BLOCK, 0, st>>>((int32_t)nCand, candIds, gv, L, cuts, best, plans);
             k_sel_init<<<blocks(nCand, kBlock), kBlock, 0, st>>>((int32_t)nCand, plans, state);
-            GLS_HIP(ctx, hipMemsetAsync(mk, 0, sizeof(uint32_t) * n, st));
-            GLS_HIP(ctx, hipMemsetAsync(cl.W, 0, sizeof(unsigned long long) * n, st));
-            GLS_HIP(ctx, hipMemsetAsync(cl.Wnr, 0, sizeof(unsigned long long) * n, st));
-            GLS_HIP(ctx, hipMemsetAsync(cl.L, 0, sizeof(unsigned long long) * n, st));
-            GLS_HIP(ctx, hipMemsetAsync(cl.M, 0, sizeof(unsigned long long) * n, st));
+            GLS_TRY(Fills(ctx)
+                        .add(mk, 0, sizeof(uint32_t) * n)
+                        .add(cl.W, 0, sizeof(unsigned long long) * n)
+                        .add(cl.Wnr, 0, sizeof(unsigned long long) * n)
+                        .add(cl.L, 0, sizeof(unsigned long long) * n)
+                        .add(cl.M, 0, sizeof(unsigned long long) * n)
+                        .run());
             for (uint32_t r = 1;; r++) {
-                GLS_HIP(ctx, hipMemsetAsync(d_cnt, 0, 4, st));
-                k_sel_claim<<<blocks(nCand, kBlock), kBlock, 0, st>>>(r, (int32_t)nCand, plans, state, cl);
+                k_sel_claim<<<blocks(nCand, kBlock), kBlock, 0, st>>>(r, (int32_t)nCand, plans, state, cl, d_cnt);
                 k_sel_decide<<<blocks(nCand, kBlock), kBlock, 0, st>>>(r, (int32_t)nCand, plans, state, cl, mk);
                 k_sel_elim<<<blocks(nCand, kBlock), kBlock, 0, st>>>((int32_t)nCand, plans, state, mk, d_cnt);
                 GLS_HIP(ctx, hipGetLastError());
                 uint32_t left = 0;
-                GLS_HIP(ctx, hipMemcpyAsync(&left, d_cnt, 4, hipMemcpyDeviceToHost, st));
-                GLS_HIP(ctx, hipStreamSynchronize(st));
+                GLS_TRY(stream_copy(ctx, &left, d_cnt, 4, hipMemcpyDeviceToHost));
                 rounds = r;
                 if (left == 0) break;
                 if (r > 60000) return gls_fail(ctx, GLS_ERR_INTERNAL, "selection did not converge");
             }
-            GLS_HIP(ctx, hipMemsetAsync(d_gain, 0, 8, st));
-            k_new_counts<<<blocks(nCand, kBlock), kBlock, 0, st>>>((int32_t)nCand, plans, state, newCnt, d_gain);
-            GLS_HIP(ctx, hipMemsetAsync(newCnt + nCand, 0, 4, st));
+            GLS_TRY(Fills(ctx).add(d_gain, 0, 16).run());
+            k_new_counts<<<blocks((int64_t)nCand + 1, kBlock), kBlock, 0, st>>>((int32_t)nCand, plans, state, newCnt, d_gain);
             size_t tb2 = 0;
             GLS_HIP(ctx, rocprim::exclusive_scan(nullptr, tb2, newCnt, newOff, 0u, (size_t)nCand + 1, rocprim::plus<uint32_t>(), st));
             void *tmp2 = t.get<uint8_t>(tb2);
             if (!tmp2) return gls_fail(ctx, GLS_ERR_NOMEM, "rewrite: scan storage");
             GLS_HIP(ctx, rocprim::exclusive_scan(tmp2, tb2, newCnt, newOff, 0u, (size_t)nCand + 1, rocprim::plus<uint32_t>(), st));
-            GLS_HIP(ctx, hipMemcpyAsync(&totalNew, newOff + nCand, 4, hipMemcpyDeviceToHost, st));
-            GLS_HIP(ctx, hipMemcpyAsync(&estGain, d_gain, 8, hipMemcpyDeviceToHost, st));
-            // count selected (state == 1)
-            std::vector<uint8_t> hs(nCand);
-            GLS_HIP(ctx, hipMemcpyAsync(hs.data(), state, nCand, hipMemcpyDeviceToHost, st));
-            GLS_HIP(ctx, hipStreamSynchronize(st));
-            for (uint8_t s : hs) nSel += (s == ST_SELECTED);
+            unsigned long long sums[2] = {};
+            GLS_TRY(fetch(ctx, {{&totalNew, newOff + nCand, 4}, {sums, d_gain, 16}}));
+            estGain = sums[0];
+            nSel = (uint32_t)sums[1];
         }
         tm.mark(); // 5
         const int32_t N = n + (int32_t)totalNew;
@@ -2319,8 +2327,7 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
         k_compose<<<grid_for(N), kBlock, 0, st>>>(n, N, nPIs, g.f0, g.f1, repl, comb.f0, comb.f1);
         if (nPOs > 0) k_compose_pos<<<blocks(nPOs, kBlock), kBlock, 0, st>>>(nPOs, g.pos, repl, comb.pos);
         GLS_HIP(ctx, hipGetLastError());
-        GLS_HIP(ctx, hipMemcpyAsync(&herr, d_err, 4, hipMemcpyDeviceToHost, st));
-        GLS_HIP(ctx, hipStreamSynchronize(st));
+        GLS_TRY(stream_copy(ctx, &herr, d_err, 4, hipMemcpyDeviceToHost));
         if (herr) return gls_fail(ctx, GLS_ERR_INTERNAL, "rewrite: inconsistent plan (%u)", herr);
         tm.mark(); // 6
         gls_op_info stInfo = {};

@@ -129,7 +129,7 @@ void gls_server::run() {
                 // the host copy is stale once a pass runs; free it now
                 std::vector<uint32_t>().swap(j->aig->h_f0);
                 std::vector<uint32_t>().swap(j->aig->h_f1);
-                j->aig->host_valid = false;
+                j->aig->host_valid = j->aig->fetched = false;
             }
         // one batched pass per command kind over the jobs whose next command it is
         std::vector<gls_aig *> group[CMD_KINDS];

@@ -1403,8 +1403,7 @@ static int run_sweep(gls_ctx *ctx, SweepCtl *d_ctl, uint32_t first, F launch, Sw
     uint32_t k = first, batch = 4;
     for (;;) {
         for (uint32_t i = 0; i < batch; ++i, ++k) launch(k, h_ctl->curSize);
-        GLS_HIP(ctx, hipMemcpyAsync(h_ctl, d_ctl, sizeof(SweepCtl), hipMemcpyDeviceToHost, ctx->stream));
-        GLS_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        GLS_TRY(stream_copy(ctx, h_ctl, d_ctl, sizeof(SweepCtl), hipMemcpyDeviceToHost));
         if (h_ctl->err) return gls_fail(ctx, GLS_ERR_INTERNAL, "strash table overflow");
         if (h_ctl->curSize == 0) break;
         if (batch < 512) batch *= 2;
@@ -1457,14 +1456,16 @@ int dev_strash(gls_ctx *ctx, const DevGraph &in, DevGraph &out, int32_t *depthOu
         !fcnt || !fstart || !d_misc || !ctl || !ht || !recs || !ofls || !adjY)
         return gls_fail(ctx, GLS_ERR_NOMEM, "strash: device allocation failed (n=%d)", n);
 
-    GLS_HIP(ctx, hipMemsetAsync(ref, 0, sizeof(uint32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(dead, 0, n, st));
-    GLS_HIP(ctx, hipMemsetAsync(cnt, 0, sizeof(uint32_t) * (n + 1), st));
-    GLS_HIP(ctx, hipMemsetAsync(rl, 0xFF, sizeof(unsigned long long) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(wave, 0, sizeof(uint32_t) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(ht, 0xFF, sizeof(unsigned long long) * 2 * cap, st));
-    GLS_HIP(ctx, hipMemsetAsync(val, 0xFF, sizeof(unsigned long long) * n, st));
-    GLS_HIP(ctx, hipMemsetAsync(ctl, 0, sizeof(SweepCtl), st));
+    GLS_TRY(Fills(ctx)
+                .add(ref, 0, sizeof(uint32_t) * n)
+                .add(dead, 0, n)
+                .add(cnt, 0, sizeof(uint32_t) * (n + 1))
+                .add(rl, 0xFF, sizeof(unsigned long long) * n)
+                .add(wave, 0, sizeof(uint32_t) * n)
+                .add(ht, 0xFF, sizeof(unsigned long long) * 2 * cap)
+                .add(val, 0xFF, sizeof(unsigned long long) * n)
+                .add(ctl, 0, sizeof(SweepCtl))
+                .run());
     const int gN = grid_for(n);
     SweepCtl h_ctl{};
     uint32_t rounds = 0;
@@ -1476,8 +1477,7 @@ int dev_strash(gls_ctx *ctx, const DevGraph &in, DevGraph &out, int32_t *depthOu
     k_zero_flags<<<gN, kBlock, 0, st>>>(n, nPIs, ref, nullptr, zflag);
     GLS_HIP(ctx, hipGetLastError());
     GLS_TRY(select_ids(ctx, t, n, zflag, order, &ctl->curSize));
-    GLS_HIP(ctx, hipMemcpyAsync(&h_ctl, ctl, sizeof(SweepCtl), hipMemcpyDeviceToHost, st));
-    GLS_HIP(ctx, hipStreamSynchronize(st));
+    GLS_TRY(stream_copy(ctx, &h_ctl, ctl, sizeof(SweepCtl), hipMemcpyDeviceToHost));
     if (h_ctl.curSize > 0) {
         GLS_TRY(run_sweep(ctx, ctl, 1, [&](uint32_t k, uint32_t hint) {
             k_dangle_round<<<sweep_grid(hint), kBlock, 0, st>>>(k, ctl, nPIs, in.f0, in.f1, ref, dead, order);
@@ -1486,10 +1486,12 @@ int dev_strash(gls_ctx *ctx, const DevGraph &in, DevGraph &out, int32_t *depthOu
 
     const uint32_t nDead = h_ctl.processed;
     // 2. fanout CSR over live AND nodes and the first frontier (wave 1)
-    GLS_HIP(ctx, hipMemsetAsync(fcnt, 0, sizeof(uint32_t) * (n + 4), st));
-    GLS_HIP(ctx, hipMemsetAsync(fstart, 0, sizeof(uint32_t) * (n + 4), st));
-    GLS_HIP(ctx, hipMemsetAsync(d_misc, 0, sizeof(uint32_t) * 8, st));
-    GLS_HIP(ctx, hipMemsetAsync(pending, 0, sizeof(uint32_t) * n, st));
+    GLS_TRY(Fills(ctx)
+                .add(fcnt, 0, sizeof(uint32_t) * (n + 4))
+                .add(fstart, 0, sizeof(uint32_t) * (n + 4))
+                .add(d_misc, 0, sizeof(uint32_t) * 8)
+                .add(pending, 0, sizeof(uint32_t) * n)
+                .run());
     k_kahn_count<<<gN, kBlock, 0, st>>>(n, nPIs, in.f0, in.f1, dead, cnt, pending);
     size_t tb = 0;
     GLS_HIP(ctx, rocprim::exclusive_scan(nullptr, tb, cnt, adjOff, 0u, (size_t)n + 1, rocprim::plus<uint32_t>(), st));
@@ -1560,13 +1562,14 @@ int dev_strash(gls_ctx *ctx, const DevGraph &in, DevGraph &out, int32_t *depthOu
     if (!tmp2) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: select storage");
     GLS_HIP(ctx, rocprim::select(tmp2, tb2, ids, surv, survIds, d_count, (size_t)n, st));
     uint32_t m = 0;
-    GLS_HIP(ctx, hipMemcpyAsync(&m, d_count, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    GLS_HIP(ctx, hipStreamSynchronize(st));
+    GLS_TRY(stream_copy(ctx, &m, d_count, sizeof(uint32_t), hipMemcpyDeviceToHost));
     const int32_t nNew = nPIs + 1 + (int32_t)m;
     GLS_TRY(dev_graph_alloc(ctx, out, nNew, nPIs, nPOs));
-    GLS_HIP(ctx, hipMemsetAsync(out.f0, 0, sizeof(uint32_t) * (nPIs + 1), st));
-    GLS_HIP(ctx, hipMemsetAsync(out.f1, 0, sizeof(uint32_t) * (nPIs + 1), st));
-    GLS_HIP(ctx, hipMemsetAsync(out.level, 0, sizeof(uint32_t) * (nPIs + 1), st));
+    GLS_TRY(Fills(ctx)
+                .add(out.f0, 0, sizeof(uint32_t) * (nPIs + 1))
+                .add(out.f1, 0, sizeof(uint32_t) * (nPIs + 1))
+                .add(out.level, 0, sizeof(uint32_t) * (nPIs + 1))
+                .run());
     const uint32_t *sorted = survIds;
     if (m > 0) {
         k_gather_u32<<<grid_for(m), kBlock, 0, st>>>((int32_t)m, survIds, wave, survWave);
@@ -1667,10 +1670,12 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
             !survIds || !survWave || !sortIds || !sortWave || !newId || !d_misc || !ctl)
             return gls_fail(ctx, GLS_ERR_NOMEM, "strash: device allocation failed (n=%d)", N);
         unsigned long long *d_probes = reinterpret_cast<unsigned long long *>(&d_misc[6]);
-        GLS_HIP(ctx, hipMemsetAsync(ref, 0, sizeof(uint32_t) * N, st));
-        GLS_HIP(ctx, hipMemsetAsync(dead, 0, N, st));
-        GLS_HIP(ctx, hipMemsetAsync(ctl, 0, sizeof(SweepCtl), st));
-        GLS_HIP(ctx, hipMemsetAsync(d_misc, 0, sizeof(uint32_t) * 16, st));
+        GLS_TRY(Fills(ctx)
+                    .add(ref, 0, sizeof(uint32_t) * N)
+                    .add(dead, 0, N)
+                    .add(ctl, 0, sizeof(SweepCtl))
+                    .add(d_misc, 0, sizeof(uint32_t) * 16)
+                    .run());
         const int gN = grid_for(N);
         SweepCtl h_ctl{};
         uint32_t rounds = 0;
@@ -1680,8 +1685,7 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
         k_zero_flags<<<gN, kBlock, 0, st>>>(N, nPIs, ref, nullptr, surv);
         GLS_HIP(ctx, hipGetLastError());
         GLS_TRY(select_ids(ctx, t, N, surv, order, &ctl->curSize));
-        GLS_HIP(ctx, hipMemcpyAsync(&h_ctl, ctl, sizeof(SweepCtl), hipMemcpyDeviceToHost, st));
-        GLS_HIP(ctx, hipStreamSynchronize(st));
+        GLS_TRY(stream_copy(ctx, &h_ctl, ctl, sizeof(SweepCtl), hipMemcpyDeviceToHost));
         if (h_ctl.curSize > 0) {
             GLS_TRY(run_sweep(ctx, ctl, 1, [&](uint32_t k, uint32_t hint) {
                 k_dangle_round<<<sweep_grid(hint), kBlock, 0, st>>>(k, ctl, nPIs, in.f0, in.f1, ref, dead, order);
@@ -1716,7 +1720,7 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
         uint32_t keyRounds = 0;
         for (;; ++keyRounds) {
             if (keyRounds >= kRwRoundLimit) return fallback("key rounds");
-            GLS_HIP(ctx, hipMemsetAsync(&d_misc[5], 0, sizeof(uint32_t), st));
+            GLS_TRY(Fills(ctx).add(&d_misc[5], 0, sizeof(uint32_t)).run());
             k_rw_key_relax<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, fa, &d_misc[5]);
             GLS_HIP(ctx, hipGetLastError());
             uint32_t moved = 0;
@@ -1793,7 +1797,7 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
                 if (!ht || !dkey || !dslot || !nrep) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: dirty table");
             }
             k_fill_u64<<<grid_for((int64_t)2 * cap), kBlock, 0, st>>>(2 * cap, ht, KEY_EMPTY);
-            GLS_HIP(ctx, hipMemsetAsync(&d_misc[3], 0, sizeof(uint32_t), st));
+            GLS_TRY(Fills(ctx).add(&d_misc[3], 0, sizeof(uint32_t)).run());
             const int gD = grid_for(nD);
             k_rw_insert<<<gD, kBlock, 0, st>>>(nD, dlist, nPIs, in.f0, in.f1, rep, wave, ht, cap - 1, dkey, dslot,
                                                nrep, &d_misc[0], d_probes);
@@ -1842,8 +1846,10 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
             GLS_HIP(ctx, hipMemcpyAsync(tags, tagIn, sizeof(uint32_t) * (nPIs + 1), hipMemcpyDeviceToDevice, st));
             *tagOut = tags;
         }
-        GLS_HIP(ctx, hipMemsetAsync(out.f0, 0, sizeof(uint32_t) * (nPIs + 1), st));
-        GLS_HIP(ctx, hipMemsetAsync(out.f1, 0, sizeof(uint32_t) * (nPIs + 1), st));
+        GLS_TRY(Fills(ctx)
+                    .add(out.f0, 0, sizeof(uint32_t) * (nPIs + 1))
+                    .add(out.f1, 0, sizeof(uint32_t) * (nPIs + 1))
+                    .run());
         k_new_ids<<<grid_for(m + nPIs + 1), kBlock, 0, st>>>(N, nPIs, (int32_t)m, sorted, newId);
         // 5. output levels: the survivors' waves when no representative lies on
         // a lower wave than its node, else a level sweep over the output (fa /
@@ -1855,7 +1861,7 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
         if (nPOs > 0) k_rw_pos_out<<<grid_for(nPOs), kBlock, 0, st>>>(nPOs, nPIs, in.pos, rep, newId, out.pos);
         GLS_HIP(ctx, hipGetLastError());
         if (sweepOut) {
-            GLS_HIP(ctx, hipMemsetAsync(&d_misc[0], 0, sizeof(uint32_t) * 2, st));
+            GLS_TRY(Fills(ctx).add(&d_misc[0], 0, sizeof(uint32_t) * 2).run());
             k_level_sweep<<<1, SW_WG, 0, st>>>((uint32_t)nNew, fa, fb, out.level, &d_misc[0], &d_misc[1]);
             GLS_HIP(ctx, hipGetLastError());
             GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
