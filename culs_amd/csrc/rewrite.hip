@@ -1464,8 +1464,12 @@ __global__ void k_sel_decide(uint32_t round, int32_t nCand, const Plan *__restri
     for (int i = 0; i < p.nM; i++) atomicOr(&mk[p.M[i]], MK_M);
 }
 
+// the first SEL_REST candidates still active also go to list, for k_sel_rest
+constexpr uint32_t SEL_REST = 256, SEL_WG = 1024, SEL_LANES = 8;
+constexpr uint32_t SEL_ROUNDS = 60000;         // stamps hold 16 bits of round
+
 __global__ void k_sel_elim(int32_t nCand, const Plan *__restrict__ plans, uint8_t *state,
-                           const uint32_t *__restrict__ mk, uint32_t *activeLeft) {
+                           const uint32_t *__restrict__ mk, uint32_t *activeLeft, uint32_t *list) {
     int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (c >= nCand || state[c] != ST_ACTIVE) return;
     const Plan &p = plans[c];
@@ -1479,8 +1483,114 @@ __global__ void k_sel_elim(int32_t nCand, const Plan *__restrict__ plans, uint8_
         if (mk[p.L[i]] & MK_WNR) conf = true;
     for (int i = 0; i < p.nM && !conf; i++)
         if (mk[p.M[i]] & MK_W) conf = true;
-    if (conf) state[c] = ST_REJECTED;
-    else atomicAdd(activeLeft, 1u);
+    if (conf) { state[c] = ST_REJECTED; return; }
+    const uint32_t k = atomicAdd(activeLeft, 1u);
+    if (k < SEL_REST) list[k] = (uint32_t)c;
+}
+
+// All remaining rounds of the selection by one workgroup, once at most SEL_REST
+// candidates are active (multipliers need 10 to 15 rounds, most of them for a
+// few).  The candidates are in LDS, eight lanes share one's nodes.  Claims and
+// marks are updated by atomics and read past the L1, which does not see them.
+// What bounds it: a round is some trips to memory between three barriers, about
+// 10 us; three kernels and the host's look at the count took 45.  With more
+// candidates left the whole device is faster (at 2048 a burst of 32 requests
+// lost 4 ms).
+__global__ void __launch_bounds__(SEL_WG) k_sel_rest(uint32_t round, uint32_t n, const uint32_t *__restrict__ list,
+                                                     const Plan *__restrict__ plans, uint8_t *state, Claims cl,
+                                                     uint32_t *mk, uint32_t *out) {
+    __shared__ uint32_t s_list[2][SEL_REST];
+    __shared__ uint8_t s_won[SEL_REST];
+    __shared__ uint32_t s_n;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, sub = tid % SEL_LANES;
+    const uint64_t group = 0xFFull << (lane - lane % SEL_LANES);
+    if (tid < n) s_list[0][tid] = list[tid];
+    __syncthreads();
+    auto ld = [](const unsigned long long *q) {
+        return __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto ldm = [](const uint32_t *q) { return __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    // a barrier that this wavefront's memory operations have passed
+    auto settle = []() {
+        __builtin_amdgcn_s_waitcnt(0x0070);     // vmcnt(0), lgkmcnt(0)
+        __syncthreads();
+    };
+    for (uint32_t b = 0; n != 0 && round < SEL_ROUNDS; round++, b ^= 1u) {
+        // node e of a plan: 0 of W, 1 of L, 2 of M
+        auto node = [](const Plan &q, int e, int &kind) -> int {
+            if (e < q.nW) { kind = 0; return q.W[e]; }
+            e -= q.nW;
+            if (e < q.nL) { kind = 1; return q.L[e]; }
+            kind = 2;
+            return q.M[e - q.nL];
+        };
+        for (uint32_t k = tid / SEL_LANES; k < n; k += SEL_WG / SEL_LANES) {
+            const Plan &q = plans[s_list[b][k]];
+            const unsigned long long st = stamp(round, q);
+            for (int e = (int)sub, all = q.nW + q.nL + q.nM; e < all; e += (int)SEL_LANES) {
+                int kind;
+                const int x = node(q, e, kind);
+                if (kind == 0) {
+                    atomicMax(&cl.W[x], st);
+                    if (x != q.id) atomicMax(&cl.Wnr[x], st);
+                } else {
+                    atomicMax(kind == 1 ? &cl.L[x] : &cl.M[x], st);
+                }
+            }
+            if (sub == 0) s_won[k] = 0;
+        }
+        settle();
+        for (uint32_t k0 = 0; k0 < n; k0 += SEL_WG / SEL_LANES) {
+            const uint32_t k = k0 + tid / SEL_LANES;
+            bool lost = k >= n;
+            if (!lost) {
+                const Plan &q = plans[s_list[b][k]];
+                const unsigned long long st = stamp(round, q);
+                for (int e = (int)sub, all = q.nW + q.nL + q.nM; e < all; e += (int)SEL_LANES) {
+                    int kind;
+                    const int x = node(q, e, kind);
+                    if (kind == 0) lost |= ld(&cl.W[x]) != st || ld(&cl.M[x]) >= st || (x != q.id && ld(&cl.L[x]) >= st);
+                    else lost |= ld(kind == 1 ? &cl.Wnr[x] : &cl.W[x]) >= st;
+                }
+            }
+            const bool win = (__ballot(lost) & group) == 0;
+            if (k < n && win) {
+                const uint32_t c = s_list[b][k];
+                const Plan &q = plans[c];
+                if (sub == 0) { s_won[k] = 1; state[c] = ST_SELECTED; }
+                for (int e = (int)sub, all = q.nW + q.nL + q.nM; e < all; e += (int)SEL_LANES) {
+                    int kind;
+                    const int x = node(q, e, kind);
+                    atomicOr(&mk[x], kind == 0 ? MK_W | (x != q.id ? MK_WNR : 0u) : kind == 1 ? (uint32_t)MK_L : (uint32_t)MK_M);
+                }
+            }
+        }
+        if (tid == 0) s_n = 0;
+        settle();
+        for (uint32_t k0 = 0; k0 < n; k0 += SEL_WG / SEL_LANES) {
+            const uint32_t k = k0 + tid / SEL_LANES;
+            const bool open = k < n && !s_won[k];
+            bool conf = false;
+            if (open) {
+                const Plan &q = plans[s_list[b][k]];
+                for (int e = (int)sub, all = q.nW + q.nL + q.nM; e < all; e += (int)SEL_LANES) {
+                    int kind;
+                    const int x = node(q, e, kind);
+                    const uint32_t m = ldm(&mk[x]);
+                    conf |= (m & (kind == 0 ? MK_W | MK_M | (x != q.id ? MK_L : 0u) : kind == 1 ? (uint32_t)MK_WNR : (uint32_t)MK_W)) != 0;
+                }
+            }
+            const bool out1 = (__ballot(conf) & group) != 0;
+            if (open && sub == 0) {
+                const uint32_t c = s_list[b][k];
+                if (out1) state[c] = ST_REJECTED;
+                else s_list[b ^ 1u][atomicAdd(&s_n, 1u)] = c;
+            }
+        }
+        settle();
+        n = s_n;
+    }
+    if (tid == 0) { out[0] = round; out[1] = n; }
 }
 
 // cnt: new nodes per candidate (0 past the last); sum: the selected ones' gain
@@ -2273,6 +2383,7 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
             state = t.get<uint8_t>(nCand);
             uint32_t *mk = t.get<uint32_t>(n), *newCnt = t.get<uint32_t>(nCand + 1);
             newOff = t.get<uint32_t>(nCand + 1);
+            uint32_t *selList = t.get<uint32_t>(SEL_REST);
             Claims cl{t.get<unsigned long long>(n), t.get<unsigned long long>(n), t.get<unsigned long long>(n),
                       t.get<unsigned long long>(n)};
             if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "rewrite: plan allocation");
@@ -2288,13 +2399,21 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
             for (uint32_t r = 1;; r++) {
                 k_sel_claim<<<blocks(nCand, kBlock), kBlock, 0, st>>>(r, (int32_t)nCand, plans, state, cl, d_cnt);
                 k_sel_decide<<<blocks(nCand, kBlock), kBlock, 0, st>>>(r, (int32_t)nCand, plans, state, cl, mk);
-                k_sel_elim<<<blocks(nCand, kBlock), kBlock, 0, st>>>((int32_t)nCand, plans, state, mk, d_cnt);
+                k_sel_elim<<<blocks(nCand, kBlock), kBlock, 0, st>>>((int32_t)nCand, plans, state, mk, d_cnt, selList);
                 GLS_HIP(ctx, hipGetLastError());
                 uint32_t left = 0;
                 GLS_TRY(stream_copy(ctx, &left, d_cnt, 4, hipMemcpyDeviceToHost));
                 rounds = r;
                 if (left == 0) break;
-                if (r > 60000) return gls_fail(ctx, GLS_ERR_INTERNAL, "selection did not converge");
+                if (r > SEL_ROUNDS) return gls_fail(ctx, GLS_ERR_INTERNAL, "selection did not converge");
+                if (left > SEL_REST) continue;
+                k_sel_rest<<<1, SEL_WG, 0, st>>>(r + 1, left, selList, plans, state, cl, mk, d_cnt);
+                GLS_HIP(ctx, hipGetLastError());
+                uint32_t rest[2] = {};
+                GLS_TRY(stream_copy(ctx, rest, d_cnt, sizeof(rest), hipMemcpyDeviceToHost));
+                if (rest[1]) return gls_fail(ctx, GLS_ERR_INTERNAL, "selection did not converge");
+                rounds = rest[0] - 1;
+                break;
             }
             GLS_TRY(Fills(ctx).add(d_gain, 0, 16).run());
             k_new_counts<<<blocks((int64_t)nCand + 1, kBlock), kBlock, 0, st>>>((int32_t)nCand, plans, state, newCnt, d_gain);
