@@ -28,10 +28,9 @@
 // new nodes take consecutive ids by a prefix sum over its covers: the ids are
 // then the output's, levels travel with the literals and the table's values,
 // and nothing is renumbered.  Which ANDs are roots is a property of their
-// fanout edges, so all covers are computed in one launch; roots that no
-// reached cover has as input are dropped by a cascade over the cover graph,
-// and a synchronous topological sweep gives the levels.  Both sweeps, and the
-// reconstruction of a level that fits its LDS, run in one persistent workgroup
+// fanout edges, so all covers are computed in one launch; one sweep over
+// them in id order tells which ones a PO reaches, and their levels.  The sweep,
+// and the reconstruction of a level that fits its LDS, run in one persistent workgroup
 // per member of a batched arena (one in all for a single AIG): a step is bound
 // by the latency of its lookups, and the members do not depend on each other.
 // Other levels run each phase of a step as a grid-wide kernel.
@@ -58,11 +57,6 @@ constexpr int COVER_THREADS = 65536;  // most threads of a cover launch (each ow
 // few inputs above BAL_MAX_COVER: room for that
 constexpr int COVER_SCRATCH = BAL_MAX_COVER + 64;
 constexpr int COVER_FAST = 16;        // first inputs of a cover, kept in LDS during its DFS
-// a frontier wider than this runs as grid-wide rounds, SWEEP_GRID_ROUNDS per
-// host check (a round costs about 1 us per 1024 covers in one workgroup, and
-// about 9 us as a launch)
-constexpr uint32_t SWEEP_WIDE = 8192;
-constexpr int SWEEP_GRID_ROUNDS = 8;
 constexpr uint32_t UNSET = 0xFFFFFFFFu;
 constexpr unsigned long long EMPTY64 = ~0ull;
 
@@ -151,6 +145,12 @@ __device__ __forceinline__ unsigned long long and_key_of(uint32_t x, uint32_t y)
     return x < y ? (unsigned long long)x << 32 | y : (unsigned long long)y << 32 | x;
 }
 
+// LDS that other wavefronts write (a volatile pointer would make these FLAT
+// loads, which wait for all memory)
+template <class T> __device__ __forceinline__ T lds_load(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // ---------------------------------------------------------------------------
 // phase 1: covers
 // ---------------------------------------------------------------------------
@@ -193,8 +193,8 @@ struct CoverArgs {
     uint64_t poolCap;
     uint32_t *scratch;               // COVER_SCRATCH entries per thread
     uint8_t *isRoot;
-    uint32_t *indeg;                 // covers that have a root as input and are not yet taken by a sweep
     uint32_t *extra, *extraLen;      // roots met at the stack / size limits
+    uint32_t *disorder;              // an AND input's id is not below its cover's root
     uint32_t *err;                   // 1: cover pool full
 };
 
@@ -259,7 +259,7 @@ __global__ void __launch_bounds__(kB) k_covers(CoverArgs a, uint32_t nList, cons
             const uint32_t lit = in[i], id = lit >> 1;
             a.pool[off + i] = lit;
             if ((int32_t)id > a.nPIs) {
-                atomicAdd(&a.indeg[id], 1u);
+                if (id >= v) *a.disorder = 1u;
                 // an AND that is no root by its edges: a limit cut the cover there
                 if (a.isRoot[id] == 0) {
                     uint32_t *word = reinterpret_cast<uint32_t *>(a.isRoot + (id & ~3u));
@@ -272,126 +272,171 @@ __global__ void __launch_bounds__(kB) k_covers(CoverArgs a, uint32_t nList, cons
     }
 }
 
-// ---- sweeps over the cover graph.  A sweep starts from the listed roots
-// without a parent cover and takes a root when its last parent cover is taken:
-//   drop: from the roots that no PO drives; they are unreached (a constant
-//         cover has no inputs, and dangling logic no PO);
-//   levels: from the PO drivers; a root taken in round L has its longest path
-//         from a PO equal to L, which is the last level the reference's
-//         sweep puts it on (again on every level it is reached on,
-//         balance.cu:958-1037).
-struct SweepArgs {
-    const uint2 *cover;
-    const uint32_t *pool;
-    int32_t nPIs;
-    const uint32_t *mark;
-    uint32_t *indeg;
-    uint32_t *lastLevel;             // round of a taken root; UNSET, or DROPPED
-    uint32_t *front[2];              // round r's frontier, in front[r & 1] from the segment's first root
-    uint32_t drop;
+// ---- the levels of the covers.  Fanins have smaller ids than their AND, so a
+// cover's inputs have smaller ids than its root.  Roots are laid
+// out by falling id, per segment, so covers stand before their inputs: one
+// workgroup per segment goes over them in chunks of 1024, and a root hands its
+// level to its cover's inputs.  A level is 1 above the reference's (0: no PO
+// reaches the root), so a root's level is the largest value handed to it.
+//
+// What bounds it is the chain of dependent roots within a chunk (an LDS
+// round trip and two LDS atomics a step), so nothing else is waited for there:
+// the levels of the next ID_RING - 1 chunks are in LDS, and so are the chunk's
+// inputs, read a chunk ahead; only a root that is further away is handed its
+// level by an atomic in memory.  A root counts the parents in its own chunk
+// that are still to come (counted by k_id_pack); those of earlier chunks are
+// done at the barrier.  LDS is double buffered, so a chunk has one barrier.
+// 2M random ANDs (1.2M covers, 1795 levels): 2.5 ms; 15.2 for a level at a
+// time, where each of a level's four dependent accesses was a miss in memory.
+// With the inputs read from LDS after the root is known, 3.5.
+constexpr uint32_t ID_CHUNK = BAL_WG;
+constexpr uint32_t ID_RING = 16;         // chunks
+constexpr uint32_t ID_INPUTS = 6144;     // inputs of a chunk in LDS; the rest is read from memory
+constexpr uint32_t IDQ_IN = ID_INPUTS / ID_CHUNK;
+constexpr uint32_t ID_NEAR = 4;          // inputs of a root that are in registers
+
+struct IdSweepArgs {
+    const uint32_t *segFirst, *segCnt;   // positions of a segment
+    const uint32_t *off, *in;            // per position its cover's inputs, as positions (UNSET: no AND)
+    const uint32_t *pend;                // parents within the position's chunk
+    uint32_t *val;                       // 1 for a PO driver, else 0; becomes the level + 1
+    uint32_t *rounds;                    // per segment: levels
 };
-constexpr uint32_t DROPPED = 0xFFFFFFFEu;
 
-// Takes root v; add(id, want) appends an input that it was the last parent of
-// (called with want false too: appends go by wavefront).  Four inputs at a
-// time: a round is bound by the latency of its loads and atomics, not by their
-// number.
-template <class Add>
-__device__ __forceinline__ void sweep_take(const SweepArgs &a, bool has, uint32_t v, uint32_t round, Add add) {
-    uint2 c = make_uint2(0u, 0u);
-    if (has) {
-        a.lastLevel[v] = a.drop ? DROPPED : round;
-        c = a.cover[v];
-    }
-    for (uint32_t i = 0; __ballot(i < c.y) != 0; i += 4) {
-        uint32_t id[4], left[4];
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++) id[j] = i + j < c.y ? a.pool[c.x + i + j] >> 1 : 0u;
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++) left[j] = (int32_t)id[j] > a.nPIs ? atomicSub(&a.indeg[id[j]], 1u) : 0u;
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++) add(id[j], left[j] == 1u && !(a.drop && (a.mark[id[j]] & RM_PO)));
+// positions by falling id within the segment (order: roots by segment and id)
+__global__ void k_id_place(uint32_t m, const uint32_t *__restrict__ order, const uint32_t *__restrict__ tag,
+                           const uint32_t *__restrict__ segFirst, const uint32_t *__restrict__ segCnt,
+                           const uint2 *__restrict__ cover, const uint32_t *__restrict__ mark, uint32_t *rootAt,
+                           uint32_t *place, uint32_t *len, uint32_t *pend, uint32_t *val) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= m; i += stride) {
+        if (i == m) { len[m] = 0; continue; }
+        const uint32_t v = order[i], s = tag ? tag[v] : 0u, first = segFirst[s];
+        const uint32_t p = first + (segCnt[s] - 1u - ((uint32_t)i - first));
+        rootAt[p] = v;
+        place[v] = p;
+        len[p] = cover[v].y;
+        pend[p] = 0;
+        val[p] = mark[v] & RM_PO ? 1u : 0u;
     }
 }
 
-// round 0 of a sweep
-__global__ void k_sweep_first(uint32_t nRoots, const uint32_t *__restrict__ roots, SweepArgs a,
-                              const uint32_t *__restrict__ tag, const uint32_t *__restrict__ segFirst,
-                              uint32_t *segLen) {
+__global__ void k_id_pack(uint32_t m, const uint32_t *__restrict__ rootAt, const uint32_t *__restrict__ tag,
+                          const uint32_t *__restrict__ segFirst, const uint2 *__restrict__ cover,
+                          const uint32_t *__restrict__ pool, const uint32_t *__restrict__ place, int32_t nPIs,
+                          const uint32_t *__restrict__ off, uint32_t *in, uint32_t *pend) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i - (threadIdx.x & 63) < (int64_t)nRoots;
-         i += stride) {
-        const bool has = i < (int64_t)nRoots;
-        const uint32_t v = has ? roots[i] : 0u;
-        const bool want = has && a.indeg[v] == 0u && a.lastLevel[v] == UNSET && ((a.mark[v] & RM_PO) == 0) == (a.drop != 0);
-        if (tag) {
-            // roots are in id order, so a wavefront's are mostly of one segment:
-            // one append per segment
-            const uint32_t s = has ? tag[v] : 0u;
-            for (uint64_t left = __ballot(want); left;) {
-                const uint32_t seg = (uint32_t)__shfl((int)s, __ffsll((unsigned long long)left) - 1);
-                const bool mine = want && s == seg;
-                const uint32_t q = wave_append(&segLen[seg], mine);
-                if (mine) a.front[0][segFirst[seg] + q] = v;
-                left &= ~__ballot(mine);
+    for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < m; p += stride) {
+        const uint32_t v = rootAt[p], first = segFirst[tag ? tag[v] : 0u], chunk = ((uint32_t)p - first) / ID_CHUNK;
+        const uint2 c = cover[v];
+        for (uint32_t j = 0; j < c.y; j++) {
+            const uint32_t id = pool[c.x + j] >> 1, q = (int32_t)id > nPIs ? place[id] : UNSET;
+            in[off[p] + j] = q;
+            if (q != UNSET && (q - first) / ID_CHUNK == chunk) atomicAdd(&pend[q], 1u);
+        }
+    }
+}
+
+__global__ void __launch_bounds__(ID_CHUNK) k_id_sweep(IdSweepArgs a) {
+    __shared__ uint32_t s_val[ID_RING * ID_CHUNK];
+    __shared__ uint32_t s_in[2][ID_INPUTS];
+    __shared__ uint32_t s_pend[2][ID_CHUNK];
+    __shared__ uint32_t s_most;
+    const uint32_t tid = threadIdx.x, first = a.segFirst[blockIdx.x], cnt = a.segCnt[blockIdx.x];
+    const uint32_t nChunk = (cnt + ID_CHUNK - 1) / ID_CHUNK;
+    // a chunk's words, one root per thread
+    struct Chunk {
+        uint32_t base, end;                  // its inputs
+        uint32_t off, stop, pend, val, in[IDQ_IN];
+    };
+    auto chunk_off = [&](uint32_t c) -> uint32_t { return c <= nChunk ? a.off[first + min(c * ID_CHUNK, cnt)] : 0u; };
+    auto load_chunk = [&](uint32_t c, uint32_t base, uint32_t end, Chunk &x) {
+        const uint32_t k = c * ID_CHUNK + tid;
+        const bool has = k < cnt;
+        x.base = base;
+        x.end = end;
+        x.off = has ? a.off[first + k] : 0u;
+        x.stop = has ? a.off[first + k + 1] : 0u;
+        x.pend = has ? a.pend[first + k] : 0u;
+        x.val = has ? __hip_atomic_load(&a.val[first + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+#pragma unroll
+        for (uint32_t q = 0; q < IDQ_IN; q++) {
+            const uint32_t i = base + tid + q * ID_CHUNK;
+            x.in[q] = i < end ? a.in[i] : 0u;
+        }
+    };
+    for (uint32_t i = tid; i < ID_RING * ID_CHUNK; i += ID_CHUNK) s_val[i] = 0;
+    if (tid == 0) s_most = 0;
+    Chunk cur;
+    uint32_t end1 = chunk_off(1), end2 = chunk_off(2), most = 0;
+    if (nChunk != 0) load_chunk(0, chunk_off(0), end1, cur);
+    __syncthreads();
+    for (uint32_t c = 0; c < nChunk; c++) {
+        const uint32_t b = c & 1u, k = c * ID_CHUNK + tid;
+        // this chunk's words; atomics of the chunk before are in memory too
+        __builtin_amdgcn_s_waitcnt(0x0F70);     // vmcnt(0)
+        uint32_t *own = &s_val[(c % ID_RING) * ID_CHUNK + tid];
+        s_pend[b][tid] = cur.pend;
+        if (cur.val) atomicMax(own, cur.val);
+#pragma unroll
+        for (uint32_t q = 0; q < IDQ_IN; q++)
+            if (cur.base + tid + q * ID_CHUNK < cur.end) s_in[b][tid + q * ID_CHUNK] = cur.in[q];
+        const uint32_t off = cur.off, stop = cur.stop, base = cur.base;
+        __syncthreads();
+        const uint32_t nextBase = end1, nextEnd = end2;
+        end1 = end2;
+        end2 = chunk_off(c + 3);
+        if (c + 1 < nChunk) load_chunk(c + 1, nextBase, nextEnd, cur);
+        bool wait = k < cnt;
+        uint32_t v = 0;
+        // the first inputs are in registers before the root's level is known
+        auto input = [&](uint32_t i) -> uint32_t {
+            if (i >= stop) return UNSET;
+            return i - base < ID_INPUTS ? s_in[b][i - base] : a.in[i];
+        };
+        uint32_t near[ID_NEAR];
+#pragma unroll
+        for (uint32_t j = 0; j < ID_NEAR; j++) near[j] = input(off + j);
+        auto hand = [&](uint32_t q) {
+            if (q == UNSET) return;
+            const uint32_t d = (q - first) / ID_CHUNK, t = (q - first) % ID_CHUNK;
+            if (v) {
+                if (d - c < ID_RING - 1) atomicMax(&s_val[(d % ID_RING) * ID_CHUNK + t], v + 1u);
+                else atomicMax(&a.val[q], v + 1u);
             }
-        } else {
-            const uint32_t q = wave_append(segLen, want);
-            if (want) a.front[0][q] = v;
+            asm volatile("" ::: "memory");       // handed over before it is counted
+            if (d == c) atomicSub(&s_pend[b][t], 1u);
+        };
+        while (__ballot(wait) != 0) {
+            const uint32_t left = lds_load(&s_pend[b][tid]);
+            asm volatile("" ::: "memory");       // the level is read after the count
+            const uint32_t x = lds_load(own);
+            if (!wait || left != 0) continue;
+            wait = false;
+            v = x;
+#pragma unroll
+            for (uint32_t j = 0; j < ID_NEAR; j++) hand(near[j]);
+            for (uint32_t i = off + ID_NEAR; i < stop; i++) hand(input(i));
         }
+        if (k < cnt) a.val[first + k] = v;
+        most = max(most, v);
+        *own = 0;                                // of the chunk that takes its place
     }
+    atomicMax(&s_most, most);
+    __syncthreads();
+    if (tid == 0) a.rounds[blockIdx.x] = s_most;
 }
 
-// One workgroup per segment: rounds until the frontier is empty (or, for a
-// single segment, wider than `wide`).  segLen: the frontier's size, in and
-// out; segRound: rounds done.
-__global__ void __launch_bounds__(BAL_WG) k_sweep_wg(SweepArgs a, const uint32_t *__restrict__ segFirst,
-                                                     uint32_t *segLen, uint32_t *segRound, uint32_t wide) {
-    __shared__ uint32_t s_next;
-    const uint32_t seg = blockIdx.x, base = segFirst[seg], tid = threadIdx.x;
-    uint32_t round = segRound[seg], cur = segLen[seg];
-    while (cur != 0 && cur <= wide) {
-        if (tid == 0) s_next = 0;
-        __syncthreads();
-        const uint32_t *front = a.front[round & 1u] + base;
-        uint32_t *next = a.front[(round & 1u) ^ 1u] + base;
-        for (uint32_t k = tid; k - (tid & 63u) < cur; k += BAL_WG) {
-            const bool has = k < cur;
-            sweep_take(a, has, has ? front[k] : 0u, round, [&](uint32_t id, bool want) {
-                const uint32_t q = wave_append(&s_next, want);
-                if (want) next[q] = id;
-            });
-        }
-        __syncthreads();
-        cur = s_next;
-        round++;
-        __syncthreads();
-    }
-    if (tid == 0) {
-        segLen[seg] = cur;
-        segRound[seg] = round;
-    }
-}
-
-// One grid-wide round: len[0] the frontier's size, len[1] collects the next
-// one's (cleared by the host's batch).
-__global__ void k_sweep_grid(SweepArgs a, uint32_t round, uint32_t *len) {
-    const uint32_t cur = len[0];
-    const uint32_t *front = a.front[round & 1u];
-    uint32_t *next = a.front[(round & 1u) ^ 1u];
+__global__ void k_id_levels(uint32_t m, const uint32_t *__restrict__ rootAt, const uint32_t *__restrict__ val,
+                            uint32_t *lastLevel) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k - (threadIdx.x & 63) < (int64_t)cur; k += stride) {
-        const bool has = k < (int64_t)cur;
-        sweep_take(a, has, has ? front[k] : 0u, round, [&](uint32_t id, bool want) {
-            const uint32_t q = wave_append(&len[1], want);
-            if (want) next[q] = id;
-        });
-    }
+    for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < m; p += stride)
+        if (val[p]) lastLevel[rootAt[p]] = val[p] - 1u;
 }
 
 __global__ void k_taken_flags(int32_t n, const uint32_t *__restrict__ lastLevel, uint8_t *flag) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += stride) flag[v] = lastLevel[v] < DROPPED;
+    for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v < n; v += stride) flag[v] = lastLevel[v] != UNSET;
 }
 
 __global__ void __launch_bounds__(kBlock) k_count_tags(uint32_t m, const uint32_t *__restrict__ roots,
@@ -403,6 +448,12 @@ __global__ void __launch_bounds__(kBlock) k_count_tags(uint32_t m, const uint32_
     tag_chunk(0, m, b, e);
     for (int64_t i = b + threadIdx.x; i < e; i += blockDim.x) tb.add(cnt, tag[roots[i]], 1u);
     tb.flush_add(cnt, 0xFFFFFFFFu);
+}
+
+__global__ void k_gather_tags(uint32_t m, const uint32_t *__restrict__ roots, const uint32_t *__restrict__ tag,
+                              uint32_t *keys) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m; i += stride) keys[i] = tag[roots[i]];
 }
 
 // sort key of every root: its level, after the levels of the segments before
@@ -561,10 +612,6 @@ __device__ __forceinline__ unsigned long long input_sig(const RecArgs &r, uint32
 }
 
 // ---- one workgroup per segment, levels within its LDS
-// (a volatile pointer would make these FLAT loads, which wait for all memory)
-template <class T> __device__ __forceinline__ T lds_load(const T *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
 constexpr uint32_t LT_INPUTS = 4096;      // inputs of a level
 constexpr uint32_t LT_COVERS = 2048;      // covers of a level
 constexpr uint32_t LT_NEW = 3072;         // ANDs that a level can create
@@ -1339,27 +1386,26 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
     Tmp t{ctx};
     const auto t0 = std::chrono::steady_clock::now();
     // ---- phase 1: covers
-    uint32_t *nFo = t.get<uint32_t>(n), *mark = t.get<uint32_t>(n), *indeg = t.get<uint32_t>(n);
+    uint32_t *nFo = t.get<uint32_t>(n), *mark = t.get<uint32_t>(n), *place = t.get<uint32_t>(n);
     uint2 *cover = t.get<uint2>(n);
     uint32_t *lastLevel = t.get<uint32_t>(n), *roots = t.get<uint32_t>(n), *rootsSorted = t.get<uint32_t>(n);
     uint8_t *flag = t.get<uint8_t>((size_t)n + 4), *flag2 = t.get<uint8_t>(n);
     uint32_t *extra = t.get<uint32_t>(n);
-    // [0] pool next, [1] error, [2] extra roots, [3] roots, [4..6] largest level, [8..9] counter
+    // [0] pool next, [1] error, [2] extra roots, [3] roots, [4..6] largest level, [7] ids out of order, [8..9] counter
     uint32_t *ctr = t.get<uint32_t>(16);
     const uint64_t poolCap = 2ull * (uint64_t)n + 64;   // cover inputs are distinct fanin edges
     uint32_t *pool = t.get<uint32_t>(poolCap);
     const int coverThreads = (int)std::min<int64_t>(COVER_THREADS, (int64_t)nblocks(n) * kB);
     uint32_t *scratch = t.get<uint32_t>((size_t)coverThreads * COVER_SCRATCH);
-    uint32_t *segInfo = t.get<uint32_t>(4 * (size_t)nSeg + 4), *flen = t.get<uint32_t>(SWEEP_GRID_ROUNDS + 1);
+    uint32_t *segInfo = t.get<uint32_t>(3 * (size_t)nSeg);
     if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: allocation (n=%d)", n);
-    uint32_t *segFirst = segInfo, *segLen = segInfo + nSeg + 1, *segRound = segLen + nSeg, *segCnt = segRound + nSeg;
+    uint32_t *segFirst = segInfo, *segRound = segInfo + nSeg, *segCnt = segRound + nSeg;
     GLS_TRY(Fills(ctx)
                 .add(nFo, 0, sizeof(uint32_t) * n)
                 .add(mark, 0, sizeof(uint32_t) * n)
-                .add(indeg, 0, sizeof(uint32_t) * n)
                 .add(lastLevel, 0xFF, sizeof(uint32_t) * n)
                 .add(ctr, 0, sizeof(uint32_t) * 16)
-                .add(segInfo, 0, sizeof(uint32_t) * (4 * (size_t)nSeg + 4))
+                .add(segInfo, 0, sizeof(uint32_t) * 3 * (size_t)nSeg)
                 .run());
     k_fanouts<<<nblocks(n), kB, 0, st>>>(n, nPIs, in.f0, in.f1, nPOs, in.pos, nFo, mark);
     if (nPOs > 0) k_po_marks<<<nblocks(nPOs), kB, 0, st>>>(nPOs, in.pos, mark);
@@ -1376,11 +1422,11 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
     };
     uint32_t nCand = 0;
     GLS_TRY(select_ids(flag, nCand));
-    const CoverArgs ca{in.f0, in.f1, nFo, nPIs, cover, pool, &ctr[0], poolCap, scratch, flag, indeg, extra, &ctr[2],
+    const CoverArgs ca{in.f0, in.f1, nFo, nPIs, cover, pool, &ctr[0], poolCap, scratch, flag, extra, &ctr[2], &ctr[7],
                        &ctr[1]};
     // covers of the roots by their edges; then of those a limit made, until
     // no cover meets another one
-    uint32_t misc[4] = {};
+    uint32_t misc[8] = {};
     bool limited = false;
     const uint32_t *list = roots;
     for (uint32_t todo = nCand, done = 0; todo > 0;) {
@@ -1388,6 +1434,7 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
         GLS_HIP(ctx, hipGetLastError());
         GLS_TRY(stream_copy(ctx, misc, ctr, sizeof(misc), hipMemcpyDeviceToHost));
         if (misc[1]) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: cover pool overflow");
+        if (misc[7]) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: input not topological");
         list = extra + done;
         todo = misc[2] - done;
         done = misc[2];
@@ -1395,7 +1442,7 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
     }
     const uint32_t poolUsed = misc[0];
     if (limited) GLS_TRY(select_ids(flag, nCand));
-    // ---- the sweeps: unreached roots dropped, then levels
+    // ---- levels
     if (tagged && nCand > 0) {
         k_count_tags<<<tag_grid(nCand), kBlock, 0, st>>>(nCand, roots, tagIn, segCnt);
         size_t tbs = 0;
@@ -1404,42 +1451,43 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
         if (!ts) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: scan storage");
         GLS_HIP(ctx, rocprim::exclusive_scan(ts, tbs, segCnt, segFirst, 0u, (size_t)nSeg, rocprim::plus<uint32_t>(), st));
     }
-    SweepArgs sa{cover, pool, nPIs, mark, indeg, lastLevel, {extra, rootsSorted}, 0u};
+    const size_t room = std::max(nCand, 1u);
+    uint32_t *keys = t.get<uint32_t>(room), *keysSorted = t.get<uint32_t>(room);
+    uint32_t *off = t.get<uint32_t>(room + 1), *len = t.get<uint32_t>(room + 1);
+    uint32_t *newLen = t.get<uint32_t>(room + 1), *newOff = t.get<uint32_t>(room + 1);
+    uint32_t *inputs = t.get<uint32_t>(std::max<size_t>(poolUsed, 1)), *inSrc = t.get<uint32_t>(std::max<size_t>(poolUsed, 1));
+    if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: order allocation");
     std::vector<uint32_t> segLevels(nSeg, 0);
-    auto sweep = [&](bool drop) -> int {
-        sa.drop = drop ? 1u : 0u;
-        GLS_TRY(Fills(ctx).add(segLen, 0, sizeof(uint32_t) * 2 * nSeg).run());
-        k_sweep_first<<<nblocks(nCand), kB, 0, st>>>(nCand, roots, sa, tagged ? tagIn : nullptr, segFirst, segLen);
-        for (;;) {
-            k_sweep_wg<<<nSeg, BAL_WG, 0, st>>>(sa, segFirst, segLen, segRound, nSeg == 1 ? SWEEP_WIDE : UNSET);
-            GLS_HIP(ctx, hipGetLastError());
-            if (nSeg > 1) break;
-            uint32_t h[2] = {};      // the frontier's size, rounds done (segLen[0], segRound[0])
-            GLS_TRY(stream_copy(ctx, h, segLen, sizeof(h), hipMemcpyDeviceToHost));
-            while (h[0] > SWEEP_WIDE) {
-                if (h[1] > (uint32_t)n) return gls_fail(ctx, GLS_ERR_INTERNAL, "balance: cover levels do not end");
-                GLS_TRY(Fills(ctx).add(flen, 0, sizeof(uint32_t) * (SWEEP_GRID_ROUNDS + 1)).run());
-                GLS_TRY(stream_copy(ctx, flen, &h[0], sizeof(uint32_t), hipMemcpyHostToDevice));
-                for (int i = 0; i < SWEEP_GRID_ROUNDS; i++)
-                    k_sweep_grid<<<nblocks(2 * (int64_t)h[0]), kB, 0, st>>>(sa, h[1] + (uint32_t)i, flen + i);
-                GLS_HIP(ctx, hipGetLastError());
-                uint32_t sizes[SWEEP_GRID_ROUNDS + 1];
-                GLS_TRY(stream_copy(ctx, sizes, flen, sizeof(sizes), hipMemcpyDeviceToHost));
-                // rounds past the last non-empty frontier did nothing
-                int last = 0;
-                while (last < SWEEP_GRID_ROUNDS && sizes[last] != 0) last++;
-                h[0] = sizes[last];
-                h[1] += (uint32_t)last;
-                GLS_TRY(stream_copy(ctx, segLen, h, sizeof(h), hipMemcpyHostToDevice));
-            }
-            if (h[0] == 0) break;
+    auto levels_by_id = [&]() -> int {
+        const uint32_t *ordered = roots;
+        size_t tbs = 0, tbk = 0;
+        GLS_HIP(ctx, rocprim::exclusive_scan(nullptr, tbs, len, off, 0u, (size_t)nCand + 1, rocprim::plus<uint32_t>(), st));
+        GLS_HIP(ctx, rocprim::radix_sort_pairs(nullptr, tbk, keys, keysSorted, roots, rootsSorted, (size_t)nCand, 0u,
+                                               bits_of(nSeg), st));
+        void *ts = t.get<uint8_t>(std::max<size_t>(std::max(tbs, tbk), 1));
+        if (!ts) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: level storage");
+        if (tagged) {
+            k_gather_tags<<<nblocks(nCand), kB, 0, st>>>(nCand, roots, tagIn, keys);
+            GLS_HIP(ctx, rocprim::radix_sort_pairs(ts, tbk, keys, keysSorted, roots, rootsSorted, (size_t)nCand, 0u,
+                                                   bits_of(nSeg), st));
+            ordered = rootsSorted;
+        } else {
+            GLS_TRY(stream_copy(ctx, segCnt, &nCand, sizeof(uint32_t), hipMemcpyHostToDevice));
         }
+        uint32_t *rootAt = extra, *pend = newLen, *val = newOff;
+        const uint32_t *tags = tagged ? tagIn : nullptr;
+        k_id_place<<<nblocks((int64_t)nCand + 1), kB, 0, st>>>(nCand, ordered, tags, segFirst, segCnt, cover, mark, rootAt,
+                                                             place, len, pend, val);
+        GLS_HIP(ctx, rocprim::exclusive_scan(ts, tbs, len, off, 0u, (size_t)nCand + 1, rocprim::plus<uint32_t>(), st));
+        k_id_pack<<<nblocks(nCand), kB, 0, st>>>(nCand, rootAt, tags, segFirst, cover, pool, place, nPIs, off, inputs, pend);
+        k_id_sweep<<<nSeg, ID_CHUNK, 0, st>>>(IdSweepArgs{segFirst, segCnt, off, inputs, pend, val, segRound});
+        k_id_levels<<<nblocks(nCand), kB, 0, st>>>(nCand, rootAt, val, lastLevel);
+        GLS_HIP(ctx, hipGetLastError());
         return GLS_OK;
     };
     uint32_t nRoots = 0, levels = 0;
     if (nCand > 0) {
-        GLS_TRY(sweep(true));
-        GLS_TRY(sweep(false));
+        GLS_TRY(levels_by_id());
         GLS_TRY(stream_copy(ctx, segLevels.data(), segRound, sizeof(uint32_t) * nSeg, hipMemcpyDeviceToHost));
         for (uint32_t x : segLevels) levels = std::max(levels, x);
         k_taken_flags<<<nblocks(n), kB, 0, st>>>(n, lastLevel, flag2);
@@ -1448,11 +1496,6 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
     // ---- roots in the order in which they are rebuilt: by (segment, level,
     // id) where every level fits the persistent workgroup, else by (level, id)
     const uint32_t fitCovers = std::min<uint32_t>(narrowMax, LT_COVERS);
-    uint32_t *keys = t.get<uint32_t>(std::max(nRoots, 1u)), *keysSorted = t.get<uint32_t>(std::max(nRoots, 1u));
-    uint32_t *off = t.get<uint32_t>((size_t)nRoots + 1), *len = t.get<uint32_t>((size_t)nRoots + 1);
-    uint32_t *newLen = t.get<uint32_t>((size_t)nRoots + 1), *newOff = t.get<uint32_t>((size_t)nRoots + 1);
-    uint32_t *inputs = t.get<uint32_t>(std::max<size_t>(poolUsed, 1)), *inSrc = t.get<uint32_t>(std::max<size_t>(poolUsed, 1));
-    if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: order allocation");
     uint32_t *d_starts = nullptr, *d_levOff = nullptr;
     LevelRec *d_lev = nullptr;
     uint32_t most[3] = {};
@@ -1479,13 +1522,13 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
         GLS_HIP(ctx, rocprim::radix_sort_pairs(tmp2, tb2, keys, keysSorted, roots, rootsSorted, (size_t)nRoots, 0u,
                                                eb, st));
         k_key_starts<<<nblocks((int64_t)nRoots + 1), kB, 0, st>>>(nRoots, keysSorted, nKeys, d_starts);
-        k_cover_lens<<<nblocks((int64_t)nRoots + 1), kB, 0, st>>>(nRoots, rootsSorted, cover, len, newLen, indeg);
+        k_cover_lens<<<nblocks((int64_t)nRoots + 1), kB, 0, st>>>(nRoots, rootsSorted, cover, len, newLen, place);
         GLS_HIP(ctx, rocprim::exclusive_scan(tmp2, tb3, len, off, 0u, (size_t)nRoots + 1, rocprim::plus<uint32_t>(), st));
         GLS_HIP(ctx, rocprim::exclusive_scan(tmp2, tb3, newLen, newOff, 0u, (size_t)nRoots + 1,
                                              rocprim::plus<uint32_t>(), st));
         GLS_TRY(Fills(ctx).add(&ctr[4], 0, sizeof(uint32_t) * 3).run());
         k_level_sizes<<<nblocks(nKeys), kB, 0, st>>>(nKeys, d_starts, off, newOff, d_lev, &ctr[4]);
-        k_pack_inputs<<<nblocks(nRoots), kB, 0, st>>>(nRoots, rootsSorted, cover, pool, off, keysSorted, d_starts, lastLevel, indeg,
+        k_pack_inputs<<<nblocks(nRoots), kB, 0, st>>>(nRoots, rootsSorted, cover, pool, off, keysSorted, d_starts, lastLevel, place,
                                                       nPIs, inputs, inSrc);
         GLS_HIP(ctx, hipGetLastError());
         return stream_copy(ctx, most, &ctr[4], sizeof(most), hipMemcpyDeviceToHost);
