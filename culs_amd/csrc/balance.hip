@@ -94,11 +94,20 @@ __device__ __forceinline__ uint64_t t_hash(const NodeTable &t, unsigned long lon
     return (h ^ h >> 15) & t.mask;
 }
 
+// the node of a key that is there: it may be on its way still (the workgroup
+// that inserts does not wait for it)
+__device__ __forceinline__ unsigned long long t_node(const NodeTable &t, uint64_t s) {
+    unsigned long long v;
+    do v = t_load(&t.v[s]);
+    while (v == EMPTY64);
+    return v;
+}
+
 // the node with this key, or EMPTY64; k is the key word at its first slot s
 __device__ __forceinline__ unsigned long long t_find_at(const NodeTable &t, unsigned long long key, uint64_t s,
                                                         unsigned long long k) {
     for (uint64_t probes = 0; probes <= t.mask; probes++) {
-        if (k == key) return t_load(&t.v[s]);
+        if (k == key) return t_node(t, s);
         if (k == EMPTY64) return EMPTY64;
         s = (s + 1) & t.mask;
         k = t_load(&t.k[s]);
@@ -509,7 +518,7 @@ __global__ void k_pack_inputs(uint32_t m, const uint32_t *__restrict__ roots, co
 }
 
 // largest level: covers, inputs, ANDs it can create; and per level its extent
-struct LevelRec {
+struct alignas(16) LevelRec {
     uint32_t s, nb, in0, T;           // first root, roots, first input, inputs
     uint32_t most, pad[3];            // ANDs it can create
 };
@@ -540,7 +549,7 @@ struct RecArgs {
     const uint32_t *starts;           // first root of every (segment, level)
     unsigned long long *newSig;       // per root id: the result
     uint32_t *of0, *of1;              // fanins of the created nodes, by id
-    uint32_t *tagOut;                 // optional: their tags
+    uint32_t *tagOut;                 // optional: their tags (where a segment holds several)
     const uint32_t *tagIn;
     uint32_t *err;                    // 2: table full
     uint32_t shuffle;                 // 1: `b -s` input order (sortDecId = 0)
@@ -636,12 +645,14 @@ constexpr uint32_t LN_FINAL = 0x80000000u, LS_NONE = 0xFFFFu;
 // What bounds it is latency, so little is left between two levels: results of
 // the level before come from LDS, other inputs are read during its steps, its
 // table insertions are under way until the lookups, and only used entries of
-// the level's table are cleared.  Cycles per level of 2M random ANDs (1795
-// levels of 668 covers and 1523 inputs): 68000, of which 12000 to place and
-// sort the inputs, 13000 for the pairs, 20000 for two full steps, 17000 for 3.9
-// more; 88000 with every lookup made at its step in memory (46 and 63 ms in
-// all).  A level of the 64-bit multiplier (77 covers, 161 inputs): 24000 and
-// 27000.  Limiting the later memory lookups pair by pair made no difference.
+// the level's table are cleared.  The 128 registers of a thread matter: what is
+// spilled is waited for, and the insertions with it, so the next level's words
+// are read after the sort.  The table in memory is at most a quarter full: a
+// wavefront waits for the longest of its lanes' probe chains.  2M random ANDs
+// (1786 levels of 668 covers and 1523 inputs): 38.8 ms; 45.1 with the next
+// level read at the start (spilled) and a table twice as full, 63 with every
+// lookup made at its step in memory.  The 64-bit multiplier (a level has 77
+// covers, 161 inputs): 2.5 ms for 414 levels, 3.4 before.
 __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *__restrict__ levOff,
                                                     const uint32_t *__restrict__ idBase, uint32_t *made, int32_t lFirst,
                                                     int32_t lLast) {
@@ -660,18 +671,26 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
     const uint32_t lev0 = levOff[seg], nLev = levOff[seg + 1] - lev0, base0 = idBase[seg];
     uint32_t counter = base0 + made[seg];            // next id
     // a level's extent, its inputs (one per thread and LQ_IN), its covers' first
-    // inputs and roots
+    // inputs and roots.  Extents are read a level before they are used, into
+    // vector registers: in scalar ones they would be waited for at once
+    struct Extent {
+        uint4 x;
+        uint32_t most;
+    };
     struct Level {
         LevelRec e;
         uint32_t lit[LQ_IN], src[LQ_IN], off[LQ_COV], root[LQ_COV];
         unsigned long long sig[LQ_IN];
     };
-    auto load_extent = [&](int32_t l) -> LevelRec {
-        LevelRec e = {};
-        if (l >= lLast) e = r.lev[lev0 + l];
-        return e;
+    auto load_extent = [&](int32_t l) -> Extent {
+        uint32_t k = lev0 + (uint32_t)max(l, 0);
+        asm volatile("" : "+v"(k));
+        return {*reinterpret_cast<const uint4 *>(&r.lev[k]), r.lev[k].most};
     };
-    auto load_level = [&](const LevelRec &e, Level &v) {
+    auto first_lane = [](uint32_t x) -> uint32_t { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
+    auto load_level = [&](int32_t l, const Extent &x, Level &v) {
+        LevelRec e = {};
+        if (l >= lLast) e = {first_lane(x.x.x), first_lane(x.x.y), first_lane(x.x.z), first_lane(x.x.w), first_lane(x.most), {}};
         v.e = e;
 #pragma unroll
         for (uint32_t q = 0; q < LQ_IN; q++) {
@@ -682,7 +701,7 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
 #pragma unroll
         for (uint32_t q = 0; q < LQ_COV; q++) {
             const uint32_t c = tid + q * BAL_WG;
-            v.off[q] = c < e.nb ? r.off[e.s + c] - e.in0 : 0u;
+            v.off[q] = c < e.nb ? r.off[e.s + c] : 0u;
             v.root[q] = c < e.nb ? r.roots[e.s + c] : 0u;
         }
     };
@@ -702,9 +721,17 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
     for (uint32_t i = tid; i < LT_HASH; i += BAL_WG) { s_key[i] = EMPTY64; s_val[i] = UNSET; }
     int32_t l = min(lFirst, (int32_t)nLev - 1);
     Level cur, next;
-    load_level(load_extent(l), cur);
-    LevelRec ahead = load_extent(l - 1);     // extents come two levels ahead, inputs one
+    load_level(l, load_extent(l), cur);
+    Extent ahead = load_extent(l - 1);
     load_inputs(true, cur);
+    // (also before the first level: a wait that the loop shares with it would include the insertions)
+    auto arrived = [&](Level &v) {
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_IN; q++) asm volatile("" : "+v"(v.sig[q]), "+v"(v.lit[q]), "+v"(v.src[q]));
+#pragma unroll
+        for (uint32_t q = 0; q < LQ_COV; q++) asm volatile("" : "+v"(v.off[q]), "+v"(v.root[q]));
+    };
+    arrived(cur);
     // the level before's nodes, on their way into the table
     unsigned long long newKey[LQ_NEW], newNode[LQ_NEW], newPrev[LQ_NEW];
     uint32_t newSlot[LQ_NEW];
@@ -725,12 +752,10 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
     };
     for (; l >= lLast; l--) {
         const uint32_t nb = cur.e.nb, T = cur.e.T, most = cur.e.most, levBase = counter;
-        load_level(ahead, next);
-        ahead = load_extent(l - 2);
 #pragma unroll
         for (uint32_t q = 0; q < LQ_COV; q++) {
             const uint32_t c = tid + q * BAL_WG;
-            if (c < nb) { s_off[c] = (uint16_t)cur.off[q]; s_mem[c] = 0; }
+            if (c < nb) { s_off[c] = (uint16_t)(cur.off[q] - cur.e.in0); s_mem[c] = 0; }
         }
         if (tid == 0) { s_off[nb] = (uint16_t)T; s_top = (int32_t)LT_NEW; s_over = 0; }
         unsigned long long mine[LQ_IN];
@@ -789,9 +814,12 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
         for (uint32_t q = 0; q < LQ_IN; q++)
             if (place[q] != UNSET) s_arr[place[q]] = mine[q];
         for (uint32_t c = tid; c < nb; c += BAL_WG) s_len[c] = (uint16_t)(s_off[c + 1] - s_off[c]);
-        finish_inserts();
-        __builtin_amdgcn_s_waitcnt(0x0F70);     // vmcnt(0): the table's words and the level before's results are written
+        finish_inserts();                       // the keys are there; the nodes are not waited for
         __syncthreads();
+        // the next level's words set out (not earlier: they take registers, and what
+        // does not fit is spilled to memory)
+        load_level(l - 1, ahead, next);
+        ahead = load_extent(l - 2);
         // the level's own table
         auto hash = [](unsigned long long key) -> uint32_t {
             const uint32_t h = (uint32_t)(key >> 32) * 0x9E3779B1u + (uint32_t)key;
@@ -819,35 +847,40 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
                 k = lds_load(&s_key[h]);
             }
         };
-        // pairs of inputs that exist
+        // pairs of inputs that exist: two of a thread's inputs at a time, two
+        // candidates of each
 #pragma unroll
-        for (uint32_t g = 0; g < LQ_IN; g++) {
-            const uint32_t j = tid + g * BAL_WG;
+        for (uint32_t g = 0; g < LQ_IN; g += 2) {
             if (g * BAL_WG >= T) break;
-            uint32_t o = 0, left = 0;        // candidates [o, left)
-            unsigned long long x = 0;
-            uint32_t border = 0;
-            if (j < T) {
+            uint32_t o[2], left[2], border[2];       // candidates [o, left)
+            unsigned long long x[2];
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const uint32_t j = tid + (g + p) * BAL_WG;
+                o[p] = left[p] = border[p] = 0;
+                x[p] = 0;
+                if (j >= T) continue;
                 // position j's cover is input j's: the order is within covers
-                o = s_off[cur.src[g] & 0xFFFFu];
-                left = j;
-                x = s_arr[j];
-                border = j > o ? sig_lev(s_arr[j - 1]) : 0u;
+                o[p] = s_off[cur.src[g + p] & 0xFFFFu];
+                left[p] = j;
+                x[p] = s_arr[j];
+                border[p] = j > o[p] ? sig_lev(s_arr[j - 1]) : 0u;
             }
-            while (__ballot(left > o) != 0) {
+            while (__ballot(left[0] > o[0] || left[1] > o[1]) != 0) {
                 unsigned long long key[4];
                 uint64_t slot[4];
                 uint32_t wait = 0;
 #pragma unroll
                 for (int q = 0; q < 4; q++) {
+                    const int p = q >> 1;
                     key[q] = EMPTY64;
                     slot[q] = 0;
-                    if (left <= o) continue;
-                    const unsigned long long y = s_arr[left - 1];
-                    if (sig_lev(y) != border) { left = o; continue; }
-                    left--;
-                    if (and_trivial(x, y) != EMPTY64) continue;
-                    key[q] = and_key_of(sig_lit(x), sig_lit(y));
+                    if (left[p] <= o[p]) continue;
+                    const unsigned long long y = s_arr[left[p] - 1];
+                    if (sig_lev(y) != border[p]) { left[p] = o[p]; continue; }
+                    left[p]--;
+                    if (and_trivial(x[p], y) != EMPTY64) continue;
+                    key[q] = and_key_of(sig_lit(x[p]), sig_lit(y));
                     slot[q] = t_hash(r.t, key[q]);
                     wait |= 1u << q;
                 }
@@ -875,15 +908,16 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
                         const uint32_t h = level_slot(kq, isNew);
                         s_ent[at] = isNew ? (uint16_t)h : (uint16_t)LS_NONE;
                         if (isNew) {
-                            s_node[at] = t_load(&r.t.v[(sq - 1) & r.t.mask]);
+                            s_node[at] = t_node(r.t, (sq - 1) & r.t.mask);
                             s_val[h] = LN_FINAL | (uint32_t)at;
                         }
                     }
                 }
             }
         }
-        load_inputs(false, next);
+        __builtin_amdgcn_s_waitcnt(0x0F70);     // vmcnt(0): the level before's results are written
         __syncthreads();
+        load_inputs(false, next);
         const bool over = s_over != 0;       // not all of them fit: every cover looks up in memory too
         // sharedNodeDrivenPermute and prepareDataToInsert (balance.cu:113-247)
         // of a cover with two inputs at least: takes its last two; returns the
@@ -1060,10 +1094,7 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
         }
         // the next level's loads have arrived: the waits for them stand here, where
         // they do not include the insertions
-#pragma unroll
-        for (uint32_t q = 0; q < LQ_IN; q++) asm volatile("" : "+v"(next.sig[q]), "+v"(next.lit[q]), "+v"(next.src[q]));
-#pragma unroll
-        for (uint32_t q = 0; q < LQ_COV; q++) asm volatile("" : "+v"(next.off[q]), "+v"(next.root[q]));
+        arrived(next);
         // the level's nodes set out for the table; its own table is cleared
 #pragma unroll
         for (uint32_t q = 0; q < LQ_NEW; q++) {
@@ -1276,7 +1307,7 @@ __global__ void k_out_emit(uint32_t m, int32_t nPIs, uint32_t nSeg, const uint32
         of0[o] = moved(if0[v], nPIs, gap);
         of1[o] = moved(if1[v], nPIs, gap);
         olevel[o] = 0;
-        if (otag) otag[o] = itag[v];
+        if (otag) otag[o] = itag ? itag[v] : lo;
     }
     for (int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; v <= nPIs; v += stride) {
         of0[v] = 0;
@@ -1578,11 +1609,11 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
 
     // ---- phase 2: reconstruction
     uint64_t cap = 1024;
-    while (cap < 2ull * ((uint64_t)poolUsed + 16)) cap <<= 1;       // a cover of k inputs creates at most k - 1 nodes
+    while (cap < 4ull * ((uint64_t)poolUsed + 16)) cap <<= 1;       // a cover of k inputs creates at most k - 1 nodes
     const size_t idEnd = (size_t)nPIs + 1 + poolUsed;
     unsigned long long *tabK = t.get<unsigned long long>(cap), *tabV = t.get<unsigned long long>(cap), *newSig = t.get<unsigned long long>(n);
     uint32_t *cf0 = t.get<uint32_t>(idEnd), *cf1 = t.get<uint32_t>(idEnd);
-    uint32_t *ctag = tagged ? t.get<uint32_t>(idEnd) : nullptr;
+    uint32_t *ctag = tagged && !bySeg ? t.get<uint32_t>(idEnd) : nullptr;     // by segment: the segment
     uint32_t *segIds = t.get<uint32_t>(3 * (size_t)ns + 3);
     if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "balance: reconstruction allocation");
     uint32_t *d_idBase = segIds, *d_made = segIds + ns, *d_outOff = segIds + 2 * (size_t)ns;
