@@ -281,9 +281,8 @@ int batch_pass(gls_ctx *ctx, gls_aig **aigs, int32_t count, Pass pass, int32_t u
     // 1.6 / 1.8, 64 of 20k 5.5 / 6.6, 512 of 2k 14.2 / 13.5, 512 of 20k 55 / 34.
     int64_t largest = 0;
     for (int32_t k = 0; k < count; k++) largest = std::max<int64_t>(largest, aigs[k]->nObjs);
-    const RwDelta whole{0, 0, nullptr, nullptr, nullptr, nullptr, nullptr};
     int rc = pass == Pass::Strash && N <= 64 * largest
-                                     ? dev_strash_rw(ctx, U, whole, R, &depth, &info, utag, &rtag, dep)
+                                     ? dev_strash_whole(ctx, U, false, R, &depth, &info, utag, &rtag, dep)
              : pass == Pass::Strash  ? dev_strash(ctx, U, R, &depth, &info, utag, &rtag, dep)
              : pass == Pass::Rewrite ? dev_rewrite(ctx, U, useZeros, flags, R, &depth, &info, utag, &rtag, dep)
                                      : dev_balance(ctx, U, R, &info, utag, &rtag, &splitTags, 1, count);

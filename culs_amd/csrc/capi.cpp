@@ -452,16 +452,13 @@ extern "C" int gls_strash(gls_aig *a, int32_t flags) {
     DevGraph out;
     int32_t depth = 0;
     gls_op_info info = {};
-    // the whole-graph mode of the incremental strash (levels by one sweep over
-    // id order, every node hashed in rounds), which gives way to the wave sweep
+    // every node hashed in rounds, levels by sweeps over id order, which gives way to the wave sweep
     // for ids that are not topological and where it needs too many rounds.
     // Against the wave sweep, ms: 521 objects 0.34 / 0.48, 2k 0.47 / 0.50, 20k
     // 0.65 / 0.84, the 64-bit multiplier 0.53 / 1.65, 200k 0.90 / 2.7, 1M of
     // 1029 to 20876 per level 2.4 / 13.0 to 2.1 / 4.3.
     if (!(flags & GLS_ST_WAVES)) {
-        RwDelta whole{0, 0, nullptr, nullptr, nullptr, nullptr, nullptr};
-        whole.allRounds = (flags & GLS_ST_LEVELS) != 0;
-        GLS_TRY(dev_strash_rw(ctx, a->dev, whole, out, &depth, &info));
+        GLS_TRY(dev_strash_whole(ctx, a->dev, (flags & GLS_ST_LEVELS) != 0, out, &depth, &info));
     } else {
         GLS_TRY(dev_strash(ctx, a->dev, out, &depth, &info));
     }

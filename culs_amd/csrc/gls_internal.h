@@ -192,11 +192,13 @@ struct RwDelta {
     const uint32_t *g0, *g1, *glevel;
     const uint32_t *tOff;
     const uint2 *tEnt;
-    bool allRounds = false;     // as many hashing rounds as it takes
 };
 int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &out, int32_t *depth,
                   gls_op_info *info, const uint32_t *tagIn = nullptr, uint32_t **tagOut = nullptr,
                   uint32_t *tagDepth = nullptr);
+// allRounds: as many hashing rounds as it takes
+int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph &out, int32_t *depth, gls_op_info *info,
+                     const uint32_t *tagIn = nullptr, uint32_t **tagOut = nullptr, uint32_t *tagDepth = nullptr);
 int dev_reorder(gls_ctx *ctx, const DevGraph &in, DevGraph &out, std::vector<int32_t> &levelStart,
                 const uint32_t *tagIn = nullptr, uint32_t **tagOut = nullptr);
 int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGraph &out, int32_t *depth,

@@ -912,14 +912,17 @@ constexpr int SW_RING = 32768;              // 128 KiB of LDS
 constexpr uint32_t NOFAN = 0xFFFFFFFFu;
 constexpr uint32_t SW_NOLEV = 0xFFFFFFFFu;
 constexpr uint32_t SW_SPIN_LIMIT = 1u << 22;
-// Rounds of the incremental strash before it gives way to the wave sweep.  A
-// round merges duplicates one level further up, so a graph that holds the same
-// deep logic twice needs one per level.  Whole graphs measured take one to
-// three, large narrow ones eight; a graph that needs more pays for the rounds
-// tried (the 32-bit multiplier twice over the same inputs 1.7 ms against 1.2 by
-// waves at once, a windowed AIG of 200k ANDs twice 9 against 5.7).
-constexpr uint32_t kRwRoundLimit = 4096, kRwManyRounds = 32, kRwFewRounds = 5;
-// objects from which a whole narrow graph may take many rounds
+// Rounds of hashing before a strash gives way to the wave sweep.  A round merges
+// duplicates one level further up, so a graph that holds the same deep logic
+// twice needs one per level; most graphs take one to three.  A rewrite takes
+// many where its graph is narrow, else few.  A whole graph's round after the
+// first costs 15 us and 4 us per million objects, its wave sweep 0.2 ms more than
+// the rounds' other work at 20k objects, 2 ms at a million on wide levels: few
+// below 2^18 objects, many from there.  Where the levels are narrow the wave
+// sweep costs 100 ms more at 10M objects: those that are still at it go on to the
+// limit (of 120 raw deep AIGs of 10M ANDs 108 took two or three, one 44).
+constexpr uint32_t kRwRoundLimit = 4096, kRwManyRounds = 128, kRwFewRounds = 5;
+// objects from which a whole graph may take many rounds
 constexpr int32_t kRwLarge = 1 << 18;
 // The line for a rewrite of one AIG lies at this many times rw_sweep_width
 // objects per level (8192 by default).  Incremental against wave sweep, ms:
@@ -933,9 +936,20 @@ __device__ __forceinline__ uint32_t sw_lds_load(const uint32_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-__global__ void __launch_bounds__(SW_WG) k_level_sweep(uint32_t nPos, const uint32_t *__restrict__ fa,
-                                                      const uint32_t *__restrict__ fb, uint32_t *lev,
-                                                      uint32_t *err, uint32_t *maxLev) {
+// One workgroup sweeps one position array: two that do not depend on each other
+// take one launch.
+struct LevelSweep {
+    uint32_t nPos;
+    const uint32_t *fa, *fb;
+    uint32_t *lev, *maxLev;
+};
+
+__global__ void __launch_bounds__(SW_WG) k_level_sweep(LevelSweep first, LevelSweep second, uint32_t *err) {
+    const LevelSweep args = blockIdx.x == 0 ? first : second;
+    const uint32_t nPos = args.nPos;
+    const uint32_t *__restrict__ fa = args.fa;
+    const uint32_t *__restrict__ fb = args.fb;
+    uint32_t *lev = args.lev, *maxLev = args.maxLev;
     __shared__ uint32_t ring[SW_RING];
     __shared__ uint2 s_fan[2][SW_WG];           // fanin positions of this chunk and the next
     __shared__ uint32_t s_max, s_bad;
@@ -1110,9 +1124,10 @@ __global__ void k_keep_flags(int32_t N, int32_t nPIs, const uint8_t *__restrict_
 // constant and the PIs have none.
 __global__ void k_full_fanpos(int32_t N, int32_t nPIs, const uint32_t *__restrict__ f0,
                               const uint32_t *__restrict__ f1, const uint8_t *__restrict__ dead,
-                              const uint32_t *__restrict__ posOf, uint32_t *fa, uint32_t *fb) {
+                              const uint32_t *__restrict__ posOf, uint32_t *fa, uint32_t *fb, uint32_t *err) {
     int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t v = tid; v < N; v += stride) {
+        if (v > nPIs && !dead[v] && (LID(f0[v]) >= v || LID(f1[v]) >= v)) { *err = 1u; continue; }
         if (v <= nPIs) {
             fa[posOf[v]] = NOFAN;
             fb[posOf[v]] = NOFAN;
@@ -1354,12 +1369,173 @@ __global__ void k_fill_u64(size_t n, unsigned long long *p, unsigned long long v
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
 }
 
+// ---------------------------------------------------------------------------
+// Strash of a whole graph (dev_strash_whole)
+// ---------------------------------------------------------------------------
+// Its table: keys apart from the smallest id of each, both kept over the
+// rounds.  rep: the representative literal, itself the representative of none.
+struct WholeArgs {
+    int32_t N, nPIs;
+    const uint32_t *f0, *f1;
+    const uint8_t *dead;
+    uint32_t *rep;
+    uint8_t *moved;                  // the representative changed in the round before
+    uint8_t *redo;                   // the representative is taken anew in this round
+    unsigned long long *key;
+    uint32_t *least;
+    uint64_t mask;
+    uint32_t *slot, *fold;           // per node: its key's slot, or NO_SLOT and the literal it folds to
+    uint32_t *err;
+    unsigned long long *probes;
+};
+
+__global__ void k_whole_init(int32_t N, uint32_t *rep) {
+    int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t v = tid; v < N; v += stride) rep[v] = 2u * (uint32_t)v;
+}
+
+// Round, step 1: keys of the live ANDs with a fanin that moved (first: of all).
+// A key over a literal that moved is never formed again, and all nodes of a key
+// move it together, so a slot's least id stays right; the node that loses its
+// place in a slot is looked at again.
+__global__ void k_whole_hash(WholeArgs a, uint32_t first, uint32_t *changed) {
+    uint32_t np = 0;
+    int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    if (tid == 0) *changed = 0;
+    for (int64_t v = a.nPIs + 1 + tid; v < a.N; v += stride) {
+        if (a.dead[v]) continue;
+        const uint32_t x = a.f0[v], y = a.f1[v];
+        if (!first && !a.moved[LID(x)] && !a.moved[LID(y)]) continue;
+        a.redo[v] = 1;
+        uint32_t l0 = a.rep[LID(x)] ^ LC(x), l1 = a.rep[LID(y)] ^ LC(y);
+        if (l0 > l1) { const uint32_t t = l0; l0 = l1; l1 = t; }
+        uint32_t r = INVALID32;
+        if (l0 == l1) r = l0;
+        else if (l0 == (l1 ^ 1u)) r = 0;
+        else if (l0 == 1u) r = l1;
+        else if (l0 == 0u) r = 0;
+        a.slot[v] = NO_SLOT;
+        a.fold[v] = r;
+        if (r != INVALID32) continue;
+        const uint64_t key = and_key(l0, l1);
+        uint64_t s = mix64(key) & a.mask;
+        for (uint64_t probe = 0; probe <= a.mask; ++probe) {
+            unsigned long long prev = KEY_EMPTY;
+            __hip_atomic_compare_exchange_strong(&a.key[s], &prev, (unsigned long long)key, __ATOMIC_RELAXED,
+                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ++np;
+            if (prev == KEY_EMPTY || prev == key) { a.slot[v] = (uint32_t)s; break; }
+            s = (s + 1) & a.mask;
+        }
+        if (a.slot[v] == NO_SLOT) { a.fold[v] = 2u * (uint32_t)v; atomicOr(a.err, 2u); continue; }
+        const uint32_t was = atomicMin(&a.least[s], (uint32_t)v);
+        if (was != INVALID32 && was > (uint32_t)v) a.redo[was] = 1;
+        ++np;
+    }
+    block_add_u64(a.probes, np);
+}
+
+// Round, step 2: their representatives, one link each.
+__global__ void k_whole_link(WholeArgs a) {
+    int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t v = a.nPIs + 1 + tid; v < a.N; v += stride) {
+        uint8_t moved = 0;
+        if (a.redo[v]) {
+            a.redo[v] = 0;
+            const uint32_t s = a.slot[v], r = s == NO_SLOT ? a.fold[v] : 2u * a.least[s];
+            if (r != a.rep[v]) {
+                a.rep[v] = r;
+                moved = 1;
+            }
+        }
+        a.moved[v] = moved;
+    }
+}
+
+// Round, step 3: links followed to their ends (ids fall along them, and an end
+// stays one during this step).
+__global__ void k_whole_follow(WholeArgs a, uint32_t *changed) {
+    int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    bool any = false;
+    for (int64_t v = a.nPIs + 1 + tid; v < a.N; v += stride) {
+        const uint32_t was = a.rep[v];
+        if (was == 2u * (uint32_t)v) continue;
+        uint32_t r = was;
+        for (;;) {
+            const uint32_t u = LID(r), q = __hip_atomic_load(&a.rep[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (q == 2u * u) break;
+            r = q ^ LC(r);
+        }
+        if (r != was) {
+            a.rep[v] = r;
+            a.moved[v] = 1;
+        }
+        any |= a.moved[v] != 0;
+    }
+    if (__ballot(any) != 0 && (threadIdx.x & 63) == 0) atomicOr(changed, 1u);
+}
+
+// fanin positions of the classes at their representatives' positions
+__global__ void k_whole_classpos(int32_t N, int32_t nPIs, const uint32_t *__restrict__ f0,
+                                 const uint32_t *__restrict__ f1, const uint8_t *__restrict__ dead,
+                                 const uint32_t *__restrict__ rep, const uint32_t *__restrict__ posOf, uint32_t *fa,
+                                 uint32_t *fb) {
+    int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t v = tid; v < N; v += stride) {
+        if (v > nPIs && dead[v]) continue;
+        const bool top = v > nPIs && rep[v] == 2u * (uint32_t)v;
+        fa[posOf[v]] = top ? posOf[LID(rep[LID(f0[v])])] : NOFAN;
+        fb[posOf[v]] = top ? posOf[LID(rep[LID(f1[v])])] : NOFAN;
+    }
+}
+
+// waves, and the smallest (wave, id) of the other nodes of each class (a node
+// that folds to a literal lies on a higher wave than the literal's node)
+__global__ void k_whole_waves(int32_t N, int32_t nPIs, const uint8_t *__restrict__ dead,
+                              const uint32_t *__restrict__ rep, const uint32_t *__restrict__ posOf,
+                              const uint32_t *__restrict__ levPos, uint32_t *wave, unsigned long long *best) {
+    int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t v = tid; v < N; v += stride) {
+        const bool live = v > nPIs && !dead[v];
+        const uint32_t w = live ? levPos[posOf[v]] : 0u;
+        wave[v] = w;
+        if (!live || rep[v] == 2u * (uint32_t)v || LC(rep[v])) continue;
+        if (LID(rep[v]) > (uint32_t)nPIs)
+            atomicMin(&best[LID(rep[v])], (unsigned long long)w << 32 | (uint32_t)v);
+    }
+}
+
+// every node's representative by (wave, id), and its class's level
+__global__ void k_whole_rep(int32_t N, int32_t nPIs, const uint8_t *__restrict__ dead,
+                            const uint32_t *__restrict__ rep, const uint32_t *__restrict__ posOf,
+                            const uint32_t *__restrict__ wave, const unsigned long long *__restrict__ best,
+                            const uint32_t *__restrict__ classLev, uint32_t *rep2, uint32_t *level) {
+    int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t v = tid; v < N; v += stride) {
+        const uint32_t r = rep[v], u = LID(r);
+        uint32_t r2 = r, lev = 0;
+        if (v > nPIs && !dead[v] && u > (uint32_t)nPIs) {
+            const unsigned long long other = best[u], own = (unsigned long long)wave[u] << 32 | u;
+            r2 = 2u * (uint32_t)(other < own ? other : own) ^ LC(r);
+            lev = classLev[posOf[u]];
+        }
+        rep2[v] = r2;
+        level[v] = lev;
+    }
+}
+
+__global__ void k_last_pos(int32_t N, const uint32_t *__restrict__ posOf, const uint32_t *__restrict__ keep, uint32_t *count) {
+    *count = posOf[N - 1] + keep[N - 1];
+}
+
 struct Tmp {
     gls_ctx *ctx;
     std::vector<void *> ptrs;
+    bool ok = true;
     template <class T> T *get(size_t n) {
         T *p = pool_get<T>(ctx, n);
         if (p) ptrs.push_back(p);
+        else ok = false;
         return p;
     }
     ~Tmp() {
@@ -1603,6 +1779,183 @@ int dev_strash(gls_ctx *ctx, const DevGraph &in, DevGraph &out, int32_t *depthOu
     return GLS_OK;
 }
 
+// Strash of a whole graph with topological ids.  The result equals dev_strash
+// array for array:
+//  1. dangling nodes, as there;
+//  2. classes of equal ANDs in rounds, each node's representative the least id
+//     of its key's nodes over representatives.  Which nodes are equal does not
+//     depend on the choice, so no levels are needed yet, and ids only fall, so
+//     one table serves all rounds and a round after the first takes only the
+//     nodes with a fanin that moved;
+//  3. levels: the waves (of the live nodes) and the output's (of the classes),
+//     two sweeps over id order in one launch;
+//  4. the class's node of smallest (wave, id) represents it in the output.
+// What bounds it are the sweeps, whose chains of dependent positions one
+// workgroup each goes through.  Raw deep AIG of 10M ANDs: 15.1 ms, of
+// which 11.1 the sweeps; 22 with the sweeps one after the other and every node
+// hashed into a new table in each round.
+// Too many rounds lead to dev_strash(in); info->final_strash tells which ran.
+int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph &out, int32_t *depthOut,
+                     gls_op_info *info, const uint32_t *tagIn, uint32_t **tagOut, uint32_t *tagDepth) {
+    const int32_t N = in.nObjs, nPIs = in.nPIs, nPOs = in.nPOs;
+    hipStream_t st = ctx->stream;
+    auto fallback = [&]() {
+        const int rc = dev_strash(ctx, in, out, depthOut, info, tagIn, tagOut, tagDepth);
+        if (info) info->final_strash = 2;
+        return rc;
+    };
+    {
+        Tmp t{ctx};
+        uint32_t *ref = t.get<uint32_t>(N), *order = t.get<uint32_t>(N), *keep = t.get<uint32_t>(N);
+        uint8_t *dead = t.get<uint8_t>(N), *flag = t.get<uint8_t>(N), *moved = t.get<uint8_t>(N), *redo = t.get<uint8_t>(N);
+        uint32_t *posOf = t.get<uint32_t>(N), *fa = t.get<uint32_t>(N), *fb = t.get<uint32_t>(N);
+        uint32_t *ca = t.get<uint32_t>(N), *cb = t.get<uint32_t>(N), *levPos = t.get<uint32_t>(N), *classLev = t.get<uint32_t>(N);
+        uint32_t *rep = t.get<uint32_t>(N), *rep2 = t.get<uint32_t>(N), *slot = t.get<uint32_t>(N), *fold = t.get<uint32_t>(N);
+        unsigned long long *best = t.get<unsigned long long>(N);
+        uint32_t *d_misc = t.get<uint32_t>(16);   // [0] err, [1] largest wave, [2..3] a round changed something,
+                                                  // [4] survivors, [5] largest level, [6..7] probes, [8] a path got shorter
+        SweepCtl *ctl = t.get<SweepCtl>(1);
+        if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: device allocation failed (n=%d)", N);
+        unsigned long long *d_probes = reinterpret_cast<unsigned long long *>(&d_misc[6]);
+        GLS_TRY(Fills(ctx)
+                    .add(ref, 0, sizeof(uint32_t) * N)
+                    .add(dead, 0, N)
+                    .add(moved, 0, N)
+                    .add(redo, 0, N)
+                    .add(best, 0xFF, sizeof(unsigned long long) * N)
+                    .add(ctl, 0, sizeof(SweepCtl))
+                    .add(d_misc, 0, sizeof(uint32_t) * 16)
+                    .run());
+        const int gN = grid_for(N);
+        SweepCtl h_ctl{};
+        uint32_t rounds = 0;
+        // 1. dangling cascade
+        k_count_refs<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, nPOs, in.pos, ref);
+        k_zero_flags<<<gN, kBlock, 0, st>>>(N, nPIs, ref, nullptr, flag);
+        GLS_HIP(ctx, hipGetLastError());
+        GLS_TRY(select_ids(ctx, t, N, flag, order, &ctl->curSize));
+        GLS_TRY(stream_copy(ctx, &h_ctl, ctl, sizeof(SweepCtl), hipMemcpyDeviceToHost));
+        if (h_ctl.curSize > 0) {
+            GLS_TRY(run_sweep(ctx, ctl, 1, [&](uint32_t k, uint32_t hint) {
+                k_dangle_round<<<sweep_grid(hint), kBlock, 0, st>>>(k, ctl, nPIs, in.f0, in.f1, ref, dead, order);
+            }, &h_ctl, &rounds));
+        }
+        // positions: the constant and the PIs, then the live ANDs in id order
+        k_keep_flags<<<gN, kBlock, 0, st>>>(N, nPIs, dead, keep);
+        size_t tbp = 0;
+        GLS_HIP(ctx, rocprim::exclusive_scan(nullptr, tbp, keep, posOf, 0u, (size_t)N, rocprim::plus<uint32_t>(), st));
+        void *tmpp = t.get<uint8_t>(std::max<size_t>(tbp, 1));
+        if (!tmpp) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: position scan storage");
+        GLS_HIP(ctx, rocprim::exclusive_scan(tmpp, tbp, keep, posOf, 0u, (size_t)N, rocprim::plus<uint32_t>(), st));
+        k_full_fanpos<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, posOf, fa, fb, &d_misc[0]);
+        k_last_pos<<<1, 1, 0, st>>>(N, posOf, keep, &d_misc[9]);
+        GLS_HIP(ctx, hipGetLastError());
+        uint32_t misc[16] = {};
+        GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
+        if (misc[0]) return fallback();      // ids are not topological
+        const uint32_t nPos = misc[9];
+        // 2. classes
+        const uint64_t nLive = nPos - (uint32_t)(nPIs + 1);
+        uint64_t cap = 1024;
+        while (cap < 4 * nLive && cap < (1ull << 31)) cap <<= 1;
+        unsigned long long *key = t.get<unsigned long long>(cap);
+        uint32_t *least = t.get<uint32_t>(cap);
+        if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: table");
+        GLS_TRY(Fills(ctx).add(key, 0xFF, sizeof(unsigned long long) * cap).add(least, 0xFF, sizeof(uint32_t) * cap).run());
+        k_whole_init<<<gN, kBlock, 0, st>>>(N, rep);
+        const WholeArgs wa{N, nPIs, in.f0, in.f1, dead, rep, moved, redo, key, least, cap - 1, slot, fold, &d_misc[0], d_probes};
+        uint32_t roundLimit = allRounds ? kRwRoundLimit : N >= kRwLarge ? kRwManyRounds : kRwFewRounds;
+        const int64_t narrowDepth = (N + (int64_t)tuning_for(ctx, N).rw_sweep_width - 1) / tuning_for(ctx, N).rw_sweep_width;
+        const LevelSweep waves{nPos, fa, fb, levPos, &d_misc[1]}, classes{nPos, ca, cb, classLev, &d_misc[5]};
+        bool swept = false;
+        uint32_t r = 0;
+        // two rounds per look at them: most graphs take two or three
+        for (bool done = nLive == 0; !done;) {
+            if (r >= roundLimit) {
+                if (roundLimit != kRwManyRounds) return fallback();
+                k_level_sweep<<<1, SW_WG, 0, st>>>(waves, waves, &d_misc[0]);
+                GLS_HIP(ctx, hipGetLastError());
+                GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
+                if (misc[0] || (int64_t)misc[1] < narrowDepth) return fallback();
+                swept = true;
+                roundLimit = kRwRoundLimit;
+            }
+            for (uint32_t i = 0; i < 2; i++) {
+                k_whole_hash<<<gN, kBlock, 0, st>>>(wa, r + i == 0 ? 1u : 0u, &d_misc[2 + i]);
+                k_whole_link<<<gN, kBlock, 0, st>>>(wa);
+                k_whole_follow<<<gN, kBlock, 0, st>>>(wa, &d_misc[2 + i]);
+            }
+            GLS_HIP(ctx, hipGetLastError());
+            GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(uint32_t) * 4, hipMemcpyDeviceToHost));
+            if (misc[0]) return fallback();
+            done = misc[2] == 0 || misc[3] == 0;
+            r += misc[2] == 0 ? 1u : 2u;
+        }
+        // 3. levels
+        k_whole_classpos<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, rep, posOf, ca, cb);
+        k_level_sweep<<<swept ? 1 : 2, SW_WG, 0, st>>>(classes, waves, &d_misc[0]);
+        // 4. representatives, survivors in (wave, id) order
+        uint32_t *wave = ref, *level = order, *survIds = fa, *survWave = fb, *sortIds = ca, *sortWave = cb, *newId = keep;
+        k_whole_waves<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep, posOf, levPos, wave, best);
+        k_whole_rep<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep, posOf, wave, best, classLev, rep2, level);
+        if (tagIn && tagDepth) k_tag_depth<<<tag_grid(N), kBlock, 0, st>>>(N, nPIs, wave, tagIn, tagDepth);
+        k_rw_shorter<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep2, wave, &d_misc[8]);
+        k_rw_survivors<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep2, flag);
+        GLS_HIP(ctx, hipGetLastError());
+        GLS_TRY(select_ids(ctx, t, N, flag, survIds, &d_misc[4]));
+        GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
+        if (misc[0]) return fallback();
+        const int32_t depth = (int32_t)misc[1];
+        // the wave sweep's limit on objects holds where it used to run
+        if (!allRounds && !(N >= kRwLarge && (int64_t)std::max(depth, 1) >= narrowDepth) &&
+            (uint64_t)tuning_for(ctx, N).strash_table_factor * (uint64_t)N > (1ull << 31))
+            return fallback();
+        const uint32_t m = misc[4];
+        const int32_t nNew = nPIs + 1 + (int32_t)m;
+        GLS_TRY(dev_graph_alloc(ctx, out, nNew, nPIs, nPOs));
+        const uint32_t *sorted = survIds;
+        if (m > 0) {
+            k_gather_u32<<<grid_for(m), kBlock, 0, st>>>((int32_t)m, survIds, wave, survWave);
+            size_t tb3 = 0;
+            const uint32_t endBit = bits_for((uint32_t)depth);
+            GLS_HIP(ctx, rocprim::radix_sort_pairs(nullptr, tb3, survWave, sortWave, survIds, sortIds, (size_t)m, 0u,
+                                                   endBit, st));
+            void *tmp3 = t.get<uint8_t>(tb3);
+            if (!tmp3) { dev_graph_free(ctx, out); return gls_fail(ctx, GLS_ERR_NOMEM, "strash: sort storage"); }
+            GLS_HIP(ctx, rocprim::radix_sort_pairs(tmp3, tb3, survWave, sortWave, survIds, sortIds, (size_t)m, 0u,
+                                                   endBit, st));
+            sorted = sortIds;
+        }
+        uint32_t *tags = nullptr;
+        if (tagIn && tagOut) {
+            tags = pool_get<uint32_t>(ctx, (size_t)nNew);
+            if (!tags) { dev_graph_free(ctx, out); return gls_fail(ctx, GLS_ERR_NOMEM, "strash: tags"); }
+            GLS_HIP(ctx, hipMemcpyAsync(tags, tagIn, sizeof(uint32_t) * (nPIs + 1), hipMemcpyDeviceToDevice, st));
+            *tagOut = tags;
+        }
+        GLS_TRY(Fills(ctx)
+                    .add(out.f0, 0, sizeof(uint32_t) * (nPIs + 1))
+                    .add(out.f1, 0, sizeof(uint32_t) * (nPIs + 1))
+                    .run());
+        k_new_ids<<<grid_for(m + nPIs + 1), kBlock, 0, st>>>(N, nPIs, (int32_t)m, sorted, newId);
+        k_rw_emit<<<grid_for(nNew), kBlock, 0, st>>>((int32_t)m, nPIs, sorted, in.f0, in.f1, rep2, newId, out.f0,
+                                                     out.f1, nullptr, nullptr, level, out.level, tagIn, tags);
+        if (nPOs > 0) k_rw_pos_out<<<grid_for(nPOs), kBlock, 0, st>>>(nPOs, nPIs, in.pos, rep2, newId, out.pos);
+        GLS_HIP(ctx, hipGetLastError());
+        // the depth reported is the number of waves of the input, as
+        // the reference's strash counts it, not the output's largest level
+        if (depthOut) *depthOut = depth;
+        if (info) {
+            info->levels_enumerated = depth;
+            info->hash_probes += (int64_t)((uint64_t)misc[6] | (uint64_t)misc[7] << 32);
+            info->final_strash = 1;
+            info->strash_rounds = (int64_t)r;
+            info->strash_sweeps = 2;
+        }
+    }
+    return GLS_OK;
+}
+
 // Strash of the graph a rewrite composed (comb: the rewrite's input graph g,
 // ids 0..n-1, with the selected roots' fanouts redirected, plus the new nodes
 // n..N-1).  The result equals dev_strash(comb) array for array; it is computed
@@ -1632,10 +1985,7 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
                   gls_op_info *info, const uint32_t *tagIn, uint32_t **tagOut, uint32_t *tagDepth) {
     const int32_t N = in.nObjs, nPIs = in.nPIs, nPOs = in.nPOs, n = d.n;
     hipStream_t st = ctx->stream;
-    // n == 0: a whole graph, every live node dirty, its levels by one sweep
-    // over id order (ids must be topological, as AIGER's are)
-    const bool full = n == 0;
-    if (!full && (!d.g0 || !d.g1 || !d.glevel || !d.tOff || !d.tEnt || n > N))
+    if (!d.g0 || !d.g1 || !d.glevel || !d.tOff || !d.tEnt || n > N)
         return gls_fail(ctx, GLS_ERR_INTERNAL, "strash: the rewrite's input graph is not available");
     auto fallback = [&](const char *why) {
         (void)why;
@@ -1646,9 +1996,9 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
     // The level sweeps below run in one workgroup, about 1 ns per object each;
     // the wave sweep costs 2.6 us per level of few nodes, 13 us of a thousand,
     // and its per-node work.  On wide graphs the wave sweep is the faster one.
-    const int64_t width = full ? 0 : (int64_t)tuning_for(ctx, d.n).rw_sweep_width;
+    const int64_t width = (int64_t)tuning_for(ctx, d.n).rw_sweep_width;
     const int64_t depth0 = std::max(d.depth, 1);
-    if (!full && (int64_t)N > width * depth0 * (tagIn ? 1 : kRwSweepScale)) {
+    if ((int64_t)N > width * depth0 * (tagIn ? 1 : kRwSweepScale)) {
         const int rc = dev_strash(ctx, in, out, depthOut, info, tagIn, tagOut, tagDepth);
         if (info) info->final_strash = 0;
         return rc;
@@ -1692,30 +2042,9 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
             }, &h_ctl, &rounds));
         }
         // 2. a topological order (keys relaxed from the input levels, then a
-        //    stable sort), and the waves by one chunked sweep over it; for a
-        //    whole graph the ids themselves
+        //    stable sort), and the waves by one chunked sweep over it
         uint32_t misc[16] = {};
         bool sweepIn = true;
-        if (full) {
-            // positions: the constant and the PIs, then the live ANDs in id
-            // order (inD is free until the dirty set is seeded)
-            k_keep_flags<<<gN, kBlock, 0, st>>>(N, nPIs, dead, inD);
-            size_t tbp = 0;
-            GLS_HIP(ctx, rocprim::exclusive_scan(nullptr, tbp, inD, posOf, 0u, (size_t)N, rocprim::plus<uint32_t>(), st));
-            void *tmpp = t.get<uint8_t>(std::max<size_t>(tbp, 1));
-            if (!tmpp) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: position scan storage");
-            GLS_HIP(ctx, rocprim::exclusive_scan(tmpp, tbp, inD, posOf, 0u, (size_t)N, rocprim::plus<uint32_t>(), st));
-            k_full_fanpos<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, posOf, fa, fb);
-            GLS_HIP(ctx, hipGetLastError());
-            uint32_t lastPos = 0, lastKeep = 0;
-            GLS_TRY(stream_copy(ctx, &lastPos, posOf + (N - 1), sizeof(uint32_t), hipMemcpyDeviceToHost));
-            GLS_TRY(stream_copy(ctx, &lastKeep, inD + (N - 1), sizeof(uint32_t), hipMemcpyDeviceToHost));
-            const uint32_t nPos = lastPos + lastKeep;
-            k_level_sweep<<<1, SW_WG, 0, st>>>(nPos, fa, fb, levPos, &d_misc[0], &d_misc[1]);
-            GLS_HIP(ctx, hipGetLastError());
-            GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
-            if (misc[0]) return fallback("ids not topological");
-        } else {
         k_rw_key_init<<<gN, kBlock, 0, st>>>(n, N, d.glevel, fa);
         uint32_t keyRounds = 0;
         for (;; ++keyRounds) {
@@ -1748,7 +2077,8 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
             GLS_HIP(ctx, hipGetLastError());
             GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
             if (misc[0]) return fallback("positions");
-            k_level_sweep<<<1, SW_WG, 0, st>>>((uint32_t)N, fa, fb, levPos, &d_misc[0], &d_misc[1]);
+            const LevelSweep ls{(uint32_t)N, fa, fb, levPos, &d_misc[1]};
+            k_level_sweep<<<1, SW_WG, 0, st>>>(ls, ls, &d_misc[0]);
             GLS_HIP(ctx, hipGetLastError());
             GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
             if (misc[0]) return fallback("sweep order");
@@ -1757,14 +2087,12 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
             GLS_HIP(ctx, hipGetLastError());
             misc[1] = misc[10];
         }
-        }
         const int32_t depth = (int32_t)misc[1];
-        const bool narrow = full ? N >= kRwLarge && (int64_t)N <= (int64_t)tuning_for(ctx, N).rw_sweep_width * std::max(depth, 1)
-                                 : (int64_t)N <= width * depth0;
+        const bool narrow = (int64_t)N <= width * depth0;
         // the wave sweep's limit on objects holds where it used to run
-        if (!narrow && !d.allRounds && (uint64_t)tuning_for(ctx, N).strash_table_factor * (uint64_t)N > (1ull << 31))
+        if (!narrow && (uint64_t)tuning_for(ctx, N).strash_table_factor * (uint64_t)N > (1ull << 31))
             return fallback("table range");
-        const uint32_t roundLimit = d.allRounds || (narrow && !full) ? kRwRoundLimit : narrow ? kRwManyRounds : kRwFewRounds;
+        const uint32_t roundLimit = narrow ? kRwRoundLimit : kRwFewRounds;
         k_rw_seed<<<gN, kBlock, 0, st>>>(n, N, nPIs, in.f0, in.f1, d.g0, d.g1, dead, posOf, levPos, wave, rep, inD);
         GLS_HIP(ctx, hipGetLastError());
         {
@@ -1862,7 +2190,8 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
         GLS_HIP(ctx, hipGetLastError());
         if (sweepOut) {
             GLS_TRY(Fills(ctx).add(&d_misc[0], 0, sizeof(uint32_t) * 2).run());
-            k_level_sweep<<<1, SW_WG, 0, st>>>((uint32_t)nNew, fa, fb, out.level, &d_misc[0], &d_misc[1]);
+            const LevelSweep ls{(uint32_t)nNew, fa, fb, out.level, &d_misc[1]};
+            k_level_sweep<<<1, SW_WG, 0, st>>>(ls, ls, &d_misc[0]);
             GLS_HIP(ctx, hipGetLastError());
             GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
             if (misc[0]) {
