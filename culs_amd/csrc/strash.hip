@@ -45,7 +45,49 @@ __global__ void k_zero_flags(int32_t n, int32_t nPIs, const uint32_t *__restrict
     for (int64_t v = tid; v < n; v += stride) flag[v] = (v > nPIs && cnt[v] == 0 && !(dead && dead[v])) ? 1u : 0u;
 }
 
-// One round of the dangling cascade (strash.cu:175-188 as a frontier).
+// The dangling cascade (strash.cu:175-188) from the flagged ANDs.  A workgroup
+// follows the cones of its tile of ids, a round of its queue at a time; what
+// does not fit the queue is left in order[0 .. ctl->curSize) for k_dangle_round.
+// Most cones hang from roots of many tiles and are a few nodes deep, so a launch
+// and a look by the host per round was most of it: the cascade of 2k ANDs took
+// 19 launches of 4 us, now one.
+constexpr uint32_t DANGLE_TILE = 2048;      // also the room of its queue
+
+__global__ void __launch_bounds__(kBlock) k_dangle(int32_t n, int32_t nPIs, const uint32_t *__restrict__ f0,
+                                                   const uint32_t *__restrict__ f1, const uint8_t *__restrict__ flag,
+                                                   uint32_t *ref, uint8_t *dead, uint32_t *order, SweepCtl *ctl) {
+    __shared__ uint32_t s_queue[2][DANGLE_TILE], s_size[2], s_dead;
+    const uint32_t tid = threadIdx.x;
+    if (tid == 0) { s_size[0] = 0; s_size[1] = 0; s_dead = 0; }
+    __syncthreads();
+    const int64_t base = blockIdx.x * (int64_t)DANGLE_TILE;
+    for (uint32_t i = tid; i < DANGLE_TILE; i += kBlock)
+        if (base + i < n && flag[base + i]) s_queue[0][atomicAdd(&s_size[0], 1u)] = (uint32_t)(base + i);
+    __syncthreads();
+    for (uint32_t h = 0;; h ^= 1u) {
+        const uint32_t size = min(s_size[h], DANGLE_TILE);
+        if (size == 0) break;
+        if (tid == 0) s_dead += size;
+        auto release = [&](uint32_t x) {
+            if (x <= (uint32_t)nPIs || atomicSub(&ref[x], 1u) != 1u) return;
+            const uint32_t at = atomicAdd(&s_size[h ^ 1u], 1u);
+            if (at < DANGLE_TILE) s_queue[h ^ 1u][at] = x;
+            else order[atomicAdd(&ctl->curSize, 1u)] = x;
+        };
+        for (uint32_t i = tid; i < size; i += kBlock) {
+            const uint32_t v = s_queue[h][i], a = LID(f0[v]), b = LID(f1[v]);
+            dead[v] = 1;
+            release(a);
+            release(b);
+        }
+        __syncthreads();
+        if (tid == 0) s_size[h] = 0;
+        __syncthreads();
+    }
+    if (tid == 0 && s_dead) atomicAdd(&ctl->processed, s_dead);
+}
+
+// One round of what is left of it, as a frontier.
 __global__ void k_dangle_round(uint32_t k, SweepCtl *ctl, int32_t nPIs, const uint32_t *__restrict__ f0,
                                const uint32_t *__restrict__ f1, uint32_t *ref, uint8_t *dead,
                                uint32_t *order) {
@@ -1524,8 +1566,11 @@ __global__ void k_whole_rep(int32_t N, int32_t nPIs, const uint8_t *__restrict__
     }
 }
 
-__global__ void k_last_pos(int32_t N, const uint32_t *__restrict__ posOf, const uint32_t *__restrict__ keep, uint32_t *count) {
-    *count = posOf[N - 1] + keep[N - 1];
+// positions, and what is left of the dangling cascade
+__global__ void k_last_pos(int32_t N, const uint32_t *__restrict__ posOf, const uint32_t *__restrict__ keep,
+                           const SweepCtl *__restrict__ ctl, uint32_t *out) {
+    out[0] = posOf[N - 1] + keep[N - 1];
+    out[1] = ctl->curSize;
 }
 
 struct Tmp {
@@ -1573,9 +1618,9 @@ uint32_t bits_for(uint32_t x) {
 } // namespace
 
 // Runs sweep rounds (kernel `launch(k)` for k = first..) in growing batches
-// until the frontier is empty.  Returns the number of rounds launched.
+// until the frontier is empty.
 template <class F>
-static int run_sweep(gls_ctx *ctx, SweepCtl *d_ctl, uint32_t first, F launch, SweepCtl *h_ctl, uint32_t *rounds) {
+static int run_sweep(gls_ctx *ctx, SweepCtl *d_ctl, uint32_t first, F launch, SweepCtl *h_ctl) {
     uint32_t k = first, batch = 4;
     for (;;) {
         for (uint32_t i = 0; i < batch; ++i, ++k) launch(k, h_ctl->curSize);
@@ -1584,8 +1629,26 @@ static int run_sweep(gls_ctx *ctx, SweepCtl *d_ctl, uint32_t first, F launch, Sw
         if (h_ctl->curSize == 0) break;
         if (batch < 512) batch *= 2;
     }
-    *rounds = k - first;
     return GLS_OK;
+}
+
+// ANDs that nothing live refers to, in dead[]; the cascade is under way when this
+// returns, and the caller looks at ctl and calls dangling_rest.
+static void dangling(gls_ctx *ctx, const DevGraph &in, uint32_t *ref, uint8_t *flag, uint8_t *dead, uint32_t *order,
+                     SweepCtl *ctl) {
+    const int32_t n = in.nObjs;
+    hipStream_t st = ctx->stream;
+    k_count_refs<<<grid_for(n), kBlock, 0, st>>>(n, in.nPIs, in.f0, in.f1, in.nPOs, in.pos, ref);
+    k_zero_flags<<<grid_for(n), kBlock, 0, st>>>(n, in.nPIs, ref, nullptr, flag);
+    k_dangle<<<(int)(((int64_t)n + DANGLE_TILE - 1) / DANGLE_TILE), kBlock, 0, st>>>(n, in.nPIs, in.f0, in.f1, flag, ref, dead, order, ctl);
+}
+
+// its rest, in rounds
+static int dangling_rest(gls_ctx *ctx, const DevGraph &in, uint32_t *ref, uint8_t *dead, uint32_t *order, SweepCtl *ctl,
+                         SweepCtl *h_ctl) {
+    return run_sweep(ctx, ctl, 1, [&](uint32_t k, uint32_t hint) {
+        k_dangle_round<<<sweep_grid(hint), kBlock, 0, ctx->stream>>>(k, ctl, in.nPIs, in.f0, in.f1, ref, dead, order);
+    }, h_ctl);
 }
 
 // tagDepth[t] = the largest wave of a node tagged t (dangling nodes have wave 0)
@@ -1644,22 +1707,14 @@ int dev_strash(gls_ctx *ctx, const DevGraph &in, DevGraph &out, int32_t *depthOu
                 .run());
     const int gN = grid_for(n);
     SweepCtl h_ctl{};
-    uint32_t rounds = 0;
 
     // 1. fanout counts and dangling cascade
     uint8_t *zflag = t.get<uint8_t>((size_t)n);
     if (!zflag) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: frontier flags");
-    k_count_refs<<<gN, kBlock, 0, st>>>(n, nPIs, in.f0, in.f1, nPOs, in.pos, ref);
-    k_zero_flags<<<gN, kBlock, 0, st>>>(n, nPIs, ref, nullptr, zflag);
+    dangling(ctx, in, ref, zflag, dead, order, ctl);
     GLS_HIP(ctx, hipGetLastError());
-    GLS_TRY(select_ids(ctx, t, n, zflag, order, &ctl->curSize));
     GLS_TRY(stream_copy(ctx, &h_ctl, ctl, sizeof(SweepCtl), hipMemcpyDeviceToHost));
-    if (h_ctl.curSize > 0) {
-        GLS_TRY(run_sweep(ctx, ctl, 1, [&](uint32_t k, uint32_t hint) {
-            k_dangle_round<<<sweep_grid(hint), kBlock, 0, st>>>(k, ctl, nPIs, in.f0, in.f1, ref, dead, order);
-        }, &h_ctl, &rounds));
-    }
-
+    if (h_ctl.curSize > 0) GLS_TRY(dangling_rest(ctx, in, ref, dead, order, ctl, &h_ctl));
     const uint32_t nDead = h_ctl.processed;
     // 2. fanout CSR over live AND nodes and the first frontier (wave 1)
     GLS_TRY(Fills(ctx)
@@ -1813,7 +1868,8 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
         uint32_t *rep = t.get<uint32_t>(N), *rep2 = t.get<uint32_t>(N), *slot = t.get<uint32_t>(N), *fold = t.get<uint32_t>(N);
         unsigned long long *best = t.get<unsigned long long>(N);
         uint32_t *d_misc = t.get<uint32_t>(16);   // [0] err, [1] largest wave, [2..3] a round changed something,
-                                                  // [4] survivors, [5] largest level, [6..7] probes, [8] a path got shorter
+                                                  // [4] survivors, [5] largest level, [6..7] probes, [8] a path got shorter,
+                                                  // [9] positions, [10] what is left of the cascade
         SweepCtl *ctl = t.get<SweepCtl>(1);
         if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: device allocation failed (n=%d)", N);
         unsigned long long *d_probes = reinterpret_cast<unsigned long long *>(&d_misc[6]);
@@ -1828,30 +1884,25 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
                     .run());
         const int gN = grid_for(N);
         SweepCtl h_ctl{};
-        uint32_t rounds = 0;
         // 1. dangling cascade
-        k_count_refs<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, nPOs, in.pos, ref);
-        k_zero_flags<<<gN, kBlock, 0, st>>>(N, nPIs, ref, nullptr, flag);
-        GLS_HIP(ctx, hipGetLastError());
-        GLS_TRY(select_ids(ctx, t, N, flag, order, &ctl->curSize));
-        GLS_TRY(stream_copy(ctx, &h_ctl, ctl, sizeof(SweepCtl), hipMemcpyDeviceToHost));
-        if (h_ctl.curSize > 0) {
-            GLS_TRY(run_sweep(ctx, ctl, 1, [&](uint32_t k, uint32_t hint) {
-                k_dangle_round<<<sweep_grid(hint), kBlock, 0, st>>>(k, ctl, nPIs, in.f0, in.f1, ref, dead, order);
-            }, &h_ctl, &rounds));
-        }
+        dangling(ctx, in, ref, flag, dead, order, ctl);
         // positions: the constant and the PIs, then the live ANDs in id order
-        k_keep_flags<<<gN, kBlock, 0, st>>>(N, nPIs, dead, keep);
         size_t tbp = 0;
         GLS_HIP(ctx, rocprim::exclusive_scan(nullptr, tbp, keep, posOf, 0u, (size_t)N, rocprim::plus<uint32_t>(), st));
         void *tmpp = t.get<uint8_t>(std::max<size_t>(tbp, 1));
         if (!tmpp) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: position scan storage");
-        GLS_HIP(ctx, rocprim::exclusive_scan(tmpp, tbp, keep, posOf, 0u, (size_t)N, rocprim::plus<uint32_t>(), st));
-        k_full_fanpos<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, posOf, fa, fb, &d_misc[0]);
-        k_last_pos<<<1, 1, 0, st>>>(N, posOf, keep, &d_misc[9]);
-        GLS_HIP(ctx, hipGetLastError());
         uint32_t misc[16] = {};
-        GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
+        for (;;) {
+            k_keep_flags<<<gN, kBlock, 0, st>>>(N, nPIs, dead, keep);
+            GLS_HIP(ctx, rocprim::exclusive_scan(tmpp, tbp, keep, posOf, 0u, (size_t)N, rocprim::plus<uint32_t>(), st));
+            k_full_fanpos<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, posOf, fa, fb, &d_misc[0]);
+            k_last_pos<<<1, 1, 0, st>>>(N, posOf, keep, ctl, &d_misc[9]);
+            GLS_HIP(ctx, hipGetLastError());
+            GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
+            if (misc[10] == 0) break;
+            h_ctl.curSize = misc[10];
+            GLS_TRY(dangling_rest(ctx, in, ref, dead, order, ctl, &h_ctl));
+        }
         if (misc[0]) return fallback();      // ids are not topological
         const uint32_t nPos = misc[9];
         // 2. classes
@@ -2028,19 +2079,11 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
                     .run());
         const int gN = grid_for(N);
         SweepCtl h_ctl{};
-        uint32_t rounds = 0;
-        // 1. dangling cascade (its first frontier, the ANDs without fanout, by
-        //    a compaction of flags)
-        k_count_refs<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, nPOs, in.pos, ref);
-        k_zero_flags<<<gN, kBlock, 0, st>>>(N, nPIs, ref, nullptr, surv);
+        // 1. dangling cascade
+        dangling(ctx, in, ref, surv, dead, order, ctl);
         GLS_HIP(ctx, hipGetLastError());
-        GLS_TRY(select_ids(ctx, t, N, surv, order, &ctl->curSize));
         GLS_TRY(stream_copy(ctx, &h_ctl, ctl, sizeof(SweepCtl), hipMemcpyDeviceToHost));
-        if (h_ctl.curSize > 0) {
-            GLS_TRY(run_sweep(ctx, ctl, 1, [&](uint32_t k, uint32_t hint) {
-                k_dangle_round<<<sweep_grid(hint), kBlock, 0, st>>>(k, ctl, nPIs, in.f0, in.f1, ref, dead, order);
-            }, &h_ctl, &rounds));
-        }
+        if (h_ctl.curSize > 0) GLS_TRY(dangling_rest(ctx, in, ref, dead, order, ctl, &h_ctl));
         // 2. a topological order (keys relaxed from the input levels, then a
         //    stable sort), and the waves by one chunked sweep over it
         uint32_t misc[16] = {};

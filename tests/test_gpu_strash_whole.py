@@ -110,3 +110,39 @@ def test_strash_of_many_rounds(gpu_ctx, pis, window, path):
     assert a.last_op()["final_strash"] == path
     b = gpu_ctx.from_arrays(*g).strash(schedule=culs_amd.GLS_ST_WAVES)
     assert same(a.rewrite().arrays(), b.rewrite().arrays())
+
+
+@pytest.mark.parametrize("leaves", [1, 2047, 2048, 2049, 9000])
+def test_dangling_cones(gpu_ctx, leaves):
+    """A tree of ANDs that nothing refers to: its cascade's rounds are as wide as
+    its levels, which fit a workgroup's queue up to 2048; beside it a live chain
+    that has ANDs of a second dangling tree between its own."""
+    print("dangling cones:", leaves)
+    sys.stdout.flush()
+    nPIs = 200
+    rng = np.random.default_rng(leaves)
+    f0, f1 = [0] * (nPIs + 1), [0] * (nPIs + 1)
+
+    def add(a, b):
+        f0.append(int(a))
+        f1.append(int(b))
+        return 2 * (len(f0) - 1)
+
+    def lit():
+        return 2 * int(rng.integers(1, nPIs + 1)) + int(rng.integers(0, 2))
+
+    def tree(row):
+        while len(row) > 1:
+            row = [add(row[i], row[i + 1] ^ 1) if i + 1 < len(row) else row[i] for i in range(0, len(row), 2)]
+
+    tree([add(lit(), lit()) for _ in range(leaves)])
+    chain, second = add(lit(), lit()), []
+    for _ in range(3000):
+        second.append(add(chain ^ 1, lit()))
+        chain = add(chain, lit())
+    tree(second)
+    g = nPIs, np.array(f0, np.uint32), np.array(f1, np.uint32), np.array([chain, chain ^ 1, 2], np.uint32)
+    want, depth = O.strash(*g)
+    for schedule in (0, culs_amd.GLS_ST_WAVES, culs_amd.GLS_ST_LEVELS):
+        a = gpu_ctx.from_arrays(*g).strash(schedule=schedule)
+        assert same(a.arrays(), want) and a.stats().levels == depth, schedule
