@@ -1517,15 +1517,17 @@ __global__ void k_whole_follow(WholeArgs a, uint32_t *changed) {
     if (__ballot(any) != 0 && (threadIdx.x & 63) == 0) atomicOr(changed, 1u);
 }
 
-// fanin positions of the classes at their representatives' positions
+// fanin positions of the classes at their representatives' positions (deadToo:
+// dangling nodes have positions, without fanins)
 __global__ void k_whole_classpos(int32_t N, int32_t nPIs, const uint32_t *__restrict__ f0,
                                  const uint32_t *__restrict__ f1, const uint8_t *__restrict__ dead,
                                  const uint32_t *__restrict__ rep, const uint32_t *__restrict__ posOf, uint32_t *fa,
-                                 uint32_t *fb) {
+                                 uint32_t *fb, uint32_t deadToo) {
     int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t v = tid; v < N; v += stride) {
-        if (v > nPIs && dead[v]) continue;
-        const bool top = v > nPIs && rep[v] == 2u * (uint32_t)v;
+        const bool gone = v > nPIs && dead[v];
+        if (gone && !deadToo) continue;
+        const bool top = v > nPIs && !gone && rep[v] == 2u * (uint32_t)v;
         fa[posOf[v]] = top ? posOf[LID(rep[LID(f0[v])])] : NOFAN;
         fb[posOf[v]] = top ? posOf[LID(rep[LID(f1[v])])] : NOFAN;
     }
@@ -1943,7 +1945,7 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
             r += misc[2] == 0 ? 1u : 2u;
         }
         // 3. levels
-        k_whole_classpos<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, rep, posOf, ca, cb);
+        k_whole_classpos<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, rep, posOf, ca, cb, 0u);
         k_level_sweep<<<swept ? 1 : 2, SW_WG, 0, st>>>(classes, waves, &d_misc[0]);
         // 4. representatives, survivors in (wave, id) order
         uint32_t *wave = ref, *level = order, *survIds = fa, *survWave = fb, *sortIds = ca, *sortWave = cb, *newId = keep;
@@ -2012,8 +2014,8 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
 // n..N-1).  The result equals dev_strash(comb) array for array; it is computed
 // from what changed instead of a wave-by-wave sweep:
 //  1. dangling nodes, as in dev_strash;
-//  2. waves (levels over the live nodes) by one chunked sweep over a
-//     topological order of comb, sorted by a key relaxed from g's levels;
+//  2. a topological order of comb, sorted by a key relaxed from g's levels; the
+//     keys are the waves (levels over the live nodes) where every one is tight;
 //  3. representatives: g is strashed, so a live old node whose fanins are
 //     unchanged and are their own representatives keeps its key, which no
 //     other such node has.  Only the other nodes (new nodes, redirected old
@@ -2027,8 +2029,14 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
 //     representatives, which is the fixpoint the wave sweep reaches (it is
 //     unique: by induction over waves, each wave's keys and minima follow
 //     from the waves before);
-//  4. survivors in (wave, id) order, fanins over representatives, and the
-//     output levels by the same chunked sweep over the output.
+//  4. where a key is loose, the keys stand for the waves in step 3, and one
+//     launch sweeps the waves and the classes' levels side by side; then each
+//     class takes its node of smallest (wave, id);
+//  5. survivors in (wave, id) order, fanins over representatives, and the
+//     output levels: the classes', or the waves where no merge lowered one, or a
+//     sweep over the output.
+// The final strash of rw on a deep AIG of 10M ANDs whose keys are loose and whose
+// output's levels fall: 20.0 ms with one sweep after the other, 11.9 side by side.
 // Where a step cannot run (a position order that is not topological, a table
 // or dirty-set overflow, too many rounds) it falls back to dev_strash(comb);
 // info->final_strash tells which path ran.
@@ -2087,7 +2095,6 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
         // 2. a topological order (keys relaxed from the input levels, then a
         //    stable sort), and the waves by one chunked sweep over it
         uint32_t misc[16] = {};
-        bool sweepIn = true;
         k_rw_key_init<<<gN, kBlock, 0, st>>>(n, N, d.glevel, fa);
         uint32_t keyRounds = 0;
         for (;; ++keyRounds) {
@@ -2109,28 +2116,19 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
             GLS_HIP(ctx, rocprim::radix_sort_pairs(tmpk, tbk, fa, fb, levPos, order, (size_t)N, 0u, 32u, st));
         }
         k_rw_pos<<<gN, kBlock, 0, st>>>(N, order, posOf);
-        // the waves: the keys themselves where every live key is tight, else a
-        // level sweep over the positions
+        // the waves: the keys themselves where every live key is tight.  Else the
+        // keys take their place in the rounds (any order in which fanins come
+        // first does), and both level sweeps follow in one launch.
         k_rw_key_loose<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, fa, &d_misc[9], &d_misc[10]);
+        k_rw_levpos<<<gN, kBlock, 0, st>>>(N, nPIs, dead, fa, posOf, levPos);
         GLS_HIP(ctx, hipGetLastError());
         GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
-        sweepIn = misc[9] != 0u;
-        if (sweepIn) {
+        const bool loose = misc[9] != 0u;
+        int32_t depth = (int32_t)misc[10];
+        if (loose) {
             k_rw_fanpos<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, posOf, fa, fb, &d_misc[0]);
             GLS_HIP(ctx, hipGetLastError());
-            GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
-            if (misc[0]) return fallback("positions");
-            const LevelSweep ls{(uint32_t)N, fa, fb, levPos, &d_misc[1]};
-            k_level_sweep<<<1, SW_WG, 0, st>>>(ls, ls, &d_misc[0]);
-            GLS_HIP(ctx, hipGetLastError());
-            GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
-            if (misc[0]) return fallback("sweep order");
-        } else {
-            k_rw_levpos<<<gN, kBlock, 0, st>>>(N, nPIs, dead, fa, posOf, levPos);
-            GLS_HIP(ctx, hipGetLastError());
-            misc[1] = misc[10];
         }
-        const int32_t depth = (int32_t)misc[1];
         const bool narrow = (int64_t)N <= width * depth0;
         // the wave sweep's limit on objects holds where it used to run
         if (!narrow && (uint64_t)tuning_for(ctx, N).strash_table_factor * (uint64_t)N > (1ull << 31))
@@ -2146,7 +2144,6 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
             if (!tmpd) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: dirty list storage");
             GLS_HIP(ctx, rocprim::select(tmpd, tbd, ids, inD, dlist, &d_misc[2], (size_t)N, st));
         }
-        if (tagIn && tagDepth) k_tag_depth<<<tag_grid(N), kBlock, 0, st>>>(N, nPIs, wave, tagIn, tagDepth);
         // 3. representatives of the dirty set, in rounds
         uint32_t nD = 0;
         GLS_TRY(stream_copy(ctx, &nD, &d_misc[2], sizeof(uint32_t), hipMemcpyDeviceToHost));
@@ -2185,8 +2182,24 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
             if (misc[3] == 0 && nD == prevD) break;
         }
         // 4. survivors in (wave, id) order
-        k_rw_shorter<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep, wave, &d_misc[8]);
-        k_rw_survivors<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep, surv);
+        const uint32_t *outRep = rep, *outLev = wave;
+        if (loose) {
+            uint32_t *ca = survIds, *cb = survWave, *classLev = sortIds, *rep2 = inD, *level = order;
+            unsigned long long *best = t.get<unsigned long long>(N);
+            if (!best) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: representatives");
+            GLS_TRY(Fills(ctx).add(best, 0xFF, sizeof(unsigned long long) * N).run());
+            k_whole_classpos<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, rep, posOf, ca, cb, 1u);
+            k_level_sweep<<<2, SW_WG, 0, st>>>(LevelSweep{(uint32_t)N, ca, cb, classLev, &d_misc[11]},
+                                               LevelSweep{(uint32_t)N, fa, fb, levPos, &d_misc[1]}, &d_misc[0]);
+            k_whole_waves<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep, posOf, levPos, wave, best);
+            k_whole_rep<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep, posOf, wave, best, classLev, rep2, level);
+            outRep = rep2;
+            outLev = level;
+        } else {
+            k_rw_shorter<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep, wave, &d_misc[8]);
+        }
+        if (tagIn && tagDepth) k_tag_depth<<<tag_grid(N), kBlock, 0, st>>>(N, nPIs, wave, tagIn, tagDepth);
+        k_rw_survivors<<<gN, kBlock, 0, st>>>(N, nPIs, dead, outRep, surv);
         size_t tb = 0;
         rocprim::counting_iterator<uint32_t> ids(0u);
         GLS_HIP(ctx, rocprim::select(nullptr, tb, ids, surv, survIds, &d_misc[4], (size_t)N, st));
@@ -2194,6 +2207,8 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
         if (!tmp) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: select storage");
         GLS_HIP(ctx, rocprim::select(tmp, tb, ids, surv, survIds, &d_misc[4], (size_t)N, st));
         GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
+        if (misc[0]) return fallback("sweep order");
+        if (loose) depth = (int32_t)misc[1];
         const uint32_t m = misc[4];
         const int32_t nNew = nPIs + 1 + (int32_t)m;
         GLS_TRY(dev_graph_alloc(ctx, out, nNew, nPIs, nPOs));
@@ -2222,14 +2237,14 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
                     .add(out.f1, 0, sizeof(uint32_t) * (nPIs + 1))
                     .run());
         k_new_ids<<<grid_for(m + nPIs + 1), kBlock, 0, st>>>(N, nPIs, (int32_t)m, sorted, newId);
-        // 5. output levels: the survivors' waves when no representative lies on
-        // a lower wave than its node, else a level sweep over the output (fa /
-        // fb are free again: they take the output's fanin ids)
-        const bool sweepOut = misc[8] != 0u;
-        k_rw_emit<<<grid_for(nNew), kBlock, 0, st>>>((int32_t)m, nPIs, sorted, in.f0, in.f1, rep, newId, out.f0,
-                                                     out.f1, fa, fb, wave, sweepOut ? nullptr : out.level, tagIn,
+        // 5. output levels: swept already, or the survivors' waves when no
+        // representative lies on a lower wave than its node, else a level sweep
+        // over the output (fa / fb are free again: they take its fanin ids)
+        const bool sweepOut = !loose && misc[8] != 0u;
+        k_rw_emit<<<grid_for(nNew), kBlock, 0, st>>>((int32_t)m, nPIs, sorted, in.f0, in.f1, outRep, newId, out.f0,
+                                                     out.f1, fa, fb, outLev, sweepOut ? nullptr : out.level, tagIn,
                                                      tags);
-        if (nPOs > 0) k_rw_pos_out<<<grid_for(nPOs), kBlock, 0, st>>>(nPOs, nPIs, in.pos, rep, newId, out.pos);
+        if (nPOs > 0) k_rw_pos_out<<<grid_for(nPOs), kBlock, 0, st>>>(nPOs, nPIs, in.pos, outRep, newId, out.pos);
         GLS_HIP(ctx, hipGetLastError());
         if (sweepOut) {
             GLS_TRY(Fills(ctx).add(&d_misc[0], 0, sizeof(uint32_t) * 2).run());
@@ -2252,7 +2267,7 @@ int dev_strash_rw(gls_ctx *ctx, const DevGraph &in, const RwDelta &d, DevGraph &
             info->hash_probes += (int64_t)((uint64_t)misc[6] | (uint64_t)misc[7] << 32);
             info->final_strash = 1;
             info->strash_rounds = (int64_t)r + 1;
-            info->strash_sweeps = (sweepIn ? 1 : 0) + (sweepOut ? 1 : 0);
+            info->strash_sweeps = loose ? 2 : sweepOut ? 1 : 0;
         }
     }
     return GLS_OK;

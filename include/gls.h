@@ -77,10 +77,10 @@ typedef struct {
     double cut_graph_ms;
     int64_t cut_graph_nodes;
     /* gls_rewrite's incremental final strash: the one-workgroup level sweeps
-     * it ran (0-2).  The composed graph's levels are swept only where its
-     * relaxed topological keys are not already its levels, and the output's
-     * only where a merge or fold put a node's representative on a lower
-     * level than the node. */
+     * it ran (0-2).  Where the composed graph's relaxed topological keys are
+     * not already its levels, these and the output's are swept side by side;
+     * else the output's are, if a merge or fold put a node's representative
+     * on a lower level than the node. */
     int32_t strash_sweeps, pad0;
 } gls_op_info;
 
