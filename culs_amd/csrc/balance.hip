@@ -649,7 +649,8 @@ constexpr uint32_t LN_FINAL = 0x80000000u, LS_NONE = 0xFFFFu;
 // spilled is waited for, and the insertions with it, so the next level's words
 // are read after the sort.  The table in memory is at most a quarter full: a
 // wavefront waits for the longest of its lanes' probe chains.  2M random ANDs
-// (1786 levels of 668 covers and 1523 inputs): 38.8 ms; 45.1 with the next
+// (1786 levels of 668 covers and 1523 inputs): 37.2 ms; 38.8 with each step's
+// pairs and nodes handed on through LDS, 45.1 before that with the next
 // level read at the start (spilled) and a table twice as full, 63 with every
 // lookup made at its step in memory.  The 64-bit multiplier (a level has 77
 // covers, 161 inputs): 2.5 ms for 414 levels, 3.4 before.
@@ -663,7 +664,7 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
     __shared__ unsigned long long s_res[LT_COVERS];  // the covers' results, for the next level
     __shared__ uint16_t s_ent[LT_NEW];               // the nodes' entries in s_key, LS_NONE: another one has it
     __shared__ uint16_t s_perm[LT_INPUTS];           // `b -s`: the shuffled inputs
-    __shared__ uint16_t s_off[LT_COVERS + 1], s_len[LT_COVERS], s_slot[LT_COVERS], s_act[64];
+    __shared__ uint16_t s_off[LT_COVERS + 1], s_len[LT_COVERS], s_act[64];
     __shared__ uint8_t s_mem[LT_COVERS];             // the cover's pairs are looked up in memory too
     __shared__ uint32_t s_cnt[LQ_COV][BAL_WG / 64], s_over;
     __shared__ int32_t s_top;
@@ -733,7 +734,7 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
     };
     arrived(cur);
     // the level before's nodes, on their way into the table
-    unsigned long long newKey[LQ_NEW], newNode[LQ_NEW], newPrev[LQ_NEW];
+    unsigned long long newKey[LQ_NEW], newPrev[LQ_NEW];
     uint32_t newSlot[LQ_NEW];
 #pragma unroll
     for (uint32_t q = 0; q < LQ_NEW; q++) newKey[q] = EMPTY64;
@@ -747,7 +748,8 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
                 newPrev[q] = t_cas(r.t, newSlot[q], newKey[q]);
             }
             if (newPrev[q] != EMPTY64 && newPrev[q] != newKey[q]) { atomicOr(r.err, 2u); continue; }
-            __hip_atomic_store(&r.t.v[newSlot[q]], newNode[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // (its place in s_node is taken by this level's nodes only later)
+            __hip_atomic_store(&r.t.v[newSlot[q]], s_node[tid + q * BAL_WG], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
     for (; l >= lLast; l--) {
@@ -921,8 +923,13 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
         const bool over = s_over != 0;       // not all of them fit: every cover looks up in memory too
         // sharedNodeDrivenPermute and prepareDataToInsert (balance.cu:113-247)
         // of a cover with two inputs at least: takes its last two; returns the
-        // existing signal, or EMPTY64 and the slot of the inserted key
-        auto prepare = [&](uint32_t c, uint32_t o, uint32_t L, uint32_t &slot) -> unsigned long long {
+        // existing signal, or EMPTY64, the inserted key, its slot (+ 1) and the
+        // level of its node
+        struct Pair {
+            unsigned long long key;
+            uint32_t slot, lev;
+        };
+        auto prepare = [&](uint32_t c, uint32_t o, uint32_t L, Pair &pair) -> unsigned long long {
             const uint32_t right = o + L - 2;
             const unsigned long long l1 = s_arr[right + 1], l2 = s_arr[right];
             const uint32_t x1 = sig_lit(l1), border = sig_lev(l2);
@@ -943,40 +950,57 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
                 i--;
                 l3 = before;
             }
-            slot = 0;
+            pair.slot = 0;
             if (found == EMPTY64) {
-                const unsigned long long key = and_key_of(x1, sig_lit(l2));
                 bool isNew;
-                const uint32_t h = level_slot(key, isNew);
+                pair.key = and_key_of(x1, sig_lit(l2));
+                pair.lev = (sig_lev(l1) > border ? sig_lev(l1) : border) + 1u;
+                const uint32_t h = level_slot(pair.key, isNew);
                 atomicMin(&s_val[h], c);
-                slot = h + 1;
-                s_arr[right + 1] = key;                  // the popped pair, and its level
-                s_arr[right] = (sig_lev(l1) > border ? sig_lev(l1) : border) + 1u;
+                pair.slot = h + 1;
             } else {
                 s_mem[c] = 1;
             }
             return found;
         };
         // the winner of a key becomes node `at` of the level
-        auto create = [&](uint32_t c, uint32_t o, uint32_t L, uint32_t slot, uint32_t at) {
-            const unsigned long long key = s_arr[o + L + 1];
+        auto create = [&](uint32_t c, const Pair &pair, uint32_t at) -> unsigned long long {
             const uint32_t id = levBase + at;
-            s_node[at] = sig(2u * id, (uint32_t)s_arr[o + L]);
-            s_val[slot - 1] = LN_FINAL | at;
-            s_ent[at] = (uint16_t)(slot - 1);
-            r.of0[id] = (uint32_t)(key >> 32);
-            r.of1[id] = (uint32_t)key;
+            const unsigned long long x = sig(2u * id, pair.lev);
+            s_node[at] = x;
+            s_val[pair.slot - 1] = LN_FINAL | at;
+            s_ent[at] = (uint16_t)(pair.slot - 1);
+            r.of0[id] = (uint32_t)(pair.key >> 32);
+            r.of1[id] = (uint32_t)pair.key;
             if (r.tagOut) r.tagOut[id] = r.tagIn[r.roots[cur.e.s + c]];
+            return x;
         };
-        // addBackLocalArrays (balance.cu:429-467); returns the new length
+        // addBackLocalArrays (balance.cu:429-467); returns the new length.  The
+        // last four inputs are read together: a step waits for these reads, and
+        // most covers have no more.
         auto add_back = [&](uint32_t o, uint32_t L, unsigned long long x) -> uint32_t {
-            for (uint32_t i = 0; i < L; i += 2)
-                if (sig_lit(s_arr[o + i]) == sig_lit(x) || sig_lit(s_arr[o + min(i + 1, L - 1)]) == sig_lit(x)) return L;
+            unsigned long long y[4];
+            bool there = false;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++) y[k] = s_arr[o + (L > k ? L - 1 - k : 0)];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++) there |= k < L && sig_lit(y[k]) == sig_lit(x);
+            for (uint32_t i = 4; i < L; i += 2)
+                there |= sig_lit(s_arr[o + L - 1 - i]) == sig_lit(x) || sig_lit(s_arr[o + (L > i + 1 ? L - 2 - i : 0)]) == sig_lit(x);
+            if (there) return L;
             uint32_t i = L;
-            while (i > 0) {
-                const unsigned long long y = s_arr[o + i - 1];
-                if (sig_lev(x) <= sig_lev(y)) break;
-                s_arr[o + i] = y;
+            bool stop = false;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k++) {
+                stop |= k >= L || sig_lev(x) <= sig_lev(y[k]);
+                if (stop) continue;
+                s_arr[o + i] = y[k];
+                i--;
+            }
+            while (!stop && i > 0) {
+                const unsigned long long z = s_arr[o + i - 1];
+                if (sig_lev(x) <= sig_lev(z)) break;
+                s_arr[o + i] = z;
                 i--;
             }
             s_arr[o + i] = x;
@@ -986,14 +1010,18 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
         uint32_t nAct = nb;
         if (nb <= 64u && tid < 64u) s_act[tid] = (uint16_t)tid;
         while (nAct > 64u) {
-            for (uint32_t c = tid; c < nb; c += BAL_WG) {
-                const uint32_t o = s_off[c], L = s_len[c];
-                s_slot[c] = 0;
-                if (L <= 1) continue;
-                uint32_t slot;
-                const unsigned long long f = prepare(c, o, L, slot);
-                s_slot[c] = (uint16_t)slot;
-                s_len[c] = (uint16_t)(slot ? L - 2 : add_back(o, L - 2, f));
+            Pair pair[LQ_COV];
+            uint32_t len[LQ_COV];
+            unsigned long long became[LQ_COV];        // what the pair became
+#pragma unroll
+            for (uint32_t q = 0; q < LQ_COV; q++) {
+                const uint32_t c = tid + q * BAL_WG;
+                pair[q].slot = 0;
+                len[q] = c < nb ? s_len[c] : 0u;
+                if (len[q] <= 1) continue;
+                const uint32_t o = s_off[c];
+                const unsigned long long f = prepare(c, o, len[q], pair[q]);
+                len[q] = pair[q].slot ? len[q] - 2 : add_back(o, len[q] - 2, f);
             }
             __syncthreads();
             // winners, counted in cover order
@@ -1001,7 +1029,7 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
 #pragma unroll
             for (uint32_t q = 0; q < LQ_COV; q++) {
                 const uint32_t c = tid + q * BAL_WG;
-                const bool win = c < nb && s_slot[c] != 0 && s_val[s_slot[c] - 1] == c;
+                const bool win = pair[q].slot != 0 && s_val[pair[q].slot - 1] == c;
                 const uint64_t m = __ballot(win);
                 rank[q] = win ? (uint32_t)__popcll(m & ((1ull << lane) - 1ull)) : UNSET;
                 if (lane == 0) s_cnt[q][wave] = (uint32_t)__popcll(m);
@@ -1017,10 +1045,7 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
                     before += w < wave ? x : 0u;
                     total += x;
                 }
-                if (rank[q] != UNSET) {
-                    const uint32_t c = tid + q * BAL_WG;
-                    create(c, s_off[c], s_len[c], s_slot[c], counter - levBase + before + rank[q]);
-                }
+                if (rank[q] != UNSET) became[q] = create(tid + q * BAL_WG, pair[q], counter - levBase + before + rank[q]);
             }
             counter += total;
             __syncthreads();
@@ -1029,16 +1054,12 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
 #pragma unroll
             for (uint32_t q = 0; q < LQ_COV; q++) {
                 const uint32_t c = tid + q * BAL_WG;
-                bool more = false;
-                if (c < nb) {
-                    uint32_t L = s_len[c];
-                    if (s_slot[c] != 0) {
-                        L = add_back(s_off[c], L, s_node[s_val[s_slot[c] - 1] & ~LN_FINAL]);
-                        s_len[c] = (uint16_t)L;
-                    }
-                    more = L > 1;
+                if (pair[q].slot != 0) {
+                    if (rank[q] == UNSET) became[q] = s_node[s_val[pair[q].slot - 1] & ~LN_FINAL];
+                    len[q] = add_back(s_off[c], len[q], became[q]);
                 }
-                am[q] = __ballot(more);
+                if (c < nb) s_len[c] = (uint16_t)len[q];
+                am[q] = __ballot(len[q] > 1);
                 if (lane == 0) s_cnt[q][wave] = (uint32_t)__popcll(am[q]);
             }
             __syncthreads();
@@ -1068,21 +1089,21 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
                 const uint32_t c = has ? s_act[lane] : 0u, o = s_off[c];
                 uint32_t L = has ? s_len[c] : 0u;
                 while (__ballot(L > 1) != 0) {
-                    uint32_t slot = 0;
+                    Pair pair = {};
                     unsigned long long f = EMPTY64;
                     const bool act = L > 1;
                     if (act) {
-                        f = prepare(c, o, L, slot);
+                        f = prepare(c, o, L, pair);
                         L -= 2;
                     }
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    const bool win = slot != 0 && lds_load(&s_val[slot - 1]) == c;
+                    const bool win = pair.slot != 0 && lds_load(&s_val[pair.slot - 1]) == c;
                     const uint64_t m = __ballot(win);
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    if (win) create(c, o, L, slot, counter - levBase + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)));
+                    if (win) f = create(c, pair, counter - levBase + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)));
                     counter += (uint32_t)__popcll(m);
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    if (slot != 0) f = s_node[lds_load(&s_val[slot - 1]) & ~LN_FINAL];
+                    if (pair.slot != 0 && !win) f = s_node[lds_load(&s_val[pair.slot - 1]) & ~LN_FINAL];
                     if (act) L = add_back(o, L, f);
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 }
@@ -1103,7 +1124,6 @@ __global__ void __launch_bounds__(BAL_WG) k_rec_lds(RecArgs r, const uint32_t *_
             if (i >= counter - levBase) continue;
             const uint32_t h = s_ent[i];
             newKey[q] = s_key[h];
-            newNode[q] = s_node[i];
             s_key[h] = EMPTY64;
             s_val[h] = UNSET;
             newSlot[q] = (uint32_t)t_hash(r.t, newKey[q]);
