@@ -264,6 +264,9 @@ int gen_multiplier_arrays(int32_t n, double redundant, uint64_t seed, std::vecto
     if (n < 2 || n > 256 || redundant < 0 || redundant > 1) return GLS_ERR_ARG;
     Rng rng(seed);
     Builder b(2 * n);
+    const size_t room = (size_t)((9.0 * n * n + 2 * n) * (1.0 + 2.1 * redundant)) + 2 * (size_t)n + 64;
+    b.f0.reserve(room);
+    b.f1.reserve(room);
     const uint32_t NONE = 0xFFFFFFFFu;
     auto AND = [&](uint32_t x, uint32_t y) -> uint32_t {
         uint32_t g = b.add(x, y);
