@@ -454,9 +454,9 @@ extern "C" int gls_strash(gls_aig *a, int32_t flags) {
     gls_op_info info = {};
     // every node hashed in rounds, levels by sweeps over id order, which gives way to the wave sweep
     // for ids that are not topological and where it needs too many rounds.
-    // Against the wave sweep, ms: 521 objects 0.34 / 0.48, 2k 0.47 / 0.50, 20k
-    // 0.65 / 0.84, the 64-bit multiplier 0.53 / 1.65, 200k 0.90 / 2.7, 1M of
-    // 1029 to 20876 per level 2.4 / 13.0 to 2.1 / 4.3.
+    // Against the wave sweep, ms: 521 objects 0.12 / 0.24, 2k 0.15 / 0.32, 20k
+    // 0.21 / 0.46, the 64-bit multiplier 0.28 / 1.38, 200k 0.46 / 2.36, 1M of
+    // 1029 per level 1.33 / 10.7, of 12711 per level 1.84 / 3.50.
     if (!(flags & GLS_ST_WAVES)) {
         GLS_TRY(dev_strash_whole(ctx, a->dev, (flags & GLS_ST_LEVELS) != 0, out, &depth, &info));
     } else {

@@ -959,7 +959,7 @@ constexpr uint32_t SW_SPIN_LIMIT = 1u << 22;
 // twice needs one per level; most graphs take one to three.  A rewrite takes
 // many where its graph is narrow, else few.  A whole graph's round after the
 // first costs 15 us and 4 us per million objects, its wave sweep 0.2 ms more than
-// the rounds' other work at 20k objects, 2 ms at a million on wide levels: few
+// the rounds' other work at 20k objects, 1.7 ms at a million on wide levels: few
 // below 2^18 objects, many from there.  Where the levels are narrow the wave
 // sweep costs 100 ms more at 10M objects: those that are still at it go on to the
 // limit (of 120 raw deep AIGs of 10M ANDs 108 took two or three, one 44).
