@@ -1361,12 +1361,24 @@ __device__ PlanCore plan_core(const GraphView &g, const Lib &L, int id, const ui
     return pc;
 }
 
-__global__ void __launch_bounds__(EVAL_BLOCK) k_plan(int32_t nCand, const uint32_t *__restrict__ candIds,
+// Candidates per wavefront of k_plan and k_build.  A lane replays its candidate's
+// cone and forest, and a wavefront takes as long as the longest of its lanes'
+// bucket scans, so few candidates are spread over more wavefronts, up to about
+// eight on a CU.  k_plan and k_build of 2k ANDs 56 and 45 us with 64 to a
+// wavefront, 36 and 29 with 4; of the 32-bit multiplier 73 and 58, 54 and 48.
+constexpr int32_t PLAN_WAVES = 2048;
+int plan_lanes(int32_t nCand) {
+    int per = 4;
+    while (per < EVAL_BLOCK && (int64_t)nCand > (int64_t)per * PLAN_WAVES) per *= 2;
+    return per;
+}
+
+__global__ void __launch_bounds__(EVAL_BLOCK) k_plan(int32_t per, int32_t nCand, const uint32_t *__restrict__ candIds,
                                                       GraphView g, Lib L, const uint32_t *__restrict__ cuts,
                                                       const int4 *__restrict__ best, Plan *plans) {
     __shared__ int32_t s_match[NMATCH * EVAL_BLOCK], s_mlev[NMATCH * EVAL_BLOCK];
-    int64_t c = blockIdx.x * (int64_t)EVAL_BLOCK + threadIdx.x;
-    if (c >= nCand) return;
+    int64_t c = blockIdx.x * (int64_t)per + threadIdx.x;
+    if ((int32_t)threadIdx.x >= per || c >= nCand) return;
     Col match{s_match + threadIdx.x}, mlev{s_mlev + threadIdx.x};
     const int id = (int)candIds[c];
     const int4 b = best[id];
@@ -1619,14 +1631,14 @@ __global__ void k_iota2(int32_t n, uint32_t *repl) {
 
 // Creates the new nodes of each selected plan at ids n + off[c] + k, in
 // ascending library index order, and records the replacement literal.
-__global__ void __launch_bounds__(EVAL_BLOCK) k_build(int32_t n, int32_t nCand, const uint32_t *__restrict__ candIds,
+__global__ void __launch_bounds__(EVAL_BLOCK) k_build(int32_t per, int32_t n, int32_t nCand, const uint32_t *__restrict__ candIds,
                                                        GraphView g, Lib L, const uint32_t *__restrict__ cuts,
                                                        const int4 *__restrict__ best, const uint8_t *__restrict__ state,
                                                        const uint32_t *__restrict__ off, uint32_t *cf0, uint32_t *cf1,
                                                        uint32_t *repl, uint32_t *err, uint32_t *ctag) {
     __shared__ int32_t s_match[NMATCH * EVAL_BLOCK], s_mlev[NMATCH * EVAL_BLOCK];
-    int64_t c = blockIdx.x * (int64_t)EVAL_BLOCK + threadIdx.x;
-    if (c >= nCand || state[c] != ST_SELECTED) return;
+    int64_t c = blockIdx.x * (int64_t)per + threadIdx.x;
+    if ((int32_t)threadIdx.x >= per || c >= nCand || state[c] != ST_SELECTED) return;
     Col match{s_match + threadIdx.x}, mlev{s_mlev + threadIdx.x};
     const int id = (int)candIds[c];
     const int4 b = best[id];
@@ -2387,7 +2399,8 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
             Claims cl{t.get<unsigned long long>(n), t.get<unsigned long long>(n), t.get<unsigned long long>(n),
                       t.get<unsigned long long>(n)};
             if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "rewrite: plan allocation");
-            k_plan<<<blocks(nCand, EVAL_BLOCK), EVAL_BLOCK, 0, st>>>((int32_t)nCand, candIds, gv, L, cuts, best, plans);
+            const int per = plan_lanes((int32_t)nCand);
+            k_plan<<<blocks(nCand, per), EVAL_BLOCK, 0, st>>>(per, (int32_t)nCand, candIds, gv, L, cuts, best, plans);
             k_sel_init<<<blocks(nCand, kBlock), kBlock, 0, st>>>((int32_t)nCand, plans, state);
             GLS_TRY(Fills(ctx)
                         .add(mk, 0, sizeof(uint32_t) * n)
@@ -2439,10 +2452,11 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
             GLS_HIP(ctx, hipMemcpyAsync(tagC, tagR, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st));
         }
         const bool fullStrash = (flags & GLS_RW_FULL_STRASH) != 0;
-        if (nCand > 0 && totalNew + nSel > 0)
-            k_build<<<blocks(nCand, EVAL_BLOCK), EVAL_BLOCK, 0, st>>>(n, (int32_t)nCand, candIds, gv, L, cuts, best,
-                                                                       state, newOff, comb.f0, comb.f1, repl, d_err,
-                                                                       tagC);
+        if (nCand > 0 && totalNew + nSel > 0) {
+            const int per = plan_lanes((int32_t)nCand);
+            k_build<<<blocks(nCand, per), EVAL_BLOCK, 0, st>>>(per, n, (int32_t)nCand, candIds, gv, L, cuts, best, state,
+                                                               newOff, comb.f0, comb.f1, repl, d_err, tagC);
+        }
         k_compose<<<grid_for(N), kBlock, 0, st>>>(n, N, nPIs, g.f0, g.f1, repl, comb.f0, comb.f1);
         if (nPOs > 0) k_compose_pos<<<blocks(nPOs, kBlock), kBlock, 0, st>>>(nPOs, g.pos, repl, comb.pos);
         GLS_HIP(ctx, hipGetLastError());
