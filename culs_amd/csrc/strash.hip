@@ -1428,7 +1428,7 @@ struct WholeArgs {
     uint64_t mask;
     uint32_t *slot, *fold;           // per node: its key's slot, or NO_SLOT and the literal it folds to
     uint32_t *err;
-    unsigned long long *probes;
+    unsigned long long *probes, *used;   // used: slots with a key
 };
 
 __global__ void k_whole_init(int32_t N, uint32_t *rep) {
@@ -1436,18 +1436,18 @@ __global__ void k_whole_init(int32_t N, uint32_t *rep) {
     for (int64_t v = tid; v < N; v += stride) rep[v] = 2u * (uint32_t)v;
 }
 
-// Round, step 1: keys of the live ANDs with a fanin that moved (first: of all).
-// A key over a literal that moved is never formed again, and all nodes of a key
-// move it together, so a slot's least id stays right; the node that loses its
-// place in a slot is looked at again.
-__global__ void k_whole_hash(WholeArgs a, uint32_t first, uint32_t *changed) {
-    uint32_t np = 0;
+// Round, step 1: keys of the live ANDs with a fanin that moved (anew: of all,
+// into an empty table).  A key over a literal that moved is never formed again,
+// and all nodes of a key move it together, so a slot's least id stays right; the
+// node that loses its place in a slot is looked at again.
+__global__ void k_whole_hash(WholeArgs a, uint32_t anew, uint32_t *changed) {
+    uint32_t np = 0, nk = 0;
     int64_t tid = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
     if (tid == 0) *changed = 0;
     for (int64_t v = a.nPIs + 1 + tid; v < a.N; v += stride) {
         if (a.dead[v]) continue;
         const uint32_t x = a.f0[v], y = a.f1[v];
-        if (!first && !a.moved[LID(x)] && !a.moved[LID(y)]) continue;
+        if (!anew && !a.moved[LID(x)] && !a.moved[LID(y)]) continue;
         a.redo[v] = 1;
         uint32_t l0 = a.rep[LID(x)] ^ LC(x), l1 = a.rep[LID(y)] ^ LC(y);
         if (l0 > l1) { const uint32_t t = l0; l0 = l1; l1 = t; }
@@ -1466,6 +1466,7 @@ __global__ void k_whole_hash(WholeArgs a, uint32_t first, uint32_t *changed) {
             __hip_atomic_compare_exchange_strong(&a.key[s], &prev, (unsigned long long)key, __ATOMIC_RELAXED,
                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             ++np;
+            nk += prev == KEY_EMPTY;
             if (prev == KEY_EMPTY || prev == key) { a.slot[v] = (uint32_t)s; break; }
             s = (s + 1) & a.mask;
         }
@@ -1475,6 +1476,7 @@ __global__ void k_whole_hash(WholeArgs a, uint32_t first, uint32_t *changed) {
         ++np;
     }
     block_add_u64(a.probes, np);
+    block_add_u64(a.used, nk);
 }
 
 // Round, step 2: their representatives, one link each.
@@ -1842,7 +1844,7 @@ int dev_strash(gls_ctx *ctx, const DevGraph &in, DevGraph &out, int32_t *depthOu
 //  2. classes of equal ANDs in rounds, each node's representative the least id
 //     of its key's nodes over representatives.  Which nodes are equal does not
 //     depend on the choice, so no levels are needed yet, and ids only fall, so
-//     one table serves all rounds and a round after the first takes only the
+//     a table serves many rounds and a round after the first takes only the
 //     nodes with a fanin that moved;
 //  3. levels: the waves (of the live nodes) and the output's (of the classes),
 //     two sweeps over id order in one launch;
@@ -1871,10 +1873,11 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
         unsigned long long *best = t.get<unsigned long long>(N);
         uint32_t *d_misc = t.get<uint32_t>(16);   // [0] err, [1] largest wave, [2..3] a round changed something,
                                                   // [4] survivors, [5] largest level, [6..7] probes, [8] a path got shorter,
-                                                  // [9] positions, [10] what is left of the cascade
+                                                  // [9] positions, [10] what is left of the cascade, [12..13] used slots
         SweepCtl *ctl = t.get<SweepCtl>(1);
         if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: device allocation failed (n=%d)", N);
         unsigned long long *d_probes = reinterpret_cast<unsigned long long *>(&d_misc[6]);
+        unsigned long long *d_used = reinterpret_cast<unsigned long long *>(&d_misc[12]);
         GLS_TRY(Fills(ctx)
                     .add(ref, 0, sizeof(uint32_t) * N)
                     .add(dead, 0, N)
@@ -1914,15 +1917,22 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
         unsigned long long *key = t.get<unsigned long long>(cap);
         uint32_t *least = t.get<uint32_t>(cap);
         if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: table");
-        GLS_TRY(Fills(ctx).add(key, 0xFF, sizeof(unsigned long long) * cap).add(least, 0xFF, sizeof(uint32_t) * cap).run());
+        // A round claims a slot for each new key and gives none back: before it
+        // could take the table beyond seven eighths the table is emptied and every
+        // node hashed anew.  A class whose least id falls in every round gives all
+        // its fanouts a new key each time, and a scan of a full table is as long
+        // as the table.
+        const uint64_t room = cap - cap / 8;
+        const uint32_t perLook = 2 * nLive <= room ? 2u : 1u;     // most graphs take two or three rounds
+        if (nLive > room) return fallback();
+        uint64_t used = room;
         k_whole_init<<<gN, kBlock, 0, st>>>(N, rep);
-        const WholeArgs wa{N, nPIs, in.f0, in.f1, dead, rep, moved, redo, key, least, cap - 1, slot, fold, &d_misc[0], d_probes};
+        const WholeArgs wa{N, nPIs, in.f0, in.f1, dead, rep, moved, redo, key, least, cap - 1, slot, fold, &d_misc[0], d_probes, d_used};
         uint32_t roundLimit = allRounds ? kRwRoundLimit : N >= kRwLarge ? kRwManyRounds : kRwFewRounds;
         const int64_t narrowDepth = (N + (int64_t)tuning_for(ctx, N).rw_sweep_width - 1) / tuning_for(ctx, N).rw_sweep_width;
         const LevelSweep waves{nPos, fa, fb, levPos, &d_misc[1]}, classes{nPos, ca, cb, classLev, &d_misc[5]};
         bool swept = false;
         uint32_t r = 0;
-        // two rounds per look at them: most graphs take two or three
         for (bool done = nLive == 0; !done;) {
             if (r >= roundLimit) {
                 if (roundLimit != kRwManyRounds) return fallback();
@@ -1933,16 +1943,24 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
                 swept = true;
                 roundLimit = kRwRoundLimit;
             }
-            for (uint32_t i = 0; i < 2; i++) {
-                k_whole_hash<<<gN, kBlock, 0, st>>>(wa, r + i == 0 ? 1u : 0u, &d_misc[2 + i]);
+            const bool anew = used + perLook * nLive > room;
+            if (anew)
+                GLS_TRY(Fills(ctx)
+                            .add(key, 0xFF, sizeof(unsigned long long) * cap)
+                            .add(least, 0xFF, sizeof(uint32_t) * cap)
+                            .add(d_used, 0, sizeof(unsigned long long))
+                            .run());
+            for (uint32_t i = 0; i < perLook; i++) {
+                k_whole_hash<<<gN, kBlock, 0, st>>>(wa, anew && i == 0 ? 1u : 0u, &d_misc[2 + i]);
                 k_whole_link<<<gN, kBlock, 0, st>>>(wa);
                 k_whole_follow<<<gN, kBlock, 0, st>>>(wa, &d_misc[2 + i]);
             }
             GLS_HIP(ctx, hipGetLastError());
-            GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(uint32_t) * 4, hipMemcpyDeviceToHost));
+            GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
             if (misc[0]) return fallback();
-            done = misc[2] == 0 || misc[3] == 0;
-            r += misc[2] == 0 ? 1u : 2u;
+            used = (uint64_t)misc[12] | (uint64_t)misc[13] << 32;
+            done = misc[2] == 0 || (perLook == 2 && misc[3] == 0);
+            r += misc[2] == 0 ? 1u : perLook;
         }
         // 3. levels
         k_whole_classpos<<<gN, kBlock, 0, st>>>(N, nPIs, in.f0, in.f1, dead, rep, posOf, ca, cb, 0u);
