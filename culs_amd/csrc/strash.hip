@@ -958,14 +958,21 @@ constexpr uint32_t SW_SPIN_LIMIT = 1u << 22;
 // duplicates one level further up, so a graph that holds the same deep logic
 // twice needs one per level; most graphs take one to three.  A rewrite takes
 // many where its graph is narrow, else few.  A whole graph's round after the
-// first costs 15 us and 4 us per million objects, its wave sweep 0.2 ms more than
-// the rounds' other work at 20k objects, 1.7 ms at a million on wide levels: few
-// below 2^18 objects, many from there.  Where the levels are narrow the wave
-// sweep costs 100 ms more at 10M objects: those that are still at it go on to the
-// limit (of 120 raw deep AIGs of 10M ANDs 108 took two or three, one 44).
-constexpr uint32_t kRwRoundLimit = 4096, kRwManyRounds = 128, kRwFewRounds = 5;
-// objects from which a whole graph may take many rounds
+// first costs 15 us and 4 us per million objects (20 us where it finds a level of
+// duplicates): four rounds below 2^18 objects, where the wave sweep costs 0.2 ms
+// more than they do, twelve from there, and then as many as it takes where the
+// levels are narrow, since the wave sweep costs 100 ms more at 10M objects (of
+// 120 raw deep AIGs of 10M ANDs 108 took two or three, two 14 and 16, one 44).
+// Graphs that hold random logic twice, ms, against the wave sweep after a sweep
+// of all levels (without one below 2^18): 1k ANDs 0.42 / 0.70, the 64-bit
+// multiplier 2.01 / 2.05, the 110-bit one 4.26 / 4.20, 150k of 7700 objects per
+// level 2.09 / 2.17, of 1580 2.97 / 3.40, 4M of 29000 19.8 / 30.7; with 128 rounds
+// in the place of twelve and the levels swept in whole, the last three 1.52 (it
+// needs 40), 5.08 and 45.1.
+constexpr uint32_t kRwRoundLimit = 4096, kRwFewRounds = 5;
+// a whole graph's, two per look at them: from 2^18 objects on, and below
 constexpr int32_t kRwLarge = 1 << 18;
+constexpr uint32_t kWholeLargeRounds = 12, kWholeSmallRounds = 4;
 // The line for a rewrite of one AIG lies at this many times rw_sweep_width
 // objects per level (8192 by default).  Incremental against wave sweep, ms:
 // 1248 objects per level 1.6 / 9.6, 2309 1.7 / 6.2, 4294 1.6 / 4.2, 6640 3.9 /
@@ -1928,18 +1935,25 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
         uint64_t used = room;
         k_whole_init<<<gN, kBlock, 0, st>>>(N, rep);
         const WholeArgs wa{N, nPIs, in.f0, in.f1, dead, rep, moved, redo, key, least, cap - 1, slot, fold, &d_misc[0], d_probes, d_used};
-        uint32_t roundLimit = allRounds ? kRwRoundLimit : N >= kRwLarge ? kRwManyRounds : kRwFewRounds;
+        uint32_t roundLimit = allRounds ? kRwRoundLimit : N >= kRwLarge ? kWholeLargeRounds : kWholeSmallRounds;
         const int64_t narrowDepth = (N + (int64_t)tuning_for(ctx, N).rw_sweep_width - 1) / tuning_for(ctx, N).rw_sweep_width;
         const LevelSweep waves{nPos, fa, fb, levPos, &d_misc[1]}, classes{nPos, ca, cb, classLev, &d_misc[5]};
         bool swept = false;
         uint32_t r = 0;
         for (bool done = nLive == 0; !done;) {
             if (r >= roundLimit) {
-                if (roundLimit != kRwManyRounds) return fallback();
-                k_level_sweep<<<1, SW_WG, 0, st>>>(waves, waves, &d_misc[0]);
-                GLS_HIP(ctx, hipGetLastError());
-                GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
-                if (misc[0] || (int64_t)misc[1] < narrowDepth) return fallback();
+                if (roundLimit != kWholeLargeRounds) return fallback();
+                // narrow levels?  A sweep of the first eighth tells most wide
+                // graphs for an eighth of the time (twice its share of the depth
+                // is allowed for)
+                LevelSweep part = waves;
+                for (uint32_t share = 8; share != 0; share = share == 8 ? 1 : 0) {
+                    part.nPos = nPos / share;
+                    k_level_sweep<<<1, SW_WG, 0, st>>>(part, part, &d_misc[0]);
+                    GLS_HIP(ctx, hipGetLastError());
+                    GLS_TRY(stream_copy(ctx, misc, d_misc, sizeof(misc), hipMemcpyDeviceToHost));
+                    if (misc[0] || (int64_t)misc[1] * (share == 8 ? 16 : 1) < narrowDepth) return fallback();
+                }
                 swept = true;
                 roundLimit = kRwRoundLimit;
             }

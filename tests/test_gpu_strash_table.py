@@ -1,6 +1,7 @@
 """Strash of graphs whose classes take a new least id in round after round, so
 that every round brings as many new keys as there are ANDs: the table of keys
-is emptied before it fills up.  Array for array against the oracle."""
+is emptied before it fills up; and of graphs that need more rounds than are worth
+it.  Array for array against the oracle."""
 import sys
 
 import numpy as np
@@ -42,14 +43,12 @@ def falling(drops, fanouts):
     return nPIs, np.array(f0, np.uint32), np.array(f1, np.uint32), np.array(pos, np.uint32)
 
 
-# (the second: at least 2^18 objects, as many as 128 rounds without being asked for)
-@pytest.mark.parametrize("drops,fanouts,schedule", [(40, 2000, culs_amd.GLS_ST_LEVELS), (30, 180_000, 0)])
-def test_keys_of_many_rounds(gpu_ctx, drops, fanouts, schedule):
-    print("strash table:", drops, fanouts, schedule)
+@pytest.mark.parametrize("drops,fanouts", [(40, 2000), (30, 180_000)])
+def test_keys_of_many_rounds(gpu_ctx, drops, fanouts):
+    print("strash table:", drops, fanouts)
     sys.stdout.flush()
     g = falling(drops, fanouts)
-    assert schedule or len(g[1]) >= 1 << 18
-    a = gpu_ctx.from_arrays(*g).strash(schedule=schedule)
+    a = gpu_ctx.from_arrays(*g).strash(schedule=culs_amd.GLS_ST_LEVELS)
     op = a.last_op()
     print("final_strash", op["final_strash"], "rounds", op["strash_rounds"], "probes", op["hash_probes"])
     want, depth = O.strash(*g)
@@ -58,3 +57,22 @@ def test_keys_of_many_rounds(gpu_ctx, drops, fanouts, schedule):
     # linear probing at seven eighths takes 32.5 probes for a new key on
     # average, and one more counts the least id; at most every AND per round
     assert op["hash_probes"] <= 34 * op["strash_rounds"] * (len(g[1]) - g[0] - 1)
+
+
+def test_wide_graph_of_many_rounds(gpu_ctx):
+    """At least 2^18 objects, the same logic twice on wide levels: after a few
+    rounds the wave sweep is the faster way, and a part of the levels tells."""
+    print("strash, wide levels, many rounds")
+    sys.stdout.flush()
+    nPIs, f0, f1, pos = gpu_ctx.gen_random(1000, 150_000, 50, 30_000, 4).arrays()
+    up = 2 * (len(f0) - nPIs - 1)
+
+    def copy(x):
+        return np.where(x >> 1 > nPIs, x + up, x).astype(np.uint32)
+
+    g = (nPIs, np.concatenate([f0, copy(f0[nPIs + 1:])]), np.concatenate([f1, copy(f1[nPIs + 1:])]),
+         np.concatenate([pos, copy(pos)]))
+    a = gpu_ctx.from_arrays(*g).strash()
+    want, depth = O.strash(*g)
+    assert all(np.array_equal(x, y) for x, y in zip(a.arrays(), want)) and a.stats().levels == depth
+    assert a.last_op()["final_strash"] == 2
