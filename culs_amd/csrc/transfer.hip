@@ -231,7 +231,7 @@ int dev_graph_copy(gls_ctx *ctx, const DevGraph &src, const DevGraph &dst) {
 // STAGE_SMALL bytes: one kernel into the staging and one copy out of it;
 // more: pieces of STAGE_SLOT bytes on up to four threads, each with its part of
 // the staging.  Through pageable copies into arrays of the handle first, 92 MB
-// took 20 ms.
+// took 20 ms.  Without pinned memory to be had they are what is left.
 int dev_graph_fetch(gls_ctx *ctx, const DevGraph &g, uint32_t *f0, uint32_t *f1, uint32_t *pos, int32_t conv) {
     const size_t n = g.nObjs, words = 2 * n + g.nPOs;
     if (4 * words <= STAGE_SMALL && mail_ready(ctx)) {
@@ -264,7 +264,14 @@ int dev_graph_fetch(gls_ctx *ctx, const DevGraph &g, uint32_t *f0, uint32_t *f1,
     add(f1, g.f1, n);
     add(pos, g.pos, g.nPOs);
     uint8_t *stage = stage_of(ctx, STAGE_SLOT * STAGE_SLOTS);
-    if (!stage) return gls_fail(ctx, GLS_ERR_NOMEM, "pinned staging");
+    if (!stage) {
+        for (const Chunk &c : chunks)
+            GLS_HIP(ctx, hipMemcpyAsync(c.dst, c.src, sizeof(uint32_t) * c.words, hipMemcpyDeviceToHost, ctx->stream));
+        GLS_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (conv == GLS_LIT_CULS)
+            for (const Chunk &c : chunks) take(c.dst, c.dst, c.words, conv);
+        return GLS_OK;
+    }
     const int workers = (int)std::min<size_t>(STAGE_SLOTS, chunks.size());
     std::atomic<int> bad{0};
     auto work = [&](int w) {
