@@ -148,6 +148,20 @@ uint8_t *stage_of(gls_ctx *ctx, size_t bytes) {
     return ctx->stage;
 }
 
+// The context's device is the calling thread's current one while this lives:
+// a program may copy or fetch on a thread that works on another device.
+struct OnDevice {
+    int was = -1, now;
+    explicit OnDevice(int device) : now(device) {
+        if (hipGetDevice(&was) != hipSuccess) was = -1;
+        if (was != now) (void)hipSetDevice(now);
+    }
+    ~OnDevice() {
+        if (was >= 0 && was != now) (void)hipSetDevice(was);
+    }
+    OnDevice(const OnDevice &) = delete;
+};
+
 uint32_t lit_in(uint32_t l, int32_t conv) { return (conv == GLS_LIT_CULS && l < 2) ? 1u - l : l; }
 
 void take(uint32_t *dst, const uint32_t *src, size_t n, int32_t conv) {
@@ -222,6 +236,7 @@ int Fills::run() {
 }
 
 int dev_graph_copy(gls_ctx *ctx, const DevGraph &src, const DevGraph &dst) {
+    const OnDevice on(ctx->device);
     k_copy_graph<<<grid_of(((size_t)std::max(src.nObjs, src.nPOs) + 3) / 4), 256, 0, ctx->stream>>>(src, dst);
     GLS_HIP(ctx, hipGetLastError());
     return GLS_OK;
@@ -233,6 +248,7 @@ int dev_graph_copy(gls_ctx *ctx, const DevGraph &src, const DevGraph &dst) {
 // the staging.  Through pageable copies into arrays of the handle first, 92 MB
 // took 20 ms.  Without pinned memory to be had they are what is left.
 int dev_graph_fetch(gls_ctx *ctx, const DevGraph &g, uint32_t *f0, uint32_t *f1, uint32_t *pos, int32_t conv) {
+    const OnDevice on(ctx->device);
     const size_t n = g.nObjs, words = 2 * n + g.nPOs;
     if (4 * words <= STAGE_SMALL && mail_ready(ctx)) {
         uint32_t *stage = reinterpret_cast<uint32_t *>(stage_of(ctx, STAGE_SMALL));

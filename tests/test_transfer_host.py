@@ -1,8 +1,9 @@
 """The host side of the array fetch (culs_amd/csrc/transfer.hip), compiled for
 the host and linked with a stand-in for the HIP runtime whose device memory is
-the host's: what the fetch does where pinned memory cannot be had.  Sizes on
-both sides of the staging (2 MiB in all) and of its pieces (4 MiB of an array),
-both literal conventions, arrays left out."""
+the host's: what the fetch does where pinned memory cannot be had, and on which
+device it and the copy of a graph run.  Sizes on both sides of the staging (2 MiB
+in all) and of its pieces (4 MiB of an array), both literal conventions, arrays
+left out."""
 import ctypes
 import os
 import subprocess
@@ -16,13 +17,19 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 RUNTIME = r"""
 #include "gls_internal.h"
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
 
 static bool g_pinned;
+static thread_local int t_device;          // the thread's current device
+static std::atomic<int> g_elsewhere;       // allocations, launches and events on another one than the context's
+constexpr int DEVICE = 3;
+static void here() { if (t_device != DEVICE) g_elsewhere++; }
 
 extern "C" {
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+    here();
     *p = g_pinned ? malloc(n) : nullptr;
     return g_pinned ? hipSuccess : hipErrorOutOfMemory;
 }
@@ -31,12 +38,13 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipSt
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "stand-in"; }
-hipError_t hipSetDevice(int) { return hipSuccess; }
-hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { *e = (hipEvent_t)1; return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = t_device; return hipSuccess; }
+hipError_t hipSetDevice(int d) { t_device = d; return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { here(); *e = (hipEvent_t)1; return hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { return hipErrorUnknown; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { here(); return hipErrorUnknown; }
 hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
 hipError_t __hipPopCallConfiguration(dim3 *, dim3 *, size_t *, hipStream_t *) { return hipSuccess; }
 void **__hipRegisterFatBinary(const void *) { static void *h; return &h; }
@@ -47,7 +55,7 @@ int run_fetch(int pinned, int32_t nPIs, int32_t n, int32_t nPOs, uint32_t *g0, u
               uint32_t *f1, uint32_t *pos, int32_t conv) {
     g_pinned = pinned != 0;
     gls_ctx ctx;
-    ctx.device = 0;
+    ctx.device = DEVICE;
     DevGraph g;
     g.nObjs = n;
     g.nPIs = nPIs;
@@ -58,6 +66,29 @@ int run_fetch(int pinned, int32_t nPIs, int32_t n, int32_t nPOs, uint32_t *g0, u
     const int rc = dev_graph_fetch(&ctx, g, f0, f1, pos, conv);
     transfer_free(&ctx);
     return rc;
+}
+
+// a copy and fetches of all sizes by a thread on `device`; returns the device that
+// it is left on, or -1 if something ran elsewhere
+int run_on(int device, int32_t n, uint32_t *words, uint32_t *out) {
+    g_elsewhere = 0;
+    t_device = device;
+    gls_ctx ctx;
+    ctx.device = DEVICE;
+    DevGraph g;
+    g.nObjs = n;
+    g.nPIs = 1;
+    g.nPOs = 0;
+    g.f0 = g.f1 = g.level = g.pos = words;
+    for (int pinned = 0; pinned < 2; pinned++) {
+        g_pinned = pinned != 0;
+        (void)dev_graph_copy(&ctx, g, g);
+        (void)dev_graph_fetch(&ctx, g, out, nullptr, nullptr, 0);
+    }
+    const int left = t_device;
+    t_device = DEVICE;
+    transfer_free(&ctx);
+    return g_elsewhere ? -1 : left;
 }
 }
 int gls_fail(gls_ctx *, int code, const char *, ...) { return code; }
@@ -103,3 +134,10 @@ def test_fetch(host, pinned, n, nPOs, conv):
         rc = host.run_fetch(int(pinned), 3, n, nPOs, *map(ptr, graph), *map(ptr, out), conv)
         assert rc == 0
         assert all(o is None or np.array_equal(o, w) for o, w in zip(out, want))
+
+
+@pytest.mark.parametrize("n", [100, 3_000_000])
+@pytest.mark.parametrize("device", [0, 3, 5])
+def test_thread_on_another_device(host, n, device):
+    words, out = np.zeros(n, np.uint32), np.zeros(n, np.uint32)
+    assert host.run_on(device, n, ptr(words), ptr(out)) == device
