@@ -622,7 +622,7 @@ __device__ __forceinline__ unsigned long long input_sig(const RecArgs &r, uint32
 
 // ---- one workgroup per segment, levels within its LDS
 constexpr uint32_t LT_INPUTS = 4096;      // inputs of a level
-constexpr uint32_t LT_COVERS = 2048;      // covers of a level
+constexpr uint32_t LT_COVERS = BAL_LDS_COVERS;   // covers of a level
 constexpr uint32_t LT_NEW = 3072;         // ANDs that a level can create
 constexpr uint32_t LT_HASH = 4096;        // entries of the level's own node table
 constexpr uint32_t LQ_IN = LT_INPUTS / BAL_WG, LQ_COV = LT_COVERS / BAL_WG, LQ_NEW = LT_NEW / BAL_WG;

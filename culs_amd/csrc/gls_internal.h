@@ -69,6 +69,7 @@ struct gls_ctx {
     // entry point chose for the pass it runs (TuneScope), else null
     gls_tuning tune[64];
     const gls_tuning *active = nullptr;
+    uint64_t wave_sweeps = 0;    // runs of dev_strash: the autotuner sees whether its settings had a part
     // pinned memory (transfer.hip): small results and their sequence number;
     // arrays on their way to the caller
     uint8_t *mail = nullptr, *stage = nullptr;
@@ -76,6 +77,9 @@ struct gls_ctx {
     size_t stage_bytes = 0;
 };
 
+// covers of a level that the persistent balance workgroup has room for:
+// balance_narrow_max beyond it changes nothing
+constexpr int32_t BAL_LDS_COVERS = 2048;
 // the defaults of gls_tuning
 constexpr gls_tuning kTuningDefault{2048, 1024, 4, 4, 4096, 3};
 int tuning_bucket(int64_t objects);

@@ -1677,6 +1677,7 @@ __global__ void __launch_bounds__(kBlock) k_tag_depth(int32_t n, int32_t nPIs, c
 
 int dev_strash(gls_ctx *ctx, const DevGraph &in, DevGraph &out, int32_t *depthOut, gls_op_info *info,
                const uint32_t *tagIn, uint32_t **tagOut, uint32_t *tagDepth) {
+    ctx->wave_sweeps++;
     const int32_t n = in.nObjs, nPIs = in.nPIs, nPOs = in.nPOs;
     hipStream_t st = ctx->stream;
     Tmp t{ctx};

@@ -237,14 +237,14 @@ int gls_batch_balance(gls_ctx *ctx, gls_aig **aigs, int32_t count, int32_t sort_
  *   rw_sweep_width: rw finishes with the incremental strash while the input
  *     has at most eight times this many objects per level on average (the
  *     arena of a batch: this many), else with the wave sweep (default 1024);
- *   strash_table_factor: the strash table has at least this many slots per
- *     object, a power of two, 4 or 8 (default 4);
- *   strash_wave_batch: wide strash waves launched per host check, 1-64
- *     (default 4);
+ *   strash_table_factor: the table of a strash by the wave sweep has at least
+ *     this many slots per object, a power of two, 4 or 8 (default 4);
+ *   strash_wave_batch: wide waves of the wave sweep launched per host check,
+ *     1-64 (default 4);
  *   balance_narrow_max: balance levels of at most this many covers are
  *     rebuilt in one persistent workgroup where they fit its LDS (2048 covers,
  *     4096 inputs, 3072 possible ANDs), others by grid-wide phase kernels
- *     (default 4096);
+ *     (default 4096; from 2048 on it changes nothing);
  *   cut_levels: levels per cut launch of the planned schedule
  *     (GLS_RW_PLAN_CUTS, currently disabled), 1-6 (default 3). */
 typedef struct {
@@ -260,7 +260,8 @@ int gls_ctx_set_tuning(gls_ctx *ctx, int64_t objects, const gls_tuning *t);
  * setting at a time from the current ones (coordinate descent, `reps` runs
  * each, the fastest kept), stores the best for the bucket of the inputs'
  * total objects and returns it with its time and the time of the settings it
- * started from.  The inputs are not changed. */
+ * started from.  Settings that had no part in the pass (the wave sweep's where
+ * none ran) are left as they are.  The inputs are not changed. */
 #define GLS_TUNE_RW 0
 #define GLS_TUNE_RWZ 1
 #define GLS_TUNE_STRASH 2
