@@ -1628,8 +1628,7 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
     const uint32_t batchLimit = tagged ? 0xFFFFFFFFu : (uint32_t)BAL_BATCH;
 
     // ---- phase 2: reconstruction
-    uint64_t cap = 1024;
-    while (cap < 4ull * ((uint64_t)poolUsed + 16)) cap <<= 1;       // a cover of k inputs creates at most k - 1 nodes
+    const uint64_t cap = balance_table_slots(poolUsed);
     const size_t idEnd = (size_t)nPIs + 1 + poolUsed;
     unsigned long long *tabK = t.get<unsigned long long>(cap), *tabV = t.get<unsigned long long>(cap), *newSig = t.get<unsigned long long>(n);
     uint32_t *cf0 = t.get<uint32_t>(idEnd), *cf1 = t.get<uint32_t>(idEnd);

@@ -80,6 +80,14 @@ struct gls_ctx {
 // covers of a level that the persistent balance workgroup has room for:
 // balance_narrow_max beyond it changes nothing
 constexpr int32_t BAL_LDS_COVERS = 2048;
+// Slots of the balance's table for covers of so many inputs (a cover of k creates
+// at most k - 1 nodes): at most a quarter full, half from 2^29 inputs on, where
+// twice the room is tens of GiB and slot 2^32 - 1 means none.
+inline uint64_t balance_table_slots(uint64_t inputs) {
+    uint64_t cap = 1024;
+    while (cap < 4 * (inputs + 16) && (cap < (1ull << 31) || cap < 2 * (inputs + 16))) cap <<= 1;
+    return cap;
+}
 // the defaults of gls_tuning
 constexpr gls_tuning kTuningDefault{2048, 1024, 4, 4, 4096, 3};
 int tuning_bucket(int64_t objects);
