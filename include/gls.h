@@ -203,6 +203,9 @@ int gls_rewrite(gls_aig *aig, int32_t use_zeros, int32_t flags);
  * level, equal levels in the order of thrust::shuffle (thrust::seq,
  * default_random_engine seeded with the cover's index in its batch,
  * balance.cu:301, 404-411), thrust's algorithm as in rocThrust.
+ * The shuffle starts from the order in which the fanins give a cover's inputs,
+ * and a handle holds an AND's fanins in ascending order, whatever order they
+ * were given in.
  * update_level = 1 strashes afterwards as the `b` command does
  * (command_manager.cpp:77); with 0 the result keeps its balance numbering
  * and its depth is unknown (levels = -1), as after `gb`. */
