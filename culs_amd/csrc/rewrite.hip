@@ -185,19 +185,6 @@ __device__ __forceinline__ uint32_t min_quads(uint32_t v) {
     return min((uint32_t)r[0], (uint32_t)r[1]);
 }
 
-// Bits 4 k .. 4 k + 3 of a table over the variables at the set bits of
-// `phase`, from the table t over variables 0, 1, ..: entry b of the result is
-// entry pext(b, phase) of t.  The two high index bits (k) give a shift of t,
-// the two low ones spread at most four of its bits over the nibble.
-__device__ __forceinline__ uint32_t tt_nibble(uint32_t t, uint32_t phase, uint32_t ext) {
-    const uint32_t lo = phase & 3u, sh8 = lo << 3;
-    const uint32_t px = (ext >> ((phase >> 1) & 6u)) & 3u;
-    const uint32_t pc = (0x94u >> (lo << 1)) & 3u;                   // bits set in lo
-    const uint32_t x = (t >> (px << pc)) & 15u;
-    // lo 0: bit 0 to all four; 1: bits 1, 0 twice; 2: bits 0 and 1 doubled; 3: as they are
-    return (x & (0x0F010301u >> sh8)) * ((0x0103050Fu >> sh8) & 15u) + (x & (0x00020000u >> sh8)) * 6u;
-}
-
 // Fence-free record format of the dataflow schedule: every 64-bit word of a
 // slot carries a valid bit, so a reader polls the words themselves with
 // relaxed device-scope atomics and needs no ordering between words.
@@ -700,7 +687,7 @@ __global__ void __launch_bounds__(CUT3_BLOCK) k_cuts_triple(int32_t s0_, int32_t
 // price of larger cones.  (Eight wavefronts per workgroup, one per lowest-level
 // node, put two of a workgroup's own wavefronts on every SIMD and measured
 // 17.9 us per launch against 10.9 for three levels.)
-constexpr int CUT4_BLOCK = 256;   // (measured 159.5 ms per pass on the 10M AIG against 138.1 for three levels)
+constexpr int CUT4_BLOCK = 256;   // (cuts of the 10M AIG 133.5 ms, 111.6 with three levels)
 
 // the record of fanin x for a cone node: its LDS slot if the cone lists it,
 // else the global records (x below the launch)
@@ -1018,11 +1005,10 @@ struct GraphView {
 };
 
 // per-thread column of an LDS array laid out [j][lane]
-template <typename T> struct ColT {
-    T *p;
-    __device__ __forceinline__ T &operator[](int j) const { return p[j * EVAL_BLOCK]; }
+struct Col {
+    int32_t *p;
+    __device__ __forceinline__ int32_t &operator[](int j) const { return p[j * EVAL_BLOCK]; }
 };
-using Col = ColT<int32_t>;
 
 struct Mffc {
     int size;
@@ -1117,12 +1103,8 @@ __device__ __forceinline__ int table_lookup(const GraphView &g, int in0, int in1
 }
 
 // library matching of one cut (rewrite.cu:391-418); returns the class
-// LV: storage of the structure nodes' levels, uint16_t when every level is
-// below 65535 (more workgroups fit a CU's LDS), else int32_t; the values are
-// the same either way.
-template <typename LV>
 __device__ int match_cut(const GraphView &g, const Lib &L, int id, uint32_t tt, const int *leaves,
-                         const Mffc &t, Col match, ColT<LV> mlev, uint32_t &isC, uint64_t &matched) {
+                         const Mffc &t, Col match, Col mlev, uint32_t &isC, uint64_t &matched) {
     uint32_t w = L.npn[tt];
     int uPhase = w & 31, perm = (w >> 5) & 31, cls = (w >> 10) & 255;
     const uint8_t *pp = L.perms4 + 4 * perm;
@@ -1136,7 +1118,7 @@ __device__ int match_cut(const GraphView &g, const Lib &L, int id, uint32_t tt, 
         const int q = pp[j];
         const int leaf = q == 0 ? leaves[0] : q == 1 ? leaves[1] : q == 2 ? leaves[2] : leaves[3];
         match[j] = leaf;
-        mlev[j] = (LV)g.level[leaf];
+        mlev[j] = (int)g.level[leaf];
         if ((uPhase >> j) & 1) isC |= 1u << j;
     }
     const int nn = lib_nn(L, cls);
@@ -1144,7 +1126,7 @@ __device__ int match_cut(const GraphView &g, const Lib &L, int id, uint32_t tt, 
         uint32_t wd = lib_word(L, cls, j);
         int a = wd & 63, b = (wd >> 6) & 63, ca = (wd >> 12) & 1, cb = (wd >> 13) & 1;
         int num = j + 4;
-        const int la = (int)mlev[a], lb = (int)mlev[b];
+        const int la = mlev[a], lb = mlev[b];
         int lev = 1 + (la > lb ? la : lb);
         const int ma = match[a], mb = match[b];
         int found = -1;
@@ -1156,7 +1138,7 @@ __device__ int match_cut(const GraphView &g, const Lib &L, int id, uint32_t tt, 
             }
         }
         match[num] = found;
-        mlev[num] = (LV)lev;
+        mlev[num] = lev;
         if (found != -1) matched |= 1ull << num;
     }
     return cls;

@@ -1880,7 +1880,7 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
         uint32_t *rep = t.get<uint32_t>(N), *rep2 = t.get<uint32_t>(N), *slot = t.get<uint32_t>(N), *fold = t.get<uint32_t>(N);
         unsigned long long *best = t.get<unsigned long long>(N);
         uint32_t *d_misc = t.get<uint32_t>(16);   // [0] err, [1] largest wave, [2..3] a round changed something,
-                                                  // [4] survivors, [5] largest level, [6..7] probes, [8] a path got shorter,
+                                                  // [4] survivors, [5] largest level, [6..7] probes,
                                                   // [9] positions, [10] what is left of the cascade, [12..13] used slots
         SweepCtl *ctl = t.get<SweepCtl>(1);
         if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "strash: device allocation failed (n=%d)", N);
@@ -1985,7 +1985,6 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
         k_whole_waves<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep, posOf, levPos, wave, best);
         k_whole_rep<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep, posOf, wave, best, classLev, rep2, level);
         if (tagIn && tagDepth) k_tag_depth<<<tag_grid(N), kBlock, 0, st>>>(N, nPIs, wave, tagIn, tagDepth);
-        k_rw_shorter<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep2, wave, &d_misc[8]);
         k_rw_survivors<<<gN, kBlock, 0, st>>>(N, nPIs, dead, rep2, flag);
         GLS_HIP(ctx, hipGetLastError());
         GLS_TRY(select_ids(ctx, t, N, flag, survIds, &d_misc[4]));

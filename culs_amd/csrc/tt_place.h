@@ -21,6 +21,10 @@
 // Entry of a phase: up to three swaps in placement order, 20 bits each (the
 // 16-bit mask of the lower entries, then d in 4 bits); an unused swap has
 // mask 0 and changes nothing.
+//
+// The cut kernels reduce with these swaps and place with tt_nibble, which gives
+// each of four lanes its part of the table; tt_place_stretch is the same table in
+// one piece.
 #pragma once
 
 #include <cstdint>
@@ -60,6 +64,20 @@ __host__ __device__ __forceinline__ uint32_t tt_place_stretch(uint32_t t, uint64
     t = tt_delta_swap(t, e, 0);
     t = tt_delta_swap(t, e, 1);
     return tt_delta_swap(t, e, 2);
+}
+
+// Bits 4 k .. 4 k + 3 of a table over the variables at the set bits of
+// `phase`, from the table t over variables 0, 1, ..: entry b of the result is
+// entry pext(b, phase) of t.  The two high index bits (k) give a shift of t,
+// the two low ones spread at most four of its bits over the nibble.  ext:
+// pext(k, 0..3), two bits each.
+__host__ __device__ __forceinline__ uint32_t tt_nibble(uint32_t t, uint32_t phase, uint32_t ext) {
+    const uint32_t lo = phase & 3u, sh8 = lo << 3;
+    const uint32_t px = (ext >> ((phase >> 1) & 6u)) & 3u;
+    const uint32_t pc = (0x94u >> (lo << 1)) & 3u;                   // bits set in lo
+    const uint32_t x = (t >> (px << pc)) & 15u;
+    // lo 0: bit 0 to all four; 1: bits 1, 0 twice; 2: bits 0 and 1 doubled; 3: as they are
+    return (x & (0x0F010301u >> sh8)) * ((0x0103050Fu >> sh8) & 15u) + (x & (0x00020000u >> sh8)) * 6u;
 }
 
 // the variables at the set bits of the entry's phase moved down to 0..k-1
