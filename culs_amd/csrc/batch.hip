@@ -56,15 +56,18 @@ __device__ __forceinline__ uint32_t to_union(uint32_t lit, const Member &m, int3
 
 __global__ void k_pack_ands(int64_t A, int count, int32_t P, const Member *__restrict__ mem,
                             const int32_t *__restrict__ andOffs, uint32_t *uf0, uint32_t *uf1, uint32_t *ulevel,
-                            uint32_t *utag) {
+                            uint32_t *utag, int32_t *constRef) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < A; i += stride) {
         const int k = find_member(andOffs, count, i);
         const Member &m = mem[k];
         const int32_t v = m.nPIs + 1 + (int32_t)(i - m.andOff);
         const int64_t u = 1 + P + i;
-        uf0[u] = to_union(m.f0[v], m, P);
-        uf1[u] = to_union(m.f1[v], m, P);
+        const uint32_t a = to_union(m.f0[v], m, P), b = to_union(m.f1[v], m, P);
+        uf0[u] = a;
+        uf1[u] = b;
+        const int32_t refs = (a < 2u) + (b < 2u);
+        if (refs && constRef) atomicAdd(&constRef[k], refs);
         ulevel[u] = m.level ? m.level[v] : 0u;
         utag[u] = (uint32_t)k;
     }
@@ -82,12 +85,14 @@ __global__ void k_pack_pis(int32_t P, int count, const int32_t *__restrict__ piO
 }
 
 __global__ void k_pack_pos(int64_t O, int count, int32_t P, const Member *__restrict__ mem,
-                           const int32_t *__restrict__ poOffs, uint32_t *upos) {
+                           const int32_t *__restrict__ poOffs, uint32_t *upos, int32_t *constRef) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < O; j += stride) {
         const int k = find_member(poOffs, count, j);
         const Member &m = mem[k];
-        upos[j] = to_union(m.pos[j - m.poOff], m, P);
+        const uint32_t l = to_union(m.pos[j - m.poOff], m, P);
+        upos[j] = l;
+        if (l < 2u && constRef) atomicAdd(&constRef[k], 1);
     }
 }
 
@@ -245,7 +250,10 @@ int batch_pass(gls_ctx *ctx, gls_aig **aigs, int32_t count, Pass pass, int32_t u
     Member *d_mem = pb.get<Member>(count);
     int32_t *d_piOffs = pb.get<int32_t>(count), *d_andOffs = pb.get<int32_t>(count), *d_poOffs = pb.get<int32_t>(count);
     uint32_t *utag = pb.get<uint32_t>(N);
-    if (!d_mem || !d_piOffs || !d_andOffs || !d_poOffs || !utag) return gls_fail(ctx, GLS_ERR_NOMEM, "batch: tables");
+    uint32_t *dep = pb.get<uint32_t>(count);        // per-member depth, as the pass alone reports it
+    // rw: per-member references to the constant
+    int32_t *constRef = pass == Pass::Rewrite ? pb.get<int32_t>(count) : nullptr;
+    if (!d_mem || !d_piOffs || !d_andOffs || !d_poOffs || !utag || !dep || (pass == Pass::Rewrite && !constRef)) return gls_fail(ctx, GLS_ERR_NOMEM, "batch: tables");
     GLS_TRY(stream_copy(ctx, d_mem, hm.data(), sizeof(Member) * count, hipMemcpyHostToDevice));
     GLS_TRY(stream_copy(ctx, d_piOffs, piOffs.data(), sizeof(int32_t) * count, hipMemcpyHostToDevice));
     GLS_TRY(stream_copy(ctx, d_andOffs, andOffs.data(), sizeof(int32_t) * count, hipMemcpyHostToDevice));
@@ -259,19 +267,18 @@ int batch_pass(gls_ctx *ctx, gls_aig **aigs, int32_t count, Pass pass, int32_t u
         DevGraph &g;
         ~GraphGuard() { dev_graph_free(c, g); }
     } uGuard{ctx, U};
+    GLS_TRY(Fills(ctx).add(dep, 0, sizeof(uint32_t) * count).add(constRef, 0, constRef ? sizeof(int32_t) * count : 0).run());
     k_pack_pis<<<nblocks(P + 1), kB, 0, st>>>((int32_t)P, count, d_piOffs, U.f0, U.f1, U.level, utag);
     if (A > 0)
-        k_pack_ands<<<nblocks(A), kB, 0, st>>>(A, count, (int32_t)P, d_mem, d_andOffs, U.f0, U.f1, U.level, utag);
-    if (O > 0) k_pack_pos<<<nblocks(O), kB, 0, st>>>(O, count, (int32_t)P, d_mem, d_poOffs, U.pos);
+        k_pack_ands<<<nblocks(A), kB, 0, st>>>(A, count, (int32_t)P, d_mem, d_andOffs, U.f0, U.f1, U.level, utag,
+                                             constRef);
+    if (O > 0) k_pack_pos<<<nblocks(O), kB, 0, st>>>(O, count, (int32_t)P, d_mem, d_poOffs, U.pos, constRef);
     GLS_HIP(ctx, hipGetLastError());
 
     // the pass
     DevGraph R;
     int32_t depth = 0;
     uint32_t *rtag = nullptr;
-    uint32_t *dep = pb.get<uint32_t>(count);   // per-member depth, as the pass alone reports it
-    if (!dep) return gls_fail(ctx, GLS_ERR_NOMEM, "batch: depth");
-    GLS_HIP(ctx, hipMemsetAsync(dep, 0, sizeof(uint32_t) * count, st));
     gls_op_info info = {};
     std::vector<uint32_t> splitTags;
     // The strash by level sweeps passes over the whole arena in one workgroup,
@@ -286,7 +293,7 @@ int batch_pass(gls_ctx *ctx, gls_aig **aigs, int32_t count, Pass pass, int32_t u
     int rc = pass == Pass::Strash && N <= 64 * largest
                                      ? dev_strash_whole(ctx, U, false, R, &depth, &info, utag, &rtag, dep)
              : pass == Pass::Strash  ? dev_strash(ctx, U, R, &depth, &info, utag, &rtag, dep)
-             : pass == Pass::Rewrite ? dev_rewrite(ctx, U, useZeros, flags, R, &depth, &info, utag, &rtag, dep)
+             : pass == Pass::Rewrite ? dev_rewrite(ctx, U, useZeros, flags, R, &depth, &info, utag, &rtag, dep, constRef, count)
                                      : dev_balance(ctx, U, R, &info, utag, &rtag, &splitTags, 1, count);
     if (rtag) pb.ptrs.push_back(rtag);
     if (rc == GLS_ERR_BATCH_SPLIT) {

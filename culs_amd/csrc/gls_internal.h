@@ -213,9 +213,11 @@ int dev_strash_whole(gls_ctx *ctx, const DevGraph &in, bool allRounds, DevGraph 
                      const uint32_t *tagIn = nullptr, uint32_t **tagOut = nullptr, uint32_t *tagDepth = nullptr);
 int dev_reorder(gls_ctx *ctx, const DevGraph &in, DevGraph &out, std::vector<int32_t> &levelStart,
                 const uint32_t *tagIn = nullptr, uint32_t **tagOut = nullptr);
+// constRef, nTags: with tags, each member's references to the constant, and how
+// many members there are
 int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGraph &out, int32_t *depth,
                 gls_op_info *info, const uint32_t *tagIn = nullptr, uint32_t **tagOut = nullptr,
-                uint32_t *tagDepth = nullptr);
+                uint32_t *tagDepth = nullptr, const int32_t *constRef = nullptr, int32_t nTags = 0);
 // tagIn / tagOut as in dev_strash.  Returns GLS_ERR_BATCH_SPLIT (without a
 // message) when a tag has more than 32768 covers on a level: that tag would
 // be rebuilt in other batches than alone.  splitTags (optional) then lists

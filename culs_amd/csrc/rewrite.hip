@@ -1002,6 +1002,11 @@ struct GraphView {
     const uint32_t *level;
     const uint32_t *tOff;       // structural table: bucket offsets (n + 1)
     const uint2 *tEnt;          // and entries (see k_table_fill)
+    // batched: the members of the nodes, and their number of objects.  Members share
+    // the constant; where a cone reaches it, member t's is object n + t, with
+    // that member's references
+    const uint32_t *tag = nullptr;
+    int32_t n = 0;
 };
 
 // per-thread column of an LDS array laid out [j][lane]
@@ -1018,10 +1023,11 @@ struct Mffc {
 // The table and the DFS stack below are indexed by constants only (a write at
 // a run-time position selects among the entries), so they live in registers
 // instead of scratch memory.
-__device__ __forceinline__ int mffc_decrease(const GraphView &g, int x, const int *leaves, int nL, Mffc &t) {
+__device__ __forceinline__ int mffc_decrease(const GraphView &g, int root, int x, const int *leaves, int nL, Mffc &t) {
 #pragma unroll
     for (int i = 0; i < 4; i++)
         if (i < nL && x == leaves[i]) return 1;
+    if (x == 0 && g.tag) x = g.n + (int)g.tag[root];
     int found = -1;
 #pragma unroll
     for (int i = 0; i < MFFC_TAB; i++)
@@ -1063,7 +1069,7 @@ __device__ int calc_mffc(const GraphView &g, int root, const int *leaves, int nL
             stg += 1u << (2 * top);
             const int cur = stk[top];
             const int x = (int)LID(stage == 0 ? g.f0[cur] : g.f1[cur]);
-            if (mffc_decrease(g, x, leaves, nL, t) == 0) {
+            if (mffc_decrease(g, root, x, leaves, nL, t) == 0) {
                 stk[sp] = x;
                 stg &= ~(3u << (2 * sp));
                 sp++;
@@ -2304,7 +2310,8 @@ int dev_evaluate(gls_ctx *ctx, const DevGraph &g, const uint32_t *d_cuts, const 
 }
 
 int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGraph &out, int32_t *depth,
-                gls_op_info *info, const uint32_t *tagIn, uint32_t **tagOut, uint32_t *tagDepth) {
+                gls_op_info *info, const uint32_t *tagIn, uint32_t **tagOut, uint32_t *tagDepth,
+                const int32_t *constRef, int32_t nTags) {
     GLS_TRY(ctx_ensure_library(ctx));
     hipStream_t st = ctx->stream;
     Timer tm{ctx};
@@ -2312,6 +2319,7 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
     DevGraph g;
     std::vector<int32_t> levelStart;
     const bool tagged = tagIn && tagOut;
+    if (tagged && !constRef) return gls_fail(ctx, GLS_ERR_INTERNAL, "rewrite: tags without their constants' references");
     uint32_t *tagR = nullptr;   // tags in the reordered numbering (freed on every return)
     struct TagGuard {
         gls_ctx *c;
@@ -2322,11 +2330,12 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
     GraphGuard gGuard{ctx, &g};   // frees the reordered graph on every return path
     tm.mark(); // 1
     const int32_t n = g.nObjs, nPIs = g.nPIs, nPOs = g.nPOs;
+    const size_t nRefs = (size_t)n + (tagged ? nTags : 0);     // objects and the members' constants
     int rc = GLS_OK;
     {
         Tmp t{ctx};
         uint32_t *cuts = t.get<uint32_t>((size_t)n * NCUT * 5);
-        int32_t *nref = t.get<int32_t>(n);
+        int32_t *nref = t.get<int32_t>(nRefs);
         int4 *best = t.get<int4>(n);
         uint8_t *flag = t.get<uint8_t>(n);
         uint32_t *candIds = t.get<uint32_t>(n), *d_cnt = t.get<uint32_t>(4), *d_err = t.get<uint32_t>(4);
@@ -2348,6 +2357,11 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
                                    sigBits, &cutRan));
         tm.mark(); // 2
         GraphView gv{g.f0, g.f1, nref, g.level, nullptr, nullptr};
+        if (tagged) {
+            gv.tag = tagR;
+            gv.n = n;
+            GLS_HIP(ctx, hipMemcpyAsync(nref + n, constRef, sizeof(int32_t) * nTags, hipMemcpyDeviceToDevice, st));
+        }
         GLS_TRY(build_table(ctx, t, g, gv));
         tm.mark(); // 3
         k_no_candidate<<<blocks(nPIs + 1, kBlock), kBlock, 0, st>>>(nPIs + 1, best);
@@ -2375,21 +2389,21 @@ int dev_rewrite(gls_ctx *ctx, const DevGraph &in, int useZeros, int flags, DevGr
         if (nCand > 0) {
             plans = t.get<Plan>(nCand);
             state = t.get<uint8_t>(nCand);
-            uint32_t *mk = t.get<uint32_t>(n), *newCnt = t.get<uint32_t>(nCand + 1);
+            uint32_t *mk = t.get<uint32_t>(nRefs), *newCnt = t.get<uint32_t>(nCand + 1);
             newOff = t.get<uint32_t>(nCand + 1);
             uint32_t *selList = t.get<uint32_t>(SEL_REST);
-            Claims cl{t.get<unsigned long long>(n), t.get<unsigned long long>(n), t.get<unsigned long long>(n),
-                      t.get<unsigned long long>(n)};
+            Claims cl{t.get<unsigned long long>(nRefs), t.get<unsigned long long>(nRefs), t.get<unsigned long long>(nRefs),
+                      t.get<unsigned long long>(nRefs)};
             if (!t.ok) return gls_fail(ctx, GLS_ERR_NOMEM, "rewrite: plan allocation");
             const int per = plan_lanes((int32_t)nCand);
             k_plan<<<blocks(nCand, per), EVAL_BLOCK, 0, st>>>(per, (int32_t)nCand, candIds, gv, L, cuts, best, plans);
             k_sel_init<<<blocks(nCand, kBlock), kBlock, 0, st>>>((int32_t)nCand, plans, state);
             GLS_TRY(Fills(ctx)
-                        .add(mk, 0, sizeof(uint32_t) * n)
-                        .add(cl.W, 0, sizeof(unsigned long long) * n)
-                        .add(cl.Wnr, 0, sizeof(unsigned long long) * n)
-                        .add(cl.L, 0, sizeof(unsigned long long) * n)
-                        .add(cl.M, 0, sizeof(unsigned long long) * n)
+                        .add(mk, 0, sizeof(uint32_t) * nRefs)
+                        .add(cl.W, 0, sizeof(unsigned long long) * nRefs)
+                        .add(cl.Wnr, 0, sizeof(unsigned long long) * nRefs)
+                        .add(cl.L, 0, sizeof(unsigned long long) * nRefs)
+                        .add(cl.M, 0, sizeof(unsigned long long) * nRefs)
                         .run());
             for (uint32_t r = 1;; r++) {
                 k_sel_claim<<<blocks(nCand, kBlock), kBlock, 0, st>>>(r, (int32_t)nCand, plans, state, cl, d_cnt);
