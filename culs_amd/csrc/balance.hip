@@ -1545,7 +1545,12 @@ int dev_balance(gls_ctx *ctx, const DevGraph &in, DevGraph &out, gls_op_info *in
         GLS_TRY(select_ids(flag2, nRoots));
     }
     // ---- roots in the order in which they are rebuilt: by (segment, level,
-    // id) where every level fits the persistent workgroup, else by (level, id)
+    // id) where every level fits the persistent workgroup's LDS, else by (level,
+    // id).  Levels that do not fit go to the grid-wide kernels; one workgroup
+    // that reads them from memory takes longer.  30 levels of 2500 covers of 3
+    // inputs 1.95 ms / 5.6, of 4000 of 3 2.5 / 7.6, of 4000 of 6 4.6 / 21.3.  One
+    // member with such a level puts a whole batch in that order: 15 members of 20k
+    // ANDs 1.6 ms alone, 9.9 with it (18.3 where all members share one workgroup).
     const uint32_t fitCovers = std::min<uint32_t>(narrowMax, LT_COVERS);
     uint32_t *d_starts = nullptr, *d_levOff = nullptr;
     LevelRec *d_lev = nullptr;

@@ -284,10 +284,11 @@ int batch_pass(gls_ctx *ctx, gls_aig **aigs, int32_t count, Pass pass, int32_t u
     // The strash by level sweeps passes over the whole arena in one workgroup,
     // the wave sweep over as many levels as the largest member has: the first
     // where the arena is at most 64 times that member.  Against the wave sweep,
-    // ms: 36 multipliers of 8 to 64 bits 3.5 / 7.0, 32 random AIGs of 2k ANDs
-    // 1.6 / 1.8, 64 of 20k 5.5 / 6.6, 512 of 2k 14.2 / 13.5, 512 of 20k 55 / 34
-    // when the line was drawn; the first side takes 2.0, 0.5 and 2.4 ms for the
-    // first three since classes come before levels, the second 2.0 for 512 of 2k.
+    // ms (arena over largest member): 36 multipliers of 8 to 64 bits (10) 2.4 /
+    // 5.1, 96 random AIGs of 1k to 200k ANDs (19) 4.6 / 9.0, 32 of 2k (32) 0.50 /
+    // 0.89, 64 of 20k (64) 2.5 / 3.5.  Above the line it depends on more than this
+    // ratio: 100 of 200k (100) 6.6 / 10.5 and 128 of 20k (128) 4.1 / 4.8, but 512 of
+    // 1k to 200k (97) 22.9 / 21.8, 512 of 2k (512) 2.03 / 2.10 and of 20k 16.2 / 14.5.
     int64_t largest = 0;
     for (int32_t k = 0; k < count; k++) largest = std::max<int64_t>(largest, aigs[k]->nObjs);
     int rc = pass == Pass::Strash && N <= 64 * largest
