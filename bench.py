@@ -45,8 +45,9 @@ B_CUT_PER_AND = 3 * K_CUTS * CUT_BYTES + 12
 # node is recomputed in the cones of its consumers within the launch.
 TRAFFIC_BYTES_PER_LAUNCH = 980_844
 TRAFFIC_NOTE = ("profiled constant of the three-level cut kernel (profiles/k_cuts_triple_rw10m_traffic.md): "
-                "FETCH_SIZE measured over the 10M pass; the WRITE_SIZE half (98,770 B) is extrapolated from a "
-                "200k-AND AIG of the same level shape at 160.0 B per node")
+                "FETCH_SIZE measured over the 10M pass with an earlier node computation (2.6% less than the present "
+                "one on a 200k-AND AIG of the same level shape); the WRITE_SIZE half (98,770 B) is extrapolated "
+                "from that AIG at 160.0 B per node")
 
 
 def cut_kernel_name(mode):
